@@ -9,24 +9,57 @@
  *      removing the precursor) binned with rint(mz / bin width), max sqrt(I)
  *      per bin (LDS atomicMax on the bit pattern: values are >= 0).
  *   2. normaliseByRegion (:84-96): 10 regions of sel = (len-75) div 10 bins,
- *      50 * e / region max (max > 1e-6 and i < 10*sel), else 0.
+ *      50 * e / region max (max > 1e-6 and i < 10*sel), else 0.  A region's
+ *      maximum is that of its peaks, taken while they are binned.
  *   3. crossCorrolation (:105-109): x_i = e_i - sum(a[max(0,i-75) .. +150]) / 150,
  *      the 151-bin window summed left to right in FP32 (mean_mode 0, the
  *      reference's foldl') or in FP64 (mean_mode 1).
+ *
+ * The window sums run over the bins that hold a peak only: a is nowhere
+ * negative, so the zeros between them leave a left-to-right sum unchanged to
+ * the last bit, and a spectrum of a few hundred peaks over 2,000 bins has about
+ * 13 of them in a window of 151.  The non-zero values are compacted in bin
+ * order (one 64-bit mask a 64-bin chunk, and the chunks' running counts), so
+ * that a window is a contiguous run of that list whose ends are two population
+ * counts.  20,000 spectra of 167 peaks take 181 us, where summing every bin
+ * took 1,075 us (151 LDS reads and additions a bin); the chain of a spectrum's
+ * steps (loads, atomics, six barriers) bounds it now, at 1.1 TB/s of rows
+ * written.
  */
 #include "hfx_common.h"
 
 #define PP_THREADS 256
+#define PP_WAVES (PP_THREADS / HFX_WAVE)
+#define PP_CHUNKS (HFX_MAX_LEN / HFX_WAVE)
+static_assert(PP_CHUNKS <= HFX_WAVE, "one lane a chunk in the scan of counts");
+
+/* dynamic LDS: the bins (ceil(cap / 64) * 64 words) and the list of non-zero
+ * values (as many), cap = the longest spectrum the stride allows */
+static size_t pp_lds_bytes(uint32_t stride)
+{
+    const uint32_t cap = min(stride, (uint32_t)HFX_MAX_LEN);
+    return 2 * (size_t)((cap + HFX_WAVE - 1) / HFX_WAVE) * HFX_WAVE * 4;
+}
+
+/* sum of list[a .. e) in order, as T */
+template <class T>
+__device__ __forceinline__ T pp_sum(const float *list, uint32_t a, uint32_t e)
+{
+    T sum = 0;
+    for (uint32_t k = a; k < e; ++k) sum = sum + (T)list[k];
+    return sum;
+}
 
 __global__ void __launch_bounds__(PP_THREADS)
     k_preprocess(float *x, uint32_t stride, uint32_t *len_out, uint32_t *status, const float *mz,
                  const float *inten, const uint32_t *off, const float *pcr_a, const float *chg_a,
                  int remove_precursor, float bw, int mean_mode)
 {
-    __shared__ uint32_t sbin[HFX_MAX_LEN];
-    __shared__ float a[HFX_MAX_LEN];
+    extern __shared__ __align__(16) uint32_t sbin[];
     __shared__ uint32_t rmax[11];
-    const uint32_t s = blockIdx.x, t = threadIdx.x;
+    __shared__ uint64_t mask[PP_CHUNKS + 1];
+    __shared__ uint32_t pre[PP_CHUNKS + 1];
+    const uint32_t s = blockIdx.x, t = threadIdx.x, lane = hfx_lane(), wave = t / HFX_WAVE;
     const uint32_t p0 = off[s], p1 = off[s + 1];
     float *xs = x + (size_t)s * stride;
     const float pcr = pcr_a[s], chg = chg_a[s];
@@ -46,9 +79,12 @@ __global__ void __launch_bounds__(PP_THREADS)
             if (len < 85) st = 2; /* sel = (len-75) div 10 <= 0 */
         }
         if (st == 0) {
-            for (uint32_t i = t; i < len; i += PP_THREADS) sbin[i] = 0;
+            const uint32_t nch = (len + HFX_WAVE - 1) / HFX_WAVE;
+            float *list = (float *)(sbin + nch * HFX_WAVE);
+            for (uint32_t i = t; i < nch * HFX_WAVE; i += PP_THREADS) sbin[i] = 0;
             if (t < 11) rmax[t] = 0;
             __syncthreads();
+            const uint32_t sel = (len - 75) / 10;
             const float plo = pcr - 15.0f, phi = pcr + 15.0f;
             for (uint32_t p = p0 + t; p < p1; p += PP_THREADS) {
                 const float m = mz[p];
@@ -56,39 +92,58 @@ __global__ void __launch_bounds__(PP_THREADS)
                                                    : (m <= cutoff);
                 if (keep) {
                     const int32_t b = (int32_t)__builtin_rintf(m / bw);
-                    const float v = __builtin_sqrtf(inten[p]);
-                    if (b >= 0 && (uint32_t)b < len)
-                        atomicMax(&sbin[b], __float_as_uint(v) & 0x7fffffffu);
+                    const uint32_t v = __float_as_uint(__builtin_sqrtf(inten[p])) & 0x7fffffffu;
+                    if (b >= 0 && (uint32_t)b < len) {
+                        atomicMax(&sbin[b], v);
+                        atomicMax(&rmax[min(10u, (uint32_t)b / sel)], v);
+                    }
                 }
             }
             __syncthreads();
-            const int32_t sel = (int32_t)(len - 75) / 10;
-            for (uint32_t i = t; i < len; i += PP_THREADS) {
-                const int32_t rg = min(10, (int32_t)i / sel);
-                atomicMax(&rmax[rg], sbin[i]);
+            /* each bin scaled in place, and the mask of its chunk */
+            for (uint32_t c = wave; c < nch; c += PP_WAVES) {
+                const uint32_t i = c * HFX_WAVE + lane;
+                const float e = __uint_as_float(sbin[i]);
+                float a = 0.0f;
+                if (sbin[i] != 0u) {
+                    const float m = __uint_as_float(rmax[min(10u, i / sel)]);
+                    a = (m > 1e-6f && i < sel * 10) ? 50.0f * (e / m) : 0.0f;
+                }
+                sbin[i] = __float_as_uint(a);
+                const uint64_t nz = __ballot(a != 0.0f);
+                if (lane == 0) mask[c] = nz;
             }
             __syncthreads();
-            for (uint32_t i = t; i < len; i += PP_THREADS) {
-                const int32_t rg = min(10, (int32_t)i / sel);
-                const float m = __uint_as_float(rmax[rg]);
-                const float e = __uint_as_float(sbin[i]);
-                a[i] = (m > 1e-6f && (int32_t)i < sel * 10) ? 50.0f * (e / m) : 0.0f;
+            /* non-zero bins before each chunk */
+            if (wave == 0) {
+                const uint32_t n = lane < nch ? (uint32_t)__builtin_popcountll(mask[lane]) : 0u;
+                uint32_t incl = n;
+#pragma unroll
+                for (uint32_t o = 1; o < HFX_WAVE; o <<= 1) {
+                    const uint32_t y = __shfl_up(incl, o, 64);
+                    if (lane >= o) incl += y;
+                }
+                pre[lane] = incl - n;
+                if (lane == HFX_WAVE - 1) pre[HFX_WAVE] = incl;
+                if (lane == 0) mask[nch] = 0;
+            }
+            __syncthreads();
+            /* non-zero bins below bin i (i <= nch * 64) */
+            auto below = [&](uint32_t i) -> uint32_t {
+                const uint64_t m = mask[i / HFX_WAVE] & ((1ull << (i % HFX_WAVE)) - 1ull);
+                return pre[i / HFX_WAVE] + (uint32_t)__builtin_popcountll(m);
+            };
+            for (uint32_t c = wave; c < nch; c += PP_WAVES) {
+                const uint32_t i = c * HFX_WAVE + lane;
+                if ((mask[c] >> lane) & 1ull) list[below(i)] = __uint_as_float(sbin[i]);
             }
             __syncthreads();
             for (uint32_t i = t; i < len; i += PP_THREADS) {
                 const uint32_t w0 = i >= 75 ? i - 75 : 0;
-                const uint32_t w1 = min(len, w0 + 151);
-                float v;
-                if (mean_mode == 0) {
-                    float sum = 0.0f;
-                    for (uint32_t j = w0; j < w1; ++j) sum = sum + a[j];
-                    v = a[i] - sum / 150.0f;
-                } else {
-                    double sum = 0.0;
-                    for (uint32_t j = w0; j < w1; ++j) sum = sum + (double)a[j];
-                    v = (float)((double)a[i] - sum / 150.0);
-                }
-                xs[i] = v;
+                const uint32_t k0 = below(w0), k1 = below(min(len, w0 + 151));
+                const float a = __uint_as_float(sbin[i]);
+                if (mean_mode == 0) xs[i] = a - pp_sum<float>(list, k0, k1) / 150.0f;
+                else xs[i] = (float)((double)a - pp_sum<double>(list, k0, k1) / 150.0);
             }
         }
     }
@@ -112,9 +167,9 @@ extern "C" int hfx_preprocess(hfx_ctx *ctx, float *d_x, uint32_t x_stride, uint3
                 mean_mode);
     if (num_spec == 0) return HFX_OK;
     const float bw = mono ? HFX_BIN_WIDTH_MONO : HFX_BIN_WIDTH_AVG;
-    hipLaunchKernelGGL(k_preprocess, dim3(num_spec), dim3(PP_THREADS), 0, hfx_stream(stream), d_x,
-                       x_stride, d_len, d_status, d_mz, d_int, d_peak_off, d_pcr, d_charge,
-                       remove_precursor, bw, mean_mode);
+    hipLaunchKernelGGL(k_preprocess, dim3(num_spec), dim3(PP_THREADS), pp_lds_bytes(x_stride),
+                       hfx_stream(stream), d_x, x_stride, d_len, d_status, d_mz, d_int, d_peak_off,
+                       d_pcr, d_charge, remove_precursor, bw, mean_mode);
     HFX_CHECK_LAUNCH();
     return HFX_OK;
 }
