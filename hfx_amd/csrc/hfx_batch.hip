@@ -27,6 +27,7 @@
  * synchronisation or allocation and can be captured in a hipGraph.
  */
 #include "hfx_cand.h"
+#include "hfx_rows.h"
 
 #include <stdio.h>
 #include <stdlib.h>
@@ -335,7 +336,11 @@ struct hfx_pepix {
     uint64_t *ent_off;
     uint16_t *ent;
     uint64_t n_ent, n_pos, bytes;
+    /* theoretical rows (hfx_rows.hip), a level at a time when a batch first
+     * needs it; never moved once written.  g_rows_mu guards them. */
+    hfx_rows rows;
 };
+static std::mutex g_rows_mu;
 
 template <class T>
 static int dalloc(T **p, size_t n)
@@ -354,7 +359,10 @@ extern "C" int hfx_pepix_destroy(hfx_pepix *ix)
 {
     if (!ix) return HFX_OK;
     (void)hipDeviceSynchronize();
-    void *ps[] = {ix->lad_mem[0], ix->lad_mem[1], ix->caps, ix->cnt, ix->ent_off, ix->ent};
+    void *ps[] = {ix->lad_mem[0], ix->lad_mem[1], ix->caps,         ix->cnt,
+                  ix->ent_off,    ix->ent,        ix->rows.rows[0], ix->rows.rows[1],
+                  ix->rows.rows[2], ix->rows.rows[3], ix->rows.ng};
+    static_assert(HFX_MAX_CHARGE == 4, "one row buffer a charge level");
     for (void *p : ps)
         if (p) (void)hipFree(p);
     free(ix);
@@ -437,6 +445,45 @@ extern "C" int hfx_pepix_build(hfx_ctx *ctx, const hfx_db *db, uint32_t forms, u
     }
     *out = ix;
     return HFX_OK;
+}
+
+/* The index's rows of charge levels 1..L, written now where they are missing
+ * (waits for the stream then): false when a quarter of the free memory does
+ * not hold them, and the batch keeps the ladder or ion-list kernels.  The rows
+ * of a level take RW_G KiB for sixteen peptides: 1.57 GB for 2.7 M. */
+static bool pepix_need_rows(hfx_pepix *ix, uint32_t L, hipStream_t st)
+{
+    std::lock_guard<std::mutex> lk(g_rows_mu);
+    const uint32_t nt = hfx_rows_tiles(ix->db.num_pep);
+    const uint64_t level = std::max<uint64_t>((uint64_t)nt * RW_G * 1024, 256);
+    hfx_rows want{};
+    want.ntiles = nt;
+    want.G = RW_G;
+    uint64_t need = 0;
+    for (uint32_t l = 0; l < L; ++l) need += ix->rows.rows[l] ? 0 : level;
+    if (need == 0) return true;
+    size_t fr = 0, tot = 0;
+    bool ok = hipMemGetInfo(&fr, &tot) == hipSuccess && need <= fr / 4;
+    if (ok && !ix->rows.ng) ok = hipMalloc((void **)&ix->rows.ng, nt + 4ull) == hipSuccess;
+    for (uint32_t l = 0; l < L && ok; ++l)
+        if (!ix->rows.rows[l]) ok = hipMalloc((void **)&want.rows[l], level) == hipSuccess;
+    want.ng = ix->rows.ng;
+    ok = ok && hfx_rows_build(&ix->db, &want, nullptr, (void *)st) == HFX_OK &&
+         hipStreamSynchronize(st) == hipSuccess;
+    for (uint32_t l = 0; l < HFX_MAX_CHARGE; ++l) {
+        if (!want.rows[l]) continue;
+        if (!ok) {
+            (void)hipFree(want.rows[l]);
+            continue;
+        }
+        ix->rows.rows[l] = want.rows[l];
+        ix->bytes += level;
+    }
+    (void)hipGetLastError();
+    if (!ok) return false;
+    ix->rows.ntiles = nt;
+    ix->rows.G = RW_G;
+    return true;
 }
 
 extern "C" int hfx_pepix_info(const hfx_pepix *ix, uint64_t *info /*[6]*/)
@@ -625,6 +672,58 @@ __global__ void k_cut_place(uint32_t *bstart, const uint32_t *seg_cuts, const ui
     if (t <= cap && t >= nb) bstart[t] = S;
 }
 
+/* buckets of the spectrum order: about two spectra a bucket on average */
+void hfx_order_shape(uint32_t S, uint32_t num_pep, hfx_order_bufs *o)
+{
+    o->sh = 0;
+    while (((uint64_t)num_pep >> o->sh) > std::max<uint64_t>(S / 2, 64)) ++o->sh;
+    o->nbz = (num_pep >> o->sh) + 1;
+    o->nb = (HFX_MAX_CHARGE + 1) * o->nbz;
+}
+
+int hfx_order_spectra(hfx_ctx *ctx, uint32_t *order, const hfx_order_bufs *o,
+                      const uint32_t *begin, const uint32_t *zmax, const float *mass, uint32_t S,
+                      void *stream)
+{
+    hipStream_t st = hfx_stream(stream);
+    const uint32_t g = (S + 255) / 256;
+    hipLaunchKernelGGL(k_ord_fill, dim3((o->nb + 255) / 256), dim3(256), 0, st, o->cnt, o->nb);
+    hipLaunchKernelGGL(k_ord_count, dim3(g), dim3(256), 0, st, o->cnt, begin, zmax, S, o->sh,
+                       o->nbz);
+    int rc;
+    if ((rc = hfx_scan_offsets(ctx, o->off, o->cnt, o->nb, stream))) return rc;
+    hipLaunchKernelGGL(k_ord_scatter, dim3(g), dim3(256), 0, st, o->tmp, o->cnt, o->off, begin,
+                       zmax, S, o->sh, o->nbz);
+    hipLaunchKernelGGL(k_ord_rank, dim3(g), dim3(256), 0, st, order, o->tmp, o->off, begin, zmax,
+                       mass, S, o->sh, o->nbz);
+    HFX_CHECK_LAUNCH();
+    return HFX_OK;
+}
+
+uint32_t hfx_cut_segs(uint32_t S) { return (S + CUT_SEG - 1) / CUT_SEG; }
+
+int hfx_cut_blocks(hfx_ctx *ctx, uint32_t ns, const hfx_cut_bufs *c, const uint32_t *order,
+                   const uint32_t *begin, const uint32_t *num, const uint32_t *zmax, uint32_t S,
+                   void *stream)
+{
+    hipStream_t st = hfx_stream(stream);
+    const uint32_t nseg = hfx_cut_segs(S);
+    const dim3 g((nseg + CUT_SPW - 1) / CUT_SPW);
+    if (ns == 16)
+        hipLaunchKernelGGL(k_cut_seg<16>, g, dim3(CUT_WG), 0, st, c->seg, c->n, order, begin, num,
+                           zmax, S);
+    else
+        hipLaunchKernelGGL(k_cut_seg<8>, g, dim3(CUT_WG), 0, st, c->seg, c->n, order, begin, num,
+                           zmax, S);
+    int rc;
+    if ((rc = hfx_scan_offsets(ctx, c->off, c->n, nseg, stream))) return rc;
+    const uint32_t nt = std::max(nseg * CUT_SEG, S + 1);
+    hipLaunchKernelGGL(k_cut_place, dim3((nt + 255) / 256), dim3(256), 0, st, c->bstart, c->seg,
+                       c->n, c->off, nseg, S, S);
+    HFX_CHECK_LAUNCH();
+    return HFX_OK;
+}
+
 /* ------------------------------------------------------------------ */
 /* The batch object                                                       */
 /* ------------------------------------------------------------------ */
@@ -659,6 +758,9 @@ struct hfx_batch {
     uint32_t *cut_seg, *cut_n;
     uint64_t *cut_off;
     uint32_t nseg;
+    bool dense_set;      /* a dense form was chosen since the plan */
+    bool rows_tried, use_rows; /* scores come from the index's rows */
+    uint32_t *rw_small;  /* rows: [3][S] quanta, levels, wide marks */
     hipGraph_t graph;
     hipGraphExec_t exec;
 };
@@ -669,7 +771,7 @@ static void bt_free(hfx_batch *b)
                   b->ntiles,   b->counter,   b->score_off, b->tile_off,  b->scores,
                   b->top_pos,  b->top_cnt,   b->flag,      b->top_exact, b->top_f32,
                   b->tx_scratch, b->ord_cnt, b->ord_tmp,   b->ord_off,   b->dn_scratch,
-                  b->dn_bstart, b->cut_seg,  b->cut_n,     b->cut_off};
+                  b->dn_bstart, b->cut_seg,  b->cut_n,     b->cut_off,   b->rw_small};
     for (void *p : ps)
         if (p) (void)hipFree(p);
     if (b->exec) (void)hipGraphExecDestroy(b->exec);
@@ -710,6 +812,7 @@ extern "C" int hfx_batch_use_index(hfx_batch *b, const hfx_pepix *ix)
                     (ix->db.d_idx_sorted == b->db.d_idx_sorted && ix->db.num_pep == b->db.num_pep),
                 HFX_ERR_ARG, "hfx_batch_use_index: the index belongs to another database");
     b->ix = ix;
+    b->rows_tried = b->use_rows = false;
     if (b->exec) {
         (void)hipGraphExecDestroy(b->exec);
         b->exec = nullptr;
@@ -755,6 +858,15 @@ static bool tune_dense_ok(uint32_t precision, uint32_t CH)
 {
     const uint32_t step = tune_dense_step(precision);
     return CH >= step && CH % step == 0 && CH <= 8192;
+}
+
+/* candidates a dense work item takes, untuned: by the rows the blocks read --
+ * about a twelfth of the pairs, but every row of the database's two usual
+ * levels once the batch covers it */
+static uint32_t bt_chunk(const hfx_batch *b)
+{
+    const uint64_t rows = std::max<uint64_t>(b->total / 12, std::min<uint64_t>(b->total, 2ull * b->db.num_pep));
+    return hfx_rows_chunk(rows, (uint32_t)hfx_ctx_num_cus(b->ctx));
 }
 
 static std::tuple<int, int, uint32_t> tune_key(const hfx_batch *b)
@@ -846,7 +958,42 @@ static int bt_need_index(hfx_batch *b, hipStream_t st)
     if (b->own) hfx_pepix_destroy(b->own);
     b->own = nx;
     b->ix = nx;
+    b->rows_tried = b->use_rows = false;
     return HFX_OK;
+}
+
+static int bt_dense_alloc(hfx_batch *b);
+
+/* the index, and its rows where they fit (decided once a plan or index, never
+ * under capture: a batch captured by its caller without a run before it keeps
+ * the other kernels) */
+static int bt_ready(hfx_batch *b, hipStream_t st)
+{
+    int rc = bt_need_index(b, st);
+    if (rc || b->rows_tried || b->S == 0) return rc;
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    HFX_CHECK_HIP(hipStreamIsCapturing(st, &cs));
+    if (cs != hipStreamCaptureStatusNone) return HFX_OK;
+    b->rows_tried = true;
+    if (b->sp.x_stride > RW_MAXK || b->db.num_pep == 0) return HFX_OK;
+    size_t fr = 0, tot = 0;
+    HFX_CHECK_HIP(hipMemGetInfo(&fr, &tot));
+    if (!b->dn_scratch && (uint64_t)b->S * 16384 > fr / 4) return HFX_OK;
+    if (!pepix_need_rows(const_cast<hfx_pepix *>(b->ix), b->L, st)) return HFX_OK;
+    if (bt_dense_alloc(b) || (!b->rw_small && dalloc(&b->rw_small, 3 * (size_t)b->S))) {
+        (void)hipGetLastError();
+        return HFX_OK;
+    }
+    b->use_rows = true;
+    return HFX_OK;
+}
+
+/* bt_ready as far as it goes without building an index of the batch's own */
+static int bt_ready_attached(hfx_batch *b, hipStream_t st)
+{
+    const uint32_t f = bt_form(b);
+    if (!b->ix || !(b->ix->forms & f) || (f == HFX_PEPIX_IONS && b->ix->L < b->L)) return HFX_OK;
+    return bt_ready(b, st);
 }
 
 /* Device bytes hfx_batch_plan allocates for S spectra with `total` scored
@@ -978,11 +1125,11 @@ extern "C" int hfx_batch_plan(hfx_batch *b, const hfx_db *db, const hfx_spectra 
     }
     b->L = std::max(L, 1u);
     b->lstr = (std::max(lmax, 8u) + 15) & ~15u;
-    /* order buckets: about two spectra a bucket on average */
-    b->ord_sh = 0;
-    while (((uint64_t)db->num_pep >> b->ord_sh) > std::max<uint64_t>(S / 2, 64)) ++b->ord_sh;
-    b->ord_nbz = (db->num_pep >> b->ord_sh) + 1;
-    b->ord_nb = (HFX_MAX_CHARGE + 1) * b->ord_nbz;
+    hfx_order_bufs o{};
+    hfx_order_shape(S, db->num_pep, &o);
+    b->ord_sh = o.sh;
+    b->ord_nbz = o.nbz;
+    b->ord_nb = o.nb;
     if ((rc = dalloc(&b->ord_cnt, b->ord_nb)) || (rc = dalloc(&b->ord_off, (size_t)b->ord_nb + 1)) ||
         (rc = dalloc(&b->ord_tmp, S)))
         return rc;
@@ -990,15 +1137,13 @@ extern "C" int hfx_batch_plan(hfx_batch *b, const hfx_db *db, const hfx_spectra 
     b->G = 8;
     b->C = 64;
     b->threads = 512;
-    b->CH = 256;
+    b->CH = bt_chunk(b);
     b->precision = HFX_BATCH_FP32_SPARSE;
     {
         std::lock_guard<std::mutex> lk(g_tune_mu);
         tune_load_locked();
         auto it = g_tune.find(tune_key(b));
         if (it != g_tune.end()) std::tie(b->G, b->C, b->threads) = it->second;
-        auto jt = g_tune_dense.find(tune_key(b));
-        if (jt != g_tune_dense.end()) b->CH = jt->second;
     }
     if ((rc = dalloc(&b->scores, b->total)) || (rc = dalloc(&b->counter, 1)) ||
         (rc = dalloc(&b->top_pos, (size_t)S * N)) || (rc = dalloc(&b->top_exact, (size_t)S * N)) ||
@@ -1015,7 +1160,7 @@ extern "C" int hfx_batch_plan(hfx_batch *b, const hfx_db *db, const hfx_spectra 
         return rc;
     b->planned = true;
     HFX_CHECK_LAUNCH();
-    return HFX_OK;
+    return bt_ready_attached(b, st);
 }
 
 extern "C" int hfx_batch_plan_ix(hfx_batch *b, const hfx_pepix *ix, const hfx_spectra *sp,
@@ -1055,41 +1200,43 @@ static int bt_windows(hfx_batch *b, hipStream_t st)
 /* spectrum order (fragment charge level, precursor mass, index) */
 static int bt_order(hfx_batch *b, hipStream_t st)
 {
-    const uint32_t S = b->S, g = (S + 255) / 256;
-    hipLaunchKernelGGL(k_ord_fill, dim3((b->ord_nb + 255) / 256), dim3(256), 0, st, b->ord_cnt,
-                       b->ord_nb);
-    hipLaunchKernelGGL(k_ord_count, dim3(g), dim3(256), 0, st, b->ord_cnt, b->begin, b->sp.d_zmax,
-                       S, b->ord_sh, b->ord_nbz);
-    int rc;
-    if ((rc = hfx_scan_offsets(b->ctx, b->ord_off, b->ord_cnt, b->ord_nb, (void *)st))) return rc;
-    hipLaunchKernelGGL(k_ord_scatter, dim3(g), dim3(256), 0, st, b->ord_tmp, b->ord_cnt,
-                       b->ord_off, b->begin, b->sp.d_zmax, S, b->ord_sh, b->ord_nbz);
-    hipLaunchKernelGGL(k_ord_rank, dim3(g), dim3(256), 0, st, b->order, b->ord_tmp, b->ord_off,
-                       b->begin, b->sp.d_zmax, b->sp.d_mass, S, b->ord_sh, b->ord_nbz);
-    HFX_CHECK_LAUNCH();
-    return HFX_OK;
+    const hfx_order_bufs o{b->ord_sh, b->ord_nbz, b->ord_nb, b->ord_cnt, b->ord_tmp, b->ord_off};
+    return hfx_order_spectra(b->ctx, b->order, &o, b->begin, b->sp.d_zmax, b->sp.d_mass, b->S,
+                             (void *)st);
 }
 
-/* dense blocks (segment DP; eight spectra a block in the BF16 form, sixteen
- * in the integer form) and the spectra's hi/lo rows or digits */
+/* the rows form of the current precision */
+static int bt_mode(const hfx_batch *b)
+{
+    return b->precision == HFX_BATCH_I8X3_DENSE     ? RW_I8X3
+           : b->precision == HFX_BATCH_BF16X2_DENSE ? RW_BF16
+                                                    : RW_I8X4;
+}
+/* dn_scratch as the rows route carves it: planes | item bookkeeping; quanta,
+ * levels and wide marks in rw_small */
+static uint8_t *bt_planes(const hfx_batch *b) { return b->dn_scratch; }
+static void *bt_items(const hfx_batch *b)
+{
+    return b->dn_scratch + (size_t)b->S * 4 * RW_MAXK;
+}
+
+/* blocks (segment DP; eight spectra a block in the BF16 form, sixteen in the
+ * others) and the spectra's hi/lo rows or digits */
 static int bt_dense_prep(hfx_batch *b, hipStream_t st)
 {
-    const uint32_t S = b->S;
-    const bool i8 = b->precision == HFX_BATCH_I8X3_DENSE;
-    if (i8)
-        hipLaunchKernelGGL(k_cut_seg<16>, dim3((b->nseg + CUT_SPW - 1) / CUT_SPW), dim3(CUT_WG), 0,
-                           st, b->cut_seg, b->cut_n, b->order, b->begin, b->num, b->sp.d_zmax, S);
-    else
-        hipLaunchKernelGGL(k_cut_seg<8>, dim3((b->nseg + CUT_SPW - 1) / CUT_SPW), dim3(CUT_WG), 0,
-                           st, b->cut_seg, b->cut_n, b->order, b->begin, b->num, b->sp.d_zmax, S);
+    const bool bf = b->precision == HFX_BATCH_BF16X2_DENSE;
+    const hfx_cut_bufs c{b->cut_seg, b->cut_n, b->cut_off, b->dn_bstart};
     int rc;
-    if ((rc = hfx_scan_offsets(b->ctx, b->cut_off, b->cut_n, b->nseg, (void *)st))) return rc;
-    const uint32_t nt = std::max(b->nseg * CUT_SEG, S + 1);
-    hipLaunchKernelGGL(k_cut_place, dim3((nt + 255) / 256), dim3(256), 0, st, b->dn_bstart,
-                       b->cut_seg, b->cut_n, b->cut_off, b->nseg, S, S);
-    HFX_CHECK_LAUNCH();
-    return i8 ? hfx_dense8_split(&b->sp, b->dn_scratch, (void *)st)
-              : hfx_dense_split(&b->sp, b->dn_scratch, (void *)st);
+    if ((rc = hfx_cut_blocks(b->ctx, bf ? 8u : 16u, &c, b->order, b->begin, b->num, b->sp.d_zmax,
+                             b->S, (void *)st)))
+        return rc;
+    if (b->use_rows) {
+        float *qs = (float *)b->rw_small;
+        return hfx_rows_split(bt_mode(b), &b->sp, bt_planes(b), qs, b->rw_small + b->S,
+                              b->rw_small + 2 * (size_t)b->S, (void *)st);
+    }
+    return bf ? hfx_dense_split(&b->sp, b->dn_scratch, (void *)st)
+              : hfx_dense8_split(&b->sp, b->dn_scratch, (void *)st);
 }
 
 /* blocks of G spectra in order + tiles for the current (G, C) */
@@ -1106,7 +1253,7 @@ static int bt_prep(hfx_batch *b, hipStream_t st)
 {
     int rc;
     if ((rc = bt_order(b, st))) return rc;
-    if (bt_is_dense(b->precision)) return bt_dense_prep(b, st);
+    if (b->use_rows || bt_is_dense(b->precision)) return bt_dense_prep(b, st);
     return bt_tiles(b, st);
 }
 
@@ -1142,9 +1289,30 @@ static int bt_score(hfx_batch *b, hipStream_t st, void **ev)
     return HFX_OK;
 }
 
+/* scores from the index's rows, in the current precision */
+static int bt_row_scores(hfx_batch *b, hipStream_t st, void **ev)
+{
+    if (b->total == 0) return HFX_OK;
+    const int mode = bt_mode(b);
+    const float *qs = (const float *)b->rw_small;
+    hfx_spectra sq = b->sp;
+    if (mode == RW_I8X4) sq.d_zmax = b->rw_small + b->S; /* wide spectra hidden */
+    int rc;
+    if ((rc = hfx_rows_blocks(b->ctx, mode, bt_items(b), b->order, b->dn_bstart, b->begin, b->num,
+                              &sq, b->CH, (void *)st)) ||
+        (rc = hfx_rows_scores(b->ctx, mode, bt_items(b), b->scores, b->score_off, b->begin, b->num,
+                              b->order, b->dn_bstart, &b->ix->rows, bt_planes(b), qs, &sq, b->CH,
+                              b->sp.d_zmax, (void *)st, ev)))
+        return rc;
+    if (mode != RW_I8X4) return HFX_OK;
+    return hfx_xcorr_wide(b->ctx, b->scores, b->score_off, b->begin, b->num, &b->db, &b->sp,
+                          b->rw_small + 2 * (size_t)b->S, (void *)st);
+}
+
 /* ev (optional): events recorded around the scoring kernel itself */
 static int bt_scores(hfx_batch *b, hipStream_t st, void **ev = nullptr)
 {
+    if (b->use_rows) return bt_row_scores(b, st, ev);
     if (b->precision == HFX_BATCH_I8X3_DENSE) {
         if (b->total == 0) return HFX_OK;
         return hfx_dense8_scores(b->ctx, b->scores, b->score_off, b->begin, b->num, b->order,
@@ -1187,7 +1355,7 @@ extern "C" int hfx_batch_run(hfx_batch *b, void *stream)
     hipStream_t st = hfx_stream(stream);
     int rc;
     if (b->S == 0) return HFX_OK;
-    if ((rc = bt_need_index(b, st))) return rc;
+    if ((rc = bt_ready(b, st))) return rc;
     if ((rc = bt_windows(b, st)) || (rc = bt_prep(b, st)) || (rc = bt_scores(b, st))) return rc;
     return bt_topn(b, st);
 }
@@ -1203,13 +1371,14 @@ extern "C" int hfx_batch_set_precision(hfx_batch *b, uint32_t precision)
                 "(x_stride %u)", hfx_dense_max_len(), b->sp.x_stride);
     int rc;
     if (bt_is_dense(precision) && (rc = bt_dense_alloc(b))) return rc;
+    if (bt_is_dense(precision)) b->dense_set = true;
     if (bt_is_dense(precision) && precision != b->precision) {
         /* the tuned chunk of this form for batches of this shape, if any */
         std::lock_guard<std::mutex> lk(g_tune_mu);
         tune_load_locked();
         auto &m = bt_tune_dense(precision);
         auto jt = m.find(tune_key(b));
-        b->CH = jt != m.end() ? jt->second : 256;
+        b->CH = jt != m.end() ? jt->second : bt_chunk(b);
     }
     if (precision != b->precision && b->exec) {
         (void)hipGraphExecDestroy(b->exec);
@@ -1218,7 +1387,7 @@ extern "C" int hfx_batch_set_precision(hfx_batch *b, uint32_t precision)
         b->graph = nullptr;
     }
     b->precision = precision;
-    return HFX_OK;
+    return bt_ready_attached(b, nullptr);
 }
 
 extern "C" int hfx_batch_capture(hfx_batch *b, void *stream)
@@ -1227,7 +1396,7 @@ extern "C" int hfx_batch_capture(hfx_batch *b, void *stream)
     HFX_REQUIRE(stream != nullptr, HFX_ERR_ARG, "hfx_batch_capture: needs a non-null stream");
     hipStream_t st = hfx_stream(stream);
     int rc;
-    if ((rc = bt_need_index(b, st))) return rc;
+    if ((rc = bt_ready(b, st))) return rc;
     if (b->exec) { (void)hipGraphExecDestroy(b->exec); b->exec = nullptr; }
     if (b->graph) { (void)hipGraphDestroy(b->graph); b->graph = nullptr; }
     /* kernel attributes are set outside the capture */
@@ -1284,7 +1453,7 @@ extern "C" int hfx_batch_autotune(hfx_batch *b, void *stream, uint32_t *out_cfg)
     float best = 1e30f;
     uint32_t bG = b->G, bC = b->C, bT = b->threads, bCH = b->CH;
     if (bt_is_dense(b->precision)) {
-        const uint32_t CHs[5] = {256, 512, 1024, 2048, 4096};
+        const uint32_t CHs[5] = {512, 1024, 2048, 4096, 8192};
         for (uint32_t CH : CHs) {
             b->CH = CH;
             float ms = 0;
@@ -1348,7 +1517,7 @@ extern "C" int hfx_batch_time(hfx_batch *b, void *stream, float *ms)
     int rc = HFX_OK;
     for (int i = 0; i < 5; ++i) ms[i] = 0.0f;
     if (b->S == 0) return HFX_OK;
-    if ((rc = bt_need_index(b, st))) return rc;
+    if ((rc = bt_ready(b, st))) return rc;
     hipEvent_t ev[7];
     for (auto &e : ev) HFX_CHECK_HIP(hipEventCreate(&e));
     void *kev[2] = {ev[5], ev[6]};
@@ -1357,7 +1526,7 @@ extern "C" int hfx_batch_time(hfx_batch *b, void *stream, float *ms)
     HFX_CHECK_HIP(hipEventRecord(ev[1], st));
     if (!rc) rc = bt_prep(b, st);
     HFX_CHECK_HIP(hipEventRecord(ev[2], st));
-    const bool scored = b->total != 0 && (bt_is_dense(b->precision) || b->B != 0);
+    const bool scored = b->total != 0 && (b->use_rows || bt_is_dense(b->precision) || b->B != 0);
     if (!rc) rc = bt_scores(b, st, kev);
     HFX_CHECK_HIP(hipEventRecord(ev[3], st));
     if (!rc) rc = bt_topn(b, st);
@@ -1393,7 +1562,7 @@ extern "C" int hfx_batch_dense_blocks(const hfx_batch *b, uint32_t *h_bstart, ui
                                       uint32_t *num_blocks)
 {
     HFX_REQUIRE(b && num_blocks, HFX_ERR_ARG, "hfx_batch_dense_blocks: null argument");
-    HFX_REQUIRE(b->planned && b->dn_scratch, HFX_ERR_ARG,
+    HFX_REQUIRE(b->planned && b->dense_set, HFX_ERR_ARG,
                 "hfx_batch_dense_blocks: no dense run of this batch");
     uint64_t nb = 0;
     HFX_CHECK_HIP(hipDeviceSynchronize());

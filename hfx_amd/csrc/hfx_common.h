@@ -88,9 +88,16 @@ enum {
     HFX_SLOT_LADDER2 = 13, /* dense ladders: positions           */
     HFX_SLOT_STATS = 14,  /* SP ion peak flags                   */
     HFX_SLOT_SCAN2 = 15,  /* tile sums of the in-place scans     */
+    HFX_SLOT_ROWS = 16,   /* sparse XCorr: spectra, order, items */
+    HFX_SLOT_ROWS2 = 17,  /* sparse XCorr: theoretical rows      */
+    HFX_SCRATCH_SLOTS = 18
 };
 /* Scratch owned by a context: grown on demand, never shrunk. */
 int hfx_ctx_scratch(hfx_ctx *ctx, int slot, size_t bytes, void **out);
+/* the same for memory a caller can do without: null (and no error left
+ * behind) when it would have to grow while `stream` is being captured, past an
+ * eighth of the device's memory or past half of what is free */
+void *hfx_ctx_scratch_spare(hfx_ctx *ctx, int slot, size_t bytes, void *stream);
 int hfx_ctx_pinned(hfx_ctx *ctx, size_t bytes, void **out);
 int hfx_ctx_num_cus(hfx_ctx *ctx);
 hfx_ctx *hfx_default_ctx(void);
@@ -155,6 +162,11 @@ int hfx_dense8_scores(hfx_ctx *ctx, float *d_scores, const uint64_t *d_off,
                       const uint32_t *d_bstart, uint32_t nblocks, const hfx_dn_ladder *lad,
                       const hfx_spectra *sp, uint32_t CH, void *scratch, int presplit,
                       void *stream, void **ev);
+/* FP32 scores of the unmodified candidates of the spectra with wide[s] != 0
+ * (hfx_xcorr_sparse's kernel, no scratch) */
+int hfx_xcorr_wide(hfx_ctx *ctx, float *d_scores, const uint64_t *d_off, const uint32_t *d_begin,
+                   const uint32_t *d_num, const hfx_db *db, const hfx_spectra *sp,
+                   const uint32_t *wide, void *stream);
 /* ev (optional): two hipEvent_t recorded right before and after the
  * contraction kernel itself */
 int hfx_dense_scores(hfx_ctx *ctx, float *d_scores, const uint64_t *d_off, const uint32_t *d_begin,

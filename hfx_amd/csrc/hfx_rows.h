@@ -1,0 +1,78 @@
+/*
+ * hfx_rows.h -- theoretical rows of 2-bit codes and their contraction
+ * (hfx_rows.hip), for the sparse and the batched forms.
+ */
+#pragma once
+
+#include "hfx_common.h"
+
+#define RW_ROWS 16     /* peptides a tile */
+#define RW_MAXK 2176   /* bins of a row */
+#define RW_G 9         /* groups of 256 bins of a row */
+
+/* precision forms: planes of a spectrum, spectra a block */
+#define RW_I8X3 0
+#define RW_I8X4 1
+#define RW_BF16 2
+#define RW_PLANES(mode) ((mode) == RW_I8X3 ? 3 : 4)
+#define RW_NS(mode) ((mode) == RW_BF16 ? 8u : 16u)
+
+/* rows[l - 1]: charge level l's tiles of G KiB each, or null; slots: tile t of
+ * level l at place slots[(l - 1) ntiles + t] of rows[l - 1] (null: place t);
+ * ng[t]: groups tile t's peaks reach (only those are written), the array padded to
+ * whole words */
+struct hfx_rows {
+    uint8_t *rows[HFX_MAX_CHARGE];
+    const uint64_t *slots;
+    uint8_t *ng;
+    uint32_t ntiles, G;
+};
+
+uint32_t hfx_rows_tiles(uint32_t num_pep);
+uint32_t hfx_rows_groups(uint32_t x_stride);
+uint32_t hfx_rows_chunk(uint64_t rows, uint32_t cus);
+/* planes [S][RW_PLANES][RW_MAXK] and quanta of the spectra; RW_I8X4 also
+ * writes each spectrum's charge level to lvl, or to wide where its digits would
+ * lose precision (0 in the other) */
+int hfx_rows_split(int mode, const hfx_spectra *sp, uint8_t *planes, float *qs, uint32_t *lvl,
+                   uint32_t *wide, void *stream);
+/* writes the rows of the wanted levels (non-null) and tiles (flags
+ * [HFX_MAX_CHARGE][ntiles], null: all) */
+int hfx_rows_build(const hfx_db *db, const hfx_rows *r, const uint32_t *flags, void *stream);
+/* work items of the blocks bstart (num_spec + 1 entries, empty blocks at the
+ * end) of CH candidates each, in scratch of hfx_rows_items_bytes(num_spec) */
+size_t hfx_rows_items_bytes(uint32_t S);
+int hfx_rows_blocks(hfx_ctx *ctx, int mode, void *scratch, const uint32_t *order,
+                    const uint32_t *bstart, const uint32_t *begin, const uint32_t *num,
+                    const hfx_spectra *sp, uint32_t CH, void *stream);
+/* flags [HFX_MAX_CHARGE][ntiles]: the tiles those items read */
+int hfx_rows_mark(void *scratch, uint32_t S, uint32_t *flags, uint32_t ntiles, void *stream);
+/* the scores of every item; spectra whose charge in zmax is not generated
+ * score 0 (sp's own d_zmax may hide spectra from the items) */
+int hfx_rows_scores(hfx_ctx *ctx, int mode, void *scratch, float *d_scores, const uint64_t *d_off,
+                    const uint32_t *begin, const uint32_t *num, const uint32_t *order,
+                    const uint32_t *bstart, const hfx_rows *r, const uint8_t *planes,
+                    const float *qs, const hfx_spectra *sp, uint32_t CH, const uint32_t *zmax,
+                    void *stream, void **ev);
+
+/* spectrum order and block cut (hfx_batch.hip) */
+struct hfx_order_bufs {
+    uint32_t sh, nbz, nb; /* buckets, from hfx_order_shape */
+    uint32_t *cnt, *tmp;  /* [nb], [S] */
+    uint64_t *off;        /* [nb + 1] */
+};
+void hfx_order_shape(uint32_t S, uint32_t num_pep, hfx_order_bufs *o);
+/* order: (fragment charge level, precursor mass, index) */
+int hfx_order_spectra(hfx_ctx *ctx, uint32_t *order, const hfx_order_bufs *o,
+                      const uint32_t *begin, const uint32_t *zmax, const float *mass, uint32_t S,
+                      void *stream);
+struct hfx_cut_bufs {
+    uint32_t *seg, *n; /* [hfx_cut_segs(S) * 32], [hfx_cut_segs(S)] */
+    uint64_t *off;     /* [hfx_cut_segs(S) + 1] */
+    uint32_t *bstart;  /* [S + 1] */
+};
+uint32_t hfx_cut_segs(uint32_t S);
+/* blocks of at most ns (8 or 16) consecutive ordered spectra */
+int hfx_cut_blocks(hfx_ctx *ctx, uint32_t ns, const hfx_cut_bufs *c, const uint32_t *order,
+                   const uint32_t *begin, const uint32_t *num, const uint32_t *zmax, uint32_t S,
+                   void *stream);

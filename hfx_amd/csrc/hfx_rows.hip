@@ -1,0 +1,883 @@
+/*
+ * hfx_rows.hip -- theoretical spectra as rows of 2-bit codes in HBM, and their
+ * contraction with blocks of spectra on the MFMA units.
+ *
+ * A candidate's theoretical spectrum depends only on its peptide and the
+ * fragment charge level, and a peptide is a candidate of every spectrum whose
+ * window holds it (hundreds, in a batch of thousands).  Its row is therefore
+ * written once -- per database for the batched forms (kept by the peptide
+ * index), per call for hfx_xcorr_sparse -- and every block of spectra then
+ * reads finished rows: the inner loop of the contraction is loads, code lookups
+ * and matrix instructions, with no ladder, no bins, no LDS atomics and no
+ * barrier.
+ *
+ * Rows.  Sixteen consecutive residual-sorted peptides form a tile, the M of a
+ * 16x16 matrix instruction.  A tile is up to RW_G groups of 256 bins, 1 KiB
+ * each: lane (row, kg) of a wave owns 16 bytes of a group, word i holding the
+ * codes of bins 64 i + 16 kg .. + 15 of the group, so a wave reads a group of
+ * a tile with one 16-byte load a lane, contiguous.  Nibble n of a word holds bin
+ * n in bits 0-1 and bin n + 8 in bits 2-3.  Codes 0, 1, 3, 2 stand for the
+ * weights 0, 10, 25, 50 (two bits of the unary code that orders them in the
+ * LDS map).  Four v_perm turn a word into 16 int8 weights in the order
+ * rw_bin_of gives; the spectra's planes are stored in the same order.
+ *
+ * Spectra.  Precision forms (see hfx_dense.hip for their bounds):
+ *   RW_I8X3  three balanced base-256 digits of X = rint(x 2^k),
+ *            max|x| 2^k <= 8355711; a block is sixteen spectra;
+ *   RW_I8X4  four digits, max|x| 2^k <= 2139062143: 32-bit fixed point, for the
+ *            FP32 forms.  |score - exact| <= max|x| 2^-31 sum w + 2^-24 |score|,
+ *            which is below the rounding of the FP32 sums it replaces while
+ *            mean|x| >= max|x| 2^-12 (the sum of T products of mean w mean|x|
+ *            rounds to about 2^-25 T w mean|x|, the digits err by
+ *            sqrt(T) w max|x| 2^-31).  A spectrum beyond that, or with a value
+ *            that is not finite, is marked wide and keeps the FP32 kernel;
+ *   RW_BF16  hi and lo BF16 of eight spectra, FP32 accumulation.
+ *
+ * Scoring kernels, 20,000 proteins (2.7 M peptides), before (rows written per
+ * block into LDS, or per pair) and after: three digits, 20,000 spectra 1,978 ->
+ * 958 us; BF16, 6,000 spectra 1,937 -> 850 us; FP32 batched, 4,000 spectra
+ * 10,114 -> 600 us.  Writing two levels' rows of the database takes 1.26 ms,
+ * once.
+ */
+#include "hfx_cand.h"
+#include "hfx_rows.h"
+
+#include <algorithm>
+#include <type_traits>
+
+typedef __bf16 rw_bf16x8 __attribute__((ext_vector_type(8)));
+typedef float rw_f32x4 __attribute__((ext_vector_type(4)));
+typedef int32_t rw_i32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t rw_u32x4 __attribute__((ext_vector_type(4)));
+
+#define RW_NKS (RW_MAXK / 64)  /* k-steps of 64 bins */
+static_assert(RW_MAXK % 64 == 0 && RW_G * 256 >= RW_MAXK, "groups cover a row");
+
+/* bin within a k-step's 64 of byte j (0..15) of k-group kg */
+__host__ __device__ inline uint32_t rw_bin_of(uint32_t kg, uint32_t j)
+{
+    return kg * 16u + ((j >> 2) & 1u) * 8u + 2u * (j & 3u) + (j >> 3);
+}
+
+/* wave-uniform tables nothing in the kernel writes, through scalar loads */
+template <class T>
+__device__ __forceinline__ T rw_sload(const T *p, uint64_t i)
+{
+    return ((const __attribute__((address_space(4))) T *)p)[i];
+}
+
+/* ------------------------------------------------------------------ */
+/* Spectra as planes                                                     */
+/* ------------------------------------------------------------------ */
+
+__device__ __forceinline__ uint32_t rw_bf16(float f)
+{
+    const uint32_t u = __float_as_uint(f);
+    return (u + 0x7fffu + ((u >> 16) & 1u)) >> 16;
+}
+
+/* planes[s][plane][RW_MAXK]: byte 64 ks + 16 kg + j of a digit plane is the
+ * digit of bin 64 ks + rw_bin_of(kg, j); the BF16 planes (hi of bytes j < 8,
+ * hi of j >= 8, lo, lo) hold eight BF16 in the 16 bytes of a k-group.
+ * qs[s] = 2^-k.  lvl (RW_I8X4): the fragment charge of the spectra the digits
+ * serve, 0 for wide ones (their charge goes to wide[s] instead). */
+template <int MODE>
+__global__ void __launch_bounds__(256)
+    k_rw_split(uint8_t *planes, float *qs, uint32_t *lvl, uint32_t *wide, hfx_spectra sp)
+{
+    constexpr uint32_t NP = RW_PLANES(MODE);
+    __shared__ float red[2][256 / HFX_WAVE];
+    __shared__ uint32_t bad;
+    const uint32_t s = blockIdx.x, tid = threadIdx.x;
+    const uint32_t len = min(sp.d_len[s], min(sp.x_stride, (uint32_t)RW_MAXK));
+    const float *x = sp.d_x + (size_t)s * sp.x_stride;
+    /* thread t takes the four bins of words t + 256 u (bytes 4 w .. 4 w + 3) */
+    constexpr uint32_t NW = RW_MAXK / 4, NU = (NW + 255) / 256;
+    float v[NU][4];
+    float m = 0.0f, x1 = 0.0f;
+    bool odd = false;
+    if (tid == 0) bad = 0;
+#pragma unroll
+    for (uint32_t u = 0; u < NU; ++u) {
+        const uint32_t w = tid + 256 * u;
+#pragma unroll
+        for (uint32_t i = 0; i < 4; ++i) {
+            const uint32_t bin = (w >> 4) * 64u + rw_bin_of((w >> 2) & 3u, (w & 3u) * 4u + i);
+            v[u][i] = w < NW && bin < len ? x[bin] : 0.0f;
+            const float a = fabsf(v[u][i]);
+            m = fmaxf(m, a);
+            x1 += a;
+            odd |= !(a < INFINITY);
+        }
+    }
+    uint8_t *o = planes + (size_t)s * NP * RW_MAXK;
+    if constexpr (MODE == RW_BF16) {
+#pragma unroll
+        for (uint32_t u = 0; u < NU; ++u) {
+            const uint32_t w = tid + 256 * u;
+            if (w >= NW) break;
+            uint32_t h[4], l[4];
+#pragma unroll
+            for (uint32_t i = 0; i < 4; ++i) {
+                h[i] = rw_bf16(v[u][i]);
+                l[i] = rw_bf16(v[u][i] - __uint_as_float(h[i] << 16));
+            }
+            /* four bins are 8 bytes; word w & 3 < 2: the first eight bins */
+            const uint32_t part = (w >> 1) & 1u;
+            const size_t at = (size_t)(w >> 2) * 16u + (w & 1u) * 8u;
+            *(uint2 *)(o + part * RW_MAXK + at) = make_uint2(h[0] | h[1] << 16, h[2] | h[3] << 16);
+            *(uint2 *)(o + (2 + part) * RW_MAXK + at) =
+                make_uint2(l[0] | l[1] << 16, l[2] | l[3] << 16);
+        }
+        return;
+    }
+    for (uint32_t k = 32; k > 0; k >>= 1) {
+        m = fmaxf(m, __shfl_xor(m, k, 64));
+        x1 += __shfl_xor(x1, k, 64);
+    }
+    if (hfx_lane() == 0) {
+        red[0][tid / HFX_WAVE] = m;
+        red[1][tid / HFX_WAVE] = x1;
+    }
+    __syncthreads();
+    if (odd) bad = 1;
+    __syncthreads();
+    m = fmaxf(fmaxf(red[0][0], red[0][1]), fmaxf(red[0][2], red[0][3]));
+    x1 = red[1][0] + red[1][1] + red[1][2] + red[1][3];
+    /* k: m 2^k in [2^(B-1), 2^B) from m's exponent, one less where that passes
+     * the largest value the digits reach; at most 126 */
+    constexpr int B = MODE == RW_I8X4 ? 31 : 23;
+    constexpr float XMAX = MODE == RW_I8X4 ? 2139062143.0f : 8355711.0f;
+    const bool w4 = MODE == RW_I8X4 && (bad || !(x1 >= m * (float)len * (1.0f / 4096.0f)));
+    int k = 0;
+    if (m > 0.0f && !w4) {
+        const int e = (int)((__float_as_uint(m) >> 23) & 255u) - 127;
+        k = B - 1 - e;
+        if (k > 126) k = 126;
+        /* XMAX of four digits rounds up to 2139062144, one past their largest */
+        else if (ldexpf(m, k) >= XMAX && (MODE == RW_I8X4 || ldexpf(m, k) > XMAX)) --k;
+    }
+    const float sc = ldexpf(1.0f, k);
+    if (tid == 0) {
+        qs[s] = ldexpf(1.0f, -k);
+        if constexpr (MODE == RW_I8X4) {
+            const uint32_t z = hfx_zeff(sp.d_zmax[s]);
+            lvl[s] = w4 ? 0u : z;
+            wide[s] = w4 ? z : 0u;
+        }
+    }
+    if (w4) return; /* its planes are never read into a score */
+#pragma unroll
+    for (uint32_t u = 0; u < NU; ++u) {
+        const uint32_t t = tid + 256 * u;
+        if (t >= NW) break;
+        uint32_t w[NP];
+#pragma unroll
+        for (uint32_t d = 0; d < NP; ++d) w[d] = 0u;
+#pragma unroll
+        for (uint32_t i = 0; i < 4; ++i) {
+            int32_t X = (int32_t)rintf(v[u][i] * sc);
+#pragma unroll
+            for (uint32_t d = 0; d < NP; ++d) {
+                const int32_t g = d + 1 < NP ? ((X + 128) & 255) - 128 : X;
+                w[d] |= (uint32_t)(g & 255) << (8 * i);
+                X = (X - g) >> 8;
+            }
+        }
+#pragma unroll
+        for (uint32_t d = 0; d < NP; ++d) ((uint32_t *)(o + d * RW_MAXK))[t] = w[d];
+    }
+}
+
+/* ------------------------------------------------------------------ */
+/* Rows                                                                  */
+/* ------------------------------------------------------------------ */
+
+/* One workgroup of two waves a tile.  The nibble map of its sixteen rows (bin
+ * x of a row in word 2 + x / 8, unary codes OR-ed = max per bin) takes 18.7 KiB
+ * of LDS, so that eight workgroups fill a CU; a row stride of 36 mod 64 words
+ * puts the 32 lanes of half an emission read on 64 different banks.  The b
+ * ladders (one lane a peptide, sequential FP32 sums as everywhere) go through
+ * LDS sixteen peptides x RB_CHUNK positions at a time, so that each thread then
+ * takes one position whatever the peptides' lengths.  A peak whose bins all lie
+ * outside the row goes to a word of its lane's own; a triple that straddles an
+ * end spills into the row's margin words, which are not emitted. */
+#define RB_THREADS 128
+#define RB_MSTR 292
+#define RB_CHUNK 64
+static_assert(RB_MSTR >= 2 + RW_MAXK / 8 + 2 && RB_MSTR % 64 == 36, "map row stride");
+#define RB_MAGIC 12582912.0f /* 1.5 * 2^23: adding it rounds to an integer, ties to even */
+#define RB_MAGIC_BITS 0x4B400000u
+
+__device__ __forceinline__ uint32_t rb_binu(float mz)
+{
+    return __float_as_uint(hfx_div(mz, HFX_BIN_WIDTH_MONO, 1.0f / HFX_BIN_WIDTH_MONO) + RB_MAGIC) -
+           RB_MAGIC_BITS;
+}
+
+/* bins past the row's last may not fit the magic sum (2^22): such m/z are cut
+ * to a value that is past the row as well */
+#define RB_MZMAX 1.0e6f
+
+struct RbPut {
+    uint32_t *row;   /* word of bin 0 */
+    uint32_t *trash; /* this thread's */
+    __device__ __forceinline__ void one(float mz) const
+    {
+        const uint32_t u = rb_binu(mz);
+        uint32_t *w = u < RW_MAXK ? row + (u >> 3) : trash;
+        atomicOr(w, HFX_CODE10 << ((u & 7u) * 4u));
+    }
+    /* 25 at x - 1, 50 at x, 25 at x + 1 for x in [-1, RW_MAXK] */
+    __device__ __forceinline__ void three(float mz) const
+    {
+        const uint32_t u = rb_binu(mz) - 1u + 8u; /* bin x - 1, counted from -8 */
+        const uint64_t t = (uint64_t)(HFX_CODE25 | HFX_CODE50 << 4 | HFX_CODE25 << 8)
+                           << ((u & 7u) * 4u);
+        const bool in = u - 6u < RW_MAXK + 2u;
+        uint32_t *w = in ? row - 1 + (u >> 3) : trash;
+        atomicOr(w, (uint32_t)t);
+        if (t >> 32) atomicOr(w + 1, (uint32_t)(t >> 32));
+    }
+};
+
+template <int Z>
+__device__ __forceinline__ void rb_peaks(const RbPut &p, float b, float y)
+{
+    constexpr float zh = HFX_DEV_H * (float)Z;
+    constexpr float h2o = HFX_DEV_H2O / (float)Z, nh3 = HFX_DEV_NH3 / (float)Z;
+    auto zdiv = [](float x) {
+        if constexpr (Z == 3) return hfx_div(x, 3.0f, 1.0f / 3.0f);
+        else return x * (1.0f / (float)Z);
+    };
+    auto cut = [](float x) { return fminf(fmaxf(x, -RB_MZMAX), RB_MZMAX); };
+    const float ma = cut(zdiv((b - HFX_DEV_CO) + zh));
+    const float mb = cut(zdiv(b + zh));
+    const float my = cut(zdiv((y + HFX_DEV_H2O) + zh));
+    p.one(ma);
+    p.three(mb);
+    p.one(mb - h2o);
+    p.one(mb - nh3);
+    p.three(my);
+    p.one(my - nh3);
+}
+
+struct RbArgs {
+    hfx_db db;
+    uint32_t ntiles;
+    uint8_t *rows[HFX_MAX_CHARGE];       /* null: level not written */
+    const uint32_t *flags;               /* [level - 1][ntiles]: tiles wanted, or null: all */
+    const uint64_t *slots;               /* their places in rows[level - 1] */
+    uint8_t *ng;                         /* [ntiles] groups a tile's peaks reach */
+    uint32_t G;                          /* groups a tile holds */
+};
+
+/* two words of eight nibbles 0 / 1 / 3 / 7 -> sixteen 2-bit codes */
+__device__ __forceinline__ uint32_t rb_pack(uint32_t a, uint32_t b)
+{
+    const uint32_t ca = (a & 0x22222222u) | ((a ^ (a >> 2)) & 0x11111111u);
+    const uint32_t cb = (b & 0x22222222u) | ((b ^ (b >> 2)) & 0x11111111u);
+    return ca | cb << 2;
+}
+
+__global__ void __launch_bounds__(RB_THREADS) k_rw_build(RbArgs a)
+{
+    __shared__ __align__(16) uint32_t maps[RW_ROWS * RB_MSTR];
+    __shared__ float lb[RW_ROWS * RB_CHUNK];
+    __shared__ uint8_t lrow[RW_ROWS * RB_CHUNK];
+    __shared__ float mtab[32], rr[RW_ROWS];
+    __shared__ uint32_t trash[RB_THREADS + 1], tot;
+    __shared__ uint32_t topb;
+    const uint32_t t = blockIdx.x, tid = threadIdx.x, lane = hfx_lane(), wave = tid / HFX_WAVE;
+    uint32_t want = 0;
+#pragma unroll
+    for (uint32_t l = 0; l < HFX_MAX_CHARGE; ++l)
+        if (a.rows[l] && (!a.flags || rw_sload(a.flags, (uint64_t)l * a.ntiles + t) != 0u))
+            want |= 1u << l;
+    if (!want) return;
+    for (uint32_t i = tid; i < RW_ROWS * RB_MSTR / 4; i += RB_THREADS)
+        ((uint4 *)maps)[i] = make_uint4(0u, 0u, 0u, 0u);
+    if (tid < 32) mtab[tid] = tid < 26 ? a.db.d_mass[tid] : 0.0f;
+    if (tid == 0) topb = 0;
+    /* lane r < 16 of wave 0: peptide r of the tile, its ladder so far */
+    uint32_t n = 0, tc = 0;
+    float r = 0.0f, bl = 0.0f;
+    const uint32_t q = t * RW_ROWS + tid;
+    if (tid < RW_ROWS && q < a.db.num_pep) {
+        const uint32_t pep = a.db.d_idx_sorted[q];
+        const uint32_t tn = a.db.d_tn[pep];
+        tc = a.db.d_tc[pep];
+        n = tn > tc ? tn - tc : 0u;
+        r = a.db.d_r[pep];
+    }
+    if (tid < RW_ROWS) rr[tid] = r;
+    uint32_t nmax = n;
+    for (uint32_t o = 8; o > 0; o >>= 1) nmax = max(nmax, (uint32_t)__shfl_xor((int)nmax, o, 64));
+    if (tid == 0) tot = nmax;
+    __syncthreads();
+    const uint32_t nch = (tot + RB_CHUNK - 1) / RB_CHUNK;
+    const uint32_t top = 31u - (uint32_t)__builtin_clz(want); /* highest level - 1 */
+    __syncthreads(); /* tot is reused below */
+
+    /* positions [c RB_CHUNK, ...) of the sixteen ladders into lb, row after row */
+    auto ladders = [&](uint32_t c) {
+        if (wave == 0) {
+            const uint32_t k0 = c * RB_CHUNK;
+            const uint32_t cn = n > k0 ? min(n - k0, (uint32_t)RB_CHUNK) : 0u;
+            uint32_t incl = lane < RW_ROWS ? cn : 0u;
+            const uint32_t mine = incl;
+#pragma unroll
+            for (uint32_t o = 1; o < RW_ROWS; o <<= 1) {
+                const uint32_t y = __shfl_up(incl, o, 64);
+                if (lane >= o) incl += y;
+            }
+            const uint32_t at = incl - mine;
+            if (lane == RW_ROWS - 1) tot = incl;
+            if (lane < RW_ROWS) {
+                if (c == 0) bl = 0.0f;
+                const uint8_t *res = a.db.d_ions + tc + k0;
+                float mx = 0.0f;
+                for (uint32_t k = 0; k < cn; k += 8) {
+                    uint32_t x[8];
+#pragma unroll
+                    for (uint32_t j = 0; j < 8; ++j) x[j] = res[min(k + j, cn - 1u)];
+#pragma unroll
+                    for (uint32_t j = 0; j < 8; ++j)
+                        if (k + j < cn) {
+                            bl = bl + mtab[HFX_ACID_IDX(x[j])];
+                            lb[at + k + j] = bl;
+                            lrow[at + k + j] = (uint8_t)lane;
+                            mx = fmaxf(mx, fmaxf(bl, r - bl));
+                        }
+                }
+                atomicMax(&topb, __float_as_uint(mx));
+            }
+        }
+        __syncthreads();
+    };
+    for (uint32_t z = 1; z <= top + 1u; ++z) {
+        for (uint32_t c = 0; c < nch; ++c) {
+            if (z == 1 || nch > 1) ladders(c);
+            const uint32_t np = tot;
+            for (uint32_t i = tid; i < np; i += RB_THREADS) {
+                const uint32_t row = lrow[i];
+                const float b = lb[i], y = rr[row] - b;
+                const RbPut p{maps + row * RB_MSTR + 2, trash + tid};
+                switch (z) {
+                case 1: rb_peaks<1>(p, b, y); break;
+                case 2: rb_peaks<2>(p, b, y); break;
+                case 3: rb_peaks<3>(p, b, y); break;
+                default: rb_peaks<4>(p, b, y); break;
+                }
+            }
+            __syncthreads();
+        }
+        /* groups the peaks reach: every bin lies below top / 1.0005 + 24 */
+        const float tf = fminf(__uint_as_float(topb), 1.0e6f);
+        const uint32_t ng = min(a.G, ((uint32_t)tf + 28u) / 256u + 1u);
+        if (z == 1 && tid == 0) a.ng[t] = (uint8_t)ng;
+        if ((want >> (z - 1u)) & 1u) {
+            const uint64_t slot = a.slots ? rw_sload(a.slots, (uint64_t)(z - 1u) * a.ntiles + t)
+                                          : (uint64_t)t;
+            rw_u32x4 *out = (rw_u32x4 *)(a.rows[z - 1u] + slot * ((size_t)a.G * 1024u));
+            const uint32_t *mrow = maps + (lane & 15u) * RB_MSTR + 2 + 2 * (lane >> 4);
+            for (uint32_t g = wave; g < ng; g += RB_THREADS / HFX_WAVE) {
+                rw_u32x4 v;
+#pragma unroll
+                for (uint32_t k = 0; k < 4; ++k) {
+                    /* the last group's words past the row hold no bins */
+                    const uint32_t w = g * 32 + k * 8;
+                    const uint2 ab = w < RW_MAXK / 8 ? *(const uint2 *)(mrow + w)
+                                                     : make_uint2(0u, 0u);
+                    v[k] = rb_pack(ab.x, ab.y);
+                }
+                out[g * 64 + lane] = v;
+            }
+            if (z <= top) __syncthreads(); /* read before the next charge's peaks */
+        }
+    }
+}
+
+/* ------------------------------------------------------------------ */
+/* Work items                                                             */
+/* ------------------------------------------------------------------ */
+
+/* block b: the tiles of its windows' hull, fragment charge levels (bit z),
+ * longest row in k-steps, work items (CT tiles each, per level) */
+template <uint32_t NS>
+__global__ void k_rw_blocks(uint32_t *tbeg, uint32_t *tend, uint32_t *binfo, uint32_t *items,
+                            const uint32_t *order, const uint32_t *bstart, const uint32_t *begin,
+                            const uint32_t *num, hfx_spectra sp, uint32_t B, uint32_t CT)
+{
+    const uint32_t b = blockIdx.x * blockDim.x + threadIdx.x;
+    if (b >= B) return;
+    uint32_t lo = 0xffffffffu, hi = 0, mask = 0, kmax = 0;
+    const uint32_t i0 = bstart[b], i1 = bstart[b + 1];
+    uint32_t sv[NS];
+#pragma unroll
+    for (uint32_t g = 0; g < NS; ++g) sv[g] = i0 + g < i1 ? order[i0 + g] : 0xffffffffu;
+#pragma unroll
+    for (uint32_t g = 0; g < NS; ++g) {
+        const uint32_t s = sv[g];
+        if (s == 0xffffffffu) continue;
+        const uint32_t z = hfx_zeff(sp.d_zmax[s]), n = num[s], bg = begin[s], ln = sp.d_len[s];
+        if (z == 0 || n == 0) continue;
+        lo = min(lo, bg);
+        hi = max(hi, bg + n);
+        mask |= 1u << z;
+        kmax = max(kmax, min(ln, min(sp.x_stride, (uint32_t)RW_MAXK)));
+    }
+    const bool any = hi > lo;
+    const uint32_t t0 = any ? lo / RW_ROWS : 0u, t1 = any ? (hi + RW_ROWS - 1) / RW_ROWS : 0u;
+    if (!any) mask = 0;
+    tbeg[b] = t0;
+    tend[b] = t1;
+    binfo[b] = (kmax + 63u) / 64u | mask << 16;
+    items[b] = ((t1 - t0 + CT - 1) / CT) * (uint32_t)__builtin_popcount(mask);
+}
+
+__global__ void k_rw_reset(uint32_t *counter) { *counter = 0; }
+
+__global__ void k_rw_fill(uint32_t *a, uint64_t n, uint32_t v)
+{
+    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n;
+         i += (uint64_t)gridDim.x * blockDim.x)
+        a[i] = v;
+}
+
+/* the tiles the blocks read: one workgroup a block (equal stores race) */
+__global__ void k_rw_mark(uint32_t *flags, const uint32_t *tbeg, const uint32_t *tend,
+                          const uint32_t *binfo, uint32_t ntiles)
+{
+    const uint32_t b = blockIdx.x, mask = binfo[b] >> 16;
+    for (uint32_t l = 1; l <= HFX_MAX_CHARGE; ++l)
+        if ((mask >> l) & 1u)
+            for (uint32_t t = tbeg[b] + threadIdx.x; t < tend[b]; t += blockDim.x)
+                flags[(size_t)(l - 1) * ntiles + t] = 1u;
+}
+
+/* spectra whose fragment charge is not generated score 0 */
+__global__ void k_rw_zero_unscored(float *scores, const uint64_t *off, const uint32_t *zmax,
+                                   uint32_t S)
+{
+    const uint32_t s = blockIdx.x;
+    if (s >= S || hfx_zeff(zmax[s]) != 0) return;
+    for (uint64_t i = off[s] + threadIdx.x; i < off[s + 1]; i += blockDim.x) scores[i] = 0.0f;
+}
+
+/* ------------------------------------------------------------------ */
+/* The contraction                                                        */
+/* ------------------------------------------------------------------ */
+
+#define RM_THREADS 512
+#define RM_WAVES (RM_THREADS / HFX_WAVE)
+#define RM_T 4 /* tiles a wave contracts at once: each B fragment read serves 64 rows */
+
+struct RmArgs {
+    float *scores;
+    const uint64_t *score_off;
+    const uint32_t *begin, *num, *order, *bstart;
+    uint32_t B, CT;
+    const uint32_t *tbeg, *tend, *binfo;
+    const uint64_t *item_off;
+    const uint8_t *planes;
+    const float *qs;
+    uint32_t *counter;
+    const uint8_t *rows[HFX_MAX_CHARGE];
+    const uint64_t *slots; /* [level - 1][ntiles], or null: tile t at place t */
+    const uint8_t *ng;
+    uint32_t ntiles, G;
+    hfx_spectra sp;
+};
+
+/* Persistent workgroups of eight waves over (block, level, CT tiles).  The
+ * block's planes stay in LDS, laid out so that a fragment read is one
+ * contiguous KiB ([k-step][plane][lane]); each wave contracts four tiles at a
+ * time over the whole row, its accumulators in registers, the next group's
+ * codes loaded while the current one is contracted.  A k-step of four tiles
+ * costs 4 x 11 code lookups, 4 x planes matrix instructions and one fragment
+ * read a plane. */
+template <int MODE>
+__global__ void __launch_bounds__(RM_THREADS, 2) k_rw_mm(RmArgs a)
+{
+    constexpr uint32_t NP = MODE == RW_BF16 ? 2 : RW_PLANES(MODE); /* planes in LDS */
+    constexpr uint32_t NS = RW_NS(MODE);
+    extern __shared__ __align__(16) uint8_t rm_lds[];
+    rw_u32x4 *Bl = (rw_u32x4 *)rm_lds; /* [k-step][plane][64 lanes] */
+    __shared__ uint32_t m_s[16], m_beg[16], m_end[16], m_z[16];
+    __shared__ float m_q[16];
+    __shared__ uint64_t m_off[16];
+    __shared__ uint32_t sh_t[2];
+    const uint32_t tid = threadIdx.x, lane = hfx_lane();
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(tid / HFX_WAVE);
+    const uint32_t col = lane & 15u, kg = lane >> 4;
+    const uint32_t g_of = MODE == RW_BF16 ? col >> 1 : col; /* spectrum of this lane's column */
+    const uint32_t nitems = (uint32_t)rw_sload(a.item_off, a.B);
+    uint32_t cur = 0xffffffffu;
+    if (tid == 0) sh_t[0] = atomicAdd(a.counter, 1u);
+    uint32_t next = 0;
+    for (uint32_t slot = 0;; slot ^= 1u) {
+        __syncthreads(); /* every wave is done with the previous item */
+        const uint32_t t0 = __builtin_amdgcn_readfirstlane(sh_t[slot]);
+        if (t0 >= nitems) break;
+        /* from the last to the first: higher charge levels and heavier
+         * precursors (longer rows) come first, the lightest finish the launch */
+        const uint32_t it = nitems - 1u - t0;
+        if (tid == 0) next = atomicAdd(a.counter, 1u);
+        uint32_t lo = 0, hi = a.B;
+        while (hi - lo > 1) {
+            const uint32_t mid = (lo + hi) >> 1;
+            if (rw_sload(a.item_off, mid) <= it) lo = mid; else hi = mid;
+        }
+        const uint32_t b = lo;
+        const uint32_t info = rw_sload(a.binfo, b);
+        const uint32_t nks = info & 0xffffu, mask = info >> 16;
+        if (b != cur) {
+            if (tid < 16) {
+                const uint32_t i = a.bstart[b] + tid;
+                uint32_t s = 0xffffffffu, be = 0, en = 0, z = 0;
+                uint64_t of = 0;
+                float q = 0.0f;
+                if (tid < NS && i < a.bstart[b + 1]) {
+                    s = a.order[i];
+                    be = a.begin[s];
+                    en = be + a.num[s];
+                    z = hfx_zeff(a.sp.d_zmax[s]);
+                    of = a.score_off[s];
+                    if (MODE != RW_BF16) q = a.qs[s];
+                }
+                m_s[tid] = s; m_beg[tid] = be; m_end[tid] = en; m_z[tid] = z; m_off[tid] = of;
+                m_q[tid] = q;
+            }
+            __syncthreads();
+            /* lanes over columns first: LDS writes are contiguous, and the four
+             * k-groups of a column are 64 bytes of its plane */
+            const uint32_t nv = nks * NP * 64u;
+            constexpr uint32_t U = 6;
+            for (uint32_t i0 = tid; i0 < nv; i0 += U * RM_THREADS) {
+                rw_u32x4 val[U];
+#pragma unroll
+                for (uint32_t u = 0; u < U; ++u) {
+                    const uint32_t i = i0 + u * RM_THREADS;
+                    const uint32_t kd = i >> 6, ks = kd / NP, d = kd - ks * NP;
+                    const uint32_t s = m_s[g_of];
+                    val[u] = rw_u32x4{0u, 0u, 0u, 0u};
+                    if (i < nv && s != 0xffffffffu) {
+                        const uint32_t pl = MODE == RW_BF16 ? (col & 1u) * 2u + d : d;
+                        val[u] = *(const rw_u32x4 *)(a.planes +
+                                                     ((size_t)s * RW_PLANES(MODE) + pl) * RW_MAXK +
+                                                     ks * 64u + kg * 16u);
+                    }
+                }
+#pragma unroll
+                for (uint32_t u = 0; u < U; ++u)
+                    if (i0 + u * RM_THREADS < nv) Bl[i0 + u * RM_THREADS] = val[u];
+            }
+            cur = b;
+            __syncthreads();
+        }
+        if (tid == 0) sh_t[slot ^ 1u] = next;
+        const uint32_t tb = rw_sload(a.tbeg, b), te = rw_sload(a.tend, b);
+        const uint32_t nch = (te - tb + a.CT - 1) / a.CT;
+        const uint32_t local = (uint32_t)(it - rw_sload(a.item_off, b));
+        const uint32_t li = local / nch, chunk = local - li * nch;
+        uint32_t m = mask;
+        for (uint32_t qq = 0; qq < li; ++qq) m &= m - 1u;
+        const uint32_t lvl = (uint32_t)__builtin_ctz(m);
+        const uint32_t c0 = tb + chunk * a.CT, c1 = min(c0 + a.CT, te);
+        const uint8_t *rows = lvl == 1 ? a.rows[0] : lvl == 2 ? a.rows[1]
+                            : lvl == 3 ? a.rows[2] : a.rows[3];
+        const uint64_t *slots = a.slots ? a.slots + (size_t)(lvl - 1u) * a.ntiles : nullptr;
+        const uint32_t beg = m_beg[g_of], end = m_end[g_of];
+        const bool mine = m_z[g_of] == lvl && (MODE != RW_BF16 || (col & 1u) == 0u);
+        const double qd = MODE == RW_BF16 ? 0.0 : (double)m_q[g_of];
+        float *const out = a.scores + m_off[g_of];
+        const size_t tile_bytes = (size_t)a.G * 1024u;
+        for (uint32_t u0 = c0 + wave * RM_T; u0 < c1; u0 += RM_WAVES * RM_T) {
+            const uint8_t *base[RM_T];
+            uint32_t ng = 0;
+#pragma unroll
+            for (uint32_t k = 0; k < RM_T; ++k) {
+                const uint32_t t = min(u0 + k, c1 - 1u);
+                const uint64_t place = slots ? rw_sload(slots, t) : (uint64_t)t;
+                base[k] = rows + place * tile_bytes;
+                const uint32_t word = rw_sload((const uint32_t *)a.ng, t >> 2);
+                ng = max(ng, (word >> ((t & 3u) * 8u)) & 255u);
+            }
+            ng = min(ng, (nks + 3u) >> 2);
+            /* groups past a tile's own are not written: read as zeros */
+            uint32_t own[RM_T];
+#pragma unroll
+            for (uint32_t k = 0; k < RM_T; ++k) {
+                const uint32_t t = min(u0 + k, c1 - 1u);
+                own[k] = (rw_sload((const uint32_t *)a.ng, t >> 2) >> ((t & 3u) * 8u)) & 255u;
+            }
+            auto load = [&](rw_u32x4(&c)[RM_T], uint32_t g) {
+#pragma unroll
+                for (uint32_t k = 0; k < RM_T; ++k) {
+                    const uint32_t gg = min(g, own[k] - 1u);
+                    c[k] = *(const rw_u32x4 *)(base[k] + gg * 1024u + lane * 16u);
+                    if (g >= own[k]) c[k] = rw_u32x4{0u, 0u, 0u, 0u};
+                }
+            };
+            rw_u32x4 ca[RM_T], cb[RM_T];
+            load(ca, 0);
+            if constexpr (MODE == RW_BF16) {
+                rw_f32x4 acc0[RM_T], acc1[RM_T];
+#pragma unroll
+                for (uint32_t k = 0; k < RM_T; ++k) {
+                    acc0[k] = rw_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+                    acc1[k] = acc0[k];
+                }
+                for (uint32_t g = 0; g < ng; ++g) {
+                    load(cb, min(g + 1u, ng - 1u));
+#pragma unroll
+                    for (uint32_t j = 0; j < 4; ++j) {
+                        const uint32_t ks = g * 4u + j;
+                        if (ks < nks) {
+                            const rw_u32x4 f0 = Bl[(ks * NP + 0) * 64u + lane];
+                            const rw_u32x4 f1 = Bl[(ks * NP + 1) * 64u + lane];
+#pragma unroll
+                            for (uint32_t k = 0; k < RM_T; ++k) {
+                                const uint32_t P = ca[k][j];
+                                uint32_t w[8];
+#pragma unroll
+                                for (uint32_t h = 0; h < 4; ++h) {
+                                    const uint32_t sel = (P >> (2 * h)) & 0x03030303u;
+                                    const uint32_t l8 = __builtin_amdgcn_perm(0u, 0xC8482000u, sel);
+                                    const uint32_t h8 = __builtin_amdgcn_perm(0u, 0x41424100u, sel);
+                                    w[2 * h] = __builtin_amdgcn_perm(h8, l8, 0x05010400u);
+                                    w[2 * h + 1] = __builtin_amdgcn_perm(h8, l8, 0x07030602u);
+                                }
+                                const rw_u32x4 a0 = {w[0], w[1], w[2], w[3]};
+                                const rw_u32x4 a1 = {w[4], w[5], w[6], w[7]};
+                                acc0[k] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                                    __builtin_bit_cast(rw_bf16x8, a0),
+                                    __builtin_bit_cast(rw_bf16x8, f0), acc0[k], 0, 0, 0);
+                                acc1[k] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                                    __builtin_bit_cast(rw_bf16x8, a1),
+                                    __builtin_bit_cast(rw_bf16x8, f1), acc1[k], 0, 0, 0);
+                            }
+                        }
+                    }
+#pragma unroll
+                    for (uint32_t k = 0; k < RM_T; ++k) ca[k] = cb[k];
+                }
+#pragma unroll
+                for (uint32_t k = 0; k < RM_T; ++k) {
+                    const uint32_t t = u0 + k;
+#pragma unroll
+                    for (uint32_t i = 0; i < 4; ++i) {
+                        const float h = acc0[k][i] + acc1[k][i];
+                        /* an even column's lane adds its odd neighbour: hi + lo */
+                        const float v = h + __uint_as_float((uint32_t)__builtin_amdgcn_update_dpp(
+                                                (int)__float_as_uint(h), (int)__float_as_uint(h),
+                                                0xb1, 0xf, 0xf, false));
+                        const uint32_t p = t * RW_ROWS + 4u * kg + i;
+                        if (mine && t < c1 && beg <= p && p < end) out[p - beg] = v;
+                    }
+                }
+            } else {
+                rw_i32x4 acc[RM_T][NP];
+#pragma unroll
+                for (uint32_t k = 0; k < RM_T; ++k)
+#pragma unroll
+                    for (uint32_t d = 0; d < NP; ++d) acc[k][d] = rw_i32x4{0, 0, 0, 0};
+                for (uint32_t g = 0; g < ng; ++g) {
+                    load(cb, min(g + 1u, ng - 1u));
+#pragma unroll
+                    for (uint32_t j = 0; j < 4; ++j) {
+                        const uint32_t ks = g * 4u + j;
+                        if (ks < nks) {
+                            rw_i32x4 f[NP];
+#pragma unroll
+                            for (uint32_t d = 0; d < NP; ++d)
+                                f[d] = __builtin_bit_cast(rw_i32x4, Bl[(ks * NP + d) * 64u + lane]);
+#pragma unroll
+                            for (uint32_t k = 0; k < RM_T; ++k) {
+                                const uint32_t P = ca[k][j];
+                                rw_i32x4 av;
+#pragma unroll
+                                for (uint32_t h = 0; h < 4; ++h)
+                                    av[h] = (int32_t)__builtin_amdgcn_perm(
+                                        0u, 0x19320A00u, (P >> (2 * h)) & 0x03030303u);
+#pragma unroll
+                                for (uint32_t d = 0; d < NP; ++d)
+                                    acc[k][d] = __builtin_amdgcn_mfma_i32_16x16x64_i8(
+                                        av, f[d], acc[k][d], 0, 0, 0);
+                            }
+                        }
+                    }
+#pragma unroll
+                    for (uint32_t k = 0; k < RM_T; ++k) ca[k] = cb[k];
+                }
+                /* digit sums are below 50 * 128 * RW_MAXK < 2^24, so the folds
+                 * are exact in FP64 and the score is rounded once */
+#pragma unroll
+                for (uint32_t k = 0; k < RM_T; ++k) {
+                    const uint32_t t = u0 + k;
+#pragma unroll
+                    for (uint32_t i = 0; i < 4; ++i) {
+                        double v = (double)acc[k][NP - 1][i];
+#pragma unroll
+                        for (int d = (int)NP - 2; d >= 0; --d)
+                            v = __builtin_fma(v, 256.0, (double)acc[k][d][i]);
+                        const uint32_t p = t * RW_ROWS + 4u * kg + i;
+                        if (mine && t < c1 && beg <= p && p < end) out[p - beg] = (float)(v * qd);
+                    }
+                }
+            }
+        }
+    }
+}
+
+/* ------------------------------------------------------------------ */
+/* Host side                                                              */
+/* ------------------------------------------------------------------ */
+
+uint32_t hfx_rows_tiles(uint32_t num_pep) { return (num_pep + RW_ROWS - 1) / RW_ROWS; }
+uint32_t hfx_rows_groups(uint32_t x_stride)
+{
+    return (std::min(x_stride, (uint32_t)RW_MAXK) + 255u) / 256u;
+}
+/* candidates a work item takes (multiple of RM_T tiles a wave): about four
+ * items a CU, but enough rows that the block's planes are worth staging */
+uint32_t hfx_rows_chunk(uint64_t rows, uint32_t cus)
+{
+    const uint64_t c = rows / (4ull * cus);
+    const uint64_t step = RM_WAVES * RM_T * RW_ROWS; /* every wave busy */
+    return (uint32_t)std::min<uint64_t>(std::max<uint64_t>((c + step - 1) / step * step, step), 8192);
+}
+
+int hfx_rows_split(int mode, const hfx_spectra *sp, uint8_t *planes, float *qs, uint32_t *lvl,
+                   uint32_t *wide, void *stream)
+{
+    HFX_REQUIRE(sp->x_stride <= RW_MAXK, HFX_ERR_ARG, "rows: spectra of up to %d bins", RW_MAXK);
+    if (sp->num_spec == 0) return HFX_OK;
+    const dim3 g(sp->num_spec), t(256);
+    hipStream_t st = hfx_stream(stream);
+    if (mode == RW_I8X3) hipLaunchKernelGGL(k_rw_split<RW_I8X3>, g, t, 0, st, planes, qs, lvl, wide, *sp);
+    else if (mode == RW_I8X4) hipLaunchKernelGGL(k_rw_split<RW_I8X4>, g, t, 0, st, planes, qs, lvl, wide, *sp);
+    else hipLaunchKernelGGL(k_rw_split<RW_BF16>, g, t, 0, st, planes, qs, lvl, wide, *sp);
+    HFX_CHECK_LAUNCH();
+    return HFX_OK;
+}
+
+int hfx_rows_build(const hfx_db *db, const hfx_rows *r, const uint32_t *flags, void *stream)
+{
+    RbArgs a{};
+    a.db = *db;
+    a.ntiles = r->ntiles;
+    for (int l = 0; l < HFX_MAX_CHARGE; ++l) a.rows[l] = r->rows[l];
+    a.flags = flags;
+    a.slots = r->slots;
+    a.ng = r->ng;
+    a.G = r->G;
+    if (r->ntiles)
+        hipLaunchKernelGGL(k_rw_build, dim3(r->ntiles), dim3(RB_THREADS), 0, hfx_stream(stream), a);
+    HFX_CHECK_LAUNCH();
+    return HFX_OK;
+}
+
+/* scratch of the work items of S spectra: tbeg, tend, binfo, items [S] each,
+ * item_off [S + 1], counter */
+size_t hfx_rows_items_bytes(uint32_t S) { return (size_t)S * 16 + ((size_t)S + 1) * 8 + 64; }
+
+static void rw_items(void *p, uint32_t S, uint32_t **tbeg, uint32_t **tend, uint32_t **binfo,
+                     uint32_t **items, uint64_t **off, uint32_t **counter)
+{
+    *off = (uint64_t *)(((uintptr_t)p + 7) & ~(uintptr_t)7);
+    *tbeg = (uint32_t *)(*off + S + 1);
+    *tend = *tbeg + S;
+    *binfo = *tend + S;
+    *items = *binfo + S;
+    *counter = *items + S;
+}
+
+int hfx_rows_blocks(hfx_ctx *ctx, int mode, void *scratch, const uint32_t *order,
+                    const uint32_t *bstart, const uint32_t *begin, const uint32_t *num,
+                    const hfx_spectra *sp, uint32_t CH, void *stream)
+{
+    const uint32_t B = sp->num_spec;
+    uint32_t *tbeg, *tend, *binfo, *items, *counter;
+    uint64_t *off;
+    rw_items(scratch, B, &tbeg, &tend, &binfo, &items, &off, &counter);
+    hipStream_t st = hfx_stream(stream);
+    const uint32_t CT = std::max(CH / RW_ROWS, 1u);
+    if (RW_NS(mode) == 16)
+        hipLaunchKernelGGL(k_rw_blocks<16>, dim3((B + 255) / 256), dim3(256), 0, st, tbeg, tend,
+                           binfo, items, order, bstart, begin, num, *sp, B, CT);
+    else
+        hipLaunchKernelGGL(k_rw_blocks<8>, dim3((B + 255) / 256), dim3(256), 0, st, tbeg, tend,
+                           binfo, items, order, bstart, begin, num, *sp, B, CT);
+    int rc = hfx_scan_offsets(ctx, off, items, B, stream);
+    if (rc) return rc;
+    hipLaunchKernelGGL(k_rw_reset, dim3(1), dim3(1), 0, st, counter);
+    HFX_CHECK_LAUNCH();
+    return HFX_OK;
+}
+
+int hfx_rows_mark(void *scratch, uint32_t S, uint32_t *flags, uint32_t ntiles, void *stream)
+{
+    uint32_t *tbeg, *tend, *binfo, *items, *counter;
+    uint64_t *off;
+    rw_items(scratch, S, &tbeg, &tend, &binfo, &items, &off, &counter);
+    hipStream_t st = hfx_stream(stream);
+    const uint64_t n = (uint64_t)HFX_MAX_CHARGE * ntiles;
+    hipLaunchKernelGGL(k_rw_fill, dim3((uint32_t)std::min<uint64_t>((n + 255) / 256, 2048)),
+                       dim3(256), 0, st, flags, n, 0u);
+    hipLaunchKernelGGL(k_rw_mark, dim3(S), dim3(256), 0, st, flags, tbeg, tend, binfo, ntiles);
+    HFX_CHECK_LAUNCH();
+    return HFX_OK;
+}
+
+int hfx_rows_scores(hfx_ctx *ctx, int mode, void *scratch, float *d_scores, const uint64_t *d_off,
+                    const uint32_t *begin, const uint32_t *num, const uint32_t *order,
+                    const uint32_t *bstart, const hfx_rows *r, const uint8_t *planes,
+                    const float *qs, const hfx_spectra *sp, uint32_t CH, const uint32_t *zmax,
+                    void *stream, void **ev)
+{
+    const uint32_t S = sp->num_spec;
+    uint32_t *tbeg, *tend, *binfo, *items, *counter;
+    uint64_t *off;
+    rw_items(scratch, S, &tbeg, &tend, &binfo, &items, &off, &counter);
+    hipStream_t st = hfx_stream(stream);
+    RmArgs a{};
+    a.scores = d_scores;
+    a.score_off = d_off;
+    a.begin = begin;
+    a.num = num;
+    a.order = order;
+    a.bstart = bstart;
+    a.B = S;
+    a.CT = std::max(CH / RW_ROWS, 1u);
+    a.tbeg = tbeg;
+    a.tend = tend;
+    a.binfo = binfo;
+    a.item_off = off;
+    a.planes = planes;
+    a.qs = qs;
+    a.counter = counter;
+    for (int l = 0; l < HFX_MAX_CHARGE; ++l) a.rows[l] = r->rows[l];
+    a.slots = r->slots;
+    a.ng = r->ng;
+    a.ntiles = r->ntiles;
+    a.G = r->G;
+    a.sp = *sp;
+    const uint32_t np = mode == RW_BF16 ? 2u : (uint32_t)RW_PLANES(mode);
+    const uint32_t lds = RW_NKS * np * 1024u;
+    const uint32_t per_cu = lds * 2 <= 156u * 1024u ? 2u : 1u;
+    const dim3 g((uint32_t)hfx_ctx_num_cus(ctx) * per_cu), t(RM_THREADS);
+    const void *fn = mode == RW_I8X3   ? (const void *)k_rw_mm<RW_I8X3>
+                     : mode == RW_I8X4 ? (const void *)k_rw_mm<RW_I8X4>
+                                       : (const void *)k_rw_mm<RW_BF16>;
+    HFX_CHECK_HIP(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    if (ev) HFX_CHECK_HIP(hipEventRecord((hipEvent_t)ev[0], st));
+    if (mode == RW_I8X3) hipLaunchKernelGGL(k_rw_mm<RW_I8X3>, g, t, lds, st, a);
+    else if (mode == RW_I8X4) hipLaunchKernelGGL(k_rw_mm<RW_I8X4>, g, t, lds, st, a);
+    else hipLaunchKernelGGL(k_rw_mm<RW_BF16>, g, t, lds, st, a);
+    if (ev) HFX_CHECK_HIP(hipEventRecord((hipEvent_t)ev[1], st));
+    hipLaunchKernelGGL(k_rw_zero_unscored, dim3(S), dim3(256), 0, st, d_scores, d_off, zmax, S);
+    HFX_CHECK_LAUNCH();
+    return HFX_OK;
+}

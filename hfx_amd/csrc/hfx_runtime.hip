@@ -26,8 +26,6 @@ void hfx_set_error(const char *fmt, ...)
 
 extern "C" const char *hfx_last_error(void) { return g_err; }
 
-#define HFX_SCRATCH_SLOTS 16
-
 struct hfx_ctx {
     int device;
     int num_cus;
@@ -84,6 +82,27 @@ int hfx_ctx_scratch(hfx_ctx *ctx, int slot, size_t bytes, void **out)
     }
     *out = ctx->scratch[slot];
     return HFX_OK;
+}
+
+void *hfx_ctx_scratch_spare(hfx_ctx *ctx, int slot, size_t bytes, void *stream)
+{
+    if (slot < 0 || slot >= HFX_SCRATCH_SLOTS) return nullptr;
+    if (ctx->scratch[slot] && ctx->scratch_bytes[slot] >= bytes) return ctx->scratch[slot];
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    size_t fr = 0, tot = 0;
+    if (hipStreamIsCapturing(hfx_stream(stream), &cs) != hipSuccess ||
+        cs != hipStreamCaptureStatusNone || hipMemGetInfo(&fr, &tot) != hipSuccess) {
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    const size_t sz = bytes + bytes / 4 + 256; /* what hfx_ctx_scratch allocates */
+    if (sz > tot / 8 || sz > (fr + ctx->scratch_bytes[slot]) / 2) return nullptr;
+    void *p = nullptr;
+    if (hfx_ctx_scratch(ctx, slot, bytes, &p) != HFX_OK) {
+        (void)hipGetLastError();
+        return nullptr;
+    }
+    return p;
 }
 
 int hfx_ctx_pinned(hfx_ctx *ctx, size_t bytes, void **out)

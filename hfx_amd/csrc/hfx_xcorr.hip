@@ -338,22 +338,13 @@ __device__ __forceinline__ void xp_pack(uint32_t *maps, uint32_t mstr, const flo
     }
 }
 
+/* the tile of spectrum s from its candidate `first` on; every thread of the
+ * workgroup calls it */
 template <class Cands>
-__global__ void __launch_bounds__(XP_THREADS)
-    k_xcorr_pack(float *scores, const uint64_t *tile_off, Cands c, hfx_spectra sp, uint32_t mstr)
+__device__ __forceinline__ void xp_tile(float *xp_lds, float *mtab, float *scores, const Cands &c,
+                                        const hfx_spectra &sp, uint32_t mstr, uint32_t s,
+                                        uint32_t first)
 {
-    extern __shared__ __align__(16) float xp_lds[];
-    __shared__ float mtab[32];
-    const uint32_t S = sp.num_spec;
-    const uint64_t t = blockIdx.x;
-    if (t >= tile_off[S]) return;
-    uint32_t lo = 0, hi = S;
-    while (hi - lo > 1) {
-        const uint32_t mid = (lo + hi) >> 1;
-        if (tile_off[mid] <= t) lo = mid; else hi = mid;
-    }
-    const uint32_t s = lo;
-    const uint32_t first = (uint32_t)(t - tile_off[s]) * XP_CHUNK;
     const uint32_t cnt = min((uint32_t)XP_CHUNK, c.count(s) - first);
     const uint32_t xstr = sp.x_stride;
     const uint32_t xf = (xstr + 2 * XP_PAD + 3) & ~3u;
@@ -454,6 +445,49 @@ __global__ void __launch_bounds__(XP_THREADS)
 }
 
 template <class Cands>
+__global__ void __launch_bounds__(XP_THREADS)
+    k_xcorr_pack(float *scores, const uint64_t *tile_off, Cands c, hfx_spectra sp, uint32_t mstr)
+{
+    extern __shared__ __align__(16) float xp_lds[];
+    __shared__ float mtab[32];
+    const uint32_t S = sp.num_spec;
+    const uint64_t t = blockIdx.x;
+    if (t >= tile_off[S]) return;
+    const uint32_t s = find_segment(tile_off, S, t);
+    xp_tile(xp_lds, mtab, scores, c, sp, mstr, s, (uint32_t)(t - tile_off[s]) * XP_CHUNK);
+}
+
+/* The spectra marked in wide (seldom any), a workgroup each at a time: the
+ * workgroups look at XP_THREADS spectra a step and walk the tiles of those
+ * marked. */
+__global__ void __launch_bounds__(XP_THREADS)
+    k_xcorr_wide(float *scores, HfxPlainCands c, hfx_spectra sp, const uint32_t *wide,
+                 uint32_t mstr)
+{
+    extern __shared__ __align__(16) float xp_lds[];
+    __shared__ float mtab[32];
+    __shared__ uint64_t marked[XP_WAVES];
+    const uint32_t S = sp.num_spec, G = gridDim.x;
+    /* this workgroup's spectra are blockIdx.x + k G, k = 0, 1, ... */
+    for (uint64_t k0 = 0; blockIdx.x + k0 * G < S; k0 += XP_THREADS) {
+        const uint64_t mine = blockIdx.x + (k0 + threadIdx.x) * G;
+        const uint64_t bal = __ballot(mine < S && wide[mine] != 0u);
+        if (hfx_lane() == 0) marked[threadIdx.x / HFX_WAVE] = bal;
+        __syncthreads();
+        for (uint32_t w = 0; w < XP_WAVES; ++w)
+            for (uint64_t m = marked[w]; m; m &= m - 1ull) {
+                const uint32_t s = (uint32_t)(blockIdx.x + (k0 + w * HFX_WAVE +
+                                                            (uint32_t)__builtin_ctzll(m)) * G);
+                for (uint32_t f = 0; f < c.count(s); f += XP_CHUNK) {
+                    xp_tile(xp_lds, mtab, scores, c, sp, mstr, s, f);
+                    __syncthreads(); /* its LDS is staged anew */
+                }
+            }
+        __syncthreads();
+    }
+}
+
+template <class Cands>
 __global__ void k_tile_count(uint32_t *tiles, Cands c, uint32_t num_spec, uint32_t chunk)
 {
     uint32_t s = blockIdx.x * blockDim.x + threadIdx.x;
@@ -523,6 +557,20 @@ static int launch_xcorr(void *scratch, float *d_scores, const Cands &c, uint64_t
         hipLaunchKernelGGL(k_xcorr<Cands>, dim3((uint32_t)grid), dim3(XC_THREADS), 0, st,
                            d_scores, tile_off, c, *sp);
     }
+    HFX_CHECK_LAUNCH();
+    return HFX_OK;
+}
+
+int hfx_xcorr_wide(hfx_ctx *ctx, float *d_scores, const uint64_t *d_off, const uint32_t *d_begin,
+                   const uint32_t *d_num, const hfx_db *db, const hfx_spectra *sp,
+                   const uint32_t *wide, void *stream)
+{
+    const uint32_t S = sp->num_spec;
+    if (S == 0) return HFX_OK;
+    HfxPlainCands c{*db, d_begin, d_num, d_off};
+    hipLaunchKernelGGL(k_xcorr_wide, dim3(min(S, (uint32_t)hfx_ctx_num_cus(ctx) * 4u)),
+                       dim3(XP_THREADS), xp_lds_bytes(sp->x_stride), hfx_stream(stream), d_scores, c,
+                       *sp, wide, xp_map_words(sp->x_stride));
     HFX_CHECK_LAUNCH();
     return HFX_OK;
 }
