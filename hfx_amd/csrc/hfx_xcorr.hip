@@ -14,6 +14,7 @@
  * wave scores one candidate at a time (ladder -> map -> dot).
  */
 #include "hfx_cand.h"
+#include "hfx_rows.h"
 
 #include <stdlib.h>
 
@@ -575,6 +576,88 @@ int hfx_xcorr_wide(hfx_ctx *ctx, float *d_scores, const uint64_t *d_off, const u
     return HFX_OK;
 }
 
+/* ------------------------------------------------------------------ */
+/* Rows route                                                            */
+/* ------------------------------------------------------------------ */
+
+/* From this many scored pairs on, hfx_xcorr_sparse writes each candidate's
+ * theoretical row once and contracts the rows with blocks of sixteen spectra
+ * (hfx_rows.hip, 32-bit fixed point) instead of building a row per pair.  Its
+ * dozen launches cost about 100 us, which the packed kernel spends on half a
+ * million pairs. */
+#define XR_MIN_PAIRS 500000ull
+
+/* *taken = 0: nothing done (too few pairs, rows longer than the form's, no
+ * memory to spare) */
+static int xcorr_rows(hfx_ctx *ctx, float *d_scores, const uint64_t *d_off,
+                      const uint32_t *d_begin, const uint32_t *d_num, uint64_t total,
+                      const hfx_db *db, const hfx_spectra *sp, void *stream, int *taken)
+{
+    *taken = 0;
+    const uint32_t S = sp->num_spec;
+    if (total < XR_MIN_PAIRS || sp->x_stride > RW_MAXK || db->num_pep == 0) return HFX_OK;
+    const uint32_t nt = hfx_rows_tiles(db->num_pep), G = hfx_rows_groups(sp->x_stride);
+    const uint64_t nf = (uint64_t)HFX_MAX_CHARGE * nt;
+    if (nf >= 0xffffffffull) return HFX_OK;
+    /* the block cut never takes more rows than the windows one by one */
+    const uint64_t slots = min(nf, total / RW_ROWS + 2ull * S);
+    hfx_order_bufs ob;
+    hfx_order_shape(S, db->num_pep, &ob);
+    const uint32_t nseg = hfx_cut_segs(S);
+    auto al = [](uint64_t n) { return (n + 255) & ~(uint64_t)255; };
+    const uint64_t sizes[] = {
+        al((uint64_t)S * RW_PLANES(RW_I8X4) * RW_MAXK), al(4ull * S), al(4ull * S), al(4ull * S),
+        al(4ull * S), al(4ull * ob.nb), al(4ull * S), al(8ull * ob.nb + 8), al(4ull * nseg * 32),
+        al(4ull * nseg), al(8ull * nseg + 8), al(4ull * S + 4), al(hfx_rows_items_bytes(S)),
+        al(4 * nf), al(8 * nf + 8), al(nt + 4ull)};
+    uint64_t bytes = 0;
+    for (uint64_t z : sizes) bytes += z;
+    uint8_t *p = (uint8_t *)hfx_ctx_scratch_spare(ctx, HFX_SLOT_ROWS, bytes, stream);
+    if (!p) return HFX_OK;
+    uint8_t *rows = (uint8_t *)hfx_ctx_scratch_spare(ctx, HFX_SLOT_ROWS2, slots * G * 1024ull, stream);
+    if (!rows) return HFX_OK;
+    uint8_t *part[sizeof sizes / sizeof *sizes];
+    for (size_t i = 0; i < sizeof sizes / sizeof *sizes; ++i) {
+        part[i] = p;
+        p += sizes[i];
+    }
+    uint8_t *planes = part[0];
+    float *qs = (float *)part[1];
+    uint32_t *lvl = (uint32_t *)part[2], *wide = (uint32_t *)part[3], *order = (uint32_t *)part[4];
+    ob.cnt = (uint32_t *)part[5];
+    ob.tmp = (uint32_t *)part[6];
+    ob.off = (uint64_t *)part[7];
+    const hfx_cut_bufs cb{(uint32_t *)part[8], (uint32_t *)part[9], (uint64_t *)part[10],
+                          (uint32_t *)part[11]};
+    void *items = part[12];
+    uint32_t *flags = (uint32_t *)part[13];
+    hfx_rows r{};
+    r.slots = (uint64_t *)part[14];
+    r.ng = part[15];
+    r.ntiles = nt;
+    r.G = G;
+    for (int l = 0; l < HFX_MAX_CHARGE; ++l) r.rows[l] = rows;
+    hfx_spectra sq = *sp;
+    sq.d_zmax = lvl; /* wide spectra hidden from the items */
+    const uint64_t est = max(total / 12, min(total, 2ull * db->num_pep));
+    const uint32_t CH = hfx_rows_chunk(est, (uint32_t)hfx_ctx_num_cus(ctx));
+    int rc;
+    if ((rc = hfx_rows_split(RW_I8X4, sp, planes, qs, lvl, wide, stream)) ||
+        (rc = hfx_order_spectra(ctx, order, &ob, d_begin, sp->d_zmax, sp->d_mass, S, stream)) ||
+        (rc = hfx_cut_blocks(ctx, 16, &cb, order, d_begin, d_num, sp->d_zmax, S, stream)) ||
+        (rc = hfx_rows_blocks(ctx, RW_I8X4, items, order, cb.bstart, d_begin, d_num, &sq, CH,
+                              stream)) ||
+        (rc = hfx_rows_mark(items, S, flags, nt, stream)) ||
+        (rc = hfx_scan_offsets(ctx, (uint64_t *)r.slots, flags, (uint32_t)nf, stream)) ||
+        (rc = hfx_rows_build(db, &r, flags, stream)) ||
+        (rc = hfx_rows_scores(ctx, RW_I8X4, items, d_scores, d_off, d_begin, d_num, order,
+                              cb.bstart, &r, planes, qs, &sq, CH, sp->d_zmax, stream, nullptr)) ||
+        (rc = hfx_xcorr_wide(ctx, d_scores, d_off, d_begin, d_num, db, sp, wide, stream)))
+        return rc;
+    *taken = 1;
+    return HFX_OK;
+}
+
 extern "C" int hfx_xcorr_sparse(hfx_ctx *ctx, float *d_scores, const uint64_t *d_off,
                                 const uint32_t *d_begin, const uint32_t *d_num, uint64_t total,
                                 const hfx_db *db, const hfx_spectra *sp, void *stream)
@@ -583,7 +666,10 @@ extern "C" int hfx_xcorr_sparse(hfx_ctx *ctx, float *d_scores, const uint64_t *d
                 "hfx_xcorr_sparse: null argument");
     HfxPlainCands c{*db, d_begin, d_num, d_off};
     void *p = nullptr;
-    int rc;
+    int rc, taken = 0;
+    if ((rc = xcorr_rows(ctx, d_scores, d_off, d_begin, d_num, total, db, sp, stream, &taken)) ||
+        taken)
+        return rc;
     if (sp->num_spec &&
         (rc = hfx_ctx_scratch(ctx, HFX_SLOT_TILES, xc_scratch_bytes(sp->num_spec), &p)) != HFX_OK)
         return rc;

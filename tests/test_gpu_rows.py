@@ -103,6 +103,44 @@ def test_batch_rows_match_the_oracle(orc, form, npep, stride):
         assert np.array_equal(bs.results(keep_scores=True).scores, first.scores)
 
 
+def test_sparse_scores_through_rows_and_wide_spectra(orc):
+    """hfx_xcorr_sparse over enough pairs that rows are taken; some spectra hold a value that
+    dwarfs the rest, or one that is not finite, and are scored in FP32 all the same."""
+    from hfx_amd import pipeline as pl
+
+    hdb = database(pl, 100003, seed=5, longest=20)
+    x, lens, zmax, mass = spectra(pl, hdb, 4000, 2112, seed=6)
+    x[7, 40], x[8, 0] = 3e5, -1e6   # 50 x 2^36 within the oracle's 64 bits
+    odd = np.array([100, 101, 102])
+    clean = x.copy()
+    clean[odd] = 0.0
+    ref, exact, scale = reference(orc, hdb, clean, lens, zmax, mass, 5)
+    n = ref["num"]
+    assert n.sum() > 1_000_000
+    x[odd[0], 3], x[odd[1], 4], x[odd[2], 5] = np.inf, -np.inf, np.nan
+    ctx = pl.Ctx(0)
+    db = pl.DeviceDB(hdb)
+    s = pl.PlainSearch(ctx, db, Spectra(pl, x, lens, zmax, mass), eps=3.0, topn=5)
+    s.window()
+    s.score()
+    pl.sync()
+    got = pl.host(s.t_scores, np.float32, s.total).astype(np.float64)
+    keep = ~np.repeat(np.isin(np.arange(len(n)), odd), n)
+    bound = 80 * 2.0**-24 * scale + 1e-6
+    off = np.repeat(np.arange(len(n)), n)[keep & ~(np.abs(got - exact) <= bound)]
+    assert len(off) == 0, np.unique(off)
+    # the plain kernel's own answer for the others, NaN where it has one
+    o = ref["off"].astype(np.int64)
+    for k in odd:
+        one = pl.PlainSearch(ctx, db, Spectra(pl, x[k:k + 1], lens[k:k + 1], zmax[k:k + 1],
+                                              mass[k:k + 1]), eps=3.0, topn=5)
+        one.window()
+        one.score()
+        pl.sync()
+        want = pl.host(one.t_scores, np.float32, one.total)
+        assert np.array_equal(got[o[k]:o[k + 1]].astype(np.float32), want, equal_nan=True)
+
+
 def test_strides_past_the_rows_keep_the_ion_lists(orc):
     from hfx_amd import pipeline as pl
 
