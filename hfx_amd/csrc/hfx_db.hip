@@ -45,29 +45,8 @@ extern "C" void prepare_ions(uint8_t *d_ions, uint32_t N, uint8_t *d_ma, uint32_
 }
 
 /* ------------------------------------------------------------------ */
-/* Stable LSD radix sort of (uint32 key, uint32 value), 4-bit digits.    */
+/* Stable sorts of float keys with uint32 values                         */
 /* ------------------------------------------------------------------ */
-
-#define RS_THREADS 256
-#define RS_ITEMS 8
-#define RS_TILE (RS_THREADS * RS_ITEMS)
-#define RS_BUCKETS 16
-
-__global__ void __launch_bounds__(RS_THREADS) k_rs_upsweep(const uint32_t *keys, uint32_t n,
-                                                          uint32_t shift, uint32_t *hist,
-                                                          uint32_t nb)
-{
-    __shared__ uint32_t cnt[RS_BUCKETS];
-    if (threadIdx.x < RS_BUCKETS) cnt[threadIdx.x] = 0;
-    __syncthreads();
-    uint32_t base = blockIdx.x * RS_TILE;
-    for (uint32_t i = threadIdx.x; i < RS_TILE; i += RS_THREADS) {
-        uint32_t g = base + i;
-        if (g < n) atomicAdd(&cnt[(keys[g] >> shift) & 15u], 1u);
-    }
-    __syncthreads();
-    if (threadIdx.x < RS_BUCKETS) hist[threadIdx.x * nb + blockIdx.x] = cnt[threadIdx.x];
-}
 
 /* Exclusive scan of n uint32 in place by one workgroup of 1024 threads. */
 __global__ void __launch_bounds__(1024) k_scan_u32_inplace(uint32_t *a, uint32_t n)
@@ -98,120 +77,346 @@ __global__ void __launch_bounds__(1024) k_scan_u32_inplace(uint32_t *a, uint32_t
     }
 }
 
-__global__ void __launch_bounds__(RS_THREADS) k_rs_downsweep(const uint32_t *kin, const uint32_t *vin,
-                                                            uint32_t *kout, uint32_t *vout,
-                                                            uint32_t n, uint32_t shift,
-                                                            const uint32_t *hist, uint32_t nb)
-{
-    __shared__ uint32_t cnt[RS_BUCKETS * RS_THREADS];
-    __shared__ uint32_t tsum[RS_THREADS];
-    __shared__ uint32_t dstart[RS_BUCKETS];
-    const uint32_t t = threadIdx.x;
-    const uint32_t base = blockIdx.x * RS_TILE + t * RS_ITEMS;
-    uint32_t k[RS_ITEMS], v[RS_ITEMS];
-#pragma unroll
-    for (int i = 0; i < RS_ITEMS; ++i) {
-        uint32_t g = base + i;
-        k[i] = g < n ? kin[g] : 0;
-        v[i] = g < n ? vin[g] : 0;
-    }
-#pragma unroll
-    for (int d = 0; d < RS_BUCKETS; ++d) cnt[d * RS_THREADS + t] = 0;
-    __syncthreads();
-#pragma unroll
-    for (int i = 0; i < RS_ITEMS; ++i)
-        if (base + i < n) cnt[((k[i] >> shift) & 15u) * RS_THREADS + t] += 1;
-    __syncthreads();
-    /* block exclusive scan over cnt in (digit, thread) order: thread t owns
-     * flat entries [16t, 16t+16) */
-    uint32_t loc[RS_BUCKETS];
-    uint32_t s = 0;
-#pragma unroll
-    for (int j = 0; j < RS_BUCKETS; ++j) {
-        loc[j] = s;
-        s += cnt[t * RS_BUCKETS + j];
-    }
-    tsum[t] = s;
-    __syncthreads();
-    if (t < 64) {
-        /* scan of 256 thread totals by one wave, 4 per lane */
-        uint32_t a0 = tsum[4 * t], a1 = tsum[4 * t + 1], a2 = tsum[4 * t + 2], a3 = tsum[4 * t + 3];
-        uint32_t tot = a0 + a1 + a2 + a3, x = tot;
-#pragma unroll
-        for (int o = 1; o < 64; o <<= 1) {
-            uint32_t y = __shfl_up(x, o, 64);
-            if (t >= (uint32_t)o) x += y;
-        }
-        uint32_t ex = x - tot;
-        tsum[4 * t] = ex;
-        tsum[4 * t + 1] = ex + a0;
-        tsum[4 * t + 2] = ex + a0 + a1;
-        tsum[4 * t + 3] = ex + a0 + a1 + a2;
-    }
-    __syncthreads();
-    uint32_t pre = tsum[t];
-#pragma unroll
-    for (int j = 0; j < RS_BUCKETS; ++j) cnt[t * RS_BUCKETS + j] = pre + loc[j];
-    __syncthreads();
-    if (t < RS_BUCKETS) dstart[t] = cnt[t * RS_THREADS];
-    __syncthreads();
-#pragma unroll
-    for (int i = 0; i < RS_ITEMS; ++i) {
-        if (base + i < n) {
-            uint32_t d = (k[i] >> shift) & 15u;
-            uint32_t lp = cnt[d * RS_THREADS + t]++;
-            uint32_t g = hist[d * nb + blockIdx.x] + (lp - dstart[d]);
-            kout[g] = k[i];
-            vout[g] = v[i];
-        }
-    }
-}
-
-
 /* keys in radix order: ascending float order, or (desc) its reverse --
  * the complement of an order-preserving key reverses the order, and a
  * stable sort of the complements is a stable descending sort */
-__global__ void k_float_to_key(const float *f, uint32_t *k, uint32_t n, uint32_t desc)
+__device__ __forceinline__ uint32_t so_key(float f, uint32_t desc)
 {
-    uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) k[i] = desc ? ~hfx_f2key(f[i]) : hfx_f2key(f[i]);
+    return desc ? ~hfx_f2key(f) : hfx_f2key(f);
 }
-__global__ void k_key_to_float(const uint32_t *k, float *f, uint32_t n, uint32_t desc)
+__device__ __forceinline__ float so_float(uint32_t k, uint32_t desc)
 {
-    uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) f[i] = hfx_key2f(desc ? ~k[i] : k[i]);
-}
-__global__ void k_iota(uint32_t *v, uint32_t n, uint32_t init)
-{
-    uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) v[i] = init + i;
+    return hfx_key2f(desc ? ~k : k);
 }
 
-/* Sorts float keys ascending with values, stably, in place. */
+/* keys among sk[ja .. jb) that come before key k of position i: smaller, or
+ * equal and earlier.  Only the positions of the wave's own 64 keys (from i0 on)
+ * need both tests.  Positions count from sk; i0 and i may lie outside it; ja, jb
+ * and i0 are multiples of 4. */
+__device__ __forceinline__ uint32_t so_before(const uint32_t *sk, int ja, int jb, int i0, int i,
+                                              uint32_t k)
+{
+    uint32_t rk = 0;
+    const uint4 *s4 = (const uint4 *)sk;
+    const int a1 = min(jb, max(ja, i0)), a2 = min(jb, max(ja, i0 + HFX_WAVE));
+    for (int j = ja / 4; j < a1 / 4; ++j) {
+        const uint4 o = s4[j];
+        rk += (o.x <= k ? 1u : 0u) + (o.y <= k ? 1u : 0u) + (o.z <= k ? 1u : 0u) +
+              (o.w <= k ? 1u : 0u);
+    }
+    for (int j = a1 / 4; j < a2 / 4; ++j) {
+        const uint4 o = s4[j];
+        rk += (o.x < k || (o.x == k && 4 * j < i)) ? 1u : 0u;
+        rk += (o.y < k || (o.y == k && 4 * j + 1 < i)) ? 1u : 0u;
+        rk += (o.z < k || (o.z == k && 4 * j + 2 < i)) ? 1u : 0u;
+        rk += (o.w < k || (o.w == k && 4 * j + 3 < i)) ? 1u : 0u;
+    }
+    for (int j = a2 / 4; j < jb / 4; ++j) {
+        const uint4 o = s4[j];
+        rk += (o.x < k ? 1u : 0u) + (o.y < k ? 1u : 0u) + (o.z < k ? 1u : 0u) +
+              (o.w < k ? 1u : 0u);
+    }
+    return rk;
+}
+
+/* Up to SO_ONE keys: one launch of one workgroup, each key's place counted
+ * against all others (key, then position: stable), four keys an LDS read, the
+ * other keys shared out among the waves that a short list leaves over: 7 us
+ * for a few hundred keys, where the radix passes' 28 launches took about 100. */
+#define SO_ONE 1024u
+__global__ void __launch_bounds__(SO_ONE) k_sort_one(float *keys, uint32_t *vals, uint32_t n,
+                                                     uint32_t iota, uint32_t init, uint32_t desc)
+{
+    __shared__ __align__(16) uint32_t sk[SO_ONE];
+    __shared__ uint32_t rank[SO_ONE];
+    const uint32_t t = threadIdx.x;
+    const uint32_t n64 = (n + HFX_WAVE - 1) / HFX_WAVE * HFX_WAVE;
+    uint32_t k = 0xffffffffu, v = 0;
+    if (t < n) {
+        k = so_key(keys[t], desc);
+        v = iota ? init + t : vals[t];
+    }
+    sk[t] = k; /* past the end: no key before another */
+    rank[t] = 0;
+    __syncthreads();
+    const uint32_t parts = SO_ONE / n64, part = t / n64, i = t % n64;
+    if (part < parts) {
+        const uint32_t step = ((n64 + parts - 1) / parts + 3u) & ~3u;
+        const uint32_t ja = min(part * step, n64), jb = min(ja + step, n64);
+        const uint32_t rk = so_before(sk, (int)ja, (int)jb,
+                                      (int)(i & ~(uint32_t)(HFX_WAVE - 1)), (int)i, sk[i]);
+        if (i < n) atomicAdd(&rank[i], rk);
+    }
+    __syncthreads();
+    /* every key and value is in registers: in place */
+    if (t < n) {
+        keys[rank[t]] = so_float(k, desc);
+        vals[rank[t]] = v;
+    }
+}
+
+/* Up to SO_RANK keys: the same count, SO_RT keys a workgroup against all of
+ * them, into scratch, which a second launch copies back.  The count grows with
+ * n^2 and meets the radix passes' twelve launches at about twice this. */
+#define SO_RANK 8192u
+#define SO_RT 256
+__global__ void __launch_bounds__(SO_RT) k_sort_rank(const float *keys, const uint32_t *vals,
+                                                     float *okeys, uint32_t *ovals, uint32_t n,
+                                                     uint32_t iota, uint32_t init, uint32_t desc)
+{
+    __shared__ __align__(16) uint32_t sk[2048];
+    const uint32_t i = blockIdx.x * SO_RT + threadIdx.x;
+    const uint32_t k = i < n ? so_key(keys[i], desc) : 0xffffffffu;
+    uint32_t rk = 0;
+    for (uint32_t b = 0; b < n; b += 2048) {
+        __syncthreads();
+#pragma unroll
+        for (uint32_t u = 0; u < 2048 / SO_RT; ++u) {
+            const uint32_t j = b + u * SO_RT + threadIdx.x;
+            sk[u * SO_RT + threadIdx.x] = j < n ? so_key(keys[j], desc) : 0xffffffffu;
+        }
+        __syncthreads();
+        rk += so_before(sk, 0, (int)((min(n - b, 2048u) + 3u) & ~3u),
+                        (int)(i & ~(uint32_t)(HFX_WAVE - 1)) - (int)b, (int)i - (int)b, k);
+    }
+    if (i < n) {
+        okeys[rk] = so_float(k, desc);
+        ovals[rk] = iota ? init + i : vals[i];
+    }
+}
+__global__ void k_sort_back(const float *k, const uint32_t *v, float *keys, uint32_t *vals,
+                            uint32_t n)
+{
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) {
+        keys[i] = k[i];
+        vals[i] = v[i];
+    }
+}
+
+/* More: stable LSD radix, four passes of eight bits, three launches each:
+ *   k_rs_count   a tile's digit counts, hist[digit][tile];
+ *   k_rs_scan    one workgroup a digit: the exclusive scan of its row, and the
+ *                digit's total;
+ *   k_rs_place   a tile's keys ranked by digit (a wave matches its lanes'
+ *                digits by eight ballots, wave after wave, so equal digits keep
+ *                their order), put in digit order in LDS and written out in
+ *                runs.
+ * The first pass reads the caller's keys, the last writes them back, so that
+ * no conversion or copy pass is left: 2.7 M keys move 44 MB a pass.  Four bits
+ * a pass, a single-workgroup scan and separate conversions took 560 us for
+ * them. */
+#define RS_THREADS 512
+#define RS_WAVES (RS_THREADS / HFX_WAVE)
+#define RS_ITEMS 8
+#define RS_TILE (RS_THREADS * RS_ITEMS)
+#define RS_BUCKETS 256
+
+struct RsArgs {
+    const void *kin;        /* float keys in the first pass, radix keys after */
+    const uint32_t *vin;    /* null in the first pass of an index sort */
+    void *kout;             /* float keys in the last pass */
+    uint32_t *vout;
+    uint32_t n, shift, nb, first, last, desc, init;
+    uint32_t *hist;         /* [RS_BUCKETS][nb] */
+    uint32_t *tot;          /* [RS_BUCKETS] */
+};
+
+__device__ __forceinline__ uint32_t rs_load(const RsArgs &a, uint32_t g)
+{
+    return a.first ? so_key(((const float *)a.kin)[g], a.desc) : ((const uint32_t *)a.kin)[g];
+}
+
+__global__ void __launch_bounds__(RS_THREADS) k_rs_count(RsArgs a)
+{
+    __shared__ uint32_t cnt[RS_BUCKETS];
+    if (threadIdx.x < RS_BUCKETS) cnt[threadIdx.x] = 0;
+    __syncthreads();
+    const uint64_t base = (uint64_t)blockIdx.x * RS_TILE;
+    uint32_t k[RS_ITEMS];
+#pragma unroll
+    for (uint32_t i = 0; i < RS_ITEMS; ++i) {
+        const uint64_t g = base + i * RS_THREADS + threadIdx.x;
+        k[i] = g < a.n ? rs_load(a, (uint32_t)g) : 0u;
+    }
+#pragma unroll
+    for (uint32_t i = 0; i < RS_ITEMS; ++i)
+        if (base + i * RS_THREADS + threadIdx.x < a.n)
+            atomicAdd(&cnt[(k[i] >> a.shift) & 255u], 1u);
+    __syncthreads();
+    if (threadIdx.x < RS_BUCKETS)
+        a.hist[(size_t)threadIdx.x * a.nb + blockIdx.x] = cnt[threadIdx.x];
+}
+
+__global__ void __launch_bounds__(256) k_rs_scan(RsArgs a)
+{
+    __shared__ uint32_t part[4];
+    uint32_t *row = a.hist + (size_t)blockIdx.x * a.nb;
+    const uint32_t lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+    uint32_t carry = 0;
+    for (uint32_t b = 0; b < a.nb; b += 256) {
+        const uint32_t i = b + threadIdx.x;
+        const uint32_t v = i < a.nb ? row[i] : 0u;
+        uint32_t x = v;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const uint32_t y = __shfl_up(x, o, 64);
+            if (lane >= (uint32_t)o) x += y;
+        }
+        if (lane == 63) part[wid] = x;
+        __syncthreads();
+        uint32_t pre = carry, all = 0;
+        for (uint32_t w = 0; w < 4; ++w) {
+            if (w < wid) pre += part[w];
+            all += part[w];
+        }
+        if (i < a.nb) row[i] = pre + x - v;
+        carry += all;
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) a.tot[blockIdx.x] = carry;
+}
+
+__global__ void __launch_bounds__(RS_THREADS) k_rs_place(RsArgs a)
+{
+    __shared__ uint32_t wcnt[RS_WAVES][RS_BUCKETS]; /* then: each wave's base in the tile */
+    __shared__ uint32_t dbase[RS_BUCKETS];          /* a digit's first place in the tile */
+    __shared__ uint32_t gbase[RS_BUCKETS];          /* in the output, less dbase */
+    __shared__ uint32_t p1[RS_BUCKETS / HFX_WAVE], p2[RS_BUCKETS / HFX_WAVE];
+    __shared__ uint32_t sk[RS_TILE], sv[RS_TILE];
+    const uint32_t t = threadIdx.x, lane = hfx_lane(), w = t / HFX_WAVE;
+    const uint64_t base = (uint64_t)blockIdx.x * RS_TILE;
+    const uint32_t cnt = (uint32_t)min((uint64_t)RS_TILE, a.n - base);
+    for (uint32_t i = t; i < RS_WAVES * RS_BUCKETS; i += RS_THREADS) (&wcnt[0][0])[i] = 0;
+    /* wave w takes items w * 512 + 64 i + lane: in order over i, then lanes */
+    uint32_t k[RS_ITEMS], v[RS_ITEMS], rank[RS_ITEMS];
+#pragma unroll
+    for (uint32_t i = 0; i < RS_ITEMS; ++i) {
+        const uint32_t e = w * (HFX_WAVE * RS_ITEMS) + i * HFX_WAVE + lane;
+        k[i] = 0;
+        v[i] = 0;
+        if (e < cnt) {
+            const uint32_t g = (uint32_t)base + e;
+            k[i] = rs_load(a, g);
+            v[i] = a.vin ? a.vin[g] : a.init + g;
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (uint32_t i = 0; i < RS_ITEMS; ++i) {
+        const uint32_t e = w * (HFX_WAVE * RS_ITEMS) + i * HFX_WAVE + lane;
+        const uint32_t d = (k[i] >> a.shift) & 255u;
+        uint64_t same = __ballot(e < cnt);
+#pragma unroll
+        for (uint32_t b = 0; b < 8; ++b) {
+            const uint64_t one = __ballot((d >> b) & 1u);
+            same &= (d >> b) & 1u ? one : ~one;
+        }
+        /* the lanes of a digit count in lane order behind the wave's earlier
+         * items; the first of them moves the counter on */
+        const uint32_t before = (uint32_t)__builtin_popcountll(same & ((1ull << lane) - 1ull));
+        uint32_t seen = 0;
+        if (e < cnt) seen = wcnt[w][d];
+        hfx_wave_sync();
+        if (e < cnt && before == 0) wcnt[w][d] = seen + (uint32_t)__builtin_popcountll(same);
+        hfx_wave_sync();
+        rank[i] = seen + before;
+    }
+    __syncthreads();
+    uint32_t ex = 0, ey = 0;
+    if (t < RS_BUCKETS) {
+        uint32_t sum = 0;
+#pragma unroll
+        for (uint32_t q = 0; q < RS_WAVES; ++q) {
+            const uint32_t c = wcnt[q][t];
+            wcnt[q][t] = sum;
+            sum += c;
+        }
+        /* exclusive scans over the digits: the tile's counts and the totals */
+        const uint32_t tt = a.tot[t];
+        uint32_t x = sum, y = tt;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const uint32_t p = __shfl_up(x, o, 64), q = __shfl_up(y, o, 64);
+            if (lane >= (uint32_t)o) {
+                x += p;
+                y += q;
+            }
+        }
+        if (lane == 63) {
+            p1[w] = x;
+            p2[w] = y;
+        }
+        ex = x - sum;
+        ey = y - tt;
+    }
+    __syncthreads();
+    if (t < RS_BUCKETS) {
+        for (uint32_t q = 0; q < w; ++q) {
+            ex += p1[q];
+            ey += p2[q];
+        }
+        dbase[t] = ex;
+        gbase[t] = ey + a.hist[(size_t)t * a.nb + blockIdx.x] - ex;
+    }
+    __syncthreads();
+#pragma unroll
+    for (uint32_t i = 0; i < RS_ITEMS; ++i) {
+        if (w * (HFX_WAVE * RS_ITEMS) + i * HFX_WAVE + lane < cnt) {
+            const uint32_t d = (k[i] >> a.shift) & 255u;
+            const uint32_t at = dbase[d] + wcnt[w][d] + rank[i];
+            sk[at] = k[i];
+            sv[at] = v[i];
+        }
+    }
+    __syncthreads();
+    for (uint32_t j = t; j < cnt; j += RS_THREADS) {
+        const uint32_t kk = sk[j];
+        const uint32_t g = gbase[(kk >> a.shift) & 255u] + j;
+        if (a.last) ((float *)a.kout)[g] = so_float(kk, a.desc);
+        else ((uint32_t *)a.kout)[g] = kk;
+        a.vout[g] = sv[j];
+    }
+}
+
+/* Sorts float keys ascending (or descending) with values, stably, in place. */
 static int radix_sort_f32(hfx_ctx *ctx, float *d_keys, uint32_t *d_vals, uint32_t n, bool iota,
                           uint32_t init, hipStream_t st, uint32_t desc = 0)
 {
     if (n == 0) return HFX_OK;
-    uint32_t nb = (n + RS_TILE - 1) / RS_TILE;
+    if (n <= SO_ONE) {
+        hipLaunchKernelGGL(k_sort_one, dim3(1), dim3(SO_ONE), 0, st, d_keys, d_vals, n,
+                           (uint32_t)iota, init, desc);
+        HFX_CHECK_LAUNCH();
+        return HFX_OK;
+    }
+    const uint32_t nb = (uint32_t)(((uint64_t)n + RS_TILE - 1) / RS_TILE);
     void *p;
     int rc;
-    if ((rc = hfx_ctx_scratch(ctx, HFX_SLOT_SORT, (size_t)n * 16 + (size_t)nb * RS_BUCKETS * 4, &p)) != HFX_OK)
+    if ((rc = hfx_ctx_scratch(ctx, HFX_SLOT_SORT,
+                              (size_t)n * 16 + ((size_t)nb + 1) * RS_BUCKETS * 4, &p)) != HFX_OK)
         return rc;
     uint32_t *ka = (uint32_t *)p, *va = ka + n, *kb = va + n, *vb = kb + n, *hist = vb + n;
-    uint32_t g = (n + 255) / 256;
-    hipLaunchKernelGGL(k_float_to_key, dim3(g), dim3(256), 0, st, d_keys, ka, n, desc);
-    if (iota) hipLaunchKernelGGL(k_iota, dim3(g), dim3(256), 0, st, va, n, init);
-    else HFX_CHECK_HIP(hipMemcpyAsync(va, d_vals, (size_t)n * 4, hipMemcpyDeviceToDevice, st));
-    for (uint32_t shift = 0; shift < 32; shift += 4) {
-        hipLaunchKernelGGL(k_rs_upsweep, dim3(nb), dim3(RS_THREADS), 0, st, ka, n, shift, hist, nb);
-        hipLaunchKernelGGL(k_scan_u32_inplace, dim3(1), dim3(1024), 0, st, hist, nb * RS_BUCKETS);
-        hipLaunchKernelGGL(k_rs_downsweep, dim3(nb), dim3(RS_THREADS), 0, st, ka, va, kb, vb, n,
-                           shift, hist, nb);
-        uint32_t *t = ka; ka = kb; kb = t;
-        t = va; va = vb; vb = t;
+    if (n <= SO_RANK) {
+        hipLaunchKernelGGL(k_sort_rank, dim3((n + SO_RT - 1) / SO_RT), dim3(SO_RT), 0, st, d_keys,
+                           d_vals, (float *)ka, va, n, (uint32_t)iota, init, desc);
+        hipLaunchKernelGGL(k_sort_back, dim3((n + 255) / 256), dim3(256), 0, st, (float *)ka, va,
+                           d_keys, d_vals, n);
+        HFX_CHECK_LAUNCH();
+        return HFX_OK;
     }
-    hipLaunchKernelGGL(k_key_to_float, dim3(g), dim3(256), 0, st, ka, d_keys, n, desc);
-    HFX_CHECK_HIP(hipMemcpyAsync(d_vals, va, (size_t)n * 4, hipMemcpyDeviceToDevice, st));
+    /* caller -> a -> b -> a -> caller */
+    const void *ks[4] = {d_keys, ka, kb, ka};
+    const uint32_t *vs[4] = {iota ? nullptr : d_vals, va, vb, va};
+    void *kd[4] = {ka, kb, ka, d_keys};
+    uint32_t *vd[4] = {va, vb, va, d_vals};
+    for (uint32_t q = 0; q < 4; ++q) {
+        const RsArgs a{ks[q],   vs[q], kd[q], vd[q], n,    8 * q, nb, q == 0, q == 3, desc,
+                       init,    hist,  hist + (size_t)nb * RS_BUCKETS};
+        hipLaunchKernelGGL(k_rs_count, dim3(nb), dim3(RS_THREADS), 0, st, a);
+        hipLaunchKernelGGL(k_rs_scan, dim3(RS_BUCKETS), dim3(256), 0, st, a);
+        hipLaunchKernelGGL(k_rs_place, dim3(nb), dim3(RS_THREADS), 0, st, a);
+    }
     HFX_CHECK_LAUNCH();
     return HFX_OK;
 }

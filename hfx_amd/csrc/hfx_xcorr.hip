@@ -754,19 +754,25 @@ extern "C" int hfx_xcorr_sparse_noalloc(float *d_scores, const uint64_t *d_off,
 /* ------------------------------------------------------------------ */
 
 /* One wave per row: map -> dense row of floats 0/10/25/50, every element
- * written (no memset needed, no cross-block race). */
+ * written (no memset needed, no cross-block race).  Lanes take consecutive
+ * bins, eight of them reading one map word, so that a store is 256 contiguous
+ * bytes (a map word a lane made eight stores of 64 separate sectors). */
 __device__ __forceinline__ void wave_map_to_row(uint32_t *map, float *row, uint32_t len)
 {
-    const uint32_t nw = (len + 7) >> 3;
-    for (uint32_t w = hfx_lane(); w < nw; w += HFX_WAVE) {
-        uint32_t word = map[w];
-        map[w] = 0;
+    const uint32_t lane = hfx_lane(), nw = (len + 7) >> 3;
+    constexpr uint32_t U = 8; /* map words read ahead of the stores */
+    for (uint32_t b0 = lane; b0 < len; b0 += U * HFX_WAVE) {
+        uint32_t w[U];
 #pragma unroll
-        for (uint32_t k = 0; k < 8; ++k) {
-            uint32_t b = (w << 3) + k;
-            if (b < len) row[b] = hfx_code_weight((word >> (4 * k)) & 0xFu);
+        for (uint32_t u = 0; u < U; ++u) w[u] = map[min(b0 + u * HFX_WAVE, len - 1u) >> 3];
+#pragma unroll
+        for (uint32_t u = 0; u < U; ++u) {
+            const uint32_t b = b0 + u * HFX_WAVE;
+            if (b < len) row[b] = hfx_code_weight((w[u] >> (4 * (b & 7u))) & 0xFu);
         }
     }
+    hfx_wave_sync();
+    for (uint32_t w = lane; w < nw; w += HFX_WAVE) map[w] = 0;
 }
 
 __global__ void __launch_bounds__(XC_THREADS)
@@ -817,6 +823,9 @@ extern "C" void addIons(float *d_spec, const float *d_residual, const float *d_m
 /* Row MVM replacing cuBLAS sgemv(T)                                    */
 /* ------------------------------------------------------------------ */
 
+/* A wave a row; a lane's products j = lane, lane + 64, ... are added in that
+ * order, eight of its loads in flight at a time (one after the other, 366 rows
+ * of 1,400 took 10.7 us: too few waves to hide the loads' latency). */
 __global__ void __launch_bounds__(256) k_mvm_rows(float *y, const float *A, uint32_t lda,
                                                   const float *x, uint32_t m, uint32_t n)
 {
@@ -824,7 +833,31 @@ __global__ void __launch_bounds__(256) k_mvm_rows(float *y, const float *A, uint
     if (row >= m) return;
     const float *a = A + (size_t)row * lda;
     float acc = 0.0f;
-    for (uint32_t j = hfx_lane(); j < n; j += HFX_WAVE) acc = acc + a[j] * x[j];
+    constexpr uint32_t U = 8;
+    uint32_t j = hfx_lane();
+    for (; j + (U - 1) * HFX_WAVE < n; j += U * HFX_WAVE) {
+        float av[U], xv[U];
+#pragma unroll
+        for (uint32_t u = 0; u < U; ++u) {
+            av[u] = a[j + u * HFX_WAVE];
+            xv[u] = x[j + u * HFX_WAVE];
+        }
+#pragma unroll
+        for (uint32_t u = 0; u < U; ++u) acc = acc + av[u] * xv[u];
+    }
+    /* the rest, clamped into the row; products past its end not added */
+    if (j < n) {
+        float av[U], xv[U];
+#pragma unroll
+        for (uint32_t u = 0; u < U; ++u) {
+            const uint32_t q = min(j + u * HFX_WAVE, n - 1u);
+            av[u] = a[q];
+            xv[u] = x[q];
+        }
+#pragma unroll
+        for (uint32_t u = 0; u < U; ++u)
+            if (j + u * HFX_WAVE < n) acc = acc + av[u] * xv[u];
+    }
     acc = hfx_wave_sum_f32(acc);
     if (hfx_lane() == 0) y[row] = acc;
 }
