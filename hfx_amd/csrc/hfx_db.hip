@@ -203,9 +203,8 @@ __global__ void k_sort_back(const float *k, const uint32_t *v, float *keys, uint
  *                their order), put in digit order in LDS and written out in
  *                runs.
  * The first pass reads the caller's keys, the last writes them back, so that
- * no conversion or copy pass is left: 2.7 M keys move 44 MB a pass.  Four bits
- * a pass, a single-workgroup scan and separate conversions took 560 us for
- * them. */
+ * no conversion or copy pass is left: 2.7 M keys take 130 us, against 560 us
+ * with four bits a pass, a single-workgroup scan and separate conversions. */
 #define RS_THREADS 512
 #define RS_WAVES (RS_THREADS / HFX_WAVE)
 #define RS_ITEMS 8

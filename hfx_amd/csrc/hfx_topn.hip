@@ -6,31 +6,39 @@
  * final order is descending score, ties by ascending candidate position
  * (stable ascending sort, then reverse twice: Search.hs:119-123, :276).
  *
- * Here one workgroup per spectrum:
- *   1. selects the T = min(N + margin, n) best FP32 scores (key desc,
- *      position asc): for T <= TN_LT in one sweep, each thread keeping its
- *      TN_LT best in registers and the waves merging them; otherwise by a
- *      radix select;
- *   2. takes the N-th best FP32 score fN and collects every other candidate
- *      whose FP32 score is >= fN - 2B (B bounds |FP32 - exact|): the N-th
- *      best exact score exN is >= fN - B, so no candidate left out can reach
- *      the top N;
- *   3. re-scores the selection and that band exactly, in one round: int64
- *      fixed point, sum of round(w*x*2^36), independent of summation order,
- *      so the GPU and the CPU oracle agree bit for bit;
- *   4. orders the re-scored set by (exact desc, position asc), writes the best
- *      N.  If the band holds more than TN_EXT candidates, the spectrum is
- *      flagged and the exact route scores every candidate at or above
- *      exN - B exactly.
+ * Here, in three launches:
+ *   1. k_topn_select, one workgroup per spectrum: the T = min(N + margin, n)
+ *      best FP32 scores (key desc, position asc), and every other candidate
+ *      whose FP32 score is >= fN - 2B, fN being the N-th best FP32 score (B
+ *      bounds |FP32 - exact|): the N-th best exact score exN is >= fN - B, so no
+ *      candidate left out can reach the top N;
+ *   2. k_topn_exact, one wave per spectrum (long lists shared out among all
+ *      waves): the exact scores of those candidates, several a wave: int64
+ *      fixed point, sum of round(w*x*2^36), independent of summation order, so
+ *      the GPU and the CPU oracle agree bit for bit;
+ *   3. k_topn_rank, one wave per spectrum: the re-scored candidates by (exact
+ *      desc, position asc), the best N written.
+ * If the band holds more than TN_EXT candidates, the spectrum is flagged and
+ * the exact route scores every candidate at or above exN - B exactly.
  * Bound: |score - exact| <= (rel0 + rel1 * z) * 50 * sum_b |x_b|
  *                           + relq * max_b |x_b| * 50 * len + 1e-6, with
  * z the spectrum's fragment charge count and sum|w*x| <= 50 * sum_b |x_b|
  * (each bin counts once, weights <= 50).  The sparse FP32 scores use
  * rel0 = 80 * 2^-24 (<= 71 roundings per score), rel1 = 0; the dense BF16
  * scores pass their own (split error + one rounding per non-zero bin).
+ *
+ * One workgroup per spectrum did all three, a wave per candidate: half of its
+ * time went to exact scores with a quarter of the lanes busy, and a spectrum
+ * with 200 tied candidates held up a small batch by itself.
+ * Now, select + exact + rank: 10,000 spectra, 1120 candidates each, top 10:
+ * 127 + 136 + 15 us, against 445 us; 20,000 spectra, top 5: 179 + 148 + 15 us,
+ * against 430; 250 spectra: 14 + 39 + 8 us, against 171.  The selection reads
+ * the scores and the spectra once (86 + 44 MB in 179 us here: the collection's
+ * ballots take the rest); the exact scores are bound by their FP64 terms and
+ * the maps' LDS atomics.
  */
 #define HFX_TOPN_REL_F32 (80.0f * 5.9604644775390625e-08f)
-#include "hfx_cand.h"
+#include "hfx_pack.h"
 
 #define TN_THREADS 256
 #define TN_WAVES (TN_THREADS / HFX_WAVE)
@@ -38,29 +46,21 @@
 #define TN_EXT 256
 #define TN_MAXC (TN_MAXT + TN_EXT)
 
-/* T at most this: the selection keeps per-thread lists in registers */
-#define TN_LT 6
+/* T at most this: a threshold from the lanes' largest scores, then one
+ * collection; above, a radix select */
+#define TN_LT 32
+/* scores a thread keeps in registers between its two looks at them: windows of
+ * up to 6144 candidates are read once */
+#define TN_HOLD 24
 
 /* the first select pass histograms the key's 11 high bits */
 #define TN_HBITS 11
 #define TN_HBINS (1u << TN_HBITS)
 
-/* The staged spectrum and the waves' maps live in dynamic LDS sized by the
- * spectra's row stride: bins of a row, rounded up to whole map words.  The
- * spectrum's region is at least TN_HBINS words: before the spectrum is
- * staged it holds the select's histogram. */
-__host__ __device__ inline uint32_t tn_xcap(uint32_t x_stride)
-{
-    return ((x_stride < HFX_MAX_LEN ? x_stride : HFX_MAX_LEN) + 7u) & ~7u;
-}
-__host__ __device__ inline size_t tn_xs_bytes(uint32_t x_stride)
-{
-    return (size_t)(tn_xcap(x_stride) > TN_HBINS ? tn_xcap(x_stride) : TN_HBINS) * 4;
-}
-__host__ __device__ inline size_t tn_dyn_bytes(uint32_t x_stride)
-{
-    return tn_xs_bytes(x_stride) + (size_t)TN_WAVES * (tn_xcap(x_stride) / 8) * 4;
-}
+/* candidates of a spectrum that its own wave re-scores; the rest of a longer
+ * list goes out in tasks of as many */
+#define TN_TASK 16
+#define TN_SPILL ((TN_MAXC - TN_TASK + TN_TASK - 1) / TN_TASK)
 
 __device__ __forceinline__ bool before_fx(int64_t fa, uint32_t pa, int64_t fb, uint32_t pb)
 {
@@ -107,17 +107,40 @@ __device__ __forceinline__ void tn_select_digit(const uint32_t *hist, uint32_t n
     __syncthreads();
 }
 
-/* the largest of the wave's 64-bit values, in every lane */
-__device__ __forceinline__ uint64_t tn_wave_max_u64(uint64_t v)
+/* The `want` first of a wave's candidates in order of (key desc, position asc):
+ * R a lane, key 0 for none.  want rounds of a wave-wide best; emit(r, key, pos)
+ * in every lane.  A few rounds where counting every candidate's place compares
+ * them all: 25 us for 261 of them. */
+template <int R, class Emit>
+__device__ __forceinline__ void tn_wave_top(uint64_t (&k)[R], uint32_t (&p)[R], uint32_t want,
+                                            Emit &&emit)
 {
+    for (uint32_t r = 0; r < want; ++r) {
+        uint64_t bk = k[0];
+        uint32_t bp = p[0];
 #pragma unroll
-    for (uint32_t o = 1; o < HFX_WAVE; o <<= 1) {
-        const uint32_t lo = __shfl_xor((uint32_t)v, o, 64);
-        const uint32_t hi = __shfl_xor((uint32_t)(v >> 32), o, 64);
-        const uint64_t y = (uint64_t)hi << 32 | lo;
-        v = y > v ? y : v;
+        for (int i = 1; i < R; ++i) {
+            const bool c = k[i] > bk || (k[i] == bk && p[i] < bp);
+            bk = c ? k[i] : bk;
+            bp = c ? p[i] : bp;
+        }
+#pragma unroll
+        for (uint32_t o = 1; o < HFX_WAVE; o <<= 1) {
+            const uint64_t ok = (uint64_t)(uint32_t)__shfl_xor((int)(uint32_t)(bk >> 32), o, 64) << 32 |
+                                (uint32_t)__shfl_xor((int)(uint32_t)bk, o, 64);
+            const uint32_t op = (uint32_t)__shfl_xor((int)bp, o, 64);
+            const bool c = ok > bk || (ok == bk && op < bp);
+            bk = c ? ok : bk;
+            bp = c ? op : bp;
+        }
+        emit(r, bk, bp);
+#pragma unroll
+        for (int i = 0; i < R; ++i)
+            if (k[i] == bk && p[i] == bp) {
+                k[i] = 0;
+                p[i] = 0xffffffffu;
+            }
     }
-    return v;
 }
 
 /* Histogram increment of digit d for the active lanes of a wave: lanes that
@@ -138,74 +161,50 @@ __device__ __forceinline__ void tn_hist_add(uint32_t *hist, uint32_t d, bool act
     if ((m >> lane) & 1ull) atomicAdd(&hist[d], 1u);
 }
 
-/* Launch order of k_topn: spectra by window size, largest first, in classes
- * of 256 candidates (any order inside a class).  A workgroup's time grows
- * with its window; started first, the long ones no longer finish last. */
-#define TN_OCLS 64
-#define TN_OTHREADS 1024
-template <class Cands>
-__global__ void __launch_bounds__(TN_OTHREADS) k_topn_order(uint32_t *order, Cands c, uint32_t S)
-{
-    __shared__ uint32_t cnt[TN_OCLS];
-    const uint32_t tid = threadIdx.x;
-    auto cls = [&](uint32_t s) -> uint32_t {
-        return TN_OCLS - 1u - min(c.count(s) >> 8, TN_OCLS - 1u);
-    };
-    if (tid < TN_OCLS) cnt[tid] = 0;
-    static_assert(TN_OCLS <= TN_OTHREADS, "one thread clears each class counter");
-    __syncthreads();
-    for (uint32_t s = tid; s < S; s += TN_OTHREADS) atomicAdd(&cnt[cls(s)], 1u);
-    __syncthreads();
-    if (tid == 0)
-        for (uint32_t k = 0, a = 0; k < TN_OCLS; ++k) {
-            const uint32_t v = cnt[k];
-            cnt[k] = a;
-            a += v;
-        }
-    __syncthreads();
-    for (uint32_t s = tid; s < S; s += TN_OTHREADS) order[atomicAdd(&cnt[cls(s)], 1u)] = s;
-}
+#define TN_BIG 0x80000000u /* in mcnt: terms may pass 2^50 */
+/* sixteen bytes at any multiple of four */
+typedef float tn_f4 __attribute__((ext_vector_type(4), aligned(4)));
+
+/* exact-route and candidate scratch of a call, see tx_carve */
+struct TnLists {
+    uint32_t *cand;  /* [S][TN_MAXC] positions: the T selected, then the band */
+    uint32_t *mcnt;  /* [S] their number, and TN_BIG */
+    uint2 *spill;    /* [S * TN_SPILL] (spectrum, first candidate) */
+    uint32_t *nspill;
+    double *tau;     /* [S] the bound, then the exact route's threshold */
+    uint32_t *band;  /* [S] band size of flagged spectra */
+};
 
 template <class Cands>
 __global__ void __launch_bounds__(TN_THREADS)
-    k_topn(uint32_t *top_pos, double *top_exact, float *top_f32, uint32_t *top_cnt,
-           uint32_t *flag, uint32_t N, uint32_t margin, const float *scores, Cands c,
-           hfx_spectra sp, float rel0, float rel1, float relq, double *tau_out,
-           uint32_t *band_out,
-           const uint32_t *order)
+    k_topn_select(TnLists o, uint32_t *flag, uint32_t N, uint32_t margin, const float *scores,
+                  Cands c, hfx_spectra sp, float rel0, float rel1, float relq)
 {
-    extern __shared__ __align__(16) unsigned char tn_dyn[];
-    const uint32_t xcap = tn_xcap(sp.x_stride), mwords = xcap / 8;
-    float *xs = (float *)tn_dyn;
-    uint32_t *hist = (uint32_t *)tn_dyn; /* until the spectrum is staged */
-    uint32_t *maps = (uint32_t *)(tn_dyn + tn_xs_bytes(sp.x_stride));
-    __shared__ float mtab[32];
+    __shared__ uint32_t hist[TN_HBINS];
+    __shared__ uint64_t kv[TN_MAXC]; /* (key, ~position) */
     __shared__ uint32_t cp[TN_MAXC];
-    __shared__ int64_t cfx[TN_MAXC];
-    __shared__ float cf32[TN_MAXC];
-    __shared__ uint32_t wcnt[TN_WAVES];
+    __shared__ uint32_t wcnt[TN_WAVES], sh_low[TN_WAVES];
     __shared__ float sh_x1[TN_WAVES], sh_xm[TN_WAVES];
-    __shared__ uint32_t sh_digit, sh_rem, sh_gt, sh_last, sh_ext, sh_wide;
-    __shared__ uint64_t sh_wtop[TN_WAVES * TN_LT];
+    __shared__ uint32_t sh_digit, sh_rem, sh_gt, sh_last, sh_ext, sh_cnt, sh_task;
     __shared__ float sh_fN;
 
-    const uint32_t s = order[blockIdx.x], tid = threadIdx.x, wave = tid / HFX_WAVE;
+    const uint32_t s = blockIdx.x, tid = threadIdx.x, wave = tid / HFX_WAVE;
     const uint32_t lane = hfx_lane();
     const uint32_t n = c.count(s);
     const float *sc = scores + c.base(s);
     if (n == 0) {
         if (tid == 0) {
-            top_cnt[s] = 0;
+            o.mcnt[s] = 0;
             flag[s] = 0;
         }
         return;
     }
     const uint32_t T = min(N + margin, n);
 
-    /* every sweep below visits this thread's keys through for_keys(f), f(i,
-     * key), eight loads in flight at a time (clamped into the window, so
-     * that none is conditional); i >= n past the window, where all lanes of
-     * a wave still take part (for the ballots) */
+    /* every sweep over memory visits this thread's keys through for_keys(f),
+     * f(i, key), eight loads in flight at a time (clamped into the window, so
+     * that none is conditional); i >= n past the window, where all lanes of a
+     * wave still take part (for the ballots) */
     auto for_keys = [&](auto &&f) {
         constexpr uint32_t U = 8;
         for (uint32_t base = 0; base < n; base += U * TN_THREADS) {
@@ -217,222 +216,279 @@ __global__ void __launch_bounds__(TN_THREADS)
             for (uint32_t u = 0; u < U; ++u) f(base + u * TN_THREADS + tid, kk[u]);
         }
     };
-
-    /* 1. the T largest keys (key desc, position asc).  Radix select, first
-     * over the key's 11 high bits (sign, exponent, two mantissa bits: a
-     * quarter octave a bucket), then 8, 8 and 5 bits; after each pass, once
-     * the keys at or above the prefix found so far -- M of them, known from
-     * the histograms -- number at most TN_MAXC, they are collected and ranked
-     * exactly.  Otherwise (long runs of near-equal scores) the full threshold
-     * key K is found and the keys above it, then the smallest positions
-     * equal to it, are collected. */
-    uint32_t prefix = 0, pmask = 0;
     if (tid == 0) {
         sh_rem = T;
         sh_gt = 0;
         sh_ext = 0;
         sh_last = 0;
-        sh_wide = 0;
-    }
-    /* T <= TN_LT: one sweep instead.  Each thread keeps its TN_LT best
-     * (key, ~position) values in registers, sorted; the waves merge them.
-     * Anything a thread left out ranks below its TN_LT-th value, which the
-     * band step uses to take the band from the lists. */
-    const bool local = T <= TN_LT;
-    uint64_t lst[TN_LT];
-#pragma unroll
-    for (uint32_t j = 0; j < TN_LT; ++j) lst[j] = 0; /* 0: empty (no score has key 0 with position ~0) */
-    bool ranked = false;
-    if (local) {
-        for_keys([&](uint32_t i, uint32_t k) {
-            uint64_t x = i < n ? (uint64_t)k << 32 | (0xffffffffu - i) : 0ull;
-            if (x > lst[TN_LT - 1]) {
-#pragma unroll
-                for (uint32_t j = 0; j < TN_LT; ++j) {
-                    const uint64_t a = lst[j];
-                    lst[j] = x > a ? x : a;
-                    x = x > a ? a : x;
-                }
-            }
-        });
-        /* the wave's T best: T rounds of a wave max over the lists' heads */
-        uint32_t h = 0;
-        for (uint32_t r = 0; r < T; ++r) {
-            uint64_t hv = 0;
-#pragma unroll
-            for (uint32_t j = 0; j < TN_LT; ++j) hv = h == j ? lst[j] : hv;
-            const uint64_t m = tn_wave_max_u64(hv);
-            if (m != 0 && hv == m) ++h;
-            if (lane == 0) sh_wtop[wave * TN_LT + r] = m;
-        }
-        __syncthreads();
-        /* the T best of the waves' 4T, ranked exactly */
-        if (tid < TN_WAVES * T) {
-            const uint64_t v = sh_wtop[(tid / T) * TN_LT + tid % T];
-            uint32_t rk = 0;
-            for (uint32_t b = 0; b < TN_WAVES * T; ++b)
-                rk += sh_wtop[(b / T) * TN_LT + b % T] > v ? 1u : 0u;
-            if (v != 0 && rk < T) {
-                const uint32_t pa = 0xffffffffu - (uint32_t)v;
-                cp[rk] = pa;
-                if (rk == N - 1u) sh_fN = hfx_key2f((uint32_t)(v >> 32));
-                if (rk == T - 1u) {
-                    sh_digit = (uint32_t)(v >> 32);
-                    sh_last = pa;
-                }
-            }
-        }
-        __syncthreads();
-        ranked = true;
-    }
-    for (int pass = 0; pass < 4 && !local; ++pass) {
-        const uint32_t shift = pass == 0 ? 32u - TN_HBITS : pass == 1 ? 13u : pass == 2 ? 5u : 0u;
-        const uint32_t nb = pass == 0 ? TN_HBINS : pass == 3 ? 32u : 256u;
-        for (uint32_t b = tid; b < nb; b += TN_THREADS) hist[b] = 0;
-        __syncthreads();
-        for_keys([&](uint32_t i, uint32_t k) {
-            tn_hist_add(hist, (k >> shift) & (nb - 1u), i < n && (k & pmask) == prefix);
-        });
-        __syncthreads();
-        tn_select_digit(hist, nb, &sh_digit, &sh_rem);
-        prefix |= sh_digit << shift;
-        pmask |= (nb - 1u) << shift;
-        const uint32_t M = T - sh_rem + hist[sh_digit];
-        __syncthreads(); /* every thread has read hist before it is cleared */
-        if (M <= TN_MAXC) {
-            /* (key, ~position) packed so that a larger value ranks first;
-             * cfx holds them until the exact scores replace them */
-            uint64_t *kv = (uint64_t *)cfx;
-            for_keys([&](uint32_t i, uint32_t k) {
-                if (i < n && (k & pmask) >= prefix)
-                    kv[atomicAdd(&sh_gt, 1u)] = (uint64_t)k << 32 | (0xffffffffu - i);
-            });
-            __syncthreads();
-            for (uint32_t a = tid; a < M; a += TN_THREADS) {
-                const uint64_t va = kv[a];
-                uint32_t rk = 0;
-                for (uint32_t b = 0; b < M; ++b) rk += kv[b] > va ? 1u : 0u;
-                const uint32_t pa = 0xffffffffu - (uint32_t)va;
-                if (rk < T) cp[rk] = pa;
-                if (rk == T - 1u) {
-                    sh_digit = (uint32_t)(va >> 32);
-                    sh_last = pa;
-                }
-            }
-            __syncthreads();
-            ranked = true;
-            break;
-        }
-    }
-    const uint32_t K = ranked ? sh_digit : prefix;
-    if (!ranked) {
-        const uint32_t need_eq = sh_rem; /* >= 1 */
-        const uint32_t n_gt = T - need_eq;
-        for_keys([&](uint32_t i, uint32_t k) {
-            if (i < n && k > K) {
-                const uint32_t slot = atomicAdd(&sh_gt, 1u);
-                if (slot < n_gt) cp[slot] = i;
-            }
-        });
-        /* keys equal to the threshold: the need_eq smallest positions */
-        uint32_t eq_base = 0;
-        for (uint32_t base = 0; base < n && eq_base < need_eq; base += TN_THREADS) {
-            const uint32_t i = base + tid;
-            const bool f = i < n && hfx_f2key(sc[i]) == K;
-            const uint64_t bal = __ballot(f);
-            const uint32_t wr = (uint32_t)__builtin_popcountll(bal & ((1ull << lane) - 1ull));
-            if (lane == 0) wcnt[wave] = (uint32_t)__builtin_popcountll(bal);
-            __syncthreads();
-            uint32_t wpre = 0, tot = 0;
-            for (uint32_t w = 0; w < TN_WAVES; ++w) {
-                if (w < wave) wpre += wcnt[w];
-                tot += wcnt[w];
-            }
-            const uint32_t r = eq_base + wpre + wr;
-            if (f && r < need_eq) {
-                cp[n_gt + r] = i;
-                if (r == need_eq - 1) sh_last = i;
-            }
-            eq_base += tot;
-            __syncthreads();
-        }
+        sh_cnt = 0;
     }
 
-    /* 2. the spectrum, the bound B on |FP32 - exact| (from sum |x|), and the
-     * N-th best FP32 score fN of the selection */
-    const uint32_t len = hfx_stage_spectrum(xs, mtab, c.db, sp, s);
-    uint32_t *map = maps + wave * mwords;
-    for (uint32_t w = lane; w < mwords; w += HFX_WAVE) map[w] = 0;
-    for (uint32_t i = tid; i < T; i += TN_THREADS) cf32[i] = sc[cp[i]];
-    __syncthreads();
+    /* 1. the scores, once, four at a time, and the largest of each thread;
+     * sum|x| and max|x| */
+    const bool held = n <= TN_HOLD * TN_THREADS;
+    const uint32_t len = min(sp.d_len[s], min(sp.x_stride, (uint32_t)HFX_MAX_LEN));
+    const float *xg = sp.d_x + (size_t)s * sp.x_stride;
+    tn_f4 v4[TN_HOLD / 4];
+    uint32_t km = 0;
+    if (held) {
+        /* thread t's scores are 1024 u + 4 t + e; absent ones are NaN, which
+         * the largest skips */
+#pragma unroll
+        for (uint32_t u = 0; u < TN_HOLD / 4; ++u) {
+            v4[u] = tn_f4{NAN, NAN, NAN, NAN};
+            const uint32_t i = u * 4 * TN_THREADS + 4 * tid;
+            if (i + 4 <= n) v4[u] = *(const tn_f4 *)(sc + i);
+            else if (i < n)
+#pragma unroll
+                for (uint32_t e = 0; e < 3; ++e)
+                    if (i + e < n) v4[u][e] = sc[i + e];
+        }
+    }
     float x1 = 0.0f, xm = 0.0f;
-    for (uint32_t i = tid; i < len; i += TN_THREADS) {
-        x1 += fabsf(xs[i]);
-        xm = fmaxf(xm, fabsf(xs[i]));
+    for (uint32_t base = 0; base < len; base += 8 * TN_THREADS) {
+        float v[8];
+#pragma unroll
+        for (uint32_t u = 0; u < 8; ++u) v[u] = xg[min(base + u * TN_THREADS + tid, len - 1u)];
+#pragma unroll
+        for (uint32_t u = 0; u < 8; ++u)
+            if (base + u * TN_THREADS + tid < len) {
+                x1 += fabsf(v[u]);
+                xm = fmaxf(xm, fabsf(v[u]));
+            }
+    }
+    /* a score that is NaN orders by its bits, as the radix select has it */
+    bool nan = false;
+    if (held) {
+        float m = -INFINITY;
+        uint32_t cnt = 0;
+#pragma unroll
+        for (uint32_t u = 0; u < TN_HOLD / 4; ++u)
+#pragma unroll
+            for (uint32_t e = 0; e < 4; ++e) {
+                m = fmaxf(m, v4[u][e]);
+                cnt += v4[u][e] == v4[u][e] ? 1u : 0u;
+            }
+        /* this thread's scores: 4 for every whole step, the rest in the last */
+        const uint32_t step = 4 * TN_THREADS, whole = n / step, rest = n % step;
+        const uint32_t mine = whole * 4 + min(4u, rest > 4 * tid ? rest - 4 * tid : 0u);
+        nan = cnt != mine;
+        km = mine ? hfx_f2key(m) : 0u;
+    } else {
+        for_keys([&](uint32_t i, uint32_t k) { km = max(km, i < n ? k : 0u); });
     }
     x1 = hfx_wave_sum_f32(x1);
-    for (uint32_t o = 32; o > 0; o >>= 1) xm = fmaxf(xm, __shfl_xor(xm, o, 64));
+    for (uint32_t q = 32; q > 0; q >>= 1) xm = fmaxf(xm, __shfl_xor(xm, q, 64));
+    /* a key that at least T of the wave's keys reach: the T-th largest of the
+     * lanes' largest, bit by bit (0 if fewer lanes have any); the low twelve
+     * bits left out, which takes a few more scores into the list */
+    uint32_t low = 0;
+    if (T <= TN_LT)
+        for (int b = 31; b >= 12; --b) {
+            const uint32_t t = low | 1u << b;
+            if ((uint32_t)__builtin_popcountll(__ballot(km >= t)) >= T) low = t;
+        }
+    const uint64_t anynan = __ballot(nan);
     if (lane == 0) {
         sh_x1[wave] = x1;
         sh_xm[wave] = xm;
+        sh_low[wave] = low;
+        wcnt[wave] = anynan != 0;
     }
-    if (n > T && !local)
-        for (uint32_t i = tid; i < T; i += TN_THREADS) {
-            const uint32_t ki = hfx_f2key(cf32[i]), pi = cp[i];
-            uint32_t rk = 0;
-            for (uint32_t j = 0; j < T; ++j) {
-                const uint32_t kj = hfx_f2key(cf32[j]);
-                rk += (kj > ki || (kj == ki && cp[j] < pi)) ? 1u : 0u;
-            }
-            if (rk == N - 1) sh_fN = cf32[i];
-        }
     __syncthreads();
+    const bool direct = T <= TN_LT && !(wcnt[0] | wcnt[1] | wcnt[2] | wcnt[3]);
+    static_assert(TN_WAVES == 4, "every wave's mark");
     const uint32_t zeff = c.zeff(sp.d_zmax[s]);
     float xa = 0.0f, xmax = 0.0f;
     for (uint32_t w = 0; w < TN_WAVES; ++w) {
         xa += sh_x1[w];
         xmax = fmaxf(xmax, sh_xm[w]);
+        low = max(low, sh_low[w]);
     }
     const double rel = (double)rel0 + (double)rel1 * (double)zeff;
     const double bound = rel * 50.0 * (double)xa * 1.001 +
                          (double)relq * (double)xmax * 50.0 * (double)len * 1.001 + 1e-6;
+    /* scores below it can be neither selected nor in the band when the N-th
+     * best is f or more (a relative 1e-12 margin covers the double roundings) */
+    auto reach = [&](float f) {
+        const double d = (double)f;
+        return d - 2.0 * bound - 1e-12 * (fabs(d) + 2.0 * bound);
+    };
 
-    /* 3. the extension: every other candidate that could reach the N-th
-     * exact score exN.  The N best FP32 scores are selected and each has an
-     * exact score >= fN - B, so exN >= fN - B: a candidate with FP32 score
-     * below fN - 2B has an exact score below exN - B + B = exN, under N
-     * others.  (A relative 1e-12 margin covers the double roundings.)  All
-     * candidates at or above fN - 2B are re-scored with the selection, in one
-     * round.  More than TN_EXT of them: the spectrum is flagged, the
-     * selection alone is re-scored, and the exact route takes every
-     * candidate at or above exN - B. */
+    /* 2. T <= TN_LT: fN >= low, so every key at or above reach(low) holds the
+     * selection and the band.  They are ranked exactly; the band is taken from
+     * them once fN is known.  Should they pass TN_MAXC (long runs of
+     * near-equal scores), the radix select below takes over. */
     uint32_t ne = 0, fl = 0;
-    if (n > T) {
-        const double fN = (double)sh_fN;
-        const double tau2 = fN - 2.0 * bound - 1e-12 * (fabs(fN) + 2.0 * bound);
-        const uint32_t last = sh_last;
-        /* from the lists: a thread whose TN_LT-th value is below tau2 left
-         * out only values below tau2; if every thread's is, the band is the
-         * lists' unselected values at or above tau2 */
-        bool wide = false;
-        if (local) {
-            const uint64_t vT = (uint64_t)K << 32 | (0xffffffffu - last);
-            wide = lst[TN_LT - 1] != 0 &&
-                   (double)hfx_key2f((uint32_t)(lst[TN_LT - 1] >> 32)) >= tau2;
-            if (wide) sh_wide = 1u;
-            __syncthreads();
-            wide = sh_wide != 0;
-            if (!wide)
+    bool done = false;
+    if (direct) {
+        uint32_t kthr = low;
+        if (low) {
+            const double thr = reach(hfx_key2f(low));
+            if (thr == thr) {
+                /* the smallest key whose value is >= thr (-0 and +0 are equal
+                 * values, but not keys) */
+                const float tf = (float)thr;
+                uint32_t kt = hfx_f2key(tf) + ((double)tf < thr ? 1u : 0u);
+                if (tf == 0.0f && !((double)tf < thr)) kt = 0x7fffffffu;
+                kthr = min(kt, low);
+            }
+        }
+        auto collect = [&](uint32_t i, uint32_t k, bool f) {
+            const uint64_t bal = __ballot(f);
+            if (bal) {
+                const uint32_t lead = (uint32_t)__builtin_ctzll(bal);
+                uint32_t at = 0;
+                if (lane == lead) at = atomicAdd(&sh_cnt, (uint32_t)__builtin_popcountll(bal));
+                at = hfx_take(at, lead) +
+                     (uint32_t)__builtin_popcountll(bal & ((1ull << lane) - 1ull));
+                if (f && at < TN_MAXC) kv[at] = (uint64_t)k << 32 | (0xffffffffu - i);
+            }
+        };
+        if (held) {
+            /* the threshold as a value: no NaN here, and -0 is taken with +0 */
+            const float fthr = kthr <= hfx_f2key(-INFINITY) ? -INFINITY : hfx_key2f(kthr);
 #pragma unroll
-                for (uint32_t j = 0; j < TN_LT; ++j) {
-                    const uint64_t v = lst[j];
-                    if (v != 0 && v < vT && (double)hfx_key2f((uint32_t)(v >> 32)) >= tau2) {
+            for (uint32_t u = 0; u < TN_HOLD / 4; ++u)
+#pragma unroll
+                for (uint32_t e = 0; e < 4; ++e)
+                    if (__ballot(v4[u][e] >= fthr))
+                        collect(u * 4 * TN_THREADS + 4 * tid + e,
+                                v4[u][e] >= fthr ? hfx_f2key(v4[u][e]) : 0u, v4[u][e] >= fthr);
+        } else {
+            for_keys([&](uint32_t i, uint32_t k) { collect(i, k, i < n && k >= kthr); });
+        }
+        __syncthreads();
+        const uint32_t M0 = sh_cnt;
+        done = M0 <= TN_MAXC;
+        if (done) {
+            uint32_t rk[(TN_MAXC + TN_THREADS - 1) / TN_THREADS];
+#pragma unroll
+            for (uint32_t q = 0; q < (TN_MAXC + TN_THREADS - 1) / TN_THREADS; ++q) {
+                const uint32_t a = q * TN_THREADS + tid;
+                rk[q] = 0xffffffffu;
+                if (a < M0) {
+                    const uint64_t v = kv[a];
+                    uint32_t r = 0;
+#pragma unroll 8
+                    for (uint32_t b = 0; b < M0; ++b) r += kv[b] > v ? 1u : 0u;
+                    rk[q] = r;
+                    if (r < T) cp[r] = 0xffffffffu - (uint32_t)v;
+                    if (r == N - 1u) sh_fN = hfx_key2f((uint32_t)(v >> 32));
+                }
+            }
+            __syncthreads();
+            if (n > T) {
+                const double tau2 = reach(sh_fN);
+#pragma unroll
+                for (uint32_t q = 0; q < (TN_MAXC + TN_THREADS - 1) / TN_THREADS; ++q) {
+                    const uint32_t a = q * TN_THREADS + tid;
+                    if (a < M0 && rk[q] >= T &&
+                        (double)hfx_key2f((uint32_t)(kv[a] >> 32)) >= tau2) {
                         const uint32_t slot = atomicAdd(&sh_ext, 1u);
-                        if (slot < TN_EXT) cp[T + slot] = 0xffffffffu - (uint32_t)v;
+                        if (slot < TN_EXT) cp[T + slot] = 0xffffffffu - (uint32_t)kv[a];
                     }
                 }
+                __syncthreads();
+                ne = sh_ext;
+            }
         }
-        if (!local || wide)
+    }
+    if (!done) {
+        /* Radix select, first over the key's 11 high bits (sign, exponent, two
+         * mantissa bits: a quarter octave a bucket), then 8, 8 and 5 bits; after
+         * each pass, once the keys at or above the prefix found so far -- M of
+         * them, known from the histograms -- number at most TN_MAXC, they are
+         * collected and ranked exactly.  Otherwise (long runs of near-equal
+         * scores) the full threshold key K is found and the keys above it, then
+         * the smallest positions equal to it, are collected. */
+        uint32_t prefix = 0, pmask = 0;
+        bool ranked = false;
+        for (int pass = 0; pass < 4; ++pass) {
+            const uint32_t shift = pass == 0 ? 32u - TN_HBITS : pass == 1 ? 13u : pass == 2 ? 5u : 0u;
+            const uint32_t nb = pass == 0 ? TN_HBINS : pass == 3 ? 32u : 256u;
+            for (uint32_t b = tid; b < nb; b += TN_THREADS) hist[b] = 0;
+            __syncthreads();
+            for_keys([&](uint32_t i, uint32_t k) {
+                tn_hist_add(hist, (k >> shift) & (nb - 1u), i < n && (k & pmask) == prefix);
+            });
+            __syncthreads();
+            tn_select_digit(hist, nb, &sh_digit, &sh_rem);
+            prefix |= sh_digit << shift;
+            pmask |= (nb - 1u) << shift;
+            const uint32_t M = T - sh_rem + hist[sh_digit];
+            __syncthreads(); /* every thread has read hist before it is cleared */
+            if (M <= TN_MAXC) {
+                for_keys([&](uint32_t i, uint32_t k) {
+                    if (i < n && (k & pmask) >= prefix)
+                        kv[atomicAdd(&sh_gt, 1u)] = (uint64_t)k << 32 | (0xffffffffu - i);
+                });
+                __syncthreads();
+                for (uint32_t a = tid; a < M; a += TN_THREADS) {
+                    const uint64_t va = kv[a];
+                    uint32_t rk = 0;
+                    for (uint32_t b = 0; b < M; ++b) rk += kv[b] > va ? 1u : 0u;
+                    const uint32_t pa = 0xffffffffu - (uint32_t)va;
+                    if (rk < T) cp[rk] = pa;
+                    if (rk == T - 1u) {
+                        sh_digit = (uint32_t)(va >> 32);
+                        sh_last = pa;
+                    }
+                }
+                __syncthreads();
+                ranked = true;
+                break;
+            }
+        }
+        const uint32_t K = ranked ? sh_digit : prefix;
+        if (!ranked) {
+            const uint32_t need_eq = sh_rem; /* >= 1 */
+            const uint32_t n_gt = T - need_eq;
+            for_keys([&](uint32_t i, uint32_t k) {
+                if (i < n && k > K) {
+                    const uint32_t slot = atomicAdd(&sh_gt, 1u);
+                    if (slot < n_gt) cp[slot] = i;
+                }
+            });
+            /* keys equal to the threshold: the need_eq smallest positions */
+            uint32_t eq_base = 0;
+            for (uint32_t base = 0; base < n && eq_base < need_eq; base += TN_THREADS) {
+                const uint32_t i = base + tid;
+                const bool f = i < n && hfx_f2key(sc[i]) == K;
+                const uint64_t bal = __ballot(f);
+                const uint32_t wr = (uint32_t)__builtin_popcountll(bal & ((1ull << lane) - 1ull));
+                if (lane == 0) wcnt[wave] = (uint32_t)__builtin_popcountll(bal);
+                __syncthreads();
+                uint32_t wpre = 0, tot = 0;
+                for (uint32_t w = 0; w < TN_WAVES; ++w) {
+                    if (w < wave) wpre += wcnt[w];
+                    tot += wcnt[w];
+                }
+                const uint32_t r = eq_base + wpre + wr;
+                if (f && r < need_eq) {
+                    cp[n_gt + r] = i;
+                    if (r == need_eq - 1) sh_last = i;
+                }
+                eq_base += tot;
+                __syncthreads();
+            }
+        }
+        __syncthreads();
+        if (n > T) {
+            /* the N-th best of the selection, then the band */
+            for (uint32_t i = tid; i < T; i += TN_THREADS) {
+                const uint32_t pi = cp[i], ki = hfx_f2key(sc[pi]);
+                kv[i] = (uint64_t)ki << 32 | (0xffffffffu - pi);
+            }
+            __syncthreads();
+            for (uint32_t i = tid; i < T; i += TN_THREADS) {
+                uint32_t rk = 0;
+                for (uint32_t j = 0; j < T; ++j) rk += kv[j] > kv[i] ? 1u : 0u;
+                if (rk == N - 1) sh_fN = hfx_key2f((uint32_t)(kv[i] >> 32));
+            }
+            __syncthreads();
+            const double tau2 = reach(sh_fN);
+            const uint32_t last = sh_last;
             for_keys([&](uint32_t i, uint32_t k) {
                 const bool selected = k > K || (k == K && i <= last);
                 if (i < n && !selected && (double)hfx_key2f(k) >= tau2) {
@@ -440,73 +496,299 @@ __global__ void __launch_bounds__(TN_THREADS)
                     if (slot < TN_EXT) cp[T + slot] = i;
                 }
             });
-        __syncthreads();
-        ne = sh_ext;
-        if (ne > TN_EXT) {
-            fl = 1;
-            if (tid == 0) band_out[s] = ne; /* sizes the exact route's tiles */
-            ne = 0;
+            __syncthreads();
+            ne = sh_ext;
         }
     }
 
-    /* 4. exact re-score of the selection and the extension: the wave's
-     * candidates i = wave + 4 j, 64 at a time, lane j fetching candidate i's
-     * metadata */
+    /* 3. the list.  More than TN_EXT in the band: the spectrum is flagged, the
+     * selection alone is re-scored, and the exact route takes every candidate at
+     * or above exN - B. */
+    if (ne > TN_EXT) {
+        fl = 1;
+        if (tid == 0) o.band[s] = ne; /* sizes the exact route's tiles */
+        ne = 0;
+    }
     const uint32_t M = T + ne;
-    for (uint32_t c0 = 0; c0 < M; c0 += TN_WAVES * HFX_WAVE) {
-        typename Cands::Prep mine{};
-        if (c0 + wave + TN_WAVES * lane < M) mine = c.prep(s, cp[c0 + wave + TN_WAVES * lane]);
-        /* the next candidate's first residues are loaded while this one is
-         * scored */
-        uint32_t res = c0 + wave < M ? c.first_res(Cands::take(mine, 0)) : 0u;
-        for (uint32_t i = c0 + wave, j = 0; i < M && j < HFX_WAVE; i += TN_WAVES, ++j) {
-            const uint32_t cur_res = res;
-            if (i + TN_WAVES < M && j + 1 < HFX_WAVE) res = c.first_res(Cands::take(mine, j + 1));
-            c.peaks_first(map, mtab, Cands::take(mine, j), cur_res, len, zeff);
-            hfx_wave_sync();
-            const int64_t fx = hfx_wave_dot_fx(map, xs, len);
-            hfx_wave_sync();
-            if (lane == 0) {
-                cfx[i] = fx;
-                if (i >= T) cf32[i] = sc[cp[i]];
+    /* spectra whose terms 50 |x| 2^36 stay below 2^50 take the short rounding
+     * (fmaxf skips a NaN, the sum keeps it) */
+    const uint32_t big = xmax < 300.0f && xa == xa ? 0u : TN_BIG;
+    for (uint32_t i = tid; i < M; i += TN_THREADS) o.cand[(size_t)s * TN_MAXC + i] = cp[i];
+    const uint32_t ntask = M > TN_TASK ? (M - 1u) / TN_TASK : 0u;
+    if (tid == 0) {
+        o.mcnt[s] = M | big;
+        flag[s] = fl;
+        o.tau[s] = bound;
+        sh_task = ntask ? atomicAdd(o.nspill, ntask) : 0u;
+    }
+    if (ntask) {
+        __syncthreads();
+        if (tid < ntask) o.spill[sh_task + tid] = make_uint2(s, (tid + 1u) * TN_TASK);
+    }
+}
+
+/* ------------------------------------------------------------------ */
+/* Exact scores, several candidates a wave                               */
+/* ------------------------------------------------------------------ */
+
+/* LDS of a wave: XP_SLOTS maps (cleared), the ladder buffer, the pack's sums */
+struct FxWave {
+    uint32_t *maps;
+    float *lb;
+    unsigned long long *acc;
+};
+static size_t fx_lds_bytes(uint32_t xstr)
+{
+    return (size_t)TN_WAVES * (XP_SLOTS * xp_map_words(xstr) + XP_LB) * 4 + TN_WAVES * XP_SLOTS * 8;
+}
+__device__ __forceinline__ FxWave fx_wave(unsigned char *lds, uint32_t mstr, uint32_t wave)
+{
+    unsigned long long *acc = (unsigned long long *)lds;
+    uint32_t *maps = (uint32_t *)(acc + TN_WAVES * XP_SLOTS);
+    float *lb = (float *)(maps + TN_WAVES * XP_SLOTS * mstr);
+    const FxWave f{maps + wave * XP_SLOTS * mstr, lb + wave * XP_LB, acc + wave * XP_SLOTS};
+    for (uint32_t i = hfx_lane(); i < XP_SLOTS * mstr; i += HFX_WAVE) f.maps[i] = 0u;
+    return f;
+}
+
+/* one pack at fragment charges 1..Z: the exact sum of each candidate into its
+ * accumulator.  The spectrum is read where it lies (a row is a few KiB, in L2
+ * after the first pack); its values come before the claims, whose codes decide
+ * what is added; bins outside [0, len) add nothing. */
+template <int Z, bool BIG>
+__device__ __forceinline__ void fx_pack(const FxWave &f, uint32_t mstr, const float *x, uint32_t len,
+                                        const XpPack pk)
+{
+    const uint32_t lane = hfx_lane();
+    const XpLane ln = xp_lane(pk, lane);
+    if (lane < XP_SLOTS) f.acc[lane] = 0ull;
+    const float b = ln.act ? f.lb[ln.lad + ln.kpos] : 0.0f;
+    const float y = ln.r - b;
+    uint32_t *rowm = f.maps + ln.slot * mstr + XP_PAD / 8 - (XP_MAGIC_BITS >> 3);
+    const uint32_t spr = (lane & (XP_SPREAD - 1)) * 8u;
+    const XpClamp cl{XP_MAGIC_BITS - 1u - spr, XP_MAGIC_BITS + len + spr,
+                     XP_MAGIC_BITS - 2u - spr, XP_MAGIC_BITS + len + 1u + spr};
+    auto put = [&](auto zc) {
+        uint32_t u[6];
+        XpPeaks p;
+        xp_bins<decltype(zc)::value>(b, y, cl, u);
+        xp_locate(rowm, u, p);
+        xp_put(p);
+    };
+    if (ln.act) {
+        put(std::integral_constant<int, 1>{});
+        if constexpr (Z >= 2) put(std::integral_constant<int, 2>{});
+        if constexpr (Z >= 3) put(std::integral_constant<int, 3>{});
+        if constexpr (Z >= 4) put(std::integral_constant<int, 4>{});
+    }
+    hfx_wave_sync();
+    if (ln.act) {
+        uint64_t sum = 0; /* modulo 2^64 */
+        /* rint(w x 2^36): x 2^36 is exact in FP32 and the product in FP64;
+         * adding 1.5 * 2^52 rounds one below 2^51 to an integer, ties to even,
+         * and leaves it in the low bits, the constant's bits taken off the
+         * sum once for all terms */
+        constexpr double MAGIC = 6755399441055744.0;
+        auto term = [&](uint32_t nib, uint32_t bin, float xv) {
+            const uint32_t w = bin < len ? __builtin_amdgcn_perm(0x32000000u, 0x19000A00u, nib & 15u) & 0xffu
+                                         : 0u;
+            if constexpr (BIG) {
+                sum += (uint64_t)hfx_fx_term((float)w, xv);
+            } else {
+                const double t = (double)w * (double)(xv * 68719476736.0f) + MAGIC;
+                sum += (uint64_t)__double_as_longlong(t);
+            }
+        };
+        /* the bins again, not kept from the first pass: eight waves a SIMD
+         * would not hold them for four charges */
+        auto claim = [&](auto zc) {
+            float b2 = b;
+            asm volatile("" : "+v"(b2));
+            uint32_t u[6];
+            XpPeaks p;
+            xp_bins<decltype(zc)::value>(b2, y, cl, u);
+            xp_locate(rowm, u, p);
+            float xv[6][3];
+#pragma unroll
+            for (int i = 0; i < 6; ++i)
+#pragma unroll
+                for (int q = 0; q < (i == 1 || i == 4 ? 3 : 1); ++q)
+                    xv[i][q] = x[min(p.u[i] - XP_MAGIC_BITS + q, len - 1u)];
+#pragma unroll
+            for (int i = 0; i < 6; ++i) {
+                const uint32_t bin = p.u[i] - XP_MAGIC_BITS, sh = p.sh[i];
+                if (i == 1 || i == 4) {
+                    const uint64_t t = (uint64_t)0xfffu << sh;
+                    const uint32_t o0 = atomicAnd(p.w[i], ~(uint32_t)t);
+                    const uint32_t o1 = atomicAnd(p.w[i] + 1, ~(uint32_t)(t >> 32));
+                    const uint32_t g = (uint32_t)(((uint64_t)o1 << 32 | o0) >> sh);
+                    term(g, bin, xv[i][0]);
+                    term(g >> 4, bin + 1u, xv[i][1]);
+                    term(g >> 8, bin + 2u, xv[i][2]);
+                } else {
+                    term(atomicAnd(p.w[i], ~(0xfu << sh)) >> sh, bin, xv[i][0]);
+                }
+            }
+        };
+        claim(std::integral_constant<int, 1>{});
+        if constexpr (Z >= 2) claim(std::integral_constant<int, 2>{});
+        if constexpr (Z >= 3) claim(std::integral_constant<int, 3>{});
+        if constexpr (Z >= 4) claim(std::integral_constant<int, 4>{});
+        if constexpr (!BIG) sum -= 10ull * Z * (uint64_t)__double_as_longlong(MAGIC);
+        atomicAdd(&f.acc[ln.slot], (unsigned long long)sum);
+    }
+    hfx_wave_sync();
+}
+
+/* the exact scores of rn <= 64 candidates of one spectrum, candidate i's
+ * metadata in lane i: emit(i, score) once each, by one lane.  BIG: terms may
+ * pass 2^50. */
+template <bool BIG, class Cands, class Emit>
+__device__ __forceinline__ void fx_scores(const FxWave &f, uint32_t mstr, const float *mtab,
+                                          const float *x, uint32_t len, uint32_t zeff,
+                                          const Cands &c, const typename Cands::Prep &pr,
+                                          uint32_t rn, Emit &&emit)
+{
+    const uint32_t lane = hfx_lane();
+    if (zeff == 0 || len == 0) {
+        /* no fragment charge generated, or no bins */
+        if (lane < rn) emit(lane, (int64_t)0);
+        return;
+    }
+    const bool general = zeff > 4;
+    const uint32_t nl = lane < rn && pr.n <= HFX_WAVE && !general ? pr.n : 0u;
+    const uint32_t incl = xp_prefix(nl, lane), pofs = incl - nl;
+    for (uint32_t p = 0; p < rn;) {
+        const uint32_t base = hfx_take(pofs, p);
+        const uint64_t fit = __ballot(lane >= p && lane < rn && incl - base <= XP_LB);
+        const uint32_t q = p + (uint32_t)__builtin_popcountll(fit);
+        if (lane >= p && lane < q && nl) c.ladder(pr, mtab, f.lb + (pofs - base), nl);
+        hfx_wave_sync();
+        while (p < q) {
+            if (hfx_take(pr.n, p) > HFX_WAVE || general) {
+                c.peaks_prep(f.maps + XP_PAD / 8, mtab, Cands::take(pr, p), len, zeff);
+                hfx_wave_sync();
+                const int64_t v = hfx_wave_dot_fx(f.maps + XP_PAD / 8, x, len);
+                hfx_wave_sync();
+                if (lane == 0) emit(p, v);
+                ++p;
+                continue;
+            }
+            const XpPack pk = xp_form(p, q, pr.n, pr.r, pofs, base);
+            switch (zeff) {
+            case 1: fx_pack<1, BIG>(f, mstr, x, len, pk); break;
+            case 2: fx_pack<2, BIG>(f, mstr, x, len, pk); break;
+            case 3: fx_pack<3, BIG>(f, mstr, x, len, pk); break;
+            default: fx_pack<4, BIG>(f, mstr, x, len, pk); break;
+            }
+            if (lane < pk.K) emit(p + lane, (int64_t)f.acc[lane]);
+            hfx_wave_sync(); /* the accumulators are cleared by the next pack */
+            p += pk.K;
+        }
+        hfx_wave_sync(); /* the buffer is rewritten by the next chunk */
+    }
+}
+
+/* exact scores of the listed candidates: wave w takes the first TN_TASK of
+ * spectrum w, then all waves share the spilled tasks.  fx: [base(s) + i] for
+ * candidate i of s's list. */
+template <class Cands>
+__global__ void __launch_bounds__(TN_THREADS)
+    k_topn_exact(int64_t *fx, TnLists o, Cands c, hfx_spectra sp, uint32_t mstr)
+{
+    extern __shared__ __align__(16) unsigned char tn_dyn[];
+    __shared__ float mtab[32];
+    const uint32_t wave = threadIdx.x / HFX_WAVE, lane = hfx_lane(), S = sp.num_spec;
+    if (threadIdx.x < 32) mtab[threadIdx.x] = threadIdx.x < 26 ? c.db.d_mass[threadIdx.x] : 0.0f;
+    const FxWave f = fx_wave(tn_dyn, mstr, wave);
+    __syncthreads();
+    auto task = [&](uint32_t s, uint32_t k0) {
+        const uint32_t mc = __builtin_amdgcn_readfirstlane(o.mcnt[s]), M = mc & ~TN_BIG;
+        const uint32_t rn = M > k0 ? min(M - k0, (uint32_t)TN_TASK) : 0u;
+        if (rn == 0) return;
+        typename Cands::Prep pr{};
+        if (lane < rn) pr = c.prep(s, o.cand[(size_t)s * TN_MAXC + k0 + lane]);
+        const uint32_t len = min(sp.d_len[s], min(sp.x_stride, (uint32_t)HFX_MAX_LEN));
+        int64_t *out = fx + c.base(s) + k0;
+        const float *x = sp.d_x + (size_t)s * sp.x_stride;
+        const uint32_t zeff = c.zeff(sp.d_zmax[s]);
+        auto emit = [&](uint32_t i, int64_t v) { out[i] = v; };
+        if (mc & TN_BIG) fx_scores<true>(f, mstr, mtab, x, len, zeff, c, pr, rn, emit);
+        else fx_scores<false>(f, mstr, mtab, x, len, zeff, c, pr, rn, emit);
+    };
+    const uint32_t w = __builtin_amdgcn_readfirstlane(blockIdx.x * TN_WAVES + wave);
+    if (w < S) task(w, 0);
+    const uint32_t ns = *o.nspill;
+    for (uint32_t i = w; i < ns; i += gridDim.x * TN_WAVES) {
+        const uint2 t = o.spill[i];
+        task(__builtin_amdgcn_readfirstlane(t.x), __builtin_amdgcn_readfirstlane(t.y));
+    }
+}
+
+/* the lists in order of (exact desc, position asc): the best N, and for
+ * flagged spectra exN - B as the exact route's threshold.  A wave a spectrum. */
+template <class Cands>
+__global__ void __launch_bounds__(TN_THREADS)
+    k_topn_rank(uint32_t *top_pos, double *top_exact, float *top_f32, uint32_t *top_cnt,
+                const uint32_t *flag, uint32_t N, const int64_t *fx, TnLists o, const float *scores,
+                Cands c, uint32_t S)
+{
+    const uint32_t wave = threadIdx.x / HFX_WAVE, lane = hfx_lane();
+    const uint32_t s = blockIdx.x * TN_WAVES + wave;
+    if (s >= S) return;
+    const uint32_t M = o.mcnt[s] & ~TN_BIG, n = c.count(s), outn = min(N, n);
+    const float *sc = scores + c.base(s);
+    const bool fl = M && flag[s] != 0u;
+    const int64_t *f = fx + c.base(s);
+    const uint32_t *p = o.cand + (size_t)s * TN_MAXC;
+    auto put = [&](uint32_t rk, uint64_t k, uint32_t pos) {
+        const double v = (double)(int64_t)(k ^ 0x8000000000000000ull) * (1.0 / HFX_FX_SCALE);
+        top_pos[(size_t)s * N + rk] = pos;
+        top_exact[(size_t)s * N + rk] = v;
+        top_f32[(size_t)s * N + rk] = sc[pos];
+        if (fl && rk == N - 1u) o.tau[s] = v - o.tau[s];
+    };
+    if (M <= HFX_WAVE) {
+        /* each lane counts its candidate's place */
+        uint64_t k = 0;
+        uint32_t pos = 0xffffffffu;
+        if (lane < M) {
+            k = (uint64_t)f[lane] ^ 0x8000000000000000ull;
+            pos = p[lane];
+        }
+        uint32_t rk = 0;
+        for (uint32_t j = 0; j < M; ++j) {
+            const uint64_t kj = (uint64_t)hfx_take((uint32_t)(k >> 32), j) << 32 |
+                                hfx_take((uint32_t)k, j);
+            const uint32_t pj = hfx_take(pos, j);
+            rk += kj > k || (kj == k && pj < pos) ? 1u : 0u;
+        }
+        if (lane < M && rk < outn) put(rk, k, pos);
+    } else {
+        constexpr int R = TN_MAXC / HFX_WAVE;
+        uint64_t k[R];
+        uint32_t pos[R];
+#pragma unroll
+        for (int i = 0; i < R; ++i) {
+            const uint32_t j = (uint32_t)i * HFX_WAVE + lane;
+            k[i] = 0;
+            pos[i] = 0xffffffffu;
+            if (j < M) {
+                k[i] = (uint64_t)f[j] ^ 0x8000000000000000ull;
+                pos[i] = p[j];
             }
         }
+        tn_wave_top<R>(k, pos, outn, [&](uint32_t rk, uint64_t kb, uint32_t pb) {
+            if (lane == 0) put(rk, kb, pb);
+        });
     }
-    __syncthreads();
-    if (fl) {
-        /* exN, the N-th best exact score of the selection, for the exact
-         * route's threshold */
-        for (uint32_t i = tid; i < T; i += TN_THREADS) {
-            uint32_t rk = 0;
-            for (uint32_t j = 0; j < T; ++j)
-                rk += before_fx(cfx[j], cp[j], cfx[i], cp[i]) ? 1u : 0u;
-            if (rk == N - 1) tau_out[s] = (double)cfx[i] * (1.0 / HFX_FX_SCALE) - bound;
-        }
-    }
-
-    /* 5. order by (exact desc, position asc), emit N */
-    const uint32_t outn = min(N, n);
-    for (uint32_t i = tid; i < M; i += TN_THREADS) {
-        const int64_t fi = cfx[i];
-        const uint32_t pi = cp[i];
-        uint32_t rk = 0;
-        for (uint32_t j = 0; j < M; ++j) rk += before_fx(cfx[j], cp[j], fi, pi) ? 1u : 0u;
-        if (rk < outn) {
-            top_pos[(size_t)s * N + rk] = pi;
-            top_exact[(size_t)s * N + rk] = (double)fi * (1.0 / HFX_FX_SCALE);
-            top_f32[(size_t)s * N + rk] = cf32[i];
-        }
-    }
-    if (tid == 0) {
-        top_cnt[s] = outn;
-        flag[s] = fl;
-    }
+    if (lane == 0) top_cnt[s] = outn;
 }
 
 /* ------------------------------------------------------------------ */
 /* Exact route: every candidate of a flagged spectrum scored exactly     */
 /* (tile-parallel, persistent), then a 64-bit radix select of the top N. */
-/* Runs on the device after k_topn without a host round trip.            */
+/* Runs on the device after the re-score without a host round trip.      */
 /* ------------------------------------------------------------------ */
 
 #define TX_MAXN 64
@@ -514,42 +796,69 @@ __global__ void __launch_bounds__(TN_THREADS)
 /* a flagged spectrum's tiles also number at least its band count / TX_LIVE,
  * so that the candidates the exact route re-scores spread over the tiles */
 #define TX_LIVE 32
-/* a wave fetches the metadata of its share of a candidate list one lane
- * per candidate */
-static_assert(TN_MAXT / TN_WAVES <= HFX_WAVE && TN_EXT / TN_WAVES <= HFX_WAVE &&
-                  TX_CHUNK / TN_WAVES <= HFX_WAVE,
+/* a wave fetches the metadata of its share of a tile one lane per candidate */
+static_assert(TX_CHUNK / TN_WAVES <= HFX_WAVE && TN_TASK <= HFX_WAVE,
               "one lane per candidate of a wave's share");
 
-/* tiles per flagged spectrum, and the flagged spectra listed (in any
- * order) for the final select; counter[1] counts them */
+/* the flagged spectra (in any order) and the first tile of each (off[their
+ * number] = all tiles), by one workgroup: few spectra are flagged, so the tiles
+ * need no table per spectrum */
+#define TX_THREADS 1024
 template <class Cands>
-__global__ void k_flag_tiles(uint32_t *tiles, uint32_t *list, uint32_t *counter,
-                             const uint32_t *flag, const uint32_t *band, Cands c, uint32_t S)
+__global__ void __launch_bounds__(TX_THREADS)
+    k_tx_plan(uint64_t *off, uint32_t *list, uint32_t *count, const uint32_t *flag,
+              const uint32_t *band, Cands c, uint32_t S)
 {
-    const uint32_t s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= S) return;
-    const bool f = flag[s] != 0u;
-    uint32_t nt = 0;
-    if (f) {
-        const uint32_t n = c.count(s), b = min(band[s], n);
-        nt = max((n + TX_CHUNK - 1) / TX_CHUNK, (b + TX_LIVE - 1) / TX_LIVE);
+    __shared__ uint32_t nl;
+    __shared__ uint64_t wt[TX_THREADS / HFX_WAVE];
+    const uint32_t lane = hfx_lane(), wave = threadIdx.x / HFX_WAVE;
+    if (threadIdx.x == 0) nl = 0;
+    __syncthreads();
+    for (uint32_t s0 = threadIdx.x; s0 < S; s0 += 8 * TX_THREADS) {
+        uint32_t fv[8];
+#pragma unroll
+        for (uint32_t u = 0; u < 8; ++u) fv[u] = flag[min(s0 + u * TX_THREADS, S - 1u)];
+#pragma unroll
+        for (uint32_t u = 0; u < 8; ++u)
+            if (s0 + u * TX_THREADS < S && fv[u] != 0u)
+                list[atomicAdd(&nl, 1u)] = s0 + u * TX_THREADS;
     }
-    tiles[s] = nt;
-    if (f) list[atomicAdd(&counter[1], 1u)] = s;
+    __syncthreads(); /* the list is this workgroup's own: visible to it from here */
+    const uint32_t F = nl;
+    uint64_t nt = 0;
+    for (uint32_t q0 = 0; q0 < F; q0 += TX_THREADS) {
+        const uint32_t q = q0 + threadIdx.x;
+        uint64_t t = 0;
+        if (q < F) {
+            const uint32_t s = list[q], n = c.count(s), b = min(band[s], n);
+            t = max((n + TX_CHUNK - 1) / TX_CHUNK, (b + TX_LIVE - 1) / TX_LIVE);
+        }
+        uint64_t x = t;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const uint64_t v = __shfl_up(x, o, 64);
+            if (lane >= (uint32_t)o) x += v;
+        }
+        if (lane == HFX_WAVE - 1) wt[wave] = x;
+        __syncthreads();
+        uint64_t to = nt + x - t;
+        for (uint32_t w = 0; w < TX_THREADS / HFX_WAVE; ++w) {
+            if (w < wave) to += wt[w];
+            nt += wt[w];
+        }
+        if (q < F) off[q] = to;
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) {
+        off[F] = nt;
+        *count = F;
+    }
 }
 
 __global__ void k_tx_reset(uint32_t *counter)
 {
     counter[0] = 0;
     counter[1] = 0;
-}
-
-/* tile -> spectrum, one thread per spectrum writing its own tiles */
-__global__ void k_tile_spec(uint32_t *tile_spec, const uint64_t *tile_off, uint32_t S)
-{
-    const uint32_t s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s < S)
-        for (uint64_t t = tile_off[s]; t < tile_off[s + 1]; ++t) tile_spec[t] = s;
 }
 
 __global__ void k_zero_flags(uint32_t *flag, uint32_t S)
@@ -575,38 +884,37 @@ __global__ void k_mark_list(uint32_t *flag, double *tau, uint32_t *band, const u
  * spread over the tiles. */
 template <class Cands>
 __global__ void __launch_bounds__(TN_THREADS)
-    k_exact_tiles(int64_t *fxbuf, const uint64_t *tile_off, const uint32_t *tile_spec, Cands c,
-                  hfx_spectra sp, const float *scores, const double *tau)
+    k_exact_tiles(int64_t *fxbuf, const uint64_t *tile_off, const uint32_t *list,
+                  const uint32_t *count, Cands c, hfx_spectra sp, const float *scores,
+                  const double *tau, uint32_t mstr)
 {
     extern __shared__ __align__(16) unsigned char tn_dyn[];
-    const uint32_t xcap = tn_xcap(sp.x_stride), mwords = xcap / 8;
-    float *xs = (float *)tn_dyn;
-    uint32_t *maps = (uint32_t *)(tn_dyn + tn_xs_bytes(sp.x_stride));
     __shared__ float mtab[32];
+    __shared__ uint32_t lpos[TN_WAVES][HFX_WAVE];
     const uint32_t wave = threadIdx.x / HFX_WAVE, lane = hfx_lane();
-    const uint32_t S = sp.num_spec;
-    const uint64_t ntiles = tile_off[S];
-    uint32_t *map = maps + wave * mwords;
-    for (uint32_t w = lane; w < mwords; w += HFX_WAVE) map[w] = 0;
-    uint32_t cur = 0xffffffffu, len = 0;
+    const uint32_t F = *count;
+    const uint64_t ntiles = tile_off[F];
+    if (blockIdx.x >= ntiles) return;
+    if (threadIdx.x < 32) mtab[threadIdx.x] = threadIdx.x < 26 ? c.db.d_mass[threadIdx.x] : 0.0f;
+    const FxWave f = fx_wave(tn_dyn, mstr, wave);
+    __syncthreads();
     for (uint64_t t = blockIdx.x; t < ntiles; t += gridDim.x) {
-        const uint32_t s = tile_spec[t];
-        if (s != cur) {
-            len = hfx_stage_spectrum(xs, mtab, c.db, sp, s);
-            cur = s;
-            __syncthreads();
+        uint32_t lo = 0, hi = F;
+        while (hi - lo > 1) {
+            const uint32_t mid = (lo + hi) >> 1;
+            if (tile_off[mid] <= t) lo = mid; else hi = mid;
         }
-        const uint32_t k = (uint32_t)(t - tile_off[s]);
-        const uint32_t nt = (uint32_t)(tile_off[s + 1] - tile_off[s]);
+        const uint32_t s = list[lo];
+        const uint32_t k = (uint32_t)(t - tile_off[lo]);
+        const uint32_t nt = (uint32_t)(tile_off[lo + 1] - tile_off[lo]);
         const uint32_t n = c.count(s);
-        const uint32_t zeff = c.zeff(sp.d_zmax[s]);
         const double ts = tau[s];
+        const uint32_t len = min(sp.d_len[s], min(sp.x_stride, (uint32_t)HFX_MAX_LEN));
         /* the wave's candidates: tile slots m = wave + 4 j (j < 64), lane j
          * reading candidate i = k + nt m's score.  A candidate below tau
          * cannot reach the top N (its exact score is below the N-th exact
          * score): it keeps the smallest key, stored by its own lane.  The
-         * others' metadata is fetched by their lanes, and the wave re-scores
-         * them one by one. */
+         * others are moved to the first lanes and re-scored. */
         const uint64_t tb = c.base(s);
         const uint64_t mi64 = k + (uint64_t)nt * (wave + TN_WAVES * lane);
         const uint32_t mi = (uint32_t)mi64;
@@ -615,24 +923,20 @@ __global__ void __launch_bounds__(TN_THREADS)
             live = !((double)scores[tb + mi] < ts);
             if (!live) fxbuf[tb + mi] = INT64_MIN;
         }
-        typename Cands::Prep mine{};
-        if (live) mine = c.prep(s, mi);
         const uint64_t lm = __ballot(live);
-        /* the next live candidate's first residues are loaded while this one
-         * is scored */
-        uint32_t res = lm ? c.first_res(Cands::take(mine, (uint32_t)__builtin_ctzll(lm))) : 0u;
-        for (uint64_t m = lm; m; m &= m - 1ull) {
-            const uint32_t j = (uint32_t)__builtin_ctzll(m);
-            const uint32_t cur_res = res;
-            const uint64_t rest = m & (m - 1ull);
-            if (rest) res = c.first_res(Cands::take(mine, (uint32_t)__builtin_ctzll(rest)));
-            c.peaks_first(map, mtab, Cands::take(mine, j), cur_res, len, zeff);
-            hfx_wave_sync();
-            const int64_t fx = hfx_wave_dot_fx(map, xs, len);
-            hfx_wave_sync();
-            if (lane == 0) fxbuf[tb + hfx_take(mi, j)] = fx;
+        const uint32_t rn = (uint32_t)__builtin_popcountll(lm);
+        if (live) lpos[wave][__builtin_popcountll(lm & ((1ull << lane) - 1ull))] = mi;
+        hfx_wave_sync();
+        uint32_t pos = 0;
+        typename Cands::Prep pr{};
+        if (lane < rn) {
+            pos = lpos[wave][lane];
+            pr = c.prep(s, pos);
         }
-        __syncthreads();
+        fx_scores<true>(f, mstr, mtab, sp.d_x + (size_t)s * sp.x_stride, len,
+                        c.zeff(sp.d_zmax[s]), c, pr, rn,
+                        [&](uint32_t i, int64_t v) { fxbuf[tb + lpos[wave][i]] = v; });
+        hfx_wave_sync();
     }
 }
 
@@ -879,38 +1183,34 @@ __global__ void __launch_bounds__(FX_THREADS)
 /* Launch helpers                                                        */
 /* ------------------------------------------------------------------ */
 
-/* tiles: max(ceil(n / TX_CHUNK), ceil(band / TX_LIVE)) per spectrum, band <= n */
-static uint64_t tx_max_tiles(uint32_t S, uint64_t total)
-{
-    return total / TX_CHUNK + total / TX_LIVE + 2ull * S;
-}
-
+/* scratch of a call:
+ * fxbuf[total] | tile_off[S+1] | tau[S] | spill[S * TN_SPILL] | counters (256 B) |
+ * list[S] | band[S] | mcnt[S] | cand[S][TN_MAXC] */
 size_t hfx_topn_scratch_bytes(uint32_t S, uint64_t total)
 {
-    return total * 8 + ((size_t)S + 1) * 8 + (size_t)S * 8 + (size_t)S * 4 + 256 +
-           tx_max_tiles(S, total) * 4 + (size_t)S * 8;
+    return total * 8 + ((size_t)S + 1) * 8 + (size_t)S * (8 + 8 * TN_SPILL) + 256 +
+           (size_t)S * 4 * (3 + TN_MAXC);
 }
 
-/* exact-route scratch:
- * fxbuf[total] | tile_off[S+1] | tau[S] | tiles[S] | counters (256 B) |
- * tile_spec[max tiles] | list[S] | band[S] */
 struct TxScratch {
     int64_t *fxbuf;
     uint64_t *tile_off;
-    double *tau;
-    uint32_t *tiles, *counter, *tile_spec, *list, *band;
+    uint32_t *counter, *list; /* counter: spilled tasks, flagged spectra */
+    TnLists l;
 };
 static TxScratch tx_carve(void *p, uint32_t S, uint64_t total)
 {
     TxScratch x;
     x.fxbuf = (int64_t *)p;
     x.tile_off = (uint64_t *)(x.fxbuf + total);
-    x.tau = (double *)(x.tile_off + S + 1);
-    x.tiles = (uint32_t *)(x.tau + S);
-    x.counter = x.tiles + S;
-    x.tile_spec = x.counter + 64;
-    x.list = x.tile_spec + tx_max_tiles(S, total);
-    x.band = x.list + S;
+    x.l.tau = (double *)(x.tile_off + S + 1);
+    x.l.spill = (uint2 *)(x.l.tau + S);
+    x.counter = (uint32_t *)(x.l.spill + (size_t)S * TN_SPILL);
+    x.l.nspill = x.counter;
+    x.list = x.counter + 64;
+    x.l.band = x.list + S;
+    x.l.mcnt = x.l.band + S;
+    x.l.cand = x.l.mcnt + S;
     return x;
 }
 static int tx_scratch(hfx_ctx *ctx, void *given, uint32_t S, uint64_t total, void **out)
@@ -933,15 +1233,11 @@ static int exact_route(hfx_ctx *ctx, uint32_t *d_top_pos, double *d_top_exact, f
     int rc;
     if ((rc = tx_scratch(ctx, scratch, S, total, &p))) return rc;
     const TxScratch x = tx_carve(p, S, total);
-    hipLaunchKernelGGL(k_tx_reset, dim3(1), dim3(1), 0, st, x.counter);
-    hipLaunchKernelGGL(k_flag_tiles<Cands>, dim3((S + 255) / 256), dim3(256), 0, st, x.tiles,
-                       x.list, x.counter, d_flag, x.band, c, S);
-    if ((rc = hfx_scan_offsets(ctx, x.tile_off, x.tiles, S, (void *)st)) != HFX_OK) return rc;
-    hipLaunchKernelGGL(k_tile_spec, dim3((S + 255) / 256), dim3(256), 0, st, x.tile_spec,
-                       x.tile_off, S);
-    hipLaunchKernelGGL(k_exact_tiles<Cands>, dim3((uint32_t)hfx_ctx_num_cus(ctx) * 8),
-                       dim3(TN_THREADS), tn_dyn_bytes(sp->x_stride), st, x.fxbuf, x.tile_off,
-                       x.tile_spec, c, *sp, d_scores, x.tau);
+    hipLaunchKernelGGL(k_tx_plan<Cands>, dim3(1), dim3(TX_THREADS), 0, st, x.tile_off, x.list,
+                       x.counter + 1, d_flag, x.l.band, c, S);
+    hipLaunchKernelGGL(k_exact_tiles<Cands>, dim3((uint32_t)hfx_ctx_num_cus(ctx) * 4),
+                       dim3(TN_THREADS), fx_lds_bytes(sp->x_stride), st, x.fxbuf, x.tile_off, x.list,
+                       x.counter + 1, c, *sp, d_scores, x.l.tau, xp_map_words(sp->x_stride));
     hipLaunchKernelGGL(k_topn_fx<Cands>, dim3(min(S, (uint32_t)hfx_ctx_num_cus(ctx))),
                        dim3(FX_THREADS), 0, st, d_top_pos, d_top_exact, d_top_f32, d_top_cnt,
                        d_flag, N, x.list, x.counter + 1, x.fxbuf, d_scores, c);
@@ -962,20 +1258,23 @@ static int launch_topn(hfx_ctx *ctx, uint32_t *d_top_pos, double *d_top_exact, f
     HFX_REQUIRE(N >= 1 && N <= TX_MAXN && N + margin <= TN_MAXT, HFX_ERR_ARG,
                 "hfx_topn: need 1 <= N <= %d and N + margin <= %d (N=%u margin=%u)", TX_MAXN,
                 TN_MAXT, N, margin);
-    if (sp->num_spec == 0) return HFX_OK;
+    const uint32_t S = sp->num_spec;
+    if (S == 0) return HFX_OK;
     hipStream_t st = hfx_stream(stream);
     void *p;
     int rc;
-    if ((rc = tx_scratch(ctx, scratch, sp->num_spec, total, &p))) return rc;
-    const TxScratch x = tx_carve(p, sp->num_spec, total);
-    /* the launch order lives in the flagged-spectrum list, which the exact
-     * route fills only after k_topn */
-    hipLaunchKernelGGL(k_topn_order<Cands>, dim3(1), dim3(TN_OTHREADS), 0, st, x.list, c,
-                       sp->num_spec);
-    hipLaunchKernelGGL(k_topn<Cands>, dim3(sp->num_spec), dim3(TN_THREADS),
-                       tn_dyn_bytes(sp->x_stride), st, d_top_pos, d_top_exact, d_top_f32,
-                       d_top_cnt, d_flag, N, margin, d_scores, c, *sp, rel0, rel1, relq, x.tau,
-                       x.band, x.list);
+    if ((rc = tx_scratch(ctx, scratch, S, total, &p))) return rc;
+    const TxScratch x = tx_carve(p, S, total);
+    const uint32_t gw = (S + TN_WAVES - 1) / TN_WAVES;
+    hipLaunchKernelGGL(k_tx_reset, dim3(1), dim3(1), 0, st, x.counter);
+    hipLaunchKernelGGL(k_topn_select<Cands>, dim3(S), dim3(TN_THREADS), 0, st, x.l, d_flag, N,
+                       margin, d_scores, c, *sp, rel0, rel1, relq);
+    /* at least a workgroup a CU: the spilled tasks spread over all of them */
+    hipLaunchKernelGGL(k_topn_exact<Cands>, dim3(max(gw, (uint32_t)hfx_ctx_num_cus(ctx))),
+                       dim3(TN_THREADS), fx_lds_bytes(sp->x_stride), st, x.fxbuf, x.l, c, *sp,
+                       xp_map_words(sp->x_stride));
+    hipLaunchKernelGGL(k_topn_rank<Cands>, dim3(gw), dim3(TN_THREADS), 0, st, d_top_pos,
+                       d_top_exact, d_top_f32, d_top_cnt, d_flag, N, x.fxbuf, x.l, d_scores, c, S);
     HFX_CHECK_LAUNCH();
     return exact_route(ctx, d_top_pos, d_top_exact, d_top_f32, d_top_cnt, N, d_flag, d_scores, c,
                        total, sp, p, st);
@@ -999,8 +1298,8 @@ static int launch_topn_exact(hfx_ctx *ctx, uint32_t *d_top_pos, double *d_top_ex
     uint32_t *flag = (uint32_t *)p;
     const TxScratch x = tx_carve(q, S, total);
     hipLaunchKernelGGL(k_zero_flags, dim3((S + 255) / 256), dim3(256), 0, st, flag, S);
-    hipLaunchKernelGGL(k_mark_list, dim3((num_list + 255) / 256), dim3(256), 0, st, flag, x.tau,
-                       x.band, d_list, num_list, S);
+    hipLaunchKernelGGL(k_mark_list, dim3((num_list + 255) / 256), dim3(256), 0, st, flag, x.l.tau,
+                       x.l.band, d_list, num_list, S);
     return exact_route(ctx, d_top_pos, d_top_exact, d_top_f32, d_top_cnt, N, flag, d_scores, c,
                        total, sp, q, st);
 }

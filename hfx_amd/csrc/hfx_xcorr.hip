@@ -10,20 +10,19 @@
  * reaches HBM.
  *
  * Work decomposition: one workgroup (4 waves) per (spectrum, chunk of
- * XC_CHUNK candidates) tile; the spectrum is staged in LDS once per tile; each
- * wave scores one candidate at a time (ladder -> map -> dot).
+ * XP_CHUNK candidates) tile; the spectrum is staged in LDS once per tile; each
+ * wave scores several short candidates at a time (ladders -> maps -> claims).
+ * Large calls write each theoretical row once instead (hfx_rows.hip).
  */
-#include "hfx_cand.h"
+#include "hfx_pack.h"
 #include "hfx_rows.h"
 
 #include <stdlib.h>
 
 #include <mutex>
-#include <type_traits>
 
 #define XC_THREADS 256
 #define XC_WAVES (XC_THREADS / HFX_WAVE)
-#define XC_CHUNK 64
 
 /* largest s with off[s] <= t, off has n+1 entries, off[0] = 0 */
 __device__ __forceinline__ uint32_t find_segment(const uint64_t *off, uint32_t n, uint64_t t)
@@ -60,133 +59,12 @@ __device__ __forceinline__ uint32_t find_segment(const uint64_t *off, uint32_t n
 #define XP_WAVES (XP_THREADS / HFX_WAVE)
 #define XP_CHUNK 128
 #define XP_RANGE (XP_CHUNK / XP_WAVES) /* candidates a wave takes from a tile */
-#define XP_SLOTS 4
-/* b-ladder positions a wave's buffer holds (a chunk of its candidates at a
- * time; any one packable candidate has at most 64) */
-#define XP_LB 256
-/* Peaks outside [0, len) are clamped onto margin bins whose spectrum values
- * are zero (so they add 0 when claimed): singles onto bin -1 - 8 (lane & 7)
- * or len + 8 (lane & 7), triple centres onto -2 - 8 (lane & 7) or
- * len + 1 + 8 (lane & 7) (none of a clamped triple's nibbles is inside
- * [0, len)), spread over eight words a side so that they do not queue on
- * one address.  Clamped nibbles lie in [-59, len + 58]; the staged spectrum
- * is zero from bin -XP_PAD to len + XP_PAD and the map words cover bins
- * -XP_PAD .. xstr + XP_PAD. */
-#define XP_SPREAD 8
-#define XP_PAD (8 * XP_SPREAD)
 static_assert(XP_RANGE <= HFX_WAVE, "a wave's candidates fit its lanes");
-static_assert(XP_PAD % 8 == 0 && XP_PAD >= 8 * (XP_SPREAD - 1) + 3, "clamped peaks inside the margins");
-
-#define XP_MAGIC 12582912.0f /* 1.5 * 2^23: x + XP_MAGIC rounds x to an integer, ties to even */
-#define XP_MAGIC_BITS 0x4B400000u
-
-/* map words per candidate for spectra of at most xstr bins: bin x in word
- * (x + XP_PAD) / 8, x in [-XP_PAD, xstr + XP_PAD) */
-static uint32_t xp_map_words(uint32_t xstr) { return (xstr + 2 * XP_PAD + 7) / 8 + 1; }
 static size_t xp_lds_bytes(uint32_t xstr)
 {
     const size_t xf = ((size_t)xstr + 2 * XP_PAD + 3) & ~(size_t)3;
     return xf * 4 + (size_t)XP_WAVES * XP_SLOTS * xp_map_words(xstr) * 4 +
            (size_t)XP_WAVES * XP_LB * 4;
-}
-
-/* rint(mz / 1.0005079) as the bits of the integer-valued float q + 1.5 2^23
- * (q the correctly rounded quotient): u - XP_MAGIC_BITS is the bin for
- * |bin| < 2^22 */
-__device__ __forceinline__ uint32_t xp_binu(float mz)
-{
-    const float R = 1.0f / HFX_BIN_WIDTH_MONO;
-    return __float_as_uint(hfx_div(mz, HFX_BIN_WIDTH_MONO, R) + XP_MAGIC);
-}
-
-/* division by the fragment charge, correctly rounded (exact products for
- * 1, 2, 4) */
-template <int Z>
-__device__ __forceinline__ float xp_zdiv(float x)
-{
-    if constexpr (Z == 3) return hfx_div(x, 3.0f, 1.0f / 3.0f);
-    else return x * (1.0f / (float)Z);
-}
-
-/* weight of a nibble holding the OR of unary codes: 0, 1, 3, 7 -> 0, 10,
- * 25, 50, one byte lookup (v_perm: selector c picks byte c of the pool
- * 0x32000000:19000A00) */
-__device__ __forceinline__ float xp_weight(uint32_t nib)
-{
-    return (float)(__builtin_amdgcn_perm(0x32000000u, 0x19000A00u, nib) & 0xffu);
-}
-
-/* median of three unsigned (one v_med3_u32; the compiler does not fold a
- * min of a max with non-constant bounds) */
-__device__ __forceinline__ uint32_t xp_med3(uint32_t v, uint32_t lo, uint32_t hi)
-{
-    uint32_t r;
-    asm("v_med3_u32 %0, %1, %2, %3" : "=v"(r) : "v"(v), "v"(lo), "v"(hi));
-    return r;
-}
-
-/* the six bins of one ladder position at charge Z, in the FP32 operation
- * order of ion_series.cu:111-156 (addIonsAB, addIonsY), as xp_binu bits
- * (XP_MAGIC_BITS + bin) clamped into [lo, hi] (singles: a, b - H2O,
- * b - NH3, y - NH3) and [lo3, hi3] (triple centres b, y) */
-struct XpClamp {
-    uint32_t lo, hi, lo3, hi3;
-};
-template <int Z>
-__device__ __forceinline__ void xp_bins(float b, float y, const XpClamp &c, uint32_t (&u)[6])
-{
-    constexpr float zh = HFX_DEV_H * (float)Z;
-    constexpr float h2o = HFX_DEV_H2O / (float)Z, nh3 = HFX_DEV_NH3 / (float)Z;
-    const float ma = xp_zdiv<Z>((b - HFX_DEV_CO) + zh);
-    const float mb = xp_zdiv<Z>(b + zh);
-    const float my = xp_zdiv<Z>((y + HFX_DEV_H2O) + zh);
-    u[0] = xp_med3(xp_binu(ma), c.lo, c.hi);
-    u[1] = xp_med3(xp_binu(mb), c.lo3, c.hi3);
-    u[2] = xp_med3(xp_binu(mb - h2o), c.lo, c.hi);
-    u[3] = xp_med3(xp_binu(mb - nh3), c.lo, c.hi);
-    u[4] = xp_med3(xp_binu(my), c.lo3, c.hi3);
-    u[5] = xp_med3(xp_binu(my - nh3), c.lo, c.hi);
-}
-
-/* the words and nibble shifts of one position's peaks: singles at word
- * w[i], triples over words w[i], w[i] + 1 from nibble shift sh[i]; u[i] the
- * bits of the single's bin or of the bin before the triple's centre.  rowm
- * and xsm are the map row and the staged spectrum shifted back by
- * XP_MAGIC_BITS bins (never dereferenced themselves): the magic constant's
- * low three bits are zero, so u >> 3 and u & 7 give the word and nibble */
-struct XpPeaks {
-    uint32_t *w[6];
-    uint32_t sh[6];
-    uint32_t u[6];
-};
-
-__device__ __forceinline__ void xp_locate(uint32_t *rowm, const uint32_t (&u)[6], XpPeaks &pk)
-{
-#pragma unroll
-    for (int i = 0; i < 6; ++i) {
-        const uint32_t ui = (i == 1 || i == 4) ? u[i] - 1u : u[i];
-        pk.u[i] = ui;
-        pk.w[i] = rowm + (ui >> 3);
-        pk.sh[i] = (ui & 7u) * 4u;
-    }
-}
-
-/* ORs the peaks of one position into the candidate's map: the four
- * weight-10 peaks alone, each 25/50/25 triple as one 12-bit field over two
- * words */
-__device__ __forceinline__ void xp_put(const XpPeaks &pk)
-{
-#pragma unroll
-    for (int i = 0; i < 6; ++i) {
-        if (i == 1 || i == 4) {
-            const uint64_t t = (uint64_t)(HFX_CODE25 | HFX_CODE50 << 4 | HFX_CODE25 << 8)
-                               << pk.sh[i];
-            atomicOr(pk.w[i], (uint32_t)t);
-            atomicOr(pk.w[i] + 1, (uint32_t)(t >> 32));
-        } else {
-            atomicOr(pk.w[i], HFX_CODE10 << pk.sh[i]);
-        }
-    }
 }
 
 /* claims the peaks of one position (clearing them) and adds weight * x of
@@ -250,16 +128,6 @@ __device__ __forceinline__ float xp_segsum(float v, uint32_t kpos, uint32_t lane
     return v;
 }
 
-/* a pack: K candidates, candidate g on lanes [st_g, st_{g+1}), first
- * residue tc_g, residual r_g; wave-uniform values (no arrays: a lane picks
- * its candidate's by comparisons) */
-struct XpPack {
-    uint32_t K;
-    uint32_t st1, st2, st3, tot;
-    uint32_t lb0, lb1, lb2, lb3; /* first ladder position of each in the wave's buffer */
-    float r0, r1, r2, r3;
-};
-
 /* one pack at fragment charges 1..Z; the candidates' b ladders are in lb */
 template <int Z>
 __device__ __forceinline__ void xp_pack(uint32_t *maps, uint32_t mstr, const float *xs,
@@ -267,17 +135,11 @@ __device__ __forceinline__ void xp_pack(uint32_t *maps, uint32_t mstr, const flo
                                         float *out)
 {
     const uint32_t lane = hfx_lane();
-    const bool g1 = lane >= pk.st1, g2 = lane >= pk.st2, g3 = lane >= pk.st3;
-    const uint32_t slot = (uint32_t)g1 + (uint32_t)g2 + (uint32_t)g3;
-    const bool act = lane < pk.tot;
-    const uint32_t k0 = g3 ? pk.st3 : g2 ? pk.st2 : g1 ? pk.st1 : 0u;
-    const uint32_t k1 = g3 ? pk.tot : g2 ? min(pk.st3, pk.tot) : g1 ? min(pk.st2, pk.tot)
-                                                                   : min(pk.st1, pk.tot);
-    const uint32_t l0 = g3 ? pk.lb3 : g2 ? pk.lb2 : g1 ? pk.lb1 : pk.lb0;
-    const float rl = g3 ? pk.r3 : g2 ? pk.r2 : g1 ? pk.r1 : pk.r0;
-    const uint32_t kpos = lane - k0;
-    const float b = act ? lb[l0 + kpos] : 0.0f;
-    const float y = rl - b;
+    const XpLane ln = xp_lane(pk, lane);
+    const uint32_t slot = ln.slot, kpos = ln.kpos, k1 = ln.k1;
+    const bool act = ln.act;
+    const float b = act ? lb[ln.lad + kpos] : 0.0f;
+    const float y = ln.r - b;
     /* bin x of this lane's candidate map is in word rowp[x >> 3]; rowm and
      * xsm index by the xp_binu bits instead */
     uint32_t *rowm = maps + slot * mstr + XP_PAD / 8 - (XP_MAGIC_BITS >> 3);
@@ -382,12 +244,7 @@ __device__ __forceinline__ void xp_tile(float *xp_lds, float *mtab, float *score
     /* ladder positions of the packable candidates (long ones take none):
      * exclusive prefix over the wave's candidates */
     const uint32_t nl = lane < rn && pr.n <= HFX_WAVE && !general ? pr.n : 0u;
-    uint32_t incl = nl;
-#pragma unroll
-    for (int o = 1; o < HFX_WAVE; o <<= 1) {
-        const uint32_t v = __shfl_up(incl, o, 64);
-        if (lane >= (uint32_t)o) incl += v;
-    }
+    const uint32_t incl = xp_prefix(nl, lane);
     const uint32_t pofs = incl - nl;
     for (uint32_t p = 0; p < rn;) {
         /* a chunk [p, q) of candidates whose ladders fit the wave's buffer,
@@ -411,28 +268,7 @@ __device__ __forceinline__ void xp_tile(float *xp_lds, float *mtab, float *score
                 ++p;
                 continue;
             }
-            /* up to XP_SLOTS consecutive candidates of the chunk with at most
-             * 64 positions in all (wave-uniform); lanes past q are not taken */
-            const uint32_t n1 = hfx_take(pr.n, min(p + 1u, (uint32_t)HFX_WAVE - 1u));
-            const uint32_t n2 = hfx_take(pr.n, min(p + 2u, (uint32_t)HFX_WAVE - 1u));
-            const uint32_t n3 = hfx_take(pr.n, min(p + 3u, (uint32_t)HFX_WAVE - 1u));
-            const bool t1 = p + 1 < q && n0 + n1 <= HFX_WAVE;
-            const bool t2 = t1 && p + 2 < q && n0 + n1 + n2 <= HFX_WAVE;
-            const bool t3 = t2 && p + 3 < q && n0 + n1 + n2 + n3 <= HFX_WAVE;
-            XpPack pk;
-            pk.K = 1u + (uint32_t)t1 + (uint32_t)t2 + (uint32_t)t3;
-            pk.st1 = t1 ? n0 : 0xffffffffu;
-            pk.st2 = t2 ? n0 + n1 : 0xffffffffu;
-            pk.st3 = t3 ? n0 + n1 + n2 : 0xffffffffu;
-            pk.tot = n0 + (t1 ? n1 : 0u) + (t2 ? n2 : 0u) + (t3 ? n3 : 0u);
-            pk.lb0 = hfx_take(pofs, p) - base;
-            pk.lb1 = hfx_take(pofs, min(p + 1u, (uint32_t)HFX_WAVE - 1u)) - base;
-            pk.lb2 = hfx_take(pofs, min(p + 2u, (uint32_t)HFX_WAVE - 1u)) - base;
-            pk.lb3 = hfx_take(pofs, min(p + 3u, (uint32_t)HFX_WAVE - 1u)) - base;
-            pk.r0 = hfx_take(pr.r, p);
-            pk.r1 = hfx_take(pr.r, min(p + 1u, (uint32_t)HFX_WAVE - 1u));
-            pk.r2 = hfx_take(pr.r, min(p + 2u, (uint32_t)HFX_WAVE - 1u));
-            pk.r3 = hfx_take(pr.r, min(p + 3u, (uint32_t)HFX_WAVE - 1u));
+            const XpPack pk = xp_form(p, q, pr.n, pr.r, pofs, base);
             switch (zeff) {
             case 1: xp_pack<1>(maps, mstr, xs, lb, len, pk, out + p); break;
             case 2: xp_pack<2>(maps, mstr, xs, lb, len, pk, out + p); break;
@@ -495,35 +331,6 @@ __global__ void k_tile_count(uint32_t *tiles, Cands c, uint32_t num_spec, uint32
     if (s < num_spec) tiles[s] = (c.count(s) + chunk - 1) / chunk;
 }
 
-template <class Cands>
-__global__ void __launch_bounds__(XC_THREADS)
-    k_xcorr(float *scores, const uint64_t *tile_off, Cands c, hfx_spectra sp)
-{
-    __shared__ float xs[HFX_MAX_LEN];
-    __shared__ uint32_t maps[XC_WAVES][HFX_MAP_WORDS];
-    __shared__ float mtab[32];
-    const uint32_t S = sp.num_spec;
-    const uint64_t t = blockIdx.x;
-    if (t >= tile_off[S]) return;
-    const uint32_t s = find_segment(tile_off, S, t);
-    const uint32_t first = (uint32_t)(t - tile_off[s]) * XC_CHUNK;
-    const uint32_t cnt = min((uint32_t)XC_CHUNK, c.count(s) - first);
-    const uint32_t wave = threadIdx.x / HFX_WAVE;
-    uint32_t *map = maps[wave];
-    const uint32_t len = hfx_stage_spectrum(xs, mtab, c.db, sp, s);
-    for (uint32_t w = hfx_lane(); w < HFX_MAP_WORDS; w += HFX_WAVE) map[w] = 0;
-    __syncthreads();
-    const uint32_t zeff = c.zeff(sp.d_zmax[s]);
-    float *out = scores + c.base(s) + first;
-    for (uint32_t i = wave; i < cnt; i += XC_WAVES) {
-        c.peaks(map, mtab, s, first + i, len, zeff);
-        hfx_wave_sync();
-        const float sc = hfx_wave_dot_f32(map, xs, len);
-        hfx_wave_sync();
-        if (hfx_lane() == 0) out[i] = sc;
-    }
-}
-
 /* device scratch of the sparse XCorr for S spectra: per-spectrum tile counts
  * and their offsets */
 static size_t xc_scratch_bytes(uint32_t S) { return (size_t)S * 4 + ((size_t)S + 1) * 8 + 64; }
@@ -536,10 +343,7 @@ static int launch_xcorr(void *scratch, float *d_scores, const Cands &c, uint64_t
     if (S == 0 || total == 0) return HFX_OK;
     HFX_REQUIRE(sp->x_stride <= HFX_MAX_LEN, HFX_ERR_ARG,
                 "sparse XCorr: spectra of up to %d bins (x_stride %u)", HFX_MAX_LEN, sp->x_stride);
-    /* unmodified and modified candidates take the packed kernel */
-    constexpr bool PACK = std::is_same<Cands, HfxPlainCands>::value ||
-                          std::is_same<Cands, HfxModCands>::value;
-    const uint32_t chunk = PACK ? XP_CHUNK : XC_CHUNK;
+    const uint32_t chunk = XP_CHUNK;
     hipStream_t st = hfx_stream(stream);
     int rc;
     uint32_t *tiles = (uint32_t *)scratch;
@@ -550,14 +354,9 @@ static int launch_xcorr(void *scratch, float *d_scores, const Cands &c, uint64_t
     /* sum_s ceil(n_s / chunk) <= total / chunk + S */
     const uint64_t grid = (total + chunk - 1) / chunk + S;
     HFX_REQUIRE(grid < (1ull << 31), HFX_ERR_ARG, "xcorr: %llu tiles", (unsigned long long)grid);
-    if constexpr (PACK) {
-        hipLaunchKernelGGL(k_xcorr_pack<Cands>, dim3((uint32_t)grid), dim3(XP_THREADS),
-                           xp_lds_bytes(sp->x_stride), st, d_scores, tile_off, c, *sp,
-                           xp_map_words(sp->x_stride));
-    } else {
-        hipLaunchKernelGGL(k_xcorr<Cands>, dim3((uint32_t)grid), dim3(XC_THREADS), 0, st,
-                           d_scores, tile_off, c, *sp);
-    }
+    hipLaunchKernelGGL(k_xcorr_pack<Cands>, dim3((uint32_t)grid), dim3(XP_THREADS),
+                       xp_lds_bytes(sp->x_stride), st, d_scores, tile_off, c, *sp,
+                       xp_map_words(sp->x_stride));
     HFX_CHECK_LAUNCH();
     return HFX_OK;
 }
