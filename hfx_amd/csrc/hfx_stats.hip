@@ -12,35 +12,42 @@
  * scores of one bin form the range [C(k-1), C(k)) of the cumulative bin counts
  * C, and the kept count of bin k is that range's overlap with the cut.  One
  * workgroup per spectrum:
- *   1. min and max of the spectrum's scores (kept in LDS when they fit);
+ *   1. min and max of the spectrum's scores, kept in registers (the part past
+ *      EV_HOLD chunks is read again);
  *   2. key(x) = 0 for (x + 1) - min <= 4000, else ceil(((x + 1) - min) / w)
  *      - kbase (>= 1), counted per key in LDS (EV_KEYS keys per pass; a wider
- *      spread takes one pass per range of keys);
+ *      spread takes one pass per range of keys).  FP32 decides the key unless
+ *      the quotient lies within its error of an edge;
  *   3. a block scan of the counts gives every key's sorted range, hence the
  *      kept counts and the histogram points (x_k, log10(c_k / w));
- *   4. least squares in FP64, two passes: means, then centred sums.
- * The score array is read once from HBM (twice when a spectrum holds more than
- * EV_CACHE scores); the rest is LDS work.
+ *   4. least squares in FP64: sums about the middle of the key range.
  *
  * SP ions (IonSeries.hs:99-147, Match.hs:33-40): extractPeaks keeps the 200
  * largest values of the spectrum and folds them by max into bins i div 3; a
  * b or y ion matches when its bin round(m/z / bin width / 3) holds a value
- * above zero.  k_sp_peaks_w turns each spectrum into those flags (one bit
- * per bin; one wave per spectrum, the row in registers, the 200th value
- * selected bit by bit over the float bits by ballot counts; k_sp_peaks does
- * the same with a workgroup for rows longer than 3072); k_sp_* match one
- * peptide per thread along its FP32 b ladder.
+ * above zero.  sp_flags turns a spectrum into those flags (one bit per bin;
+ * one wave per spectrum, the row in registers, the 200th value selected bit by
+ * bit over the float bits by ballot counts; k_sp_peaks does the same with a
+ * workgroup for rows longer than 3072); sp_matches matches peptides along their
+ * FP32 b ladders, a position a lane.  k_sp_topn does both, a wave a spectrum.
  */
 #include "hfx_common.h"
 
 #include <math.h>
+#include <type_traits>
 
 #define ST_THREADS 256
 #define ST_WAVES (ST_THREADS / HFX_WAVE)
 
-#define EV_CACHE 8192               /* scores of a spectrum kept in LDS       */
+#define EV_THREADS 256
+#define EV_WAVES (EV_THREADS / HFX_WAVE)
+#define EV_CHUNK (4 * EV_THREADS)    /* scores a workgroup loads at once       */
+#define EV_HOLD 6                   /* chunks kept in registers               */
 #define EV_KEYS 1024                /* histogram keys per pass                */
-#define EV_KPT (EV_KEYS / ST_THREADS)
+#define EV_KPT (EV_KEYS / EV_THREADS)
+#define EV_COPY_SHIFT 4             /* 16 counts of a key where keys are few  */
+#define EV_MAGIC 12582912.0f        /* 1.5 * 2^23: adding it rounds to an integer */
+#define EV_MAGIC_BITS 0x4B400000u
 
 #define SP_TOP 200                  /* IonSeries.hs:104                       */
 #define SP_CACHE 8192               /* spectrum values kept in LDS            */
@@ -145,6 +152,28 @@ __device__ __forceinline__ double st_wsum_f64(double v)
     return __longlong_as_double(r);
 }
 
+/* least lo and greatest hi of the wave, in every lane */
+__device__ __forceinline__ void st_wave_minmax(float &lo, float &hi)
+{
+    auto step = [&](auto ctrl, auto rm) {
+        const uint32_t l = ST_DPP32(__float_as_uint(lo), __float_as_uint(lo), decltype(ctrl)::value,
+                                    decltype(rm)::value);
+        const uint32_t h = ST_DPP32(__float_as_uint(hi), __float_as_uint(hi), decltype(ctrl)::value,
+                                    decltype(rm)::value);
+        lo = fminf(lo, __uint_as_float(l));
+        hi = fmaxf(hi, __uint_as_float(h));
+    };
+    using std::integral_constant;
+    step(integral_constant<int, 0xB1>{}, integral_constant<int, 0xF>{});
+    step(integral_constant<int, 0x4E>{}, integral_constant<int, 0xF>{});
+    step(integral_constant<int, 0x141>{}, integral_constant<int, 0xF>{});
+    step(integral_constant<int, 0x140>{}, integral_constant<int, 0xF>{});
+    step(integral_constant<int, 0x142>{}, integral_constant<int, 0xA>{});
+    step(integral_constant<int, 0x143>{}, integral_constant<int, 0xC>{});
+    lo = __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(lo), 63));
+    hi = __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(hi), 63));
+}
+
 /* inclusive prefix sum of uint32 over the wave: row_shr 1, 2, 4, 8 within
  * rows of 16, then row_bcast15 / row_bcast31 across rows */
 __device__ __forceinline__ uint32_t st_wave_incl_scan32(uint32_t x)
@@ -170,30 +199,52 @@ struct EvArgs {
     const uint64_t *oa;
     const float *sb;    /* second score set, opt.      */
     const uint64_t *ob;
-    double w;
+    double w, rw, kb;   /* bin width, RN(1 / w), kbase */
     float perc;
 };
 
-#define EV_NSUM 6   /* sum dx, sum y, sum dx^2, sum dx y, points, kept */
+#define EV_NSUM 4   /* sum dx, sum y, sum dx^2, sum dx y */
 
 struct EvShared {
-    float cache[EV_CACHE];
-    uint32_t hist[EV_KEYS];       /* counts per key, then kept counts of the points */
-    uint16_t pkey[EV_KEYS];       /* key (less the range's base) of each point      */
-    double redd[EV_NSUM * ST_WAVES];
-    uint64_t redu[2 * ST_WAVES];
-    uint32_t red32[ST_WAVES];
+    uint32_t hist[EV_KEYS];       /* counts per key (several of each, if few) */
+    uint32_t red32[EV_KPT * EV_WAVES];
+    double redd[EV_NSUM * EV_WAVES];
+    uint64_t redu[2 * EV_WAVES];
+    uint32_t redn[2 * EV_WAVES];
 };
 
-/* one spectrum's view: n scores, the cut, the key map */
+/* sixteen bytes at any multiple of four */
+typedef float ev_f4 __attribute__((ext_vector_type(4), aligned(4)));
+
+/* one spectrum's view: n scores in chunks of EV_CHUNK (the first ca of set a,
+ * the rest of set b), the cut, the key map */
 struct EvSpec {
     const float *sa, *sb;
-    uint64_t na, n;
-    bool cached;
+    uint64_t na, nb, n;
+    uint64_t ca, nch;
     int64_t cb, ce;
     double h0, w, kb, x0;
+    double rw;          /* RN(1 / w) */
+    /* the key map in FP32: q = fma(v, rwf, cf) is within eps of the quotient
+     * ((v + 1) - h0) / w less a half; above qhi the score is kept for certain,
+     * below qlo filtered out, and within in of an integer its ceiling holds */
+    float rwf, cf, qlo, qhi, in;
 
-    double rw;   /* RN(1 / w) */
+    /* thread tid's four scores of chunk u; NaN past the end, which no key
+     * counts */
+    __device__ __forceinline__ ev_f4 load(uint64_t u) const
+    {
+        const bool a = u < ca;
+        const float *p = a ? sa : sb;
+        const uint64_t i = (a ? u : u - ca) * EV_CHUNK + 4 * threadIdx.x, m = a ? na : nb;
+        ev_f4 v = {NAN, NAN, NAN, NAN};
+        if (i + 4 <= m) v = *(const ev_f4 *)(p + i);
+        else if (i < m)
+#pragma unroll
+            for (int e = 0; e < 3; ++e)
+                if (i + e < m) v[e] = p[i + e];
+        return v;
+    }
 
     /* 0 for (x + 1) - min <= 4000 (filtered out, Statistics.hs:76), else
      * the bin ceiling(y / w) less kbase: monotone in x.  q = y * RN(1/w) is
@@ -219,172 +270,279 @@ struct EvSpec {
     }
 };
 
+/* a thread's part of the histogram points */
+struct EvSums {
+    double v[EV_NSUM];
+    uint32_t points, kept;
+};
+
+/* f(score, its place in the group) for every score of thread tid, group(first
+ * chunk) after each group of up to 8 chunks: H = EV_HOLD from the registers that hold
+ * them (none if H = 0), then two at a time from memory */
+template <int H, class F, class G>
+__device__ __forceinline__ void ev_each(const EvSpec &e, const ev_f4 (&v)[EV_HOLD], F &&f, G &&group)
+{
+    if constexpr (H > 0) {
+#pragma unroll
+        for (int u = 0; u < H; ++u) {
+            if ((uint64_t)u < e.nch) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) f(v[u][i], 4 * (u % 8) + i);
+            }
+            if (u % 8 == 7) group((uint64_t)u - 7);
+        }
+        if (H % 8) group((uint64_t)(H - H % 8));
+    }
+    for (uint64_t u = H; u < e.nch; u += 2) {
+        ev_f4 t[2];
+        t[0] = e.load(u);
+        t[1] = e.load(u + 1); /* past the last chunk: NaN */
+#pragma unroll
+        for (int i = 0; i < 8; ++i) f(t[i >> 2][i & 3], i);
+        group(u);
+    }
+}
+
 /* Histogram of keys [base, base + EV_KEYS); the kept part of each key's
  * scores becomes a point (x, logh), added to the thread's sums (x shifted by
- * x0).  Key 0 (filtered) is counted with the keys below the range, in
- * registers.  next = the smallest key above the range (~0 if none). */
-__device__ __forceinline__ void ev_window(const EvSpec &e, EvShared &sh, uint64_t base,
-                                          double *acc, uint64_t &next)
+ * x0).  ALL: no score lies above the range.  next = the smallest key above the
+ * range (~0 if none).  hist is clear, and left so if not ALL. */
+template <bool ALL>
+__device__ __forceinline__ void ev_window(const EvSpec &e, EvShared &sh, const ev_f4 (&v)[EV_HOLD],
+                                          uint64_t base, uint64_t khi, EvSums &acc, uint64_t &next)
 {
     const uint32_t tid = threadIdx.x, lane = tid % HFX_WAVE, wv = tid / HFX_WAVE;
-    for (uint32_t k = tid; k < EV_KEYS; k += ST_THREADS) sh.hist[k] = 0;
-    __syncthreads();
-    uint32_t below = 0;
-    uint64_t nxt = ~(uint64_t)0;
-    auto count = [&](float v) {
-        const uint64_t k = e.key(v);
-        if (k < base || k == 0)
-            ++below;
-        else if (k - base < EV_KEYS)
-            atomicAdd(&sh.hist[k - base], 1u);
-        else
+    /* few keys: up to 16 counts of each, by lane, so that fewer lanes of an
+     * atomic meet on a word */
+    uint32_t shl = 0;
+    if (ALL)
+        while (shl < EV_COPY_SHIFT && (khi + 1) << (shl + 1) <= EV_KEYS) ++shl;
+    const uint32_t cp = lane & ((1u << shl) - 1u);
+    uint64_t above = 0, nxt = ~(uint64_t)0;
+    auto add = [&](uint64_t k) {
+        if (k < base || k == 0) return;
+        if (ALL || k - base < EV_KEYS) {
+            atomicAdd(&sh.hist[(uint32_t)(k - base) << shl | cp], 1u);
+        } else {
+            ++above;
             nxt = k < nxt ? k : nxt;
-    };
-    if (e.cached) {
-        /* four scores per thread at a time: their keys' latencies overlap */
-        uint64_t i = tid;
-        for (; i + 3 * ST_THREADS < e.n; i += 4 * ST_THREADS) {
-            float v[4];
-#pragma unroll
-            for (int u = 0; u < 4; ++u) v[u] = sh.cache[i + u * ST_THREADS];
-#pragma unroll
-            for (int u = 0; u < 4; ++u) count(v[u]);
         }
-        for (; i < e.n; i += ST_THREADS) count(sh.cache[i]);
-    } else {
-        for (uint64_t i = tid; i < e.na; i += ST_THREADS) count(e.sa[i]);
-        for (uint64_t i = tid; i < e.n - e.na; i += ST_THREADS) count(e.sb[i]);
-    }
-    /* block: sum of below, min of nxt (one barrier pair; the first barrier
-     * also ends the counting) */
-    const uint64_t bsum = st_wave_reduce64(below, 0ull, [](uint64_t a, uint64_t b) { return a + b; });
-    nxt = st_wave_reduce64(nxt, ~0ull, [](uint64_t a, uint64_t b) { return a < b ? a : b; });
-    __syncthreads();
-    if (lane == 0) {
-        sh.redu[2 * wv] = bsum;
-        sh.redu[2 * wv + 1] = nxt;
-    }
-    __syncthreads();
-    uint64_t tb = sh.redu[0];
-    next = sh.redu[1];
-#pragma unroll
-    for (int i = 1; i < ST_WAVES; ++i) {
-        tb += sh.redu[2 * i];
-        next = sh.redu[2 * i + 1] < next ? sh.redu[2 * i + 1] : next;
-    }
-    /* sorted position of each key: exclusive block scan of the counts */
-    uint32_t c[EV_KPT];
-    uint32_t tot = 0;
-#pragma unroll
-    for (int j = 0; j < EV_KPT; ++j) {
-        c[j] = sh.hist[tid * EV_KPT + j];
-        tot += c[j];
-    }
-    const uint32_t incl = st_wave_incl_scan32(tot);
-    if (lane == HFX_WAVE - 1) sh.red32[wv] = incl;
-    __syncthreads();
-    uint32_t woff = 0;
-    for (uint32_t i = 0; i < wv; ++i) woff += sh.red32[i];
-    int64_t pre = (int64_t)tb + (int64_t)(woff + incl - tot);
-    uint32_t kept[EV_KPT], nv = 0;
-#pragma unroll
-    for (int j = 0; j < EV_KPT; ++j) {
-        const uint64_t kk = base + tid * EV_KPT + j;
-        const int64_t lo = pre, hi = pre + c[j];
-        pre = hi;
-        const int64_t kp = min(hi, e.ce) - max(lo, e.cb);
-        kept[j] = (kk >= 1 && kp > 0) ? (uint32_t)kp : 0u;
-        nv += kept[j] != 0;
-    }
-    /* the points, compacted in key order, one per thread at a time */
-    const uint32_t incl2 = st_wave_incl_scan32(nv);
-    __syncthreads();   /* every thread has read its counts and the first scan */
-    if (lane == HFX_WAVE - 1) sh.red32[wv] = incl2;
-    __syncthreads();
-    uint32_t o = incl2 - nv, npt = 0;
-#pragma unroll
-    for (int i = 0; i < ST_WAVES; ++i) {
-        o += i < (int)wv ? sh.red32[i] : 0u;
-        npt += sh.red32[i];
-    }
-#pragma unroll
-    for (int j = 0; j < EV_KPT; ++j)
-        if (kept[j]) {
-            sh.hist[o] = kept[j];
-            sh.pkey[o] = (uint16_t)(tid * EV_KPT + j);
-            ++o;
-        }
-    __syncthreads();
-    for (uint32_t i = tid; i < npt; i += ST_THREADS) {
-        /* logh = logBase 10 (count / w) = log h / log 10 (here log10: within
-         * an ulp) */
-        const double dx = e.xof(base + sh.pkey[i]) - e.x0;
-        const double y = log10((double)sh.hist[i] / e.w);
-        acc[0] += dx;
-        acc[1] += y;
-        acc[2] += dx * dx;
-        acc[3] += dx * y;
-        acc[4] += 1.0;
-        acc[5] += (double)sh.hist[i];
-    }
-    __syncthreads();   /* the next range reuses hist */
-}
-
-/* min and max of p[0..cnt), copied to dst[0..cnt) when COPY; 16-byte loads
- * over the aligned middle, up to eight per thread in flight */
-template <bool COPY>
-__device__ __forceinline__ void ev_scan(const float *p, uint64_t cnt, float *dst, float &lo,
-                                        float &hi)
-{
-    const uint32_t tid = threadIdx.x;
-    const uint64_t h = min(cnt, (uint64_t)(((16u - ((uint32_t)(uintptr_t)p & 15u)) & 15u) / 4u));
-    auto one = [&](uint64_t i, float v) {
-        lo = fminf(lo, v);
-        hi = fmaxf(hi, v);
-        if (COPY) dst[i] = v;
     };
-    if (tid < h) one(tid, p[tid]);
-    const float4 *p4 = (const float4 *)(p + h);
-    const uint64_t n4 = (cnt - h) / 4;
-    for (uint64_t i = tid; i < n4; i += 8 * ST_THREADS) {
-        float4 q[8];
-#pragma unroll
-        for (int u = 0; u < 8; ++u)
-            q[u] = i + u * ST_THREADS < n4 ? p4[i + u * ST_THREADS]
-                                           : make_float4(p[0], p[0], p[0], p[0]);
-#pragma unroll
-        for (int u = 0; u < 8; ++u) {
-            const uint64_t o = h + 4 * (i + u * ST_THREADS);
-            lo = fminf(fminf(lo, q[u].x), fminf(q[u].y, fminf(q[u].z, q[u].w)));
-            hi = fmaxf(fmaxf(hi, q[u].x), fmaxf(q[u].y, fmaxf(q[u].z, q[u].w)));
-            if (COPY && i + u * ST_THREADS < n4) {
-                dst[o] = q[u].x;
-                dst[o + 1] = q[u].y;
-                dst[o + 2] = q[u].z;
-                dst[o + 3] = q[u].w;
+    uint32_t edge = 0; /* scores of the group that FP32 cannot decide */
+    const uint32_t kofs = EV_MAGIC_BITS - 1u + (uint32_t)e.kb;
+    /* several ranges are rare: their passes read the scores again */
+    ev_each<ALL ? EV_HOLD : 0>(
+        e, v,
+        [&](float x, int i) {
+            /* the sum with 1.5 * 2^23 rounds quotient - 1/2: its ceiling less 1 */
+            const float q = __builtin_fmaf(x, e.rwf, e.cf), t = q + EV_MAGIC;
+            const bool ok = fabsf(q - (t - EV_MAGIC)) < e.in && q > e.qhi;
+            if (ok) {
+                const uint32_t k = __float_as_uint(t) - kofs; /* the key */
+                if constexpr (ALL) atomicAdd(&sh.hist[k << shl | cp], 1u); /* base 0, none above */
+                else add(k);
             }
+            edge |= (!ok && q >= e.qlo ? 1u : 0u) << i;
+        },
+        [&](uint64_t u) {
+            while (edge) {
+                const uint32_t i = (uint32_t)__builtin_ctz(edge);
+                edge &= edge - 1u;
+                const uint64_t c = u + i / 4;
+                const bool a = c < e.ca;
+                add(e.key((a ? e.sa : e.sb)[(a ? c : c - e.ca) * EV_CHUNK + 4 * threadIdx.x + i % 4]));
+            }
+        });
+    if constexpr (!ALL) {
+        above = st_wave_reduce64(above, 0ull, [](uint64_t a, uint64_t b) { return a + b; });
+        nxt = st_wave_reduce64(nxt, ~0ull, [](uint64_t a, uint64_t b) { return a < b ? a : b; });
+        if (lane == 0) {
+            sh.redu[2 * wv] = above;
+            sh.redu[2 * wv + 1] = nxt;
         }
     }
-    for (uint64_t t = h + 4 * n4 + tid; t < cnt; t += ST_THREADS) one(t, p[t]);
+    __syncthreads();
+    next = ~(uint64_t)0;
+    uint64_t ta = 0;
+    if constexpr (!ALL) {
+#pragma unroll
+        for (int i = 0; i < EV_WAVES; ++i) {
+            ta += sh.redu[2 * i];
+            next = sh.redu[2 * i + 1] < next ? sh.redu[2 * i + 1] : next;
+        }
+    }
+    /* thread t's keys are t + 256 j: the sorted position of each from a scan of
+     * the counts */
+    const uint32_t nj = max((uint32_t)EV_KPT >> shl, 1u);
+    auto counted = [&](uint32_t j) {
+        const uint32_t k = j * EV_THREADS + tid;
+        if (shl < 2) return sh.hist[k << shl] + (shl ? sh.hist[k << 1 | 1u] : 0u);
+        uint32_t n = 0;
+        if (k << shl < EV_KEYS)
+            for (uint32_t i = 0; i < 1u << shl; i += 4) {
+                const uint4 q = *(const uint4 *)&sh.hist[(k << shl) + ((i + 4 * k) & ((1u << shl) - 4u))];
+                n += q.x + q.y + q.z + q.w;
+            }
+        return n;
+    };
+#pragma unroll 1
+    for (uint32_t j = 0; j < nj; ++j) {
+        const uint32_t incl = st_wave_incl_scan32(counted(j));
+        if (lane == HFX_WAVE - 1) sh.red32[j * EV_WAVES + wv] = incl;
+    }
+    __syncthreads();
+    /* scores of keys below the range: all but those counted or above */
+    uint32_t pre = (uint32_t)(e.n - ta);
+    for (uint32_t i = 0; i < nj * EV_WAVES; ++i) pre -= sh.red32[i];
+#pragma unroll 1
+    for (uint32_t j = 0; j < nj; ++j) {
+        const uint32_t c = counted(j);
+        uint32_t o = pre + st_wave_incl_scan32(c) - c;
+#pragma unroll
+        for (uint32_t i = 0; i < EV_WAVES; ++i) {
+            o += i < wv ? sh.red32[j * EV_WAVES + i] : 0u;
+            pre += sh.red32[j * EV_WAVES + i];
+        }
+        if (!ALL) sh.hist[j * EV_THREADS + tid] = 0;
+        const int64_t kp = min((int64_t)o + c, e.ce) - max((int64_t)o, e.cb);
+        if (c && kp > 0) {
+            /* logh = logBase 10 (count / w) = log h / log 10 (here log10:
+             * within an ulp) */
+            const double dx = e.xof(base + j * EV_THREADS + tid) - e.x0;
+            const double y = log10((double)kp / e.w);
+            acc.v[0] += dx;
+            acc.v[1] += y;
+            acc.v[2] += dx * dx;
+            acc.v[3] += dx * y;
+            acc.points += 1;
+            acc.kept += (uint32_t)kp;
+        }
+    }
+    if constexpr (!ALL) __syncthreads(); /* the next range counts in hist again */
 }
 
-__global__ __launch_bounds__(ST_THREADS) void k_evfit(EvArgs a)
+/* spectrum s's sets */
+__device__ __forceinline__ EvSpec ev_sets(const EvArgs &a, uint32_t s)
 {
-    __shared__ EvShared sh;
-    const uint32_t s = blockIdx.x, tid = threadIdx.x, lane = tid % HFX_WAVE;
-    const uint32_t wv = tid / HFX_WAVE;
     EvSpec e;
     const uint64_t a0 = a.oa[s];
     e.na = a.oa[s + 1] - a0;
     e.sa = a.sa + a0;
-    uint64_t nb = 0;
+    e.nb = 0;
     e.sb = nullptr;
     if (a.sb) {
         const uint64_t b0 = a.ob[s];
-        nb = a.ob[s + 1] - b0;
+        e.nb = a.ob[s + 1] - b0;
         e.sb = a.sb + b0;
     }
-    e.n = e.na + nb;
+    e.n = e.na + e.nb;
+    e.ca = (e.na + EV_CHUNK - 1) / EV_CHUNK;
+    e.nch = e.ca + (e.nb + EV_CHUNK - 1) / EV_CHUNK;
+    return e;
+}
+
+/* its cut and key map, the scores lying in [lo, hi]; the key of hi */
+__device__ __forceinline__ uint64_t ev_map(EvSpec &e, const EvArgs &a, float lo, float hi)
+{
+    /* the cut (Statistics.hs:72-73): Float for cut_end, Double for cut_beg,
+     * halves to even */
+    const float fe = (1.0f - a.perc / 100.0f) * (float)e.n;
+    e.ce = min((int64_t)e.n, max((int64_t)0, (int64_t)__builtin_rintf(fe)));
+    e.cb = max((int64_t)0, (int64_t)rint((30.0 / 100.0) * (double)e.n));
+    e.h0 = (double)lo;
+    e.w = a.w;
+    e.rw = a.rw;
+    e.kb = a.kb;
+    /* rwf, cf and the sum are each within 2^-24 relative, of |v| rw, |cf| and no
+     * more than both together; eps is more than twice that.  Nothing is decided
+     * in FP32 where it passes a quarter of a bin. */
+    e.rwf = (float)e.rw;
+    e.cf = (float)((1.0 - e.h0) * e.rw - 0.5);
+    const float q4 = (float)(4000.0 * e.rw - 0.5);
+    const float eps =
+        (fmaxf(fabsf(lo), fabsf(hi)) * e.rwf + fabsf(e.cf) + fabsf(q4) + 1.0f) * 2.4e-7f * 2.0f;
+    const bool use = eps < 0.25f;
+    e.in = use ? 0.5f - eps : -1.0f;
+    e.qhi = q4 + eps;
+    e.qlo = use ? q4 - eps : -INFINITY;
+    /* sums are taken about x0, the middle of the key range of the scores,
+     * and centred at the end (no cancellation beyond the data's own spread) */
+    const uint64_t khi = e.key(hi);
+    e.x0 = khi ? 0.5 * (e.xof(1) + e.xof(khi)) : 0.0;
+    return khi;
+}
+
+/* the sums' least squares: over the block in wave order (deterministic) */
+__device__ __forceinline__ void ev_solve(const EvArgs &a, EvShared &sh, uint32_t s, double x0, EvSums acc)
+{
+    const uint32_t tid = threadIdx.x, lane = tid % HFX_WAVE, wv = tid / HFX_WAVE;
+    if (__ballot(acc.points != 0)) { /* often the first wave only */
+#pragma unroll
+        for (int q = 0; q < EV_NSUM; ++q) acc.v[q] = st_wsum_f64(acc.v[q]);
+        const uint64_t pk = st_wave_reduce64((uint64_t)acc.points << 32 | acc.kept, 0ull,
+                                             [](uint64_t x, uint64_t y) { return x + y; });
+        acc.points = (uint32_t)(pk >> 32);
+        acc.kept = (uint32_t)pk;
+    }
+    if (lane == 0) {
+#pragma unroll
+        for (int q = 0; q < EV_NSUM; ++q) sh.redd[EV_NSUM * wv + q] = acc.v[q];
+        sh.redn[2 * wv] = acc.points;
+        sh.redn[2 * wv + 1] = acc.kept;
+    }
+    __syncthreads();
+    if (tid == 0) {
+        double t[EV_NSUM];
+        uint32_t points = 0, kept = 0;
+        for (int i = 0; i < EV_WAVES; ++i) {
+            points += sh.redn[2 * i];
+            kept += sh.redn[2 * i + 1];
+        }
+#pragma unroll
+        for (int q = 0; q < EV_NSUM; ++q) {
+            t[q] = sh.redd[q];
+            for (int i = 1; i < EV_WAVES; ++i) t[q] += sh.redd[EV_NSUM * i + q];
+        }
+        const double m = (double)points;
+        const double sxx = t[2] - t[0] * t[0] / m;
+        const double sxy = t[3] - t[0] * t[1] / m;
+        const double beta = sxy / sxx;
+        const double mx = x0 + t[0] / m, my = t[1] / m;
+        a.fit[2 * s] = my - beta * mx;
+        a.fit[2 * s + 1] = beta;
+        if (a.npts) a.npts[s] = points;
+        if (a.nused) a.nused[s] = kept;
+    }
+}
+
+/* a spectrum whose keys take several ranges: a function of its own (the
+ * kernel's arguments through their segment), called last, so that its registers are not those of the usual case */
+__device__ __attribute__((noinline)) void
+ev_wide(const __attribute__((address_space(4))) void *args, EvShared &sh, uint32_t s, float lo, float hi)
+{
+    const EvArgs a = *(const EvArgs *)args;
+    EvSpec e = ev_sets(a, s);
+    const uint64_t khi = ev_map(e, a, lo, hi);
+    const ev_f4 v[EV_HOLD] = {};
+    EvSums acc{};
+    uint64_t next = 0;
+    for (uint64_t base = 0; base <= khi; base = next) /* no key passes khi */
+        ev_window<false>(e, sh, v, base, khi, acc, next);
+    ev_solve(a, sh, s, e.x0, acc);
+}
+
+/* A workgroup a spectrum, eight of them a CU (64 registers, 4.5 KiB of LDS):
+ * each step waits on the one before it (loads, least, counts, scan, logarithms,
+ * sums), so the CU is kept busy by the other workgroups.  With the scores in
+ * LDS four workgroups fitted, and keys in FP64 alone took a dozen FP64 operations
+ * a score.  10,000 spectra of 4600 scores on average: 162 -> 70 us (185 MB,
+ * 2.6 TB/s; 128 threads and 5120 scores held: 75, one wave and 4096: 110). */
+__global__ __launch_bounds__(EV_THREADS, 8) void k_evfit(EvArgs a)
+{
+    __shared__ __align__(16) EvShared sh;
+    const uint32_t s = blockIdx.x, tid = threadIdx.x, lane = tid % HFX_WAVE;
+    const uint32_t wv = tid / HFX_WAVE;
+    EvSpec e = ev_sets(a, s);
     auto no_fit = [&]() {
         if (tid == 0) {
             a.fit[2 * s] = NAN;
@@ -398,34 +556,29 @@ __global__ __launch_bounds__(ST_THREADS) void k_evfit(EvArgs a)
         no_fit();
         return;
     }
-    e.cached = e.n <= EV_CACHE;
 
-    /* 1. min, max (and the LDS copy) */
+    /* 1. the scores, their min and max */
+    ev_f4 v[EV_HOLD];
+#pragma unroll
+    for (int u = 0; u < EV_HOLD; ++u) v[u] = (uint64_t)u < e.nch ? e.load(u) : ev_f4{NAN, NAN, NAN, NAN};
+    for (uint32_t k = tid; k < EV_KEYS / 4; k += EV_THREADS)
+        ((uint4 *)sh.hist)[k] = make_uint4(0u, 0u, 0u, 0u);
     float lo = INFINITY, hi = -INFINITY;
-    if (e.cached) {
-        ev_scan<true>(e.sa, e.na, sh.cache, lo, hi);
-        if (nb) ev_scan<true>(e.sb, nb, sh.cache + e.na, lo, hi);
-    } else {
-        ev_scan<false>(e.sa, e.na, nullptr, lo, hi);
-        if (nb) ev_scan<false>(e.sb, nb, nullptr, lo, hi);
-    }
+    ev_each<EV_HOLD>(
+        e, v,
+        [&](float x, int) {
+            lo = fminf(lo, x);
+            hi = fmaxf(hi, x);
+        },
+        [](uint64_t) {});
     {
-        const uint64_t mm = ((uint64_t)__float_as_uint(hi) << 32) | __float_as_uint(lo);
-        const uint64_t r = st_wave_reduce64(mm, ((uint64_t)__float_as_uint(-INFINITY) << 32) |
-                                                    __float_as_uint(INFINITY),
-                                            [](uint64_t x, uint64_t y) {
-            const float l = fminf(__uint_as_float((uint32_t)x), __uint_as_float((uint32_t)y));
-            const float h = fmaxf(__uint_as_float((uint32_t)(x >> 32)),
-                                  __uint_as_float((uint32_t)(y >> 32)));
-            return ((uint64_t)__float_as_uint(h) << 32) | __float_as_uint(l);
-        });
-        __syncthreads();
-        if (lane == 0) sh.redu[wv] = r;
+        st_wave_minmax(lo, hi);
+        if (lane == 0) sh.redu[wv] = (uint64_t)__float_as_uint(hi) << 32 | __float_as_uint(lo);
         __syncthreads();
         lo = INFINITY;
         hi = -INFINITY;
 #pragma unroll
-        for (int i = 0; i < ST_WAVES; ++i) {
+        for (int i = 0; i < EV_WAVES; ++i) {
             lo = fminf(lo, __uint_as_float((uint32_t)sh.redu[i]));
             hi = fmaxf(hi, __uint_as_float((uint32_t)(sh.redu[i] >> 32)));
         }
@@ -436,50 +589,18 @@ __global__ __launch_bounds__(ST_THREADS) void k_evfit(EvArgs a)
         return;
     }
 
-    /* the cut (Statistics.hs:72-73): Float for cut_end, Double for cut_beg,
-     * halves to even */
-    const float fe = (1.0f - a.perc / 100.0f) * (float)e.n;
-    e.ce = min((int64_t)e.n, max((int64_t)0, (int64_t)__builtin_rintf(fe)));
-    e.cb = max((int64_t)0, (int64_t)rint((30.0 / 100.0) * (double)e.n));
-    e.h0 = (double)lo;
-    e.w = a.w;
-    e.rw = 1.0 / a.w;
-    e.kb = fmax(floor(4000.0 / a.w) - 1.0, 0.0);
-    /* sums are taken about x0, the middle of the key range of the scores,
-     * and centred at the end (no cancellation beyond the data's own spread) */
-    const uint64_t khi = e.key(hi);
-    e.x0 = khi ? 0.5 * (e.xof(1) + e.xof(khi)) : 0.0;
+    const uint64_t khi = ev_map(e, a, lo, hi);
 
-    /* 2-3. histogram points, one pass per occupied range of EV_KEYS keys */
-    double acc[EV_NSUM] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
-    uint64_t next = 0;
-    for (uint64_t base = 0; base != ~(uint64_t)0; base = next) ev_window(e, sh, base, acc, next);
-
-    /* 4. least squares: sums over the block (wave order, deterministic) */
-#pragma unroll
-    for (int q = 0; q < EV_NSUM; ++q) acc[q] = st_wsum_f64(acc[q]);
-    __syncthreads();
-    if (lane == 0)
-#pragma unroll
-        for (int q = 0; q < EV_NSUM; ++q) sh.redd[EV_NSUM * wv + q] = acc[q];
-    __syncthreads();
-    if (tid == 0) {
-        double t[EV_NSUM];
-#pragma unroll
-        for (int q = 0; q < EV_NSUM; ++q) {
-            t[q] = sh.redd[q];
-            for (int i = 1; i < ST_WAVES; ++i) t[q] += sh.redd[EV_NSUM * i + q];
-        }
-        const double m = t[4];
-        const double sxx = t[2] - t[0] * t[0] / m;
-        const double sxy = t[3] - t[0] * t[1] / m;
-        const double beta = sxy / sxx;
-        const double mx = e.x0 + t[0] / m, my = t[1] / m;
-        a.fit[2 * s] = my - beta * mx;
-        a.fit[2 * s + 1] = beta;
-        if (a.npts) a.npts[s] = (uint32_t)m;
-        if (a.nused) a.nused[s] = (uint64_t)t[5];
+    /* 2-4. histogram points and their least squares */
+    if (khi >= EV_KEYS) {
+        __syncthreads(); /* redu is written again */
+        ev_wide((const __attribute__((address_space(4))) void *)__builtin_amdgcn_kernarg_segment_ptr(), sh, s, lo, hi);
+        return;
     }
+    EvSums acc{};
+    uint64_t next = 0;
+    ev_window<true>(e, sh, v, 0, khi, acc, next);
+    ev_solve(a, sh, s, e.x0, acc);
 }
 
 /* Statistics.hs:41: E = 10 ** (alpha + beta * (score / 10000)) */
@@ -567,76 +688,132 @@ __global__ __launch_bounds__(ST_THREADS) void k_sp_peaks(uint32_t *on, uint32_t 
 #define SPW_MAXE 48                                          /* values per lane */
 #define SPW_WORDS ((SPW_MAXE * HFX_WAVE / 3 + 1 + 31) / 32)     /* 33 flag words  */
 
-/* k_sp_peaks for rows of at most E * 64 values (E <= SPW_MAXE): one wave per
- * spectrum, the row in registers (value j of a lane is position lane + 64 j,
- * 0 past the row, which no count sees), every count a ballot; the flag words
- * go through LDS. */
+/* k_sp_peaks' flags for a row of L <= E * 64 values (E <= SPW_MAXE, a multiple
+ * of 4) by one wave: the row in registers (values 4 q .. 4 q + 3 of a lane are
+ * positions 256 q + 4 lane + 0 .. 3, 0 past the row, which no count sees), every
+ * count a ballot.  The 200th value is found bit by bit; once 64 values or fewer
+ * share its leading bits -- a dozen steps, where a spectrum's largest value and
+ * its 200th differ by a few octaves -- those go one to a lane, and a step is one
+ * ballot instead of E.  fw: the wave's flag words, clear; u: 64 words of LDS. */
 template <int E>
-__global__ __launch_bounds__(ST_THREADS) void k_sp_peaks_w(uint32_t *on, uint32_t W,
-                                                            hfx_spectra sp)
+__device__ __forceinline__ void sp_flags(uint32_t *fw, uint32_t *u, const float *row, uint32_t L)
 {
-    __shared__ uint32_t words[ST_WAVES * SPW_WORDS];
-    const uint32_t wv = threadIdx.x / HFX_WAVE, lane = threadIdx.x % HFX_WAVE;
-    const uint32_t s = blockIdx.x * ST_WAVES + wv;
-    uint32_t *fw = words + wv * SPW_WORDS;
-    for (uint32_t k = lane; k < SPW_WORDS; k += HFX_WAVE) fw[k] = 0;
-    __syncthreads();
-    const bool live = s < sp.num_spec;
-    const uint32_t L = live ? min(min(sp.d_len[s], sp.x_stride), (uint32_t)(E * HFX_WAVE)) : 0u;
-    const float *row = sp.d_x + (size_t)(live ? s : 0) * sp.x_stride;
-    float v[E];
-#pragma unroll
-    for (int j = 0; j < E; ++j) {
-        /* unconditional loads (past the row: its first value, discarded) */
-        const uint32_t i = lane + HFX_WAVE * j;
-        const float t = row[i < L ? i : 0u];
-        v[j] = i < L ? t : 0.0f;
-    }
+    const uint32_t lane = hfx_lane();
     uint32_t kv[E];
 #pragma unroll
-    for (int j = 0; j < E; ++j) kv[j] = sp_key(v[j]);
-    uint32_t P = 0;
+    for (int q = 0; q < E / 4; ++q) {
+        const uint32_t i = 4 * (HFX_WAVE * q + lane);
+        ev_f4 t = {0.0f, 0.0f, 0.0f, 0.0f};
+        if (i + 4 <= L) t = *(const ev_f4 *)(row + i);
+        else if (i < L)
 #pragma unroll
-    for (int j = 0; j < E; ++j) P += __popcll(__builtin_amdgcn_ballot_w64(kv[j] != 0));
-    uint32_t T = 0, need = 0;
-    const bool all_pos = P <= SP_TOP;
-    if (!all_pos) {
-        /* T = key of the 200th largest value, bit by bit from the top */
-        for (int bit = 30; bit >= 0; --bit) {
+            for (int e = 0; e < 3; ++e)
+                if (i + e < L) t[e] = row[i + e];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) kv[4 * q + e] = __float_as_uint(t[e]);
+    }
+    uint32_t P = 0, top = 0;
+#pragma unroll
+    for (int j = 0; j < E; ++j) {
+        kv[j] = sp_key(__uint_as_float(kv[j]));
+        P += __popcll(__builtin_amdgcn_ballot_w64(kv[j] != 0));
+        top = max(top, kv[j]);
+    }
+    uint32_t T = 1, need = 0, eq = 0; /* all positive values */
+    if (P > SP_TOP) {
+#pragma unroll
+        for (int m = 1; m < HFX_WAVE; m <<= 1) top = max(top, (uint32_t)__shfl_xor((int)top, m, 64));
+        top = __builtin_amdgcn_readfirstlane(top);
+        /* T: the largest with ge = #{key >= T} >= 200; hi = #{key >= T + 2^(bit + 1)} */
+        T = 0;
+        uint32_t ge = P, hi = 0;
+        int bit = 31 - __builtin_clz(top);
+        for (; bit >= 0 && ge - hi > HFX_WAVE; --bit) {
             const uint32_t cand = T | (1u << bit);
             uint32_t c = 0;
 #pragma unroll
             for (int j = 0; j < E; ++j) c += __popcll(__builtin_amdgcn_ballot_w64(kv[j] >= cand));
-            if (c >= SP_TOP) T = cand;
+            if (c >= SP_TOP) {
+                T = cand;
+                ge = c;
+            } else {
+                hi = c;
+            }
         }
-        uint32_t gt = 0;
+        if (bit >= 0) {
+            /* the ge - hi <= 64 keys of [T, T + 2^(bit + 1)), one to a lane */
+            const uint32_t end = T + (2u << bit), lo = max(T, 1u);
+            const uint64_t below = __lanemask_lt();
+            uint32_t at = 0;
 #pragma unroll
-        for (int j = 0; j < E; ++j) gt += __popcll(__builtin_amdgcn_ballot_w64(kv[j] > T));
-        need = SP_TOP - gt;
-    }
-    /* ties of T in position order: rows in order, lanes in order within */
-    const uint64_t below = __lanemask_lt();
-    uint32_t base = 0;
-#pragma unroll
-    for (int j = 0; j < E; ++j) {
-        const uint32_t k = kv[j];
-        bool sel;
-        if (all_pos) {
-            sel = k != 0;
+            for (int j = 0; j < E; ++j) {
+                const bool in = kv[j] >= lo && kv[j] < end;
+                const uint64_t m = __builtin_amdgcn_ballot_w64(in);
+                if (in) u[at + (uint32_t)__popcll(m & below)] = kv[j];
+                at += (uint32_t)__popcll(m);
+            }
+            hfx_wave_sync();
+            const uint32_t w = lane < at ? u[lane] : 0u;
+            for (; bit >= 0; --bit) {
+                const uint32_t cand = T | (1u << bit);
+                const uint32_t c = hi + (uint32_t)__popcll(__builtin_amdgcn_ballot_w64(w >= cand));
+                if (c >= SP_TOP) {
+                    T = cand;
+                    ge = c;
+                }
+            }
+            eq = (uint32_t)__popcll(__builtin_amdgcn_ballot_w64(w == T));
         } else {
-            const uint64_t m = __builtin_amdgcn_ballot_w64(k == T);
-            sel = k > T || (k == T && base + (uint32_t)__popcll(m & below) < need);
-            base += (uint32_t)__popcll(m);
+            eq = ge - hi; /* of [T, T + 1) */
         }
-        if (sel) {
-            const uint32_t t = (lane + HFX_WAVE * j) / 3;
-            atomicOr(&fw[t >> 5], 1u << (t & 31));
+        need = SP_TOP - (ge - eq);
+    }
+    auto flag = [&](int q, int e) {
+        const uint32_t t = (4 * (HFX_WAVE * q + lane) + e) / 3;
+        atomicOr(&fw[t >> 5], 1u << (t & 31));
+    };
+    if (need == eq) {
+#pragma unroll
+        for (int j = 0; j < E; ++j)
+            if (kv[j] >= T) flag(j / 4, j % 4);
+    } else {
+        /* ties of T past the 200: the lowest positions */
+        const uint64_t below = __lanemask_lt();
+        uint32_t base = 0;
+#pragma unroll
+        for (int q = 0; q < E / 4; ++q) {
+            uint32_t before = base;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const uint64_t m = __builtin_amdgcn_ballot_w64(kv[4 * q + e] == T);
+                before += (uint32_t)__popcll(m & below);
+                base += (uint32_t)__popcll(m);
+            }
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const uint32_t k = kv[4 * q + e];
+                if (k > T || (k == T && before < need)) flag(q, e);
+                before += k == T;
+            }
         }
     }
-    __syncthreads();
-    if (live)
-        for (uint32_t k = lane; k < W; k += HFX_WAVE)
-            on[(size_t)s * W + k] = k < SPW_WORDS ? fw[k] : 0u;
+    hfx_wave_sync();
+}
+
+template <int E>
+__global__ __launch_bounds__(ST_THREADS) void k_sp_peaks_w(uint32_t *on, uint32_t W,
+                                                            hfx_spectra sp)
+{
+    __shared__ uint32_t words[ST_WAVES * SPW_WORDS], und[ST_THREADS];
+    const uint32_t wv = threadIdx.x / HFX_WAVE, lane = threadIdx.x % HFX_WAVE;
+    const uint32_t s = blockIdx.x * ST_WAVES + wv;
+    if (s >= sp.num_spec) return;
+    uint32_t *fw = words + wv * SPW_WORDS;
+    for (uint32_t k = lane; k < SPW_WORDS; k += HFX_WAVE) fw[k] = 0;
+    hfx_wave_sync();
+    sp_flags<E>(fw, und + wv * HFX_WAVE, sp.d_x + (size_t)s * sp.x_stride,
+                min(min(sp.d_len[s], sp.x_stride), (uint32_t)(E * HFX_WAVE)));
+    for (uint32_t k = lane; k < W; k += HFX_WAVE) on[(size_t)s * W + k] = k < SPW_WORDS ? fw[k] : 0u;
 }
 
 struct SpArgs {
@@ -659,89 +836,210 @@ __device__ __forceinline__ uint32_t sp_on(const uint32_t *f, uint32_t npk, float
     return (f[i >> 5] >> (i & 31)) & 1u;
 }
 
-/* lookup (Location.hs:42-58) + matchIonSequence (IonSeries.hs:136-147) +
- * scoreSP (Match.hs:33-40) of peptide p against spectrum s */
-__device__ __forceinline__ void sp_match(const SpArgs &a, uint64_t m, uint32_t p, uint32_t s,
-                                         uint32_t nmod)
+/* Matches of a wave, SPM_ROWS at a time: lane i < SPM_ROWS holds match i.  Its
+ * lane sums the FP32 ladder (in order, as everywhere) into LDS, SPM_POS positions
+ * at a time; then the wave's lanes take one position each, whatever the peptides'
+ * lengths.  One thread a match took 70 us for 50,000 of them, most lanes waiting
+ * on the residues, masses and flags of the longest. */
+#define SPM_ROWS 16
+#define SPM_POS 32
+
+struct SpMatch {
+    uint32_t tc, n;   /* first residue, residues taken (Location.hs:42-58) */
+    uint32_t nz, npk; /* fragment charges, peak bins */
+    uint32_t nmod, s;
+    float r;
+    bool live;
+};
+
+struct SpLds {
+    float b[SPM_ROWS * SPM_POS];
+    uint8_t row[SPM_ROWS * SPM_POS];
+    uint32_t first[SPM_ROWS]; /* ladder position of b[0], were it this row's */
+    uint32_t n[SPM_ROWS], nz[SPM_ROWS], npk[SPM_ROWS], s[SPM_ROWS];
+    float r[SPM_ROWS];
+    uint32_t nb[SPM_ROWS], ny[SPM_ROWS];
+};
+
+/* peptide p against spectrum s, s < num_spec; live: p < num_pep */
+__device__ __forceinline__ SpMatch sp_get(const SpArgs &a, uint32_t p, uint32_t s, uint32_t nmod,
+                                          bool live)
 {
-    const uint32_t tc = a.db.d_tc[p], tn = a.db.d_tn[p];
-    const uint32_t ntake = (uint64_t)tn < a.db.num_ions ? tn - tc + 1 : tn - tc;
-    const float r = (a.db.d_r[p] + SP_H) + SP_H2O;
-    const uint32_t npk = min(a.len[s], a.stride) / 3 + 1;
-    const uint32_t *f = a.on + (size_t)s * a.W;
-    const uint32_t nz = max(a.zmax[s], 1u);
-    const uint64_t nI = (uint64_t)ntake * nz;
-    uint32_t nb = 0, ny = 0;
-    uint64_t j = 0;
-    for (uint32_t c = 1; c <= nz; ++c) {
-        const float cf = (float)c;
-        const float hc = SP_H * cf;
-        float pm = 0.0f;
-        for (uint32_t k = 0; k < ntake; ++k, ++j) {
-            pm = pm + a.db.d_mass[HFX_ACID_IDX(a.db.d_ions[tc + k])];
-            const float mz = (pm + hc) / cf;
-            if (j + 1 < nI) nb += sp_on(f, npk, mz, a.bw);     /* init */
-            if (j >= 1) ny += sp_on(f, npk, r - mz, a.bw);     /* tail */
+    SpMatch m{};
+    m.live = live;
+    if (!live) return m;
+    m.tc = a.db.d_tc[p];
+    const uint32_t tn = a.db.d_tn[p];
+    m.n = (uint64_t)tn < a.db.num_ions ? tn - m.tc + 1 : tn - m.tc;
+    m.r = (a.db.d_r[p] + SP_H) + SP_H2O;
+    m.npk = min(a.len[s], a.stride) / 3 + 1;
+    m.nz = max(a.zmax[s], 1u);
+    m.nmod = nmod;
+    m.s = s;
+    return m;
+}
+
+/* lookup + matchIonSequence (IonSeries.hs:136-147) + scoreSP (Match.hs:33-40) of
+ * cnt <= SPM_ROWS matches, results to out + i; flags(s) = words of spectrum s */
+template <class Flags>
+__device__ __forceinline__ void sp_matches(const SpArgs &a, SpLds &w, const float *mtab,
+                                           const SpMatch &m, uint32_t cnt, uint64_t out,
+                                           Flags &&flags)
+{
+    const uint32_t lane = hfx_lane();
+    const uint32_t n = lane < cnt && m.live ? m.n : 0u;
+    if (lane < SPM_ROWS) {
+        w.n[lane] = n;
+        w.nz[lane] = m.nz;
+        w.npk[lane] = m.npk;
+        w.s[lane] = m.s;
+        w.r[lane] = m.r;
+        w.nb[lane] = 0;
+        w.ny[lane] = 0;
+    }
+    uint32_t nmax = lane < SPM_ROWS ? n : 0u;
+#pragma unroll
+    for (uint32_t o = 1; o < SPM_ROWS; o <<= 1) nmax = max(nmax, (uint32_t)__shfl_xor((int)nmax, o, 64));
+    nmax = __builtin_amdgcn_readfirstlane(nmax);
+    const uint8_t *res = a.db.d_ions + m.tc;
+    float pm = 0.0f;
+    for (uint32_t k0 = 0; k0 < nmax; k0 += SPM_POS) {
+        const uint32_t cn = n > k0 ? min(n - k0, (uint32_t)SPM_POS) : 0u;
+        uint32_t incl = lane < SPM_ROWS ? cn : 0u;
+#pragma unroll
+        for (uint32_t o = 1; o < SPM_ROWS; o <<= 1) {
+            const uint32_t y = __shfl_up(incl, o, 64);
+            if (lane >= o) incl += y;
         }
+        const uint32_t np = __builtin_amdgcn_readlane(incl, SPM_ROWS - 1);
+        if (cn) {
+            const uint32_t at = incl - cn;
+            w.first[lane] = k0 - at; /* modulo 2^32 */
+            for (uint32_t k = 0; k < cn; k += 8) {
+                uint32_t x[8];
+#pragma unroll
+                for (uint32_t j = 0; j < 8; ++j) x[j] = res[k0 + min(k + j, cn - 1u)];
+#pragma unroll
+                for (uint32_t j = 0; j < 8; ++j)
+                    if (k + j < cn) {
+                        pm = pm + mtab[HFX_ACID_IDX(x[j])];
+                        w.b[at + k + j] = pm;
+                        w.row[at + k + j] = (uint8_t)lane;
+                    }
+            }
+        }
+        hfx_wave_sync();
+        for (uint32_t i = lane; i < np; i += HFX_WAVE) {
+            const uint32_t q = w.row[i], k = w.first[q] + i, nq = w.n[q], nz = w.nz[q];
+            const uint32_t npk = w.npk[q];
+            const uint32_t *f = flags(w.s[q]);
+            const float b = w.b[i], r = w.r[q];
+            uint32_t nb = 0, ny = 0;
+            for (uint32_t c = 1; c <= nz; ++c) {
+                const float cf = (float)c;
+                const float mz = (b + SP_H * cf) / cf;
+                if (c < nz || k + 1u < nq) nb += sp_on(f, npk, mz, a.bw);   /* init */
+                if (c > 1 || k > 0) ny += sp_on(f, npk, r - mz, a.bw);      /* tail */
+            }
+            if (nb) atomicAdd(&w.nb[q], nb);
+            if (ny) atomicAdd(&w.ny[q], ny);
+        }
+        hfx_wave_sync();
     }
-    a.nb[m] = nb;
-    a.ny[m] = ny;
-    a.tot[m] = (ntake - 1 + nmod) * 2;
+    hfx_wave_sync();
+    if (lane < cnt) {
+        a.nb[out + lane] = m.live ? w.nb[lane] : 0u;
+        a.ny[out + lane] = m.live ? w.ny[lane] : 0u;
+        a.tot[out + lane] = m.live ? (m.n - 1 + m.nmod) * 2 : 0u;
+    }
+    hfx_wave_sync(); /* the rows are set again by the next matches */
 }
 
-__device__ __forceinline__ void sp_none(const SpArgs &a, uint64_t m)
+__global__ __launch_bounds__(ST_THREADS) void k_sp_list(SpArgs a, const uint32_t *pep,
+                                                        const uint32_t *spec, const uint32_t *nmod,
+                                                        uint64_t M)
 {
-    a.nb[m] = 0;
-    a.ny[m] = 0;
-    a.tot[m] = 0;
-}
-
-__global__ void k_sp_list(SpArgs a, const uint32_t *pep, const uint32_t *spec,
-                          const uint32_t *nmod, uint64_t M)
-{
-    const uint64_t m = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (m >= M) return;
-    const uint32_t p = pep[m], s = spec[m];
-    if (p >= a.db.num_pep || s >= a.num_spec) {   /* 0xFFFFFFFF: no peptide */
-        sp_none(a, m);
-        return;
+    __shared__ SpLds lds[ST_WAVES];
+    __shared__ float mtab[32];
+    const uint32_t wv = threadIdx.x / HFX_WAVE, lane = hfx_lane();
+    if (threadIdx.x < 32) mtab[threadIdx.x] = threadIdx.x < 26 ? a.db.d_mass[threadIdx.x] : 0.0f;
+    __syncthreads();
+    const uint64_t m0 = ((uint64_t)blockIdx.x * ST_WAVES + wv) * SPM_ROWS;
+    if (m0 >= M) return;
+    const uint32_t cnt = (uint32_t)min(M - m0, (uint64_t)SPM_ROWS);
+    SpMatch m{};
+    if (lane < cnt) {
+        const uint32_t p = pep[m0 + lane], s = spec[m0 + lane];
+        /* 0xFFFFFFFF: no peptide */
+        m = sp_get(a, p, s, nmod ? nmod[m0 + lane] : 0u, p < a.db.num_pep && s < a.num_spec);
     }
-    sp_match(a, m, p, s, nmod ? nmod[m] : 0u);
+    sp_matches(a, lds[wv], mtab, m, cnt, m0, [&](uint32_t s) { return a.on + (size_t)s * a.W; });
 }
 
 /* top-N of an unmodified search: entry k of spectrum s is the window
  * position top_pos[s][k] (sorted peptide begin[s] + position) */
-__global__ void k_sp_topn(SpArgs a, const uint32_t *top_pos, const uint32_t *top_cnt,
-                          const uint32_t *begin, uint32_t N, uint32_t S)
-{
-    const uint64_t m = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (m >= (uint64_t)N * S) return;
-    const uint32_t s = (uint32_t)(m / N), k = (uint32_t)(m % N);
-    if (k >= top_cnt[s]) {
-        sp_none(a, m);
-        return;
+struct SpPlainTop {
+    const uint32_t *top_pos, *top_cnt, *begin;
+    uint32_t N;
+    __device__ __forceinline__ SpMatch get(const SpArgs &a, uint32_t s, uint32_t k) const
+    {
+        const bool live = k < top_cnt[s];
+        return sp_get(a, live ? a.db.d_idx_sorted[begin[s] + top_pos[(uint64_t)s * N + k]] : 0u, s, 0u,
+                      live);
     }
-    sp_match(a, m, a.db.d_idx_sorted[begin[s] + top_pos[m]], s, 0u);
-}
+};
 
 /* top-N of a modified search: entry k of spectrum s is modified peptide
  * mp_off[s] + top_pos[s][k]; matched on its unmodified peptide
  * (Search.hs:296-299), the printed length grows by its modified sites */
-__global__ void k_sp_topn_mod(SpArgs a, const uint32_t *top_pos, const uint32_t *top_cnt,
-                              const uint64_t *mp_off, uint32_t N, uint32_t S, hfx_modset ms)
-{
-    const uint64_t m = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (m >= (uint64_t)N * S) return;
-    const uint32_t s = (uint32_t)(m / N), k = (uint32_t)(m % N);
-    if (k >= top_cnt[s]) {
-        sp_none(a, m);
-        return;
+struct SpModTop {
+    const uint32_t *top_pos, *top_cnt;
+    const uint64_t *mp_off;
+    uint32_t N;
+    hfx_modset ms;
+    __device__ __forceinline__ SpMatch get(const SpArgs &a, uint32_t s, uint32_t k) const
+    {
+        if (k >= top_cnt[s]) return SpMatch{};
+        const uint64_t i = mp_off[s] + top_pos[(uint64_t)s * N + k];
+        const uint32_t md = ms.d_mpep_mod_idx[i];
+        uint32_t nmod = 0;
+        for (uint32_t q = 0; q < ms.num_ma; ++q) nmod += ms.d_mod_ma_count[(size_t)md * ms.num_ma + q];
+        return sp_get(a, ms.d_mpep_pep_idx[i], s, nmod, true);
     }
-    const uint64_t i = mp_off[s] + top_pos[m];
-    const uint32_t md = ms.d_mpep_mod_idx[i];
-    uint32_t nmod = 0;
-    for (uint32_t q = 0; q < ms.num_ma; ++q) nmod += ms.d_mod_ma_count[(size_t)md * ms.num_ma + q];
-    sp_match(a, m, ms.d_mpep_pep_idx[i], s, nmod);
+};
+
+/* a wave a spectrum: its N matches, the flags of its row found here (E > 0) or
+ * read from a.on (E = 0).  10,000 spectra of 2176 bins, top 5: 54 us, where the
+ * flags took 53 us (31 steps of 36 ballots) and the matches 70 (a thread each).
+ * The chains of reads and of select steps bound it, 24 waves a CU; 64 registers
+ * for 32 waves spill (61 us). */
+template <int E, class Top>
+__global__ __launch_bounds__(ST_THREADS) void k_sp_topn(SpArgs a, Top top, const float *x)
+{
+    __shared__ uint32_t words[ST_WAVES * SPW_WORDS], und[ST_THREADS];
+    __shared__ SpLds lds[ST_WAVES];
+    __shared__ float mtab[32];
+    const uint32_t wv = threadIdx.x / HFX_WAVE, lane = hfx_lane();
+    const uint32_t s = blockIdx.x * ST_WAVES + wv;
+    uint32_t *fw = words + wv * SPW_WORDS;
+    if constexpr (E > 0)
+        for (uint32_t k = lane; k < SPW_WORDS; k += HFX_WAVE) fw[k] = 0;
+    if (threadIdx.x < 32) mtab[threadIdx.x] = threadIdx.x < 26 ? a.db.d_mass[threadIdx.x] : 0.0f;
+    __syncthreads();
+    if (s >= a.num_spec) return;
+    /* the first matches' chain of reads starts before the row's */
+    SpMatch m{};
+    if (lane < min(top.N, (uint32_t)SPM_ROWS)) m = top.get(a, s, lane);
+    if constexpr (E > 0)
+        sp_flags<E>(fw, und + wv * HFX_WAVE, x + (size_t)s * a.stride,
+                    min(min(a.len[s], a.stride), (uint32_t)(E * HFX_WAVE)));
+    for (uint32_t k = 0; k < top.N; k += SPM_ROWS) {
+        const uint32_t cnt = min(top.N - k, (uint32_t)SPM_ROWS);
+        if (k && lane < cnt) m = top.get(a, s, k + lane);
+        sp_matches(a, lds[wv], mtab, m, cnt, (uint64_t)s * top.N + k, [&](uint32_t) {
+            return E > 0 ? (const uint32_t *)fw : a.on + (size_t)s * a.W;
+        });
+    }
 }
 
 /* ------------------------------------------------------------------ */
@@ -763,8 +1061,9 @@ extern "C" int hfx_evalue_fit(hfx_ctx *ctx, double *d_fit, uint32_t *d_npts, uin
                 "hfx_evalue_fit: cut-off percentage %g outside [0, 100]", (double)cutoff_perc);
     if (num_spec == 0) return HFX_OK;
     EvArgs a{d_fit, d_npts, d_nused, d_scores_a, d_off_a, d_scores_b, d_off_b,
-             (double)bin_width, cutoff_perc};
-    hipLaunchKernelGGL(k_evfit, dim3(num_spec), dim3(ST_THREADS), 0, hfx_stream(stream), a);
+             (double)bin_width, 1.0 / bin_width,
+             fmax(floor(4000.0 / bin_width) - 1.0, 0.0), cutoff_perc};
+    hipLaunchKernelGGL(k_evfit, dim3(num_spec), dim3(EV_THREADS), 0, hfx_stream(stream), a);
     HFX_CHECK_LAUNCH();
     return HFX_OK;
 }
@@ -785,6 +1084,18 @@ extern "C" int hfx_evalues(hfx_ctx *ctx, double *d_ev, const double *d_fit,
 
 extern "C" uint32_t hfx_sp_peak_words(uint32_t x_stride) { return (x_stride / 3 + 1 + 31) / 32; }
 
+/* run(values per lane) for rows that a wave holds; 0 for longer ones */
+template <class F>
+static int sp_rows(const hfx_spectra *sp, F &&run)
+{
+    const uint32_t rows = (sp->x_stride + HFX_WAVE - 1) / HFX_WAVE;
+    if (rows <= 12) return run(std::integral_constant<int, 12>{});
+    if (rows <= 24) return run(std::integral_constant<int, 24>{});
+    if (rows <= 36) return run(std::integral_constant<int, 36>{});
+    if (rows <= SPW_MAXE) return run(std::integral_constant<int, SPW_MAXE>{});
+    return 0;
+}
+
 extern "C" int hfx_sp_peaks(hfx_ctx *ctx, uint32_t *d_on, uint32_t words, const hfx_spectra *sp,
                             void *stream)
 {
@@ -798,22 +1109,14 @@ extern "C" int hfx_sp_peaks(hfx_ctx *ctx, uint32_t *d_on, uint32_t words, const 
                 3u * (32u * SP_WORDS - 1u) + 2u);
     if (sp->num_spec == 0) return HFX_OK;
     const dim3 gw((sp->num_spec + ST_WAVES - 1) / ST_WAVES);
-    const uint32_t rows = (sp->x_stride + HFX_WAVE - 1) / HFX_WAVE;
-    if (rows <= 12)
-        hipLaunchKernelGGL(k_sp_peaks_w<12>, gw, dim3(ST_THREADS), 0, hfx_stream(stream), d_on,
-                           words, *sp);
-    else if (rows <= 24)
-        hipLaunchKernelGGL(k_sp_peaks_w<24>, gw, dim3(ST_THREADS), 0, hfx_stream(stream), d_on,
-                           words, *sp);
-    else if (rows <= 36)
-        hipLaunchKernelGGL(k_sp_peaks_w<36>, gw, dim3(ST_THREADS), 0, hfx_stream(stream), d_on,
-                           words, *sp);
-    else if (rows <= SPW_MAXE)
-        hipLaunchKernelGGL(k_sp_peaks_w<SPW_MAXE>, gw, dim3(ST_THREADS), 0, hfx_stream(stream),
-                           d_on, words, *sp);
-    else
-        hipLaunchKernelGGL(k_sp_peaks, dim3(sp->num_spec), dim3(ST_THREADS), 0,
+    const int rc = sp_rows(sp, [&](auto e) {
+        hipLaunchKernelGGL(k_sp_peaks_w<decltype(e)::value>, gw, dim3(ST_THREADS), 0,
                            hfx_stream(stream), d_on, words, *sp);
+        return 1;
+    });
+    if (!rc)
+        hipLaunchKernelGGL(k_sp_peaks, dim3(sp->num_spec), dim3(ST_THREADS), 0, hfx_stream(stream),
+                           d_on, words, *sp);
     HFX_CHECK_LAUNCH();
     return HFX_OK;
 }
@@ -851,22 +1154,45 @@ extern "C" int hfx_sp_ions(hfx_ctx *ctx, uint32_t *d_nb, uint32_t *d_ny, uint32_
     if (rc) return rc;
     HFX_REQUIRE(d_pep && d_spec, HFX_ERR_ARG, "hfx_sp_ions: null match list");
     if (num_match == 0) return HFX_OK;
-    hipLaunchKernelGGL(k_sp_list, dim3((unsigned)((num_match + 255) / 256)), dim3(256), 0,
+    const uint64_t per = (uint64_t)ST_WAVES * SPM_ROWS;
+    hipLaunchKernelGGL(k_sp_list, dim3((unsigned)((num_match + per - 1) / per)), dim3(ST_THREADS), 0,
                        hfx_stream(stream), a, d_pep, d_spec, d_nmod, num_match);
     HFX_CHECK_LAUNCH();
     return HFX_OK;
 }
 
-static int sp_topn_flags(hfx_ctx *ctx, const hfx_spectra *sp, uint32_t **on, uint32_t *W,
-                         void *stream)
+/* the matches of every spectrum's top N: rows that a wave holds in one launch
+ * without scratch, longer ones through their flags in scratch */
+template <class Top>
+static int sp_topn(hfx_ctx *ctx, uint32_t *d_nb, uint32_t *d_ny, uint32_t *d_total, const Top &top,
+                   const hfx_db *db, const hfx_spectra *sp, int mono, void *stream)
 {
-    HFX_REQUIRE(ctx && sp, HFX_ERR_ARG, "hfx_sp_ions_topn: null argument");
-    *W = hfx_sp_peak_words(sp->x_stride);
-    void *p = nullptr;
-    int rc = hfx_ctx_scratch(ctx, HFX_SLOT_STATS, (size_t)4 * *W * (sp->num_spec ? sp->num_spec : 1), &p);
+    HFX_REQUIRE(ctx, HFX_ERR_ARG, "hfx_sp_ions_topn: null argument");
+    const uint32_t W = hfx_sp_peak_words(sp->x_stride);
+    HFX_REQUIRE(W <= SP_WORDS, HFX_ERR_ARG, "hfx_sp_ions_topn: spectrum stride %u above %u",
+                sp->x_stride, 3u * (32u * SP_WORDS - 1u) + 2u);
+    const dim3 g((sp->num_spec + ST_WAVES - 1) / ST_WAVES), t(ST_THREADS);
+    SpArgs a;
+    /* any non-null flags: not read where the kernel finds them */
+    int rc = sp_args(a, d_nb, d_ny, d_total, (const uint32_t *)sp, W, db, sp, mono);
     if (rc) return rc;
-    *on = (uint32_t *)p;
-    return hfx_sp_peaks(ctx, *on, *W, sp, stream);
+    if (top.N == 0 || sp->num_spec == 0) return HFX_OK;
+    if (!sp_rows(sp, [&](auto e) {
+            a.on = nullptr;
+            hipLaunchKernelGGL((k_sp_topn<decltype(e)::value, Top>), g, t, 0, hfx_stream(stream), a,
+                               top, sp->d_x);
+            return 1;
+        })) {
+        void *p = nullptr;
+        rc = hfx_ctx_scratch(ctx, HFX_SLOT_STATS, (size_t)4 * W * sp->num_spec, &p);
+        if (rc) return rc;
+        rc = hfx_sp_peaks(ctx, (uint32_t *)p, W, sp, stream);
+        if (rc) return rc;
+        a.on = (const uint32_t *)p;
+        hipLaunchKernelGGL((k_sp_topn<0, Top>), g, t, 0, hfx_stream(stream), a, top, sp->d_x);
+    }
+    HFX_CHECK_LAUNCH();
+    return HFX_OK;
 }
 
 extern "C" int hfx_sp_ions_topn(hfx_ctx *ctx, uint32_t *d_nb, uint32_t *d_ny, uint32_t *d_total,
@@ -876,18 +1202,8 @@ extern "C" int hfx_sp_ions_topn(hfx_ctx *ctx, uint32_t *d_nb, uint32_t *d_ny, ui
 {
     HFX_REQUIRE(d_top_pos && d_top_cnt && d_begin && db && sp, HFX_ERR_ARG,
                 "hfx_sp_ions_topn: null argument");
-    uint32_t *on = nullptr, W = 0;
-    int rc = sp_topn_flags(ctx, sp, &on, &W, stream);
-    if (rc) return rc;
-    SpArgs a;
-    rc = sp_args(a, d_nb, d_ny, d_total, on, W, db, sp, mono);
-    if (rc) return rc;
-    const uint64_t M = (uint64_t)N * sp->num_spec;
-    if (M == 0) return HFX_OK;
-    hipLaunchKernelGGL(k_sp_topn, dim3((unsigned)((M + 255) / 256)), dim3(256), 0,
-                       hfx_stream(stream), a, d_top_pos, d_top_cnt, d_begin, N, sp->num_spec);
-    HFX_CHECK_LAUNCH();
-    return HFX_OK;
+    return sp_topn(ctx, d_nb, d_ny, d_total, SpPlainTop{d_top_pos, d_top_cnt, d_begin, N}, db, sp, mono,
+                   stream);
 }
 
 extern "C" int hfx_sp_ions_topn_mod(hfx_ctx *ctx, uint32_t *d_nb, uint32_t *d_ny,
@@ -898,17 +1214,6 @@ extern "C" int hfx_sp_ions_topn_mod(hfx_ctx *ctx, uint32_t *d_nb, uint32_t *d_ny
 {
     HFX_REQUIRE(d_top_pos && d_top_cnt && d_mp_off && ms && db && sp, HFX_ERR_ARG,
                 "hfx_sp_ions_topn_mod: null argument");
-    uint32_t *on = nullptr, W = 0;
-    int rc = sp_topn_flags(ctx, sp, &on, &W, stream);
-    if (rc) return rc;
-    SpArgs a;
-    rc = sp_args(a, d_nb, d_ny, d_total, on, W, db, sp, mono);
-    if (rc) return rc;
-    const uint64_t M = (uint64_t)N * sp->num_spec;
-    if (M == 0) return HFX_OK;
-    hipLaunchKernelGGL(k_sp_topn_mod, dim3((unsigned)((M + 255) / 256)), dim3(256), 0,
-                       hfx_stream(stream), a, d_top_pos, d_top_cnt, d_mp_off, N, sp->num_spec,
-                       *ms);
-    HFX_CHECK_LAUNCH();
-    return HFX_OK;
+    return sp_topn(ctx, d_nb, d_ny, d_total, SpModTop{d_top_pos, d_top_cnt, d_mp_off, N, *ms}, db, sp,
+                   mono, stream);
 }
