@@ -451,7 +451,7 @@ extern "C" int hfx_pepix_build(hfx_ctx *ctx, const hfx_db *db, uint32_t forms, u
  * (waits for the stream then): false when a quarter of the free memory does
  * not hold them, and the batch keeps the ladder or ion-list kernels.  The rows
  * of a level take RW_G KiB for sixteen peptides: 1.57 GB for 2.7 M. */
-static bool pepix_need_rows(hfx_pepix *ix, uint32_t L, hipStream_t st)
+static bool pepix_need_rows(hfx_pepix *ix, uint32_t L, uint32_t cus, hipStream_t st)
 {
     std::lock_guard<std::mutex> lk(g_rows_mu);
     const uint32_t nt = hfx_rows_tiles(ix->db.num_pep);
@@ -468,7 +468,7 @@ static bool pepix_need_rows(hfx_pepix *ix, uint32_t L, hipStream_t st)
     for (uint32_t l = 0; l < L && ok; ++l)
         if (!ix->rows.rows[l]) ok = hipMalloc((void **)&want.rows[l], level) == hipSuccess;
     want.ng = ix->rows.ng;
-    ok = ok && hfx_rows_build(&ix->db, &want, nullptr, (void *)st) == HFX_OK &&
+    ok = ok && hfx_rows_build(cus, &ix->db, &want, nullptr, (void *)st) == HFX_OK &&
          hipStreamSynchronize(st) == hipSuccess;
     for (uint32_t l = 0; l < HFX_MAX_CHARGE; ++l) {
         if (!want.rows[l]) continue;
@@ -979,7 +979,7 @@ static int bt_ready(hfx_batch *b, hipStream_t st)
     size_t fr = 0, tot = 0;
     HFX_CHECK_HIP(hipMemGetInfo(&fr, &tot));
     if (!b->dn_scratch && (uint64_t)b->S * 16384 > fr / 4) return HFX_OK;
-    if (!pepix_need_rows(const_cast<hfx_pepix *>(b->ix), b->L, st)) return HFX_OK;
+    if (!pepix_need_rows(const_cast<hfx_pepix *>(b->ix), b->L, (uint32_t)hfx_ctx_num_cus(b->ctx), st)) return HFX_OK;
     if (bt_dense_alloc(b) || (!b->rw_small && dalloc(&b->rw_small, 3 * (size_t)b->S))) {
         (void)hipGetLastError();
         return HFX_OK;

@@ -38,7 +38,8 @@ int hfx_rows_split(int mode, const hfx_spectra *sp, uint8_t *planes, float *qs, 
                    uint32_t *wide, void *stream);
 /* writes the rows of the wanted levels (non-null) and tiles (flags
  * [HFX_MAX_CHARGE][ntiles], null: all) */
-int hfx_rows_build(const hfx_db *db, const hfx_rows *r, const uint32_t *flags, void *stream);
+int hfx_rows_build(uint32_t cus, const hfx_db *db, const hfx_rows *r, const uint32_t *flags,
+                   void *stream);
 /* work items of the blocks bstart (num_spec + 1 entries, empty blocks at the
  * end) of CH candidates each, in scratch of hfx_rows_items_bytes(num_spec) */
 size_t hfx_rows_items_bytes(uint32_t S);

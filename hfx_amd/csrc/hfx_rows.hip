@@ -36,7 +36,7 @@
  * Scoring kernels, 20,000 proteins (2.7 M peptides), before (rows written per
  * block into LDS, or per pair) and after: three digits, 20,000 spectra 1,978 ->
  * 958 us; BF16, 6,000 spectra 1,937 -> 850 us; FP32 batched, 4,000 spectra
- * 10,114 -> 600 us.  Writing two levels' rows of the database takes 1.26 ms,
+ * 10,114 -> 600 us.  Writing two levels' rows of the database takes 0.87 ms,
  * once.
  */
 #include "hfx_cand.h"
@@ -193,51 +193,65 @@ __global__ void __launch_bounds__(256)
 /* Rows                                                                  */
 /* ------------------------------------------------------------------ */
 
-/* One workgroup of two waves a tile.  The nibble map of its sixteen rows (bin
- * x of a row in word 2 + x / 8, unary codes OR-ed = max per bin) takes 18.7 KiB
- * of LDS, so that eight workgroups fill a CU; a row stride of 36 mod 64 words
- * puts the 32 lanes of half an emission read on 64 different banks.  The b
- * ladders (one lane a peptide, sequential FP32 sums as everywhere) go through
- * LDS sixteen peptides x RB_CHUNK positions at a time, so that each thread then
- * takes one position whatever the peptides' lengths.  A peak whose bins all lie
- * outside the row goes to a word of its lane's own; a triple that straddles an
- * end spills into the row's margin words, which are not emitted. */
-#define RB_THREADS 128
+/* Persistent workgroups of four waves, a tile at a time.  The nibble map of its
+ * sixteen rows (bin x of a row in word 2 + x / 8, unary codes OR-ed = max per
+ * bin) takes 18.7 KiB of LDS, so that seven workgroups fill a CU; a row stride of
+ * 36 mod 64 words puts the 32 lanes of half an emission read on 64 different
+ * banks.  A tile is a chain: order, offsets, residues, masses, sums, peaks,
+ * codes.  The reads of the next three tiles are under way while one is written;
+ * masses are looked up a position a lane and only their sums (one lane a
+ * peptide, sequential FP32 as everywhere) go one after the other.  Ladders lie
+ * in LDS one peptide after the other, sixteen peptides x RB_CHUNK positions at a
+ * time, so that each thread then takes one position whatever the peptides'
+ * lengths.  A peak whose bins all lie outside the row goes to one of the words
+ * past it, by lane; a triple that straddles an end spills into the row's margin
+ * words.  Neither is emitted.  Words are cleared as they are emitted for the last
+ * time.  Rows go out past the caches: they are read again only after gigabytes
+ * of others.
+ * Two levels of 2.7 M peptides (2.2 GB written, 0.7 GB of scattered reads): 1,340
+ * us with a workgroup of two waves a tile, no reads ahead and a lane a peptide
+ * for residues, masses and sums; 880 us now (960 through the caches; 6
+ * workgroups a CU 50 us more, 5 150 more).  Memory at 3.3 TB/s and vector
+ * instructions (61 % of issue) share the rest. */
+#define RB_THREADS 256
+#define RB_WAVES (RB_THREADS / HFX_WAVE)
+#define RB_PER_CU 7
 #define RB_MSTR 292
-#define RB_CHUNK 64
+#define RB_CHUNK 48
 static_assert(RB_MSTR >= 2 + RW_MAXK / 8 + 2 && RB_MSTR % 64 == 36, "map row stride");
+static_assert(RB_THREADS == 16 * RW_ROWS && RB_CHUNK % 16 == 0, "sixteen threads a peptide");
 #define RB_MAGIC 12582912.0f /* 1.5 * 2^23: adding it rounds to an integer, ties to even */
 #define RB_MAGIC_BITS 0x4B400000u
 
+/* bin + RB_MAGIC_BITS: |mz| < 2^21 */
 __device__ __forceinline__ uint32_t rb_binu(float mz)
 {
-    return __float_as_uint(hfx_div(mz, HFX_BIN_WIDTH_MONO, 1.0f / HFX_BIN_WIDTH_MONO) + RB_MAGIC) -
-           RB_MAGIC_BITS;
+    return __float_as_uint(hfx_div(mz, HFX_BIN_WIDTH_MONO, 1.0f / HFX_BIN_WIDTH_MONO) + RB_MAGIC);
 }
 
-/* bins past the row's last may not fit the magic sum (2^22): such m/z are cut
- * to a value that is past the row as well */
+/* ladder masses are cut to this, whose peaks are past the row at any charge and
+ * do not pass the magic sum's 2^22 bins */
 #define RB_MZMAX 1.0e6f
+/* bins past the row that a lane's peaks outside it go to: words 276 .. 291 */
+#define RB_OUT(lane) (RW_MAXK + 16u + ((lane) & 7u) * 16u)
+static_assert(2 + RB_OUT(7u) / 8 + 1 < RB_MSTR, "the last word outside the row");
 
 struct RbPut {
-    uint32_t *row;   /* word of bin 0 */
-    uint32_t *trash; /* this thread's */
+    uint32_t *row; /* word of bin -16 */
+    uint32_t out;  /* RB_OUT + 16 */
     __device__ __forceinline__ void one(float mz) const
     {
-        const uint32_t u = rb_binu(mz);
-        uint32_t *w = u < RW_MAXK ? row + (u >> 3) : trash;
-        atomicOr(w, HFX_CODE10 << ((u & 7u) * 4u));
+        const uint32_t u = min(rb_binu(mz) - (RB_MAGIC_BITS - 16u), out);
+        atomicOr(row + (u >> 3), HFX_CODE10 << ((u << 2) & 31u));
     }
-    /* 25 at x - 1, 50 at x, 25 at x + 1 for x in [-1, RW_MAXK] */
+    /* 25 at x - 1, 50 at x, 25 at x + 1 */
     __device__ __forceinline__ void three(float mz) const
     {
-        const uint32_t u = rb_binu(mz) - 1u + 8u; /* bin x - 1, counted from -8 */
+        const uint32_t u = min(rb_binu(mz) - (RB_MAGIC_BITS - 15u), out); /* x - 1 */
         const uint64_t t = (uint64_t)(HFX_CODE25 | HFX_CODE50 << 4 | HFX_CODE25 << 8)
-                           << ((u & 7u) * 4u);
-        const bool in = u - 6u < RW_MAXK + 2u;
-        uint32_t *w = in ? row - 1 + (u >> 3) : trash;
-        atomicOr(w, (uint32_t)t);
-        if (t >> 32) atomicOr(w + 1, (uint32_t)(t >> 32));
+                           << ((u << 2) & 31u);
+        atomicOr(row + (u >> 3), (uint32_t)t);
+        if (t >> 32) atomicOr(row + (u >> 3) + 1, (uint32_t)(t >> 32));
     }
 };
 
@@ -250,10 +264,9 @@ __device__ __forceinline__ void rb_peaks(const RbPut &p, float b, float y)
         if constexpr (Z == 3) return hfx_div(x, 3.0f, 1.0f / 3.0f);
         else return x * (1.0f / (float)Z);
     };
-    auto cut = [](float x) { return fminf(fmaxf(x, -RB_MZMAX), RB_MZMAX); };
-    const float ma = cut(zdiv((b - HFX_DEV_CO) + zh));
-    const float mb = cut(zdiv(b + zh));
-    const float my = cut(zdiv((y + HFX_DEV_H2O) + zh));
+    const float ma = zdiv((b - HFX_DEV_CO) + zh);
+    const float mb = zdiv(b + zh);
+    const float my = zdiv((y + HFX_DEV_H2O) + zh);
     p.one(ma);
     p.three(mb);
     p.one(mb - h2o);
@@ -280,120 +293,171 @@ __device__ __forceinline__ uint32_t rb_pack(uint32_t a, uint32_t b)
     return ca | cb << 2;
 }
 
-__global__ void __launch_bounds__(RB_THREADS) k_rw_build(RbArgs a)
+__global__ void __launch_bounds__(RB_THREADS, RB_PER_CU) k_rw_build(RbArgs a)
 {
     __shared__ __align__(16) uint32_t maps[RW_ROWS * RB_MSTR];
     __shared__ float lb[RW_ROWS * RB_CHUNK];
     __shared__ uint8_t lrow[RW_ROWS * RB_CHUNK];
     __shared__ float mtab[32], rr[RW_ROWS];
-    __shared__ uint32_t trash[RB_THREADS + 1], tot;
-    __shared__ uint32_t topb;
-    const uint32_t t = blockIdx.x, tid = threadIdx.x, lane = hfx_lane(), wave = tid / HFX_WAVE;
-    uint32_t want = 0;
-#pragma unroll
-    for (uint32_t l = 0; l < HFX_MAX_CHARGE; ++l)
-        if (a.rows[l] && (!a.flags || rw_sload(a.flags, (uint64_t)l * a.ntiles + t) != 0u))
-            want |= 1u << l;
-    if (!want) return;
+    __shared__ float topb;
+    const uint32_t tid = threadIdx.x, lane = hfx_lane(), wave = tid / HFX_WAVE;
     for (uint32_t i = tid; i < RW_ROWS * RB_MSTR / 4; i += RB_THREADS)
         ((uint4 *)maps)[i] = make_uint4(0u, 0u, 0u, 0u);
     if (tid < 32) mtab[tid] = tid < 26 ? a.db.d_mass[tid] : 0.0f;
-    if (tid == 0) topb = 0;
-    /* lane r < 16 of wave 0: peptide r of the tile, its ladder so far */
-    uint32_t n = 0, tc = 0;
-    float r = 0.0f, bl = 0.0f;
-    const uint32_t q = t * RW_ROWS + tid;
-    if (tid < RW_ROWS && q < a.db.num_pep) {
-        const uint32_t pep = a.db.d_idx_sorted[q];
-        const uint32_t tn = a.db.d_tn[pep];
-        tc = a.db.d_tc[pep];
-        n = tn > tc ? tn - tc : 0u;
-        r = a.db.d_r[pep];
-    }
-    if (tid < RW_ROWS) rr[tid] = r;
-    uint32_t nmax = n;
-    for (uint32_t o = 8; o > 0; o >>= 1) nmax = max(nmax, (uint32_t)__shfl_xor((int)nmax, o, 64));
-    if (tid == 0) tot = nmax;
+    /* lane: peptide lane & 15 of a tile; thread: residues lk, lk + 16, ... of its
+     * peptide lr */
+    const uint32_t lr = tid >> 4, lk = tid & 15u;
+    const uint32_t G = gridDim.x;
+    auto order = [&](uint64_t t) {
+        const uint64_t q = t * RW_ROWS + (lane & 15u);
+        return q < a.db.num_pep ? a.db.d_idx_sorted[q] : 0xffffffffu;
+    };
+    struct Meta {
+        uint32_t tc, tn;
+        float r;
+    };
+    auto meta = [&](uint32_t pep) {
+        Meta m{0u, 0u, 0.0f};
+        if (pep != 0xffffffffu) m = Meta{a.db.d_tc[pep], a.db.d_tn[pep], a.db.d_r[pep]};
+        return m;
+    };
+    auto count = [](const Meta &m) { return m.tn > m.tc ? m.tn - m.tc : 0u; };
+    auto residues = [&](const Meta &m, uint32_t (&x)[2]) {
+        const uint32_t tc = (uint32_t)__shfl((int)m.tc, (int)lr, 64);
+        const uint32_t n = (uint32_t)__shfl((int)count(m), (int)lr, 64);
+#pragma unroll
+        for (uint32_t j = 0; j < 2; ++j) x[j] = lk + 16 * j < n ? a.db.d_ions[tc + lk + 16 * j] : 0u;
+    };
+    uint32_t want_next = 0;
+    auto wanted = [&](uint64_t t) {
+        uint32_t w = 0;
+#pragma unroll
+        for (uint32_t l = 0; l < HFX_MAX_CHARGE; ++l)
+            if (a.rows[l] && (!a.flags || rw_sload(a.flags, (uint64_t)l * a.ntiles + t) != 0u))
+                w |= 1u << l;
+        return w;
+    };
+    /* tile t: its residues; t + G: its offsets; t + 2 G: its order */
+    Meta m0 = meta(order(blockIdx.x)), m1 = meta(order((uint64_t)blockIdx.x + G));
+    uint32_t pep = order((uint64_t)blockIdx.x + 2ull * G), x[2];
+    residues(m0, x);
+    if (blockIdx.x < a.ntiles) want_next = wanted(blockIdx.x);
+    uint32_t turn = blockIdx.x;
     __syncthreads();
-    const uint32_t nch = (tot + RB_CHUNK - 1) / RB_CHUNK;
-    const uint32_t top = 31u - (uint32_t)__builtin_clz(want); /* highest level - 1 */
-    __syncthreads(); /* tot is reused below */
+    for (uint64_t t = blockIdx.x; t < a.ntiles; t += G, ++turn) {
+        const Meta m = m0;
+        const uint32_t want = want_next, x0 = x[0], x1 = x[1];
+        m0 = m1;
+        residues(m0, x);
+        m1 = meta(pep);
+        pep = order(t + 3ull * G);
+        if (t + G < a.ntiles) want_next = wanted(t + G);
+        if (!want) continue;
+        const uint32_t n = count(m);
+        uint32_t nmax = n;
+#pragma unroll
+        for (uint32_t o = 8; o > 0; o >>= 1) nmax = max(nmax, (uint32_t)__shfl_xor((int)nmax, o, 64));
+        nmax = __builtin_amdgcn_readfirstlane(nmax);
+        const uint32_t nch = max((nmax + RB_CHUNK - 1) / RB_CHUNK, 1u);
+        const uint32_t top = 31u - (uint32_t)__builtin_clz(want); /* highest level - 1 */
+        const uint32_t wv = (wave + turn) % RB_WAVES; /* the sums go round the SIMDs */
+        if (tid < RW_ROWS) rr[tid] = m.r;
+        float bl = 0.0f;
 
-    /* positions [c RB_CHUNK, ...) of the sixteen ladders into lb, row after row */
-    auto ladders = [&](uint32_t c) {
-        if (wave == 0) {
+        /* positions [c RB_CHUNK, ...) of the sixteen ladders into lb, row after
+         * row; their number */
+        auto ladders = [&](uint32_t c) {
             const uint32_t k0 = c * RB_CHUNK;
             const uint32_t cn = n > k0 ? min(n - k0, (uint32_t)RB_CHUNK) : 0u;
-            uint32_t incl = lane < RW_ROWS ? cn : 0u;
-            const uint32_t mine = incl;
+            uint32_t incl = cn;
 #pragma unroll
             for (uint32_t o = 1; o < RW_ROWS; o <<= 1) {
-                const uint32_t y = __shfl_up(incl, o, 64);
-                if (lane >= o) incl += y;
+                const uint32_t y = __shfl_up(incl, o, 16);
+                if ((lane & 15u) >= o) incl += y;
             }
-            const uint32_t at = incl - mine;
-            if (lane == RW_ROWS - 1) tot = incl;
-            if (lane < RW_ROWS) {
-                if (c == 0) bl = 0.0f;
-                const uint8_t *res = a.db.d_ions + tc + k0;
-                float mx = 0.0f;
-                for (uint32_t k = 0; k < cn; k += 8) {
-                    uint32_t x[8];
+            const uint32_t at = incl - cn;
+            const uint32_t la = (uint32_t)__shfl((int)at, (int)lr, 64);
+            const uint32_t ln = (uint32_t)__shfl((int)cn, (int)lr, 64);
+            const uint32_t ltc = (uint32_t)__shfl((int)m.tc, (int)lr, 64);
 #pragma unroll
-                    for (uint32_t j = 0; j < 8; ++j) x[j] = res[min(k + j, cn - 1u)];
-#pragma unroll
-                    for (uint32_t j = 0; j < 8; ++j)
-                        if (k + j < cn) {
-                            bl = bl + mtab[HFX_ACID_IDX(x[j])];
-                            lb[at + k + j] = bl;
-                            lrow[at + k + j] = (uint8_t)lane;
-                            mx = fmaxf(mx, fmaxf(bl, r - bl));
-                        }
-                }
-                atomicMax(&topb, __float_as_uint(mx));
-            }
-        }
-        __syncthreads();
-    };
-    for (uint32_t z = 1; z <= top + 1u; ++z) {
-        for (uint32_t c = 0; c < nch; ++c) {
-            if (z == 1 || nch > 1) ladders(c);
-            const uint32_t np = tot;
-            for (uint32_t i = tid; i < np; i += RB_THREADS) {
-                const uint32_t row = lrow[i];
-                const float b = lb[i], y = rr[row] - b;
-                const RbPut p{maps + row * RB_MSTR + 2, trash + tid};
-                switch (z) {
-                case 1: rb_peaks<1>(p, b, y); break;
-                case 2: rb_peaks<2>(p, b, y); break;
-                case 3: rb_peaks<3>(p, b, y); break;
-                default: rb_peaks<4>(p, b, y); break;
+            for (uint32_t j = 0; j < RB_CHUNK / 16; ++j) {
+                const uint32_t k = lk + 16 * j;
+                if (k < ln) {
+                    const uint32_t xr = c == 0 && j < 2 ? (j ? x1 : x0) : a.db.d_ions[ltc + k0 + k];
+                    lb[la + k] = mtab[HFX_ACID_IDX(xr)];
+                    lrow[la + k] = (uint8_t)lr;
                 }
             }
             __syncthreads();
-        }
-        /* groups the peaks reach: every bin lies below top / 1.0005 + 24 */
-        const float tf = fminf(__uint_as_float(topb), 1.0e6f);
-        const uint32_t ng = min(a.G, ((uint32_t)tf + 28u) / 256u + 1u);
-        if (z == 1 && tid == 0) a.ng[t] = (uint8_t)ng;
-        if ((want >> (z - 1u)) & 1u) {
-            const uint64_t slot = a.slots ? rw_sload(a.slots, (uint64_t)(z - 1u) * a.ntiles + t)
-                                          : (uint64_t)t;
-            rw_u32x4 *out = (rw_u32x4 *)(a.rows[z - 1u] + slot * ((size_t)a.G * 1024u));
-            const uint32_t *mrow = maps + (lane & 15u) * RB_MSTR + 2 + 2 * (lane >> 4);
-            for (uint32_t g = wave; g < ng; g += RB_THREADS / HFX_WAVE) {
-                rw_u32x4 v;
+            if (wv == 0) {
+                float mx = 0.0f;
+                if (lane < RW_ROWS) {
+                    if (c == 0) bl = 0.0f;
+                    for (uint32_t k = 0; k < cn; k += 8) {
+                        float v[8];
 #pragma unroll
-                for (uint32_t k = 0; k < 4; ++k) {
-                    /* the last group's words past the row hold no bins */
-                    const uint32_t w = g * 32 + k * 8;
-                    const uint2 ab = w < RW_MAXK / 8 ? *(const uint2 *)(mrow + w)
-                                                     : make_uint2(0u, 0u);
-                    v[k] = rb_pack(ab.x, ab.y);
+                        for (uint32_t j = 0; j < 8; ++j) v[j] = lb[at + min(k + j, cn - 1u)];
+#pragma unroll
+                        for (uint32_t j = 0; j < 8; ++j)
+                            if (k + j < cn) {
+                                bl = bl + v[j];
+                                lb[at + k + j] = bl;
+                                mx = fmaxf(mx, fmaxf(bl, m.r - bl));
+                            }
+                    }
                 }
-                out[g * 64 + lane] = v;
+#pragma unroll
+                for (uint32_t o = 8; o > 0; o >>= 1) mx = fmaxf(mx, __shfl_xor(mx, o, 64));
+                if (lane == 0) topb = c == 0 ? mx : fmaxf(topb, mx);
             }
-            if (z <= top) __syncthreads(); /* read before the next charge's peaks */
+            __syncthreads();
+            return (uint32_t)__builtin_amdgcn_readlane((int)incl, RW_ROWS - 1);
+        };
+        uint32_t np = 0;
+        for (uint32_t z = 1; z <= top + 1u; ++z) {
+            for (uint32_t c = 0; c < nch; ++c) {
+                if (z == 1 || nch > 1) np = ladders(c);
+                for (uint32_t i = tid; i < np; i += RB_THREADS) {
+                    const uint32_t row = lrow[i];
+                    const float b0 = lb[i];
+                    const float b = __builtin_amdgcn_fmed3f(b0, -RB_MZMAX, RB_MZMAX);
+                    const float y = __builtin_amdgcn_fmed3f(rr[row] - b0, -RB_MZMAX, RB_MZMAX);
+                    const RbPut p{maps + row * RB_MSTR, RB_OUT(lane) + 16u};
+                    switch (z) {
+                    case 1: rb_peaks<1>(p, b, y); break;
+                    case 2: rb_peaks<2>(p, b, y); break;
+                    case 3: rb_peaks<3>(p, b, y); break;
+                    default: rb_peaks<4>(p, b, y); break;
+                    }
+                }
+                __syncthreads();
+            }
+            /* groups the peaks reach: every bin lies below top / 1.0005 + 24 */
+            const float tf = fminf(topb, 1.0e6f);
+            const uint32_t ng = min(a.G, ((uint32_t)tf + 28u) / 256u + 1u);
+            if (z == 1 && tid == 0) a.ng[t] = (uint8_t)ng;
+            if ((want >> (z - 1u)) & 1u) {
+                const bool last = z > top;
+                const uint64_t slot = a.slots ? rw_sload(a.slots, (uint64_t)(z - 1u) * a.ntiles + t) : t;
+                rw_u32x4 *out = (rw_u32x4 *)(a.rows[z - 1u] + slot * ((size_t)a.G * 1024u));
+                uint32_t *mrow = maps + (lane & 15u) * RB_MSTR + 2 + 2 * (lane >> 4);
+                for (uint32_t g = wv; g < ng; g += RB_WAVES) {
+                    rw_u32x4 v;
+#pragma unroll
+                    for (uint32_t k = 0; k < 4; ++k) {
+                        /* the last group's words past the row hold no bins */
+                        const uint32_t w = g * 32 + k * 8;
+                        uint2 ab = make_uint2(0u, 0u);
+                        if (w < RW_MAXK / 8) {
+                            ab = *(const uint2 *)(mrow + w);
+                            if (last) *(uint2 *)(mrow + w) = make_uint2(0u, 0u);
+                        }
+                        v[k] = rb_pack(ab.x, ab.y);
+                    }
+                    __builtin_nontemporal_store(v, out + g * 64 + lane);
+                }
+                if (!last) __syncthreads(); /* read before the next charge's peaks */
+            }
         }
     }
 }
@@ -763,7 +827,8 @@ int hfx_rows_split(int mode, const hfx_spectra *sp, uint8_t *planes, float *qs, 
     return HFX_OK;
 }
 
-int hfx_rows_build(const hfx_db *db, const hfx_rows *r, const uint32_t *flags, void *stream)
+int hfx_rows_build(uint32_t cus, const hfx_db *db, const hfx_rows *r, const uint32_t *flags,
+                   void *stream)
 {
     RbArgs a{};
     a.db = *db;
@@ -774,7 +839,7 @@ int hfx_rows_build(const hfx_db *db, const hfx_rows *r, const uint32_t *flags, v
     a.ng = r->ng;
     a.G = r->G;
     if (r->ntiles)
-        hipLaunchKernelGGL(k_rw_build, dim3(r->ntiles), dim3(RB_THREADS), 0, hfx_stream(stream), a);
+        hipLaunchKernelGGL(k_rw_build, dim3(std::min(r->ntiles, cus * RB_PER_CU)), dim3(RB_THREADS), 0, hfx_stream(stream), a);
     HFX_CHECK_LAUNCH();
     return HFX_OK;
 }

@@ -448,7 +448,7 @@ static int xcorr_rows(hfx_ctx *ctx, float *d_scores, const uint64_t *d_off,
                               stream)) ||
         (rc = hfx_rows_mark(items, S, flags, nt, stream)) ||
         (rc = hfx_scan_offsets(ctx, (uint64_t *)r.slots, flags, (uint32_t)nf, stream)) ||
-        (rc = hfx_rows_build(db, &r, flags, stream)) ||
+        (rc = hfx_rows_build((uint32_t)hfx_ctx_num_cus(ctx), db, &r, flags, stream)) ||
         (rc = hfx_rows_scores(ctx, RW_I8X4, items, d_scores, d_off, d_begin, d_num, order,
                               cb.bstart, &r, planes, qs, &sq, CH, sp->d_zmax, stream, nullptr)) ||
         (rc = hfx_xcorr_wide(ctx, d_scores, d_off, d_begin, d_num, db, sp, wide, stream)))
