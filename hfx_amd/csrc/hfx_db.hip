@@ -499,41 +499,97 @@ extern "C" void sort_b40c_f(float *d_keys, uint32_t *d_vals, uint32_t N)
 /* Precursor windows                                                     */
 /* ------------------------------------------------------------------ */
 
-/* lower_bound / upper_bound over r[idx[i]] (thrust's permutation_iterator
- * form, filter.cu:101-115); idx == nullptr reads r directly (sorted copy). */
-__device__ __forceinline__ uint32_t lb_perm(const float *r, const uint32_t *idx, uint32_t n, float v)
+/* lower_bound of lo and upper_bound of hi over r[idx[i]] (thrust's
+ * permutation_iterator form, filter.cu:101-115); idx == nullptr reads r directly
+ * (sorted copy).  Both at once by a wave, a probe a lane: four steps for 2.7 M
+ * peptides, where a thread that bisects waits for 44 reads one after the other
+ * (250 spectra: 20 -> 5.0 us a launch; 10,000: 18.8 -> 12.8).  All lanes return both. */
+__device__ __forceinline__ void db_bounds_wave(const float *r, const uint32_t *idx, uint32_t n,
+                                               float lo, float hi, uint32_t *begin, uint32_t *end)
 {
-    uint32_t lo = 0, hi = n;
-    while (lo < hi) {
-        uint32_t mid = lo + ((hi - lo) >> 1);
-        float e = idx ? r[idx[mid]] : r[mid];
-        if (e < v) lo = mid + 1; else hi = mid;
+    const uint32_t lane = threadIdx.x & 63u;
+    /* the result lies in [at, at + left] */
+    uint32_t at[2] = {0, 0}, left[2] = {n, n};
+    while (left[0] | left[1]) {
+        uint32_t k[2], step[2];
+        float v[2];
+#pragma unroll
+        for (int w = 0; w < 2; ++w) {
+            step[w] = left[w] / 64 + (left[w] % 64 ? 1u : 0u);
+            /* the last of part `lane`; of a search that is done, anything */
+            const uint64_t last = min((uint64_t)step[w] * (lane + 1u), (uint64_t)left[w]);
+            k[w] = min(at[w] + (last ? (uint32_t)last - 1u : 0u), n - 1u);
+        }
+        if (idx) {
+            k[0] = idx[k[0]];
+            k[1] = idx[k[1]];
+        }
+        v[0] = r[k[0]];
+        v[1] = r[k[1]];
+        const uint64_t in[2] = {__ballot(v[0] < lo), __ballot(!(hi < v[1]))};
+#pragma unroll
+        for (int w = 0; w < 2; ++w) {
+            const uint32_t c = (uint32_t)__popcll(in[w]);
+            const uint32_t go = (uint32_t)min((uint64_t)c * step[w], (uint64_t)left[w]);
+            at[w] += go;
+            /* into the part whose last is not below */
+            left[w] = go == left[w] ? 0u : min(step[w], left[w] - go) - 1u;
+        }
     }
-    return lo;
-}
-__device__ __forceinline__ uint32_t ub_perm(const float *r, const uint32_t *idx, uint32_t n, float v)
-{
-    uint32_t lo = 0, hi = n;
-    while (lo < hi) {
-        uint32_t mid = lo + ((hi - lo) >> 1);
-        float e = idx ? r[idx[mid]] : r[mid];
-        if (v < e) hi = mid; else lo = mid + 1;
-    }
-    return lo;
+    *begin = at[0];
+    *end = at[1];
 }
 
-__global__ void k_window(uint32_t *begin, uint32_t *end, uint32_t *num, const float *r,
-                         const uint32_t *idx, uint32_t num_pep, const float *mass, uint32_t num_spec,
-                         float eps)
+/* the same by a thread, seven probes a step of each, all in flight: eight steps
+ * for 2.7 M */
+template <bool IDX>
+__device__ __forceinline__ void db_bounds(const float *r, const uint32_t *idx, uint32_t n, float lo,
+                                          float hi, uint32_t *begin, uint32_t *end)
 {
-    uint32_t s = blockIdx.x * blockDim.x + threadIdx.x;
+    uint32_t at[2] = {0, 0}, left[2] = {n, n};
+    while (left[0] | left[1]) {
+        uint32_t step[2], k[2][7];
+        float v[2][7];
+#pragma unroll
+        for (int w = 0; w < 2; ++w) {
+            step[w] = (left[w] + 7) / 8;
+#pragma unroll
+            for (uint32_t j = 0; j < 7; ++j)
+                k[w][j] = min(at[w] + max(min(step[w] * (j + 1), left[w]), 1u) - 1u, n - 1u);
+        }
+        if constexpr (IDX)
+#pragma unroll
+            for (uint32_t j = 0; j < 14; ++j) k[j / 7][j % 7] = idx[k[j / 7][j % 7]];
+#pragma unroll
+        for (uint32_t j = 0; j < 14; ++j) v[j / 7][j % 7] = r[k[j / 7][j % 7]];
+#pragma unroll
+        for (int w = 0; w < 2; ++w) {
+            uint32_t c = 0;
+#pragma unroll
+            for (uint32_t j = 0; j < 7; ++j) c += (w == 0 ? v[w][j] < lo : !(hi < v[w][j])) ? 1u : 0u;
+            const uint32_t go = min(c * step[w], left[w]), rest = left[w] - go;
+            at[w] += go;
+            /* past seven parts: the eighth; else a part whose last is not below */
+            left[w] = c == 7 ? rest : min(step[w], rest) - (rest ? 1u : 0u);
+        }
+    }
+    *begin = at[0];
+    *end = at[1];
+}
+
+__global__ void __launch_bounds__(256)
+    k_window(uint32_t *begin, uint32_t *end, uint32_t *num, const float *r, const uint32_t *idx,
+             uint32_t num_pep, const float *mass, uint32_t num_spec, float eps)
+{
+    const uint32_t s = blockIdx.x * 4 + threadIdx.x / 64;
     if (s >= num_spec) return;
-    float lo = mass[s] - eps, hi = mass[s] + eps;
-    uint32_t b = lb_perm(r, idx, num_pep, lo);
-    uint32_t e = ub_perm(r, idx, num_pep, hi);
-    if (begin) begin[s] = b;
-    if (end) end[s] = e;
-    num[s] = e - b;
+    uint32_t b, e;
+    db_bounds_wave(r, idx, num_pep, mass[s] - eps, mass[s] + eps, &b, &e);
+    if ((threadIdx.x & 63u) == 0) {
+        if (begin) begin[s] = b;
+        if (end) end[s] = e;
+        num[s] = e - b;
+    }
 }
 
 /* sum of n uint32 (wrapping, like thrust::reduce on uint32) into *out */
@@ -606,7 +662,7 @@ extern "C" uint32_t findSpecCandsByMass(uint32_t *d_spec_begin_raw, uint32_t *d_
     if (num_spec == 0) return 0;
     hfx_ctx *ctx = hfx_default_ctx();
     if (!ctx) return 0;
-    hipLaunchKernelGGL(k_window, dim3((num_spec + 255) / 256), dim3(256), 0, 0, d_spec_begin_raw,
+    hipLaunchKernelGGL(k_window, dim3((num_spec + 3) / 4), dim3(256), 0, 0, d_spec_begin_raw,
                        d_spec_end_raw, d_spec_num_pep_raw, d_r_raw, d_pep_idx_r_sorted_raw, num_pep,
                        d_spec_masses_raw, num_spec, eps);
     return hfx_sum_u32_to_host(ctx, d_spec_num_pep_raw, num_spec);
@@ -619,7 +675,7 @@ extern "C" int hfx_window(hfx_ctx *ctx, uint32_t *d_begin, uint32_t *d_num, cons
     if (num_spec == 0) return HFX_OK;
     const float *r = db->d_r_sorted ? db->d_r_sorted : db->d_r;
     const uint32_t *idx = db->d_r_sorted ? nullptr : db->d_idx_sorted;
-    hipLaunchKernelGGL(k_window, dim3((num_spec + 255) / 256), dim3(256), 0, hfx_stream(stream),
+    hipLaunchKernelGGL(k_window, dim3((num_spec + 3) / 4), dim3(256), 0, hfx_stream(stream),
                        d_begin, (uint32_t *)nullptr, d_num, r, idx, db->num_pep, d_spec_mass,
                        num_spec, eps);
     HFX_CHECK_LAUNCH();
@@ -632,8 +688,9 @@ __global__ void k_begin_end_mod(uint32_t *begin, uint32_t *end, uint32_t *cnt, c
 {
     uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= num_mod) return;
-    float lo = lo0 - delta[i], hi = hi0 - delta[i];
-    uint32_t b = lb_perm(r, idx, num_pep, lo), e = ub_perm(r, idx, num_pep, hi);
+    uint32_t b, e;
+    if (idx) db_bounds<true>(r, idx, num_pep, lo0 - delta[i], hi0 - delta[i], &b, &e);
+    else db_bounds<false>(r, idx, num_pep, lo0 - delta[i], hi0 - delta[i], &b, &e);
     begin[i] = b;
     end[i] = e;
     cnt[i] = e - b;
@@ -658,28 +715,39 @@ extern "C" uint32_t findBeginEnd_f(uint32_t *d_begin_raw, uint32_t *d_end_raw,
     return total;
 }
 
-/* findBeginEnd_f for many spectra in one launch: one thread per spectrum
- * walks the modifications in order, so its exclusive scan of the window sizes
- * is the reference's per-spectrum scan. */
-__global__ void k_mod_windows(uint32_t *begin, uint32_t *end, uint32_t *scan, uint32_t *spec_cand,
-                              const float *r, const uint32_t *idx, uint32_t num_pep,
-                              const float *delta, uint32_t num_mod, const float *mass,
-                              uint32_t num_spec, float eps)
+/* findBeginEnd_f for many spectra in one launch: a wave a spectrum, a lane a
+ * modification; the prefix sums of its lanes are the reference's per-spectrum
+ * scan.  One thread a spectrum took 205 us for 5,000 spectra and 34
+ * modifications, 18 now. */
+template <bool IDX>
+__global__ void __launch_bounds__(256)
+    k_mod_windows(uint32_t *begin, uint32_t *end, uint32_t *scan, uint32_t *spec_cand,
+                  const float *r, const uint32_t *idx, uint32_t num_pep, const float *delta,
+                  uint32_t num_mod, const float *mass, uint32_t num_spec, float eps)
 {
-    const uint32_t s = blockIdx.x * blockDim.x + threadIdx.x;
+    const uint32_t s = blockIdx.x * 4 + threadIdx.x / 64, lane = threadIdx.x & 63;
     if (s >= num_spec) return;
     const float lo0 = mass[s] - eps, hi0 = mass[s] + eps;
     uint32_t acc = 0;
-    for (uint32_t i = 0; i < num_mod; ++i) {
-        const float lo = lo0 - delta[i], hi = hi0 - delta[i];
-        const uint32_t b = lb_perm(r, idx, num_pep, lo), e = ub_perm(r, idx, num_pep, hi);
-        const size_t o = (size_t)s * num_mod + i;
-        begin[o] = b;
-        end[o] = e;
-        scan[o] = acc;
-        acc += e - b;
+    for (uint32_t i0 = 0; i0 < num_mod; i0 += 64) {
+        const uint32_t i = i0 + lane;
+        uint32_t b = 0, e = 0;
+        if (i < num_mod) db_bounds<IDX>(r, idx, num_pep, lo0 - delta[i], hi0 - delta[i], &b, &e);
+        uint32_t x = e - b;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const uint32_t y = __shfl_up(x, o, 64);
+            if (lane >= (uint32_t)o) x += y;
+        }
+        if (i < num_mod) {
+            const size_t o = (size_t)s * num_mod + i;
+            begin[o] = b;
+            end[o] = e;
+            scan[o] = acc + x - (e - b);
+        }
+        acc += (uint32_t)__shfl((int)x, 63, 64);
     }
-    spec_cand[s] = acc;
+    if (lane == 0) spec_cand[s] = acc;
 }
 
 extern "C" int hfx_mod_windows(hfx_ctx *ctx, uint32_t *d_begin, uint32_t *d_end,
@@ -694,7 +762,8 @@ extern "C" int hfx_mod_windows(hfx_ctx *ctx, uint32_t *d_begin, uint32_t *d_end,
     if (num_spec == 0) return HFX_OK;
     const float *r = db->d_r_sorted ? db->d_r_sorted : db->d_r;
     const uint32_t *idx = db->d_r_sorted ? nullptr : db->d_idx_sorted;
-    hipLaunchKernelGGL(k_mod_windows, dim3((num_spec + 255) / 256), dim3(256), 0,
+    hipLaunchKernelGGL(idx ? k_mod_windows<true> : k_mod_windows<false>, dim3((num_spec + 3) / 4),
+                       dim3(256), 0,
                        hfx_stream(stream), d_begin, d_end, d_num_scan, d_spec_cand, r, idx,
                        db->num_pep, d_mod_delta, num_mod, d_spec_mass, num_spec, eps);
     HFX_CHECK_LAUNCH();
@@ -705,34 +774,112 @@ extern "C" int hfx_mod_windows(hfx_ctx *ctx, uint32_t *d_begin, uint32_t *d_end,
 /* Offsets and candidate lists                                           */
 /* ------------------------------------------------------------------ */
 
-/* Exclusive scan of n uint32 counts into n+1 uint64 offsets, one workgroup. */
+/* inclusive prefix sum over the wave by lane moves: rows of 16 by shifts of 1,
+ * 2, 4 and 8, then across rows */
+template <int CTRL, int ROWS>
+__device__ __forceinline__ uint64_t sc_step(uint64_t x)
+{
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)x, CTRL, ROWS, 0xf, false);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(x >> 32), CTRL, ROWS,
+                                                              0xf, false);
+    return x + ((uint64_t)hi << 32 | lo);
+}
+__device__ __forceinline__ uint64_t sc_wave_incl(uint64_t x)
+{
+    x = sc_step<0x111, 0xf>(x);
+    x = sc_step<0x112, 0xf>(x);
+    x = sc_step<0x114, 0xf>(x);
+    x = sc_step<0x118, 0xf>(x);
+    x = sc_step<0x142, 0xa>(x);
+    x = sc_step<0x143, 0xc>(x);
+    return x;
+}
+__device__ __forceinline__ uint64_t sc_last(uint64_t x)
+{
+    return (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)(x >> 32), 63) << 32 |
+           (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)x, 63);
+}
+/* exclusive prefix sums of a wave's counts v[q], in order of (q, lane); returns
+ * their sum */
+template <int Q>
+__device__ __forceinline__ uint64_t sc_wave_scan(const uint32_t (&v)[Q], uint64_t (&x)[Q])
+{
+    uint64_t sum = 0;
+#pragma unroll
+    for (int q = 0; q < Q; ++q) {
+        const uint64_t incl = sc_wave_incl(v[q]);
+        x[q] = sum + incl - v[q];
+        sum += sc_last(incl);
+    }
+    return sum;
+}
+
+/* four counts / two offsets beside each other, at their own alignment */
+typedef uint32_t sc_u4 __attribute__((ext_vector_type(4), aligned(4)));
+typedef uint64_t sc_l2 __attribute__((ext_vector_type(2), aligned(8)));
+
+/* Exclusive scan of n uint32 counts into n+1 uint64 offsets, one workgroup, Q
+ * counts beside each other a thread: one pass for 1024 Q of them.  (A single CU
+ * cannot afford a wave scan for each count: 7.5 us for 5000, Q = 1 over five
+ * passes 8.5, 4.3 now.) */
+template <int Q>
 __global__ void __launch_bounds__(1024) k_scan_offsets(uint64_t *off, const uint32_t *cnt, uint32_t n)
 {
-    __shared__ uint64_t warp_tot[16];
-    __shared__ uint64_t carry_s;
-    if (threadIdx.x == 0) carry_s = 0;
-    __syncthreads();
+    __shared__ uint64_t warp_tot[2][16];
     const uint32_t lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-    for (uint32_t base = 0; base < n; base += 1024) {
-        uint32_t i = base + threadIdx.x;
-        uint64_t v = i < n ? cnt[i] : 0;
-        uint64_t x = v;
+    uint64_t carry = 0;
+    uint32_t turn = 0;
+    for (uint64_t base = 0; base < n; base += 1024 * Q, turn ^= 1) {
+        const uint64_t first = base + (uint64_t)threadIdx.x * Q;
+        const bool all = Q % 4 == 0 && first + Q <= n;
+        uint32_t v[Q];
+        if (all) {
 #pragma unroll
-        for (int o = 1; o < 64; o <<= 1) {
-            uint64_t y = __shfl_up(x, o, 64);
-            if (lane >= (uint32_t)o) x += y;
+            for (int q = 0; q + 3 < Q; q += 4) {
+                const sc_u4 t = *(const sc_u4 *)(cnt + first + q);
+                v[q] = t[0];
+                v[q + 1] = t[1];
+                v[q + 2] = t[2];
+                v[q + 3] = t[3];
+            }
+        } else {
+#pragma unroll
+            for (int q = 0; q < Q; ++q) v[q] = first + q < n ? cnt[first + q] : 0u;
         }
-        if (lane == 63) warp_tot[wid] = x;
+        uint64_t sum = 0;
+#pragma unroll
+        for (int q = 0; q < Q; ++q) sum += v[q];
+        const uint64_t incl = sc_wave_incl(sum);
+        if (lane == 63) warp_tot[turn][wid] = incl;
         __syncthreads();
-        uint64_t wpre = 0;
-        for (uint32_t w = 0; w < wid; ++w) wpre += warp_tot[w];
-        uint64_t carry = carry_s;
-        if (i < n) off[i] = carry + wpre + x - v;
-        __syncthreads();
-        if (threadIdx.x == 1023) carry_s = carry + wpre + x;
-        __syncthreads();
+        uint64_t x = carry + incl - sum;
+#pragma unroll
+        for (uint32_t w = 0; w < 16; ++w) {
+            x += w < wid ? warp_tot[turn][w] : 0;
+            carry += warp_tot[turn][w];
+        }
+        if (all) {
+#pragma unroll
+            for (int q = 0; q + 1 < Q; q += 2) {
+                *(sc_l2 *)(off + first + q) = sc_l2{x, x + v[q]};
+                x += (uint64_t)v[q] + v[q + 1];
+            }
+        } else {
+#pragma unroll
+            for (int q = 0; q < Q; ++q) {
+                if (first + q < n) off[first + q] = x;
+                x += v[q];
+            }
+        }
     }
-    if (threadIdx.x == 0) off[n] = carry_s;
+    if (threadIdx.x == 0) off[n] = carry;
+}
+
+static void scan_offsets_one(uint64_t *off, const uint32_t *cnt, uint32_t n, hipStream_t st)
+{
+    if (n <= 1024) hipLaunchKernelGGL(k_scan_offsets<1>, dim3(1), dim3(1024), 0, st, off, cnt, n);
+    else if (n <= 4096) hipLaunchKernelGGL(k_scan_offsets<4>, dim3(1), dim3(1024), 0, st, off, cnt, n);
+    else hipLaunchKernelGGL(k_scan_offsets<16>, dim3(1), dim3(1024), 0, st, off, cnt, n);
 }
 
 /* Multi-workgroup form (reduce, then scan), with no scratch: the offsets
@@ -749,8 +896,10 @@ __global__ void __launch_bounds__(1024) k_scan_offsets(uint64_t *off, const uint
 #define SC_THREADS 1024
 #define SC_ITEMS 8
 #define SC_TILE (SC_THREADS * SC_ITEMS)
-/* below this count one workgroup's pass is quicker than three launches */
-#define SC_SMALL 8192u
+/* below this count one workgroup's passes are quicker than three launches:
+ * 10,000 counts take 5.8 us, the launches 4.7 + 2.5 + 6.4 and their gaps; a
+ * second pass adds 3 */
+#define SC_SMALL 32768u
 
 __device__ __forceinline__ uint64_t sc_block_sum(uint64_t v, uint64_t *part)
 {
@@ -818,31 +967,21 @@ __global__ void __launch_bounds__(SC_THREADS) k_scan_tiles(uint64_t *off, const 
     __shared__ uint64_t warp_tot[SC_THREADS / 64];
     const uint64_t base = (uint64_t)blockIdx.x * SC_TILE;
     const uint64_t tile_base = off[base];
-    /* thread t takes counts t * SC_ITEMS .. + SC_ITEMS - 1 of the tile */
-    const uint64_t first = base + (uint64_t)threadIdx.x * SC_ITEMS;
-    uint32_t v[SC_ITEMS];
-    uint64_t s = 0;
-#pragma unroll
-    for (uint32_t k = 0; k < SC_ITEMS; ++k) {
-        v[k] = first + k < n ? cnt[first + k] : 0u;
-        s += v[k];
-    }
+    /* a wave takes SC_ITEMS * 64 counts, its lanes beside each other */
     const uint32_t lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-    uint64_t x = s;
+    const uint64_t first = base + wid * 64 * SC_ITEMS + lane;
+    uint32_t v[SC_ITEMS];
+    uint64_t x[SC_ITEMS];
 #pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-        const uint64_t y = __shfl_up(x, o, 64);
-        if (lane >= (uint32_t)o) x += y;
-    }
-    if (lane == 63) warp_tot[wid] = x;
+    for (uint32_t k = 0; k < SC_ITEMS; ++k) v[k] = first + 64 * k < n ? cnt[first + 64 * k] : 0u;
+    const uint64_t sum = sc_wave_scan(v, x);
+    if (lane == 0) warp_tot[wid] = sum;
     __syncthreads();
-    uint64_t pre = tile_base + x - s;
+    uint64_t pre = tile_base;
     for (uint32_t w = 0; w < wid; ++w) pre += warp_tot[w];
 #pragma unroll
-    for (uint32_t k = 0; k < SC_ITEMS; ++k) {
-        if (first + k < n) off[first + k] = pre;
-        pre += v[k];
-    }
+    for (uint32_t k = 0; k < SC_ITEMS; ++k)
+        if (first + 64 * k < n) off[first + 64 * k] = pre + x[k];
 }
 
 /* In-place exclusive scan of n uint32 (wrapping) over many workgroups:
@@ -867,30 +1006,20 @@ __global__ void __launch_bounds__(SC_THREADS) k_scan32_tiles(uint32_t *a, uint32
                                                              const uint32_t *sums)
 {
     __shared__ uint32_t warp_tot[SC_THREADS / 64];
-    const uint64_t first = (uint64_t)blockIdx.x * SC_TILE + (uint64_t)threadIdx.x * SC_ITEMS;
-    uint32_t v[SC_ITEMS];
-    uint32_t s = 0;
-#pragma unroll
-    for (uint32_t k = 0; k < SC_ITEMS; ++k) {
-        v[k] = first + k < n ? a[first + k] : 0u;
-        s += v[k];
-    }
     const uint32_t lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-    uint32_t x = s;
+    const uint64_t first = (uint64_t)blockIdx.x * SC_TILE + wid * 64 * SC_ITEMS + lane;
+    uint32_t v[SC_ITEMS];
+    uint64_t x[SC_ITEMS];
 #pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-        const uint32_t y = __shfl_up(x, o, 64);
-        if (lane >= (uint32_t)o) x += y;
-    }
-    if (lane == 63) warp_tot[wid] = x;
+    for (uint32_t k = 0; k < SC_ITEMS; ++k) v[k] = first + 64 * k < n ? a[first + 64 * k] : 0u;
+    const uint64_t sum = sc_wave_scan(v, x);
+    if (lane == 0) warp_tot[wid] = (uint32_t)sum;
     __syncthreads();
-    uint32_t pre = sums[blockIdx.x] + x - s;
+    uint32_t pre = sums[blockIdx.x];
     for (uint32_t w = 0; w < wid; ++w) pre += warp_tot[w];
 #pragma unroll
-    for (uint32_t k = 0; k < SC_ITEMS; ++k) {
-        if (first + k < n) a[first + k] = pre;
-        pre += v[k];
-    }
+    for (uint32_t k = 0; k < SC_ITEMS; ++k)
+        if (first + 64 * k < n) a[first + 64 * k] = pre + (uint32_t)x[k];
 }
 
 int hfx_scan_u32_inplace(uint32_t *d_a, uint32_t n, void *stream)
@@ -922,7 +1051,7 @@ extern "C" int hfx_scan_offsets(hfx_ctx *ctx, uint64_t *d_off, const uint32_t *d
     HFX_REQUIRE(d_off != nullptr, HFX_ERR_ARG, "hfx_scan_offsets: null output");
     hipStream_t st = hfx_stream(stream);
     if (n < SC_SMALL) {
-        hipLaunchKernelGGL(k_scan_offsets, dim3(1), dim3(1024), 0, st, d_off, d_count, n);
+        scan_offsets_one(d_off, d_count, n, st);
     } else {
         const uint32_t nt = (uint32_t)(((uint64_t)n + SC_TILE - 1) / SC_TILE);
         hipLaunchKernelGGL(k_scan_tile_sums, dim3(nt), dim3(SC_THREADS), 0, st, d_off, d_count, n);
@@ -952,7 +1081,7 @@ extern "C" void prepare_scoring(uint32_t *d_out_spec_pep_idx, const uint32_t *d_
     void *p;
     if (hfx_ctx_scratch(ctx, HFX_SLOT_SCAN, ((size_t)num_spec + 1) * 8, &p) != HFX_OK) return;
     uint64_t *off = (uint64_t *)p;
-    hipLaunchKernelGGL(k_scan_offsets, dim3(1), dim3(1024), 0, 0, off, d_spec_num_pep, num_spec);
+    scan_offsets_one(off, d_spec_num_pep, num_spec, 0);
     hipLaunchKernelGGL(k_prepare_scoring, dim3(num_spec), dim3(256), 0, 0, d_out_spec_pep_idx,
                        d_pep_idx_r_sorted_raw, d_spec_begin, d_spec_num_pep, off);
     hipError_t e = hipGetLastError();
