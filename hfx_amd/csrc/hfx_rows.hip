@@ -35,8 +35,8 @@
  *
  * Scoring kernels, 20,000 proteins (2.7 M peptides), before (rows written per
  * block into LDS, or per pair) and after: three digits, 20,000 spectra 1,978 ->
- * 958 us; BF16, 6,000 spectra 1,937 -> 850 us; FP32 batched, 4,000 spectra
- * 10,114 -> 600 us.  Writing two levels' rows of the database takes 0.87 ms,
+ * 864 us; BF16, 6,000 spectra 1,937 -> 773 us; FP32 batched, 4,000 spectra
+ * 10,114 -> 547 us.  Writing two levels' rows of the database takes 0.87 ms,
  * once.
  */
 #include "hfx_cand.h"
@@ -533,7 +533,7 @@ __global__ void k_rw_zero_unscored(float *scores, const uint64_t *off, const uin
 /* The contraction                                                        */
 /* ------------------------------------------------------------------ */
 
-#define RM_THREADS 512
+#define RM_THREADS 768
 #define RM_WAVES (RM_THREADS / HFX_WAVE)
 #define RM_T 4 /* tiles a wave contracts at once: each B fragment read serves 64 rows */
 
@@ -554,15 +554,23 @@ struct RmArgs {
     hfx_spectra sp;
 };
 
-/* Persistent workgroups of eight waves over (block, level, CT tiles).  The
+/* Persistent workgroups of twelve waves over (block, level, CT tiles).  The
  * block's planes stay in LDS, laid out so that a fragment read is one
  * contiguous KiB ([k-step][plane][lane]); each wave contracts four tiles at a
  * time over the whole row, its accumulators in registers, the next group's
  * codes loaded while the current one is contracted.  A k-step of four tiles
  * costs 4 x 11 code lookups, 4 x planes matrix instructions and one fragment
- * read a plane. */
+ * read a plane.
+ * The two kinds add up: vector and matrix instructions together fill 96 % of
+ * the cycles, with rows from cache as well, and interleaving them by hand
+ * changes nothing.  So what is not a lookup was taken out of the loop (copies of
+ * the codes, per-lane addresses, FP64 folds) and a third wave a SIMD fills its
+ * waits: three digits, 20,000 spectra 963 -> 881 (the wave) -> 864 us; four, a
+ * plain search of 10,000, 840 -> 767 -> 757; BF16 850 -> 812 -> 773.  Sixteen
+ * waves spill (983 us, three digits); three groups of codes on their way, also
+ * across tiles, cost more scalar work than they hide (1,134). */
 template <int MODE>
-__global__ void __launch_bounds__(RM_THREADS, 2) k_rw_mm(RmArgs a)
+__global__ void __launch_bounds__(RM_THREADS, 3) k_rw_mm(RmArgs a)
 {
     constexpr uint32_t NP = MODE == RW_BF16 ? 2 : RW_PLANES(MODE); /* planes in LDS */
     constexpr uint32_t NS = RW_NS(MODE);
@@ -654,7 +662,7 @@ __global__ void __launch_bounds__(RM_THREADS, 2) k_rw_mm(RmArgs a)
         const uint64_t *slots = a.slots ? a.slots + (size_t)(lvl - 1u) * a.ntiles : nullptr;
         const uint32_t beg = m_beg[g_of], end = m_end[g_of];
         const bool mine = m_z[g_of] == lvl && (MODE != RW_BF16 || (col & 1u) == 0u);
-        const double qd = MODE == RW_BF16 ? 0.0 : (double)m_q[g_of];
+        const float qf = MODE == RW_BF16 ? 0.0f : m_q[g_of];
         float *const out = a.scores + m_off[g_of];
         const size_t tile_bytes = (size_t)a.G * 1024u;
         for (uint32_t u0 = c0 + wave * RM_T; u0 < c1; u0 += RM_WAVES * RM_T) {
@@ -676,16 +684,36 @@ __global__ void __launch_bounds__(RM_THREADS, 2) k_rw_mm(RmArgs a)
                 const uint32_t t = min(u0 + k, c1 - 1u);
                 own[k] = (rw_sload((const uint32_t *)a.ng, t >> 2) >> ((t & 3u) * 8u)) & 255u;
             }
+            const uint32_t own_min = min(min(own[0], own[1]), min(own[2], own[3]));
+            static_assert(RM_T == 4, "the least of its tiles' groups");
             auto load = [&](rw_u32x4(&c)[RM_T], uint32_t g) {
 #pragma unroll
                 for (uint32_t k = 0; k < RM_T; ++k) {
-                    const uint32_t gg = min(g, own[k] - 1u);
-                    c[k] = *(const rw_u32x4 *)(base[k] + gg * 1024u + lane * 16u);
-                    if (g >= own[k]) c[k] = rw_u32x4{0u, 0u, 0u, 0u};
+                    const uint8_t *p = base[k] + min(g, own[k] - 1u) * 1024u; /* uniform */
+                    c[k] = *(const rw_u32x4 *)(p + lane * 16u);
                 }
             };
+            auto past = [&](rw_u32x4(&c)[RM_T], uint32_t g) {
+                if (g < own_min) return;
+#pragma unroll
+                for (uint32_t k = 0; k < RM_T; ++k)
+                    if (g >= own[k]) c[k] = rw_u32x4{0u, 0u, 0u, 0u};
+            };
+            /* use(codes, group) for every group, the next one's codes on their
+             * way meanwhile */
             rw_u32x4 ca[RM_T], cb[RM_T];
-            load(ca, 0);
+            auto groups = [&](auto &&use) {
+                load(ca, 0);
+                for (uint32_t g = 0; g < ng; g += 2) {
+                    load(cb, min(g + 1u, ng - 1u));
+                    past(ca, g);
+                    use(ca, g);
+                    if (g + 1u >= ng) break;
+                    load(ca, min(g + 2u, ng - 1u));
+                    past(cb, g + 1u);
+                    use(cb, g + 1u);
+                }
+            };
             if constexpr (MODE == RW_BF16) {
                 rw_f32x4 acc0[RM_T], acc1[RM_T];
 #pragma unroll
@@ -693,8 +721,7 @@ __global__ void __launch_bounds__(RM_THREADS, 2) k_rw_mm(RmArgs a)
                     acc0[k] = rw_f32x4{0.0f, 0.0f, 0.0f, 0.0f};
                     acc1[k] = acc0[k];
                 }
-                for (uint32_t g = 0; g < ng; ++g) {
-                    load(cb, min(g + 1u, ng - 1u));
+                groups([&](const rw_u32x4(&c)[RM_T], uint32_t g) {
 #pragma unroll
                     for (uint32_t j = 0; j < 4; ++j) {
                         const uint32_t ks = g * 4u + j;
@@ -703,7 +730,7 @@ __global__ void __launch_bounds__(RM_THREADS, 2) k_rw_mm(RmArgs a)
                             const rw_u32x4 f1 = Bl[(ks * NP + 1) * 64u + lane];
 #pragma unroll
                             for (uint32_t k = 0; k < RM_T; ++k) {
-                                const uint32_t P = ca[k][j];
+                                const uint32_t P = c[k][j];
                                 uint32_t w[8];
 #pragma unroll
                                 for (uint32_t h = 0; h < 4; ++h) {
@@ -724,9 +751,7 @@ __global__ void __launch_bounds__(RM_THREADS, 2) k_rw_mm(RmArgs a)
                             }
                         }
                     }
-#pragma unroll
-                    for (uint32_t k = 0; k < RM_T; ++k) ca[k] = cb[k];
-                }
+                });
 #pragma unroll
                 for (uint32_t k = 0; k < RM_T; ++k) {
                     const uint32_t t = u0 + k;
@@ -747,8 +772,7 @@ __global__ void __launch_bounds__(RM_THREADS, 2) k_rw_mm(RmArgs a)
                 for (uint32_t k = 0; k < RM_T; ++k)
 #pragma unroll
                     for (uint32_t d = 0; d < NP; ++d) acc[k][d] = rw_i32x4{0, 0, 0, 0};
-                for (uint32_t g = 0; g < ng; ++g) {
-                    load(cb, min(g + 1u, ng - 1u));
+                groups([&](const rw_u32x4(&c)[RM_T], uint32_t g) {
 #pragma unroll
                     for (uint32_t j = 0; j < 4; ++j) {
                         const uint32_t ks = g * 4u + j;
@@ -759,7 +783,7 @@ __global__ void __launch_bounds__(RM_THREADS, 2) k_rw_mm(RmArgs a)
                                 f[d] = __builtin_bit_cast(rw_i32x4, Bl[(ks * NP + d) * 64u + lane]);
 #pragma unroll
                             for (uint32_t k = 0; k < RM_T; ++k) {
-                                const uint32_t P = ca[k][j];
+                                const uint32_t P = c[k][j];
                                 rw_i32x4 av;
 #pragma unroll
                                 for (uint32_t h = 0; h < 4; ++h)
@@ -772,22 +796,26 @@ __global__ void __launch_bounds__(RM_THREADS, 2) k_rw_mm(RmArgs a)
                             }
                         }
                     }
-#pragma unroll
-                    for (uint32_t k = 0; k < RM_T; ++k) ca[k] = cb[k];
-                }
-                /* digit sums are below 50 * 128 * RW_MAXK < 2^24, so the folds
-                 * are exact in FP64 and the score is rounded once */
+                });
+                /* Digit sums are below 50 * 128 * RW_MAXK < 2^23.8.  Carries go up
+                 * until the highest digit is followed by 16 or 24 bits; both parts
+                 * are exact in FP32, and the fused sum rounds once. */
 #pragma unroll
                 for (uint32_t k = 0; k < RM_T; ++k) {
                     const uint32_t t = u0 + k;
 #pragma unroll
                     for (uint32_t i = 0; i < 4; ++i) {
-                        double v = (double)acc[k][NP - 1][i];
+                        int32_t top = acc[k][0][i];
+                        uint32_t low = 0;
 #pragma unroll
-                        for (int d = (int)NP - 2; d >= 0; --d)
-                            v = __builtin_fma(v, 256.0, (double)acc[k][d][i]);
+                        for (uint32_t d = 1; d < NP; ++d) {
+                            low |= ((uint32_t)top & 255u) << (8 * (d - 1));
+                            top = acc[k][d][i] + (top >> 8);
+                        }
+                        const float v = __builtin_fmaf((float)top, (float)(1u << (8 * (NP - 1))),
+                                                       (float)low) * qf;
                         const uint32_t p = t * RW_ROWS + 4u * kg + i;
-                        if (mine && t < c1 && beg <= p && p < end) out[p - beg] = (float)(v * qd);
+                        if (mine && t < c1 && beg <= p && p < end) out[p - beg] = v;
                     }
                 }
             }
