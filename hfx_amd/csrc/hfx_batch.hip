@@ -760,7 +760,7 @@ struct hfx_batch {
     uint32_t nseg;
     bool dense_set;      /* a dense form was chosen since the plan */
     bool rows_tried, use_rows; /* scores come from the index's rows */
-    uint32_t *rw_small;  /* rows: [3][S] quanta, levels, wide marks */
+    uint32_t *rw_small;  /* rows: [S] sum and max of |x|, [3][S] quanta, levels, wide marks */
     hipGraph_t graph;
     hipGraphExec_t exec;
 };
@@ -980,7 +980,7 @@ static int bt_ready(hfx_batch *b, hipStream_t st)
     HFX_CHECK_HIP(hipMemGetInfo(&fr, &tot));
     if (!b->dn_scratch && (uint64_t)b->S * 16384 > fr / 4) return HFX_OK;
     if (!pepix_need_rows(const_cast<hfx_pepix *>(b->ix), b->L, (uint32_t)hfx_ctx_num_cus(b->ctx), st)) return HFX_OK;
-    if (bt_dense_alloc(b) || (!b->rw_small && dalloc(&b->rw_small, 3 * (size_t)b->S))) {
+    if (bt_dense_alloc(b) || (!b->rw_small && dalloc(&b->rw_small, 5 * (size_t)b->S))) {
         (void)hipGetLastError();
         return HFX_OK;
     }
@@ -1212,8 +1212,12 @@ static int bt_mode(const hfx_batch *b)
            : b->precision == HFX_BATCH_BF16X2_DENSE ? RW_BF16
                                                     : RW_I8X4;
 }
-/* dn_scratch as the rows route carves it: planes | item bookkeeping; quanta,
- * levels and wide marks in rw_small */
+/* dn_scratch as the rows route carves it: planes | item bookkeeping; norms,
+ * quanta, levels and wide marks in rw_small */
+static float2 *bt_norms(const hfx_batch *b) { return (float2 *)b->rw_small; }
+static float *bt_quanta(const hfx_batch *b) { return (float *)(b->rw_small + 2 * (size_t)b->S); }
+static uint32_t *bt_levels(const hfx_batch *b) { return b->rw_small + 3 * (size_t)b->S; }
+static uint32_t *bt_wide(const hfx_batch *b) { return b->rw_small + 4 * (size_t)b->S; }
 static uint8_t *bt_planes(const hfx_batch *b) { return b->dn_scratch; }
 static void *bt_items(const hfx_batch *b)
 {
@@ -1231,9 +1235,8 @@ static int bt_dense_prep(hfx_batch *b, hipStream_t st)
                              b->S, (void *)st)))
         return rc;
     if (b->use_rows) {
-        float *qs = (float *)b->rw_small;
-        return hfx_rows_split(bt_mode(b), &b->sp, bt_planes(b), qs, b->rw_small + b->S,
-                              b->rw_small + 2 * (size_t)b->S, (void *)st);
+        return hfx_rows_split(bt_mode(b), &b->sp, bt_planes(b), bt_quanta(b), bt_levels(b),
+                              bt_wide(b), bt_norms(b), (void *)st);
     }
     return bf ? hfx_dense_split(&b->sp, b->dn_scratch, (void *)st)
               : hfx_dense8_split(&b->sp, b->dn_scratch, (void *)st);
@@ -1294,9 +1297,9 @@ static int bt_row_scores(hfx_batch *b, hipStream_t st, void **ev)
 {
     if (b->total == 0) return HFX_OK;
     const int mode = bt_mode(b);
-    const float *qs = (const float *)b->rw_small;
+    const float *qs = bt_quanta(b);
     hfx_spectra sq = b->sp;
-    if (mode == RW_I8X4) sq.d_zmax = b->rw_small + b->S; /* wide spectra hidden */
+    if (mode == RW_I8X4) sq.d_zmax = bt_levels(b); /* wide spectra hidden */
     int rc;
     if ((rc = hfx_rows_blocks(b->ctx, mode, bt_items(b), b->order, b->dn_bstart, b->begin, b->num,
                               &sq, b->CH, (void *)st)) ||
@@ -1306,7 +1309,7 @@ static int bt_row_scores(hfx_batch *b, hipStream_t st, void **ev)
         return rc;
     if (mode != RW_I8X4) return HFX_OK;
     return hfx_xcorr_wide(b->ctx, b->scores, b->score_off, b->begin, b->num, &b->db, &b->sp,
-                          b->rw_small + 2 * (size_t)b->S, (void *)st);
+                          bt_wide(b), (void *)st);
 }
 
 /* ev (optional): events recorded around the scoring kernel itself */
@@ -1345,8 +1348,8 @@ static int bt_topn(hfx_batch *b, hipStream_t st)
                                                                              : BT_REL_F32;
     return hfx_topn_device(b->ctx, b->top_pos, b->top_exact, b->top_f32, b->top_cnt, b->flag,
                            b->N, b->margin, b->scores, b->score_off, b->total, b->begin, b->num,
-                           &b->db, &b->sp, rel0, 0.0f, i8 ? BT_RELQ_I8 : 0.0f, b->tx_scratch,
-                           (void *)st);
+                           &b->db, &b->sp, rel0, 0.0f, i8 ? BT_RELQ_I8 : 0.0f,
+                           b->use_rows ? bt_norms(b) : nullptr, b->tx_scratch, (void *)st);
 }
 
 extern "C" int hfx_batch_run(hfx_batch *b, void *stream)

@@ -116,7 +116,7 @@ int hfx_topn_device(hfx_ctx *ctx, uint32_t *d_top_pos, double *d_top_exact, floa
                     uint32_t *d_top_cnt, uint32_t *d_flag, uint32_t N, uint32_t margin,
                     const float *d_scores, const uint64_t *d_off, uint64_t total,
                     const uint32_t *d_begin, const uint32_t *d_num, const hfx_db *db,
-                    const hfx_spectra *sp, float rel0, float rel1, float relq, void *scratch,
+                    const hfx_spectra *sp, float rel0, float rel1, float relq, const float2 *norms, void *scratch,
                     void *stream);
 /* b ladders of the peptides in residual-sorted positions [q0, q0 + nq), for
  * the dense path.  Position k < tn - tc of sorted peptide q is

@@ -33,9 +33,9 @@ uint32_t hfx_rows_groups(uint32_t x_stride);
 uint32_t hfx_rows_chunk(uint64_t rows, uint32_t cus);
 /* planes [S][RW_PLANES][RW_MAXK] and quanta of the spectra; RW_I8X4 also
  * writes each spectrum's charge level to lvl, or to wide where its digits would
- * lose precision (0 in the other) */
+ * lose precision (0 in the other); norms [S], if any: sum and max of |x| */
 int hfx_rows_split(int mode, const hfx_spectra *sp, uint8_t *planes, float *qs, uint32_t *lvl,
-                   uint32_t *wide, void *stream);
+                   uint32_t *wide, float2 *norms, void *stream);
 /* writes the rows of the wanted levels (non-null) and tiles (flags
  * [HFX_MAX_CHARGE][ntiles], null: all) */
 int hfx_rows_build(uint32_t cus, const hfx_db *db, const hfx_rows *r, const uint32_t *flags,

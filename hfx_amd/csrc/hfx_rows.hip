@@ -79,11 +79,12 @@ __device__ __forceinline__ uint32_t rw_bf16(float f)
 /* planes[s][plane][RW_MAXK]: byte 64 ks + 16 kg + j of a digit plane is the
  * digit of bin 64 ks + rw_bin_of(kg, j); the BF16 planes (hi of bytes j < 8,
  * hi of j >= 8, lo, lo) hold eight BF16 in the 16 bytes of a k-group.
- * qs[s] = 2^-k.  lvl (RW_I8X4): the fragment charge of the spectra the digits
+ * qs[s] = 2^-k.  norms (if any): sum and max of |x|.  lvl (RW_I8X4): the fragment charge of the spectra the digits
  * serve, 0 for wide ones (their charge goes to wide[s] instead). */
 template <int MODE>
 __global__ void __launch_bounds__(256)
-    k_rw_split(uint8_t *planes, float *qs, uint32_t *lvl, uint32_t *wide, hfx_spectra sp)
+    k_rw_split(uint8_t *planes, float *qs, uint32_t *lvl, uint32_t *wide, float2 *norms,
+               hfx_spectra sp)
 {
     constexpr uint32_t NP = RW_PLANES(MODE);
     __shared__ float red[2][256 / HFX_WAVE];
@@ -110,6 +111,20 @@ __global__ void __launch_bounds__(256)
             odd |= !(a < INFINITY);
         }
     }
+    for (uint32_t k = 32; k > 0; k >>= 1) {
+        m = fmaxf(m, __shfl_xor(m, k, 64));
+        x1 += __shfl_xor(x1, k, 64);
+    }
+    if (hfx_lane() == 0) {
+        red[0][tid / HFX_WAVE] = m;
+        red[1][tid / HFX_WAVE] = x1;
+    }
+    __syncthreads();
+    if (odd) bad = 1;
+    __syncthreads();
+    m = fmaxf(fmaxf(red[0][0], red[0][1]), fmaxf(red[0][2], red[0][3]));
+    x1 = red[1][0] + red[1][1] + red[1][2] + red[1][3];
+    if (tid == 0 && norms) norms[s] = make_float2(x1, m);
     uint8_t *o = planes + (size_t)s * NP * RW_MAXK;
     if constexpr (MODE == RW_BF16) {
 #pragma unroll
@@ -131,19 +146,6 @@ __global__ void __launch_bounds__(256)
         }
         return;
     }
-    for (uint32_t k = 32; k > 0; k >>= 1) {
-        m = fmaxf(m, __shfl_xor(m, k, 64));
-        x1 += __shfl_xor(x1, k, 64);
-    }
-    if (hfx_lane() == 0) {
-        red[0][tid / HFX_WAVE] = m;
-        red[1][tid / HFX_WAVE] = x1;
-    }
-    __syncthreads();
-    if (odd) bad = 1;
-    __syncthreads();
-    m = fmaxf(fmaxf(red[0][0], red[0][1]), fmaxf(red[0][2], red[0][3]));
-    x1 = red[1][0] + red[1][1] + red[1][2] + red[1][3];
     /* k: m 2^k in [2^(B-1), 2^B) from m's exponent, one less where that passes
      * the largest value the digits reach; at most 126 */
     constexpr int B = MODE == RW_I8X4 ? 31 : 23;
@@ -842,15 +844,15 @@ uint32_t hfx_rows_chunk(uint64_t rows, uint32_t cus)
 }
 
 int hfx_rows_split(int mode, const hfx_spectra *sp, uint8_t *planes, float *qs, uint32_t *lvl,
-                   uint32_t *wide, void *stream)
+                   uint32_t *wide, float2 *norms, void *stream)
 {
     HFX_REQUIRE(sp->x_stride <= RW_MAXK, HFX_ERR_ARG, "rows: spectra of up to %d bins", RW_MAXK);
     if (sp->num_spec == 0) return HFX_OK;
     const dim3 g(sp->num_spec), t(256);
     hipStream_t st = hfx_stream(stream);
-    if (mode == RW_I8X3) hipLaunchKernelGGL(k_rw_split<RW_I8X3>, g, t, 0, st, planes, qs, lvl, wide, *sp);
-    else if (mode == RW_I8X4) hipLaunchKernelGGL(k_rw_split<RW_I8X4>, g, t, 0, st, planes, qs, lvl, wide, *sp);
-    else hipLaunchKernelGGL(k_rw_split<RW_BF16>, g, t, 0, st, planes, qs, lvl, wide, *sp);
+    if (mode == RW_I8X3) hipLaunchKernelGGL(k_rw_split<RW_I8X3>, g, t, 0, st, planes, qs, lvl, wide, norms, *sp);
+    else if (mode == RW_I8X4) hipLaunchKernelGGL(k_rw_split<RW_I8X4>, g, t, 0, st, planes, qs, lvl, wide, norms, *sp);
+    else hipLaunchKernelGGL(k_rw_split<RW_BF16>, g, t, 0, st, planes, qs, lvl, wide, norms, *sp);
     HFX_CHECK_LAUNCH();
     return HFX_OK;
 }

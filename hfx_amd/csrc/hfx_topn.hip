@@ -31,10 +31,9 @@
  * time went to exact scores with a quarter of the lanes busy, and a spectrum
  * with 200 tied candidates held up a small batch by itself.
  * Now, select + exact + rank: 10,000 spectra, 1120 candidates each, top 10:
- * 127 + 136 + 15 us, against 445 us; 20,000 spectra, top 5: 179 + 148 + 15 us,
- * against 430; 250 spectra: 14 + 39 + 8 us, against 171.  The selection reads
- * the scores and the spectra once (86 + 44 MB in 179 us here: the collection's
- * ballots take the rest); the exact scores are bound by their FP64 terms and
+ * 127 + 136 + 15 us, against 445 us; 20,000 spectra, top 5: 160 + 148 + 15 us,
+ * against 430 (179 where the selection reads the spectra for their norms); 250 spectra: 14 + 39 + 8 us, against 171.  The selection is a
+ * chain of short steps, half of its waves waiting; the exact scores are bound by their FP64 terms and
  * the maps' LDS atomics.
  */
 #define HFX_TOPN_REL_F32 (80.0f * 5.9604644775390625e-08f)
@@ -178,7 +177,7 @@ struct TnLists {
 template <class Cands>
 __global__ void __launch_bounds__(TN_THREADS)
     k_topn_select(TnLists o, uint32_t *flag, uint32_t N, uint32_t margin, const float *scores,
-                  Cands c, hfx_spectra sp, float rel0, float rel1, float relq)
+                  Cands c, hfx_spectra sp, float rel0, float rel1, float relq, const float2 *norms)
 {
     __shared__ uint32_t hist[TN_HBINS];
     __shared__ uint64_t kv[TN_MAXC]; /* (key, ~position) */
@@ -225,7 +224,7 @@ __global__ void __launch_bounds__(TN_THREADS)
     }
 
     /* 1. the scores, once, four at a time, and the largest of each thread;
-     * sum|x| and max|x| */
+     * sum|x| and max|x|, where the caller does not have them (norms) */
     const bool held = n <= TN_HOLD * TN_THREADS;
     const uint32_t len = min(sp.d_len[s], min(sp.x_stride, (uint32_t)HFX_MAX_LEN));
     const float *xg = sp.d_x + (size_t)s * sp.x_stride;
@@ -246,7 +245,7 @@ __global__ void __launch_bounds__(TN_THREADS)
         }
     }
     float x1 = 0.0f, xm = 0.0f;
-    for (uint32_t base = 0; base < len; base += 8 * TN_THREADS) {
+    for (uint32_t base = 0; !norms && base < len; base += 8 * TN_THREADS) {
         float v[8];
 #pragma unroll
         for (uint32_t u = 0; u < 8; ++u) v[u] = xg[min(base + u * TN_THREADS + tid, len - 1u)];
@@ -304,6 +303,10 @@ __global__ void __launch_bounds__(TN_THREADS)
         xa += sh_x1[w];
         xmax = fmaxf(xmax, sh_xm[w]);
         low = max(low, sh_low[w]);
+    }
+    if (norms) {
+        xa = norms[s].x;
+        xmax = norms[s].y;
     }
     const double rel = (double)rel0 + (double)rel1 * (double)zeff;
     const double bound = rel * 50.0 * (double)xa * 1.001 +
@@ -1249,8 +1252,8 @@ template <class Cands>
 static int launch_topn(hfx_ctx *ctx, uint32_t *d_top_pos, double *d_top_exact, float *d_top_f32,
                        uint32_t *d_top_cnt, uint32_t *d_flag, uint32_t N, uint32_t margin,
                        const float *d_scores, const Cands &c, uint64_t total,
-                       const hfx_spectra *sp, float rel0, float rel1, float relq, void *scratch,
-                       void *stream)
+                       const hfx_spectra *sp, float rel0, float rel1, float relq,
+                       const float2 *norms, void *scratch, void *stream)
 {
     HFX_REQUIRE(ctx && d_top_pos && d_top_exact && d_top_f32 && d_top_cnt && d_flag && d_scores &&
                     sp,
@@ -1268,7 +1271,7 @@ static int launch_topn(hfx_ctx *ctx, uint32_t *d_top_pos, double *d_top_exact, f
     const uint32_t gw = (S + TN_WAVES - 1) / TN_WAVES;
     hipLaunchKernelGGL(k_tx_reset, dim3(1), dim3(1), 0, st, x.counter);
     hipLaunchKernelGGL(k_topn_select<Cands>, dim3(S), dim3(TN_THREADS), 0, st, x.l, d_flag, N,
-                       margin, d_scores, c, *sp, rel0, rel1, relq);
+                       margin, d_scores, c, *sp, rel0, rel1, relq, norms);
     /* at least a workgroup a CU: the spilled tasks spread over all of them */
     hipLaunchKernelGGL(k_topn_exact<Cands>, dim3(max(gw, (uint32_t)hfx_ctx_num_cus(ctx))),
                        dim3(TN_THREADS), fx_lds_bytes(sp->x_stride), st, x.fxbuf, x.l, c, *sp,
@@ -1309,8 +1312,8 @@ int hfx_topn_device(hfx_ctx *ctx, uint32_t *d_top_pos, double *d_top_exact, floa
                     uint32_t *d_top_cnt, uint32_t *d_flag, uint32_t N, uint32_t margin,
                     const float *d_scores, const uint64_t *d_off, uint64_t total,
                     const uint32_t *d_begin, const uint32_t *d_num, const hfx_db *db,
-                    const hfx_spectra *sp, float rel0, float rel1, float relq, void *scratch,
-                    void *stream)
+                    const hfx_spectra *sp, float rel0, float rel1, float relq, const float2 *norms,
+                    void *scratch, void *stream)
 {
     HFX_REQUIRE(rel0 >= 0.0f && rel1 >= 0.0f && relq >= 0.0f && rel0 < 1.0f && rel1 < 1.0f &&
                     relq < 1.0f,
@@ -1319,7 +1322,7 @@ int hfx_topn_device(hfx_ctx *ctx, uint32_t *d_top_pos, double *d_top_exact, floa
                 rel1, relq);
     HfxPlainCands c{*db, d_begin, d_num, d_off};
     return launch_topn(ctx, d_top_pos, d_top_exact, d_top_f32, d_top_cnt, d_flag, N, margin,
-                       d_scores, c, total, sp, rel0, rel1, relq, scratch, stream);
+                       d_scores, c, total, sp, rel0, rel1, relq, norms, scratch, stream);
 }
 
 extern "C" int hfx_topn(hfx_ctx *ctx, uint32_t *d_top_pos, double *d_top_exact, float *d_top_f32,
@@ -1331,7 +1334,7 @@ extern "C" int hfx_topn(hfx_ctx *ctx, uint32_t *d_top_pos, double *d_top_exact, 
     HFX_REQUIRE(d_off && d_begin && d_num && db, HFX_ERR_ARG, "hfx_topn: null argument");
     return hfx_topn_device(ctx, d_top_pos, d_top_exact, d_top_f32, d_top_cnt, d_flag, N, margin,
                            d_scores, d_off, total, d_begin, d_num, db, sp, HFX_TOPN_REL_F32, 0.0f,
-                           0.0f, nullptr, stream);
+                           0.0f, nullptr, nullptr, stream);
 }
 
 extern "C" int hfx_topn_rel(hfx_ctx *ctx, uint32_t *d_top_pos, double *d_top_exact,
@@ -1344,7 +1347,7 @@ extern "C" int hfx_topn_rel(hfx_ctx *ctx, uint32_t *d_top_pos, double *d_top_exa
     HFX_REQUIRE(d_off && d_begin && d_num && db, HFX_ERR_ARG, "hfx_topn_rel: null argument");
     return hfx_topn_device(ctx, d_top_pos, d_top_exact, d_top_f32, d_top_cnt, d_flag, N, margin,
                            d_scores, d_off, total, d_begin, d_num, db, sp, rel0, rel1, 0.0f,
-                           nullptr, stream);
+                           nullptr, nullptr, stream);
 }
 
 extern "C" int hfx_topn_rel_q(hfx_ctx *ctx, uint32_t *d_top_pos, double *d_top_exact,
@@ -1357,7 +1360,7 @@ extern "C" int hfx_topn_rel_q(hfx_ctx *ctx, uint32_t *d_top_pos, double *d_top_e
     HFX_REQUIRE(d_off && d_begin && d_num && db, HFX_ERR_ARG, "hfx_topn_rel_q: null argument");
     return hfx_topn_device(ctx, d_top_pos, d_top_exact, d_top_f32, d_top_cnt, d_flag, N, margin,
                            d_scores, d_off, total, d_begin, d_num, db, sp, rel0, rel1, relq,
-                           nullptr, stream);
+                           nullptr, nullptr, stream);
 }
 
 extern "C" int hfx_topn_exact(hfx_ctx *ctx, uint32_t *d_top_pos, double *d_top_exact,
@@ -1385,7 +1388,7 @@ extern "C" int hfx_topn_mod(hfx_ctx *ctx, uint32_t *d_top_pos, double *d_top_exa
     HfxModCands c{*db, *ms, d_mp_off};
     return launch_topn(ctx, d_top_pos, d_top_exact, d_top_f32, d_top_cnt, d_flag, N, margin,
                        d_scores, c, ms->num_mpep, sp, HFX_TOPN_REL_F32, 0.0f, 0.0f, nullptr,
-                       stream);
+                       nullptr, stream);
 }
 
 extern "C" int hfx_topn_exact_mod(hfx_ctx *ctx, uint32_t *d_top_pos, double *d_top_exact,
