@@ -32,8 +32,9 @@
  * with 200 tied candidates held up a small batch by itself.
  * Now, select + exact + rank: 10,000 spectra, 1120 candidates each, top 10:
  * 127 + 136 + 15 us, against 445 us; 20,000 spectra, top 5: 160 + 148 + 15 us,
- * against 430 (179 where the selection reads the spectra for their norms); 250 spectra: 14 + 39 + 8 us, against 171.  The selection is a
- * chain of short steps, half of its waves waiting; the exact scores are bound by their FP64 terms and
+ * against 430 (179 where the selection reads the spectra for their norms); 250
+ * spectra: 14 + 39 + 8 us, against 171.  The selection is a chain of short steps,
+ * half of its waves waiting; the exact scores are bound by their FP64 terms and
  * the maps' LDS atomics.
  */
 #define HFX_TOPN_REL_F32 (80.0f * 5.9604644775390625e-08f)
