@@ -312,7 +312,7 @@ __global__ void __launch_bounds__(RB_THREADS, RB_PER_CU) k_rw_build(RbArgs a)
     const uint32_t G = gridDim.x;
     auto order = [&](uint64_t t) {
         const uint64_t q = t * RW_ROWS + (lane & 15u);
-        return q < a.db.num_pep ? a.db.d_idx_sorted[q] : 0xffffffffu;
+        return t < a.ntiles && q < a.db.num_pep ? a.db.d_idx_sorted[q] : 0xffffffffu;
     };
     struct Meta {
         uint32_t tc, tn;
@@ -330,31 +330,50 @@ __global__ void __launch_bounds__(RB_THREADS, RB_PER_CU) k_rw_build(RbArgs a)
 #pragma unroll
         for (uint32_t j = 0; j < 2; ++j) x[j] = lk + 16 * j < n ? a.db.d_ions[tc + lk + 16 * j] : 0u;
     };
-    uint32_t want_next = 0;
-    auto wanted = [&](uint64_t t) {
-        uint32_t w = 0;
+    /* the wanted tiles among blockIdx.x, blockIdx.x + G, ...: 64 looked at at once,
+     * a tile a lane; ~0 past the last */
+    uint64_t look = blockIdx.x, from = 0, left = 0;
+    uint32_t lane_want = 0;
+    auto next = [&](uint32_t &want) -> uint64_t {
+        while (!left) {
+            want = 0;
+            if (look >= a.ntiles) return ~0ull;
+            from = look;
+            const uint64_t t = from + (uint64_t)lane * G;
+            lane_want = 0;
 #pragma unroll
-        for (uint32_t l = 0; l < HFX_MAX_CHARGE; ++l)
-            if (a.rows[l] && (!a.flags || rw_sload(a.flags, (uint64_t)l * a.ntiles + t) != 0u))
-                w |= 1u << l;
-        return w;
+            for (uint32_t l = 0; l < HFX_MAX_CHARGE; ++l)
+                if (a.rows[l] && t < a.ntiles && (!a.flags || a.flags[(size_t)l * a.ntiles + t] != 0u))
+                    lane_want |= 1u << l;
+            left = __ballot(lane_want != 0u);
+            look += 64ull * G;
+        }
+        const uint32_t i = (uint32_t)__builtin_ctzll(left);
+        left &= left - 1ull;
+        want = (uint32_t)__builtin_amdgcn_readlane((int)lane_want, (int)i);
+        return from + (uint64_t)i * G;
     };
-    /* tile t: its residues; t + G: its offsets; t + 2 G: its order */
-    Meta m0 = meta(order(blockIdx.x)), m1 = meta(order((uint64_t)blockIdx.x + G));
-    uint32_t pep = order((uint64_t)blockIdx.x + 2ull * G), x[2];
+    /* the tile written: its offsets and residues; the one after it: its offsets;
+     * the one after that: its order */
+    uint32_t w0, w1, w2, x[2];
+    uint64_t t0 = next(w0), t1 = next(w1), t2 = next(w2);
+    Meta m0 = meta(order(t0)), m1 = meta(order(t1));
+    uint32_t pep = order(t2);
     residues(m0, x);
-    if (blockIdx.x < a.ntiles) want_next = wanted(blockIdx.x);
-    uint32_t turn = blockIdx.x;
     __syncthreads();
-    for (uint64_t t = blockIdx.x; t < a.ntiles; t += G, ++turn) {
+    for (uint32_t turn = blockIdx.x; t0 != ~0ull; ++turn) {
+        const uint64_t t = t0;
         const Meta m = m0;
-        const uint32_t want = want_next, x0 = x[0], x1 = x[1];
+        const uint32_t want = w0, x0 = x[0], x1 = x[1];
+        t0 = t1;
+        t1 = t2;
+        w0 = w1;
+        w1 = w2;
         m0 = m1;
         residues(m0, x);
         m1 = meta(pep);
-        pep = order(t + 3ull * G);
-        if (t + G < a.ntiles) want_next = wanted(t + G);
-        if (!want) continue;
+        t2 = next(w2);
+        pep = order(t2);
         const uint32_t n = count(m);
         uint32_t nmax = n;
 #pragma unroll
