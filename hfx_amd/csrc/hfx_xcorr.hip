@@ -9,7 +9,7 @@
  * and are dotted straight against the spectrum held in LDS: no dense row ever
  * reaches HBM.
  *
- * Work decomposition: one workgroup (4 waves) per (spectrum, chunk of
+ * Work decomposition: one workgroup (4 waves) per (spectrum, chunk of up to
  * XP_CHUNK candidates) tile; the spectrum is staged in LDS once per tile; each
  * wave scores several short candidates at a time (ladders -> maps -> claims).
  * Large calls write each theoretical row once instead (hfx_rows.hip).
@@ -39,7 +39,7 @@ __device__ __forceinline__ uint32_t find_segment(const uint64_t *off, uint32_t n
 /* Plain candidates, packed: several candidates per wave                 */
 /* ------------------------------------------------------------------ */
 
-/* One workgroup (four waves) per tile of XP_CHUNK candidates of one
+/* One workgroup (four waves) per tile of up to XP_CHUNK candidates of one
  * spectrum; each wave takes a quarter of the tile and packs up to XP_SLOTS
  * consecutive candidates of at most 64 ladder positions in all into its 64
  * lanes, one lane per (candidate, ladder position):
@@ -58,8 +58,7 @@ __device__ __forceinline__ uint32_t find_segment(const uint64_t *off, uint32_t n
 #define XP_THREADS 256
 #define XP_WAVES (XP_THREADS / HFX_WAVE)
 #define XP_CHUNK 128
-#define XP_RANGE (XP_CHUNK / XP_WAVES) /* candidates a wave takes from a tile */
-static_assert(XP_RANGE <= HFX_WAVE, "a wave's candidates fit its lanes");
+static_assert(XP_CHUNK / XP_WAVES <= HFX_WAVE, "a wave's candidates fit its lanes");
 static size_t xp_lds_bytes(uint32_t xstr)
 {
     const size_t xf = ((size_t)xstr + 2 * XP_PAD + 3) & ~(size_t)3;
@@ -91,40 +90,32 @@ __device__ __forceinline__ float xp_claim(const XpPeaks &pk, const float *xsm, f
     return acc;
 }
 
-/* v + (the value of the lane DPP control CTRL selects; 0 where none, and in
- * rows outside ROWS) */
-template <int CTRL, int ROWS>
-__device__ __forceinline__ float xp_dpp_add(float v)
+/* the value of the lane before (0 in lane 0) */
+__device__ __forceinline__ float xp_prev(float v)
 {
-    return v + __uint_as_float((uint32_t)__builtin_amdgcn_update_dpp(
-                   0, (int)__float_as_uint(v), CTRL, ROWS, 0xf, true));
+    return __uint_as_float((uint32_t)__builtin_amdgcn_update_dpp(0, (int)__float_as_uint(v),
+                                                                 0x138 /* wave_shr:1 */, 0xf, 0xf, false));
 }
 
-/* Inclusive segmented sum over the wave: lane l ends with the sum of the
- * lanes of its segment from the segment's first lane (kpos = 0) to l, added
- * in a fixed tree (at most six additions on any term's path).  Within rows
- * of 16 lanes by row shifts of 1, 2, 4, 8, then the last lanes of rows 0
- * and 2 into rows 1 and 3 and the last lane of row 1 into rows 2 and 3 (the
- * wave scan of gfx9 DPP), each step taken only where the source lane lies in
- * the same segment. */
+/* Inclusive segmented sum over the wave: lane l ends with the sum of the lanes of
+ * its segment from the segment's first lane (kpos = 0) to l, by doubling steps
+ * taken where kpos reaches back that far: the order of the additions is that of the
+ * candidate's positions alone, so that a score has the same bits wherever its
+ * candidate lies in a pack. */
 __device__ __forceinline__ float xp_segsum(float v, uint32_t kpos, uint32_t lane)
 {
-    const uint32_t r = lane & 15u;
-    float t;
-    t = xp_dpp_add<0x111 /* row_shr:1 */, 0xf>(v);
-    v = kpos >= 1 && r >= 1 ? t : v;
-    t = xp_dpp_add<0x112 /* row_shr:2 */, 0xf>(v);
-    v = kpos >= 2 && r >= 2 ? t : v;
-    t = xp_dpp_add<0x114 /* row_shr:4 */, 0xf>(v);
-    v = kpos >= 4 && r >= 4 ? t : v;
-    t = xp_dpp_add<0x118 /* row_shr:8 */, 0xf>(v);
-    v = kpos >= 8 && r >= 8 ? t : v;
-    /* lane 15 of rows 0 and 2 into rows 1 and 3 */
-    t = xp_dpp_add<0x142 /* row_bcast:15 */, 0xa>(v);
-    v = (lane & 16u) && kpos > r ? t : v;
-    /* lane 31 into rows 2 and 3 */
-    t = xp_dpp_add<0x143 /* row_bcast:31 */, 0xc>(v);
-    v = lane >= 32u && kpos > lane - 32u ? t : v;
+#pragma unroll
+    for (uint32_t o = 1; o < HFX_WAVE; o <<= 1) {
+        float t = v;
+        if (o <= 4) {
+#pragma unroll
+            for (uint32_t i = 0; i < o; ++i) t = xp_prev(t);
+        } else {
+            t = __uint_as_float((uint32_t)__builtin_amdgcn_ds_bpermute((int)((lane - o) << 2),
+                                                                       (int)__float_as_uint(v)));
+        }
+        v = kpos >= o ? v + t : v;
+    }
     return v;
 }
 
@@ -206,9 +197,9 @@ __device__ __forceinline__ void xp_pack(uint32_t *maps, uint32_t mstr, const flo
 template <class Cands>
 __device__ __forceinline__ void xp_tile(float *xp_lds, float *mtab, float *scores, const Cands &c,
                                         const hfx_spectra &sp, uint32_t mstr, uint32_t s,
-                                        uint32_t first)
+                                        uint32_t first, uint32_t chunk)
 {
-    const uint32_t cnt = min((uint32_t)XP_CHUNK, c.count(s) - first);
+    const uint32_t cnt = min(chunk, c.count(s) - first);
     const uint32_t xstr = sp.x_stride;
     const uint32_t xf = (xstr + 2 * XP_PAD + 3) & ~3u;
     float *xs = xp_lds + XP_PAD;
@@ -224,9 +215,9 @@ __device__ __forceinline__ void xp_tile(float *xp_lds, float *mtab, float *score
     __syncthreads();
     const uint32_t zeff = c.zeff(sp.d_zmax[s]);
     /* this wave's candidates [c0, c0 + rn) of the tile */
-    const uint32_t c0 = wave * XP_RANGE;
+    const uint32_t range = chunk / XP_WAVES, c0 = wave * range;
     const uint32_t rn = __builtin_amdgcn_readfirstlane(
-        c0 < cnt ? min((uint32_t)XP_RANGE, cnt - c0) : 0u);
+        c0 < cnt ? min(range, cnt - c0) : 0u);
     float *out = scores + c.base(s) + first + c0;
     if (rn == 0) return;
     if (zeff == 0) {
@@ -283,7 +274,8 @@ __device__ __forceinline__ void xp_tile(float *xp_lds, float *mtab, float *score
 
 template <class Cands>
 __global__ void __launch_bounds__(XP_THREADS)
-    k_xcorr_pack(float *scores, const uint64_t *tile_off, Cands c, hfx_spectra sp, uint32_t mstr)
+    k_xcorr_pack(float *scores, const uint64_t *tile_off, Cands c, hfx_spectra sp, uint32_t mstr,
+                 uint32_t chunk)
 {
     extern __shared__ __align__(16) float xp_lds[];
     __shared__ float mtab[32];
@@ -291,7 +283,7 @@ __global__ void __launch_bounds__(XP_THREADS)
     const uint64_t t = blockIdx.x;
     if (t >= tile_off[S]) return;
     const uint32_t s = find_segment(tile_off, S, t);
-    xp_tile(xp_lds, mtab, scores, c, sp, mstr, s, (uint32_t)(t - tile_off[s]) * XP_CHUNK);
+    xp_tile(xp_lds, mtab, scores, c, sp, mstr, s, (uint32_t)(t - tile_off[s]) * chunk, chunk);
 }
 
 /* The spectra marked in wide (seldom any), a workgroup each at a time: the
@@ -316,12 +308,24 @@ __global__ void __launch_bounds__(XP_THREADS)
                 const uint32_t s = (uint32_t)(blockIdx.x + (k0 + w * HFX_WAVE +
                                                             (uint32_t)__builtin_ctzll(m)) * G);
                 for (uint32_t f = 0; f < c.count(s); f += XP_CHUNK) {
-                    xp_tile(xp_lds, mtab, scores, c, sp, mstr, s, f);
+                    xp_tile(xp_lds, mtab, scores, c, sp, mstr, s, f, XP_CHUNK);
                     __syncthreads(); /* its LDS is staged anew */
                 }
             }
         __syncthreads();
     }
+}
+
+/* Candidates a tile takes, a multiple of XP_WAVES up to XP_CHUNK.  A wave's share
+ * is a chain of packs, and few tiles leave CUs idle; many small ones stage the
+ * spectrum too often.  Scores of 100 spectra (33,460 pairs of short peptides):
+ * 25 us with 16, 21 with 32, 31 with 64, 48 with 128; 16,183 pairs 17.4, 17.8,
+ * 26, 41; 131,032 pairs 69, 51, 49, 56; 457,000 pairs 207, 140, 121, 124; long
+ * peptides move the lines up (48,347 pairs 33, 37, 55, 87; 365,831 pairs 186, 146,
+ * 151, 157); 10.2 million modified ones take 9 % more with 64 than with 128. */
+static uint32_t xp_chunk(uint64_t total)
+{
+    return total <= 24000 ? 16u : total <= 160000 ? 32u : total <= 1000000 ? 64u : XP_CHUNK;
 }
 
 template <class Cands>
@@ -343,7 +347,7 @@ static int launch_xcorr(void *scratch, float *d_scores, const Cands &c, uint64_t
     if (S == 0 || total == 0) return HFX_OK;
     HFX_REQUIRE(sp->x_stride <= HFX_MAX_LEN, HFX_ERR_ARG,
                 "sparse XCorr: spectra of up to %d bins (x_stride %u)", HFX_MAX_LEN, sp->x_stride);
-    const uint32_t chunk = XP_CHUNK;
+    const uint32_t chunk = xp_chunk(total);
     hipStream_t st = hfx_stream(stream);
     int rc;
     uint32_t *tiles = (uint32_t *)scratch;
@@ -356,7 +360,7 @@ static int launch_xcorr(void *scratch, float *d_scores, const Cands &c, uint64_t
     HFX_REQUIRE(grid < (1ull << 31), HFX_ERR_ARG, "xcorr: %llu tiles", (unsigned long long)grid);
     hipLaunchKernelGGL(k_xcorr_pack<Cands>, dim3((uint32_t)grid), dim3(XP_THREADS),
                        xp_lds_bytes(sp->x_stride), st, d_scores, tile_off, c, *sp,
-                       xp_map_words(sp->x_stride));
+                       xp_map_words(sp->x_stride), chunk);
     HFX_CHECK_LAUNCH();
     return HFX_OK;
 }
@@ -379,12 +383,22 @@ int hfx_xcorr_wide(hfx_ctx *ctx, float *d_scores, const uint64_t *d_off, const u
 /* Rows route                                                            */
 /* ------------------------------------------------------------------ */
 
-/* From this many scored pairs on, hfx_xcorr_sparse writes each candidate's
- * theoretical row once and contracts the rows with blocks of sixteen spectra
- * (hfx_rows.hip, 32-bit fixed point) instead of building a row per pair.  Its
- * dozen launches cost about 100 us, which the packed kernel spends on half a
- * million pairs. */
-#define XR_MIN_PAIRS 500000ull
+/* hfx_xcorr_sparse writes each candidate's theoretical row once and contracts the
+ * rows with blocks of sixteen spectra (hfx_rows.hip, 32-bit fixed point) instead
+ * of building a row per pair, where that is quicker.  In ns: a pair costs 230 ps
+ * to score by itself, 30 through its row; the rows' dozen launches 80,000 more
+ * than the packed kernel's three; a tile of the database 1/3 to look at and, if a
+ * window holds it, 2.7 at each charge level to write and read (as many as the
+ * pairs fill, at most two levels of all).  Measured, packed and rows, us: 2000
+ * proteins, short peptides (7,293 tiles) 520,778 pairs 138 and 161, 1,043,828
+ * pairs 243 and 174; longer ones (16,900 tiles) 365,831 pairs 156 and 181, 733,473
+ * pairs 233 and 216; 20,000 proteins (73,000 and 170,000 tiles) 1,240,720 pairs
+ * 268 and 333, 1,839,460 pairs 453 and 549; 46 million pairs 9,409 and 1,800. */
+static bool xr_pays(uint64_t total, uint32_t tiles)
+{
+    const uint64_t read = min(total / RW_ROWS, 2ull * tiles);
+    return total / 5 > 80000ull + tiles / 3 + read * 27 / 10;
+}
 
 /* *taken = 0: nothing done (too few pairs, rows longer than the form's, no
  * memory to spare) */
@@ -394,8 +408,8 @@ static int xcorr_rows(hfx_ctx *ctx, float *d_scores, const uint64_t *d_off,
 {
     *taken = 0;
     const uint32_t S = sp->num_spec;
-    if (total < XR_MIN_PAIRS || sp->x_stride > RW_MAXK || db->num_pep == 0) return HFX_OK;
     const uint32_t nt = hfx_rows_tiles(db->num_pep), G = hfx_rows_groups(sp->x_stride);
+    if (!xr_pays(total, nt) || sp->x_stride > RW_MAXK || db->num_pep == 0) return HFX_OK;
     const uint64_t nf = (uint64_t)HFX_MAX_CHARGE * nt;
     if (nf >= 0xffffffffull) return HFX_OK;
     /* the block cut never takes more rows than the windows one by one */
