@@ -13,8 +13,10 @@
 
 #define XP_SLOTS 4
 /* b-ladder positions a wave's buffer holds (a chunk of its candidates at a
- * time; any one packable candidate has at most 64) */
-#define XP_LB 256
+ * time; any one packable candidate has at most 64): the more, the more lanes walk
+ * ladders at once; past 288 a CU holds four workgroups instead of five (10.2
+ * million modified candidates: 2,945 us with 256, 2,897 with 288, 3,131 with 320) */
+#define XP_LB 288
 /* Peaks outside [0, len) are clamped onto margin bins whose spectrum values
  * are zero (so they add 0 when claimed): singles onto bin -1 - 8 (lane & 7)
  * or len + 8 (lane & 7), triple centres onto -2 - 8 (lane & 7) or

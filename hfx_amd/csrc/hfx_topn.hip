@@ -701,9 +701,10 @@ __global__ void __launch_bounds__(TN_THREADS)
     k_topn_exact(int64_t *fx, TnLists o, Cands c, hfx_spectra sp, uint32_t mstr)
 {
     extern __shared__ __align__(16) unsigned char tn_dyn[];
-    __shared__ float mtab[32];
+    __shared__ float mtab[HFX_MTAB];
     const uint32_t wave = threadIdx.x / HFX_WAVE, lane = hfx_lane(), S = sp.num_spec;
     if (threadIdx.x < 32) mtab[threadIdx.x] = threadIdx.x < 26 ? c.db.d_mass[threadIdx.x] : 0.0f;
+    c.stage(mtab);
     const FxWave f = fx_wave(tn_dyn, mstr, wave);
     __syncthreads();
     auto task = [&](uint32_t s, uint32_t k0) {
@@ -893,13 +894,14 @@ __global__ void __launch_bounds__(TN_THREADS)
                   const double *tau, uint32_t mstr)
 {
     extern __shared__ __align__(16) unsigned char tn_dyn[];
-    __shared__ float mtab[32];
+    __shared__ float mtab[HFX_MTAB];
     __shared__ uint32_t lpos[TN_WAVES][HFX_WAVE];
     const uint32_t wave = threadIdx.x / HFX_WAVE, lane = hfx_lane();
     const uint32_t F = *count;
     const uint64_t ntiles = tile_off[F];
     if (blockIdx.x >= ntiles) return;
     if (threadIdx.x < 32) mtab[threadIdx.x] = threadIdx.x < 26 ? c.db.d_mass[threadIdx.x] : 0.0f;
+    c.stage(mtab);
     const FxWave f = fx_wave(tn_dyn, mstr, wave);
     __syncthreads();
     for (uint64_t t = blockIdx.x; t < ntiles; t += gridDim.x) {

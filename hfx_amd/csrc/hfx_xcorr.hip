@@ -208,6 +208,7 @@ __device__ __forceinline__ void xp_tile(float *xp_lds, float *mtab, float *score
     uint32_t *maps = maps_all + wave * XP_SLOTS * mstr;
     float *lb = (float *)(maps_all + XP_WAVES * XP_SLOTS * mstr) + wave * XP_LB;
     const uint32_t len = hfx_stage_spectrum(xs, mtab, c.db, sp, s);
+    c.stage(mtab);
     /* zeros around the spectrum: clamped peaks read them */
     for (uint32_t i = len + threadIdx.x; i < xf - XP_PAD; i += XP_THREADS) xs[i] = 0.0f;
     for (uint32_t i = threadIdx.x; i < XP_PAD; i += XP_THREADS) xp_lds[i] = 0.0f;
@@ -278,7 +279,7 @@ __global__ void __launch_bounds__(XP_THREADS)
                  uint32_t chunk)
 {
     extern __shared__ __align__(16) float xp_lds[];
-    __shared__ float mtab[32];
+    __shared__ float mtab[HFX_MTAB];
     const uint32_t S = sp.num_spec;
     const uint64_t t = blockIdx.x;
     if (t >= tile_off[S]) return;
@@ -294,7 +295,7 @@ __global__ void __launch_bounds__(XP_THREADS)
                  uint32_t mstr)
 {
     extern __shared__ __align__(16) float xp_lds[];
-    __shared__ float mtab[32];
+    __shared__ float mtab[HFX_MTAB];
     __shared__ uint64_t marked[XP_WAVES];
     const uint32_t S = sp.num_spec, G = gridDim.x;
     /* this workgroup's spectra are blockIdx.x + k G, k = 0, 1, ... */
