@@ -89,19 +89,19 @@ struct HfxPlainCands {
     }
     __device__ __forceinline__ void stage(float *) const {}
     /* one lane: the candidate's b ladder (sequential FP32 prefix of its
-     * first nl residue masses) into dst, four residues loaded ahead (the
+     * first nl residue masses) into dst, eight residues loaded ahead (the
      * last one re-read past the end) */
     __device__ __forceinline__ void ladder(const Prep &p, const float *mtab, float *dst,
                                            uint32_t nl) const
     {
         const uint8_t *res = db.d_ions + p.tc;
         float bl = 0.0f;
-        for (uint32_t k = 0; k < nl; k += 4) {
-            uint32_t a[4];
+        for (uint32_t k = 0; k < nl; k += 8) {
+            uint32_t a[8];
 #pragma unroll
-            for (uint32_t j = 0; j < 4; ++j) a[j] = res[min(k + j, nl - 1u)];
+            for (uint32_t j = 0; j < 8; ++j) a[j] = res[min(k + j, nl - 1u)];
 #pragma unroll
-            for (uint32_t j = 0; j < 4; ++j) {
+            for (uint32_t j = 0; j < 8; ++j) {
                 if (k + j < nl) {
                     bl = bl + mtab[HFX_ACID_IDX(a[j])];
                     dst[k + j] = bl;
@@ -160,9 +160,9 @@ struct HfxModCands {
      * i-th of its acid in the peptide weighs table + ma_mass[a] when i is in
      * the acid's part of the unrank slice (HfxModMass's rule, per lane).
      * One word holds the acids' occurrence masks (64 / num_ma bits each) and one
-     * their counters, and eight residues are on their way at a time: a mask and a
-     * test for each acid took 940 of 3,206 us of 10.2 million candidates, this
-     * 640 of 2,905.  Occurrences that the masks do not hold (the sixteenth of an acid,
+     * their counters; four entries of the slice and eight residues are on their way at
+     * a time.  A mask and a test for each acid took 940 of 3,206 us of 10.2 million
+     * candidates; they take 2,800 now.  Occurrences that the masks do not hold (the sixteenth of an acid,
      * with four acids) are looked up in the slice. */
     __device__ __forceinline__ void ladder(const Prep &p, const float *mtab, float *dst,
                                            uint32_t nl) const
@@ -171,18 +171,29 @@ struct HfxModCands {
         const uint32_t w = min(64u / max(na, 1u), 16u); /* bits of a mask */
         const uint32_t *row = ms.d_mod_ma_count + (size_t)p.mod * ms.num_ma;
         const uint32_t *u = ms.d_unrank + p.uoff;
+        /* the acids' shares of the slice end here; then its entries, four reads at
+         * a time */
+        uint32_t ends[HFX_MAX_MA], tot = 0;
+#pragma unroll
+        for (uint32_t a = 0; a < HFX_MAX_MA; ++a) ends[a] = a < na ? row[a] : 0u;
+#pragma unroll
+        for (uint32_t a = 0; a < HFX_MAX_MA; ++a) ends[a] = tot += ends[a];
         uint64_t mask = 0;
         bool fits = true;
-        uint32_t off = 0;
-        for (uint32_t a = 0; a < na; ++a) {
-            const uint32_t k = row[a];
-            for (uint32_t q = 0; q < k; ++q) {
-                const uint32_t i = u[off + q];
-                /* the last bit stays clear: it stands for every later occurrence */
-                if (i + 1u < w) mask |= 1ull << (w * a + i);
-                else fits = false;
-            }
-            off += k;
+        for (uint32_t q = 0; q < tot; q += 4) {
+            uint32_t e[4];
+#pragma unroll
+            for (uint32_t j = 0; j < 4; ++j) e[j] = u[min(q + j, tot - 1u)];
+#pragma unroll
+            for (uint32_t j = 0; j < 4; ++j)
+                if (q + j < tot) {
+                    uint32_t a = 0;
+#pragma unroll
+                    for (uint32_t i = 0; i + 1 < HFX_MAX_MA; ++i) a += q + j >= ends[i] ? 1u : 0u;
+                    /* the last bit stays clear: it stands for every later occurrence */
+                    if (e[j] + 1u < w) mask |= 1ull << (w * a + e[j]);
+                    else fits = false;
+                }
         }
         const uint8_t *res = db.d_ions + p.tc;
         uint32_t occ = 0; /* four bits an acid, staying at fifteen */
