@@ -1236,7 +1236,7 @@ static int bt_dense_prep(hfx_batch *b, hipStream_t st)
         return rc;
     if (b->use_rows) {
         return hfx_rows_split(bt_mode(b), &b->sp, bt_planes(b), bt_quanta(b), bt_levels(b),
-                              bt_wide(b), bt_norms(b), (void *)st);
+                              bt_wide(b), bt_norms(b), b->scores, b->score_off, (void *)st);
     }
     return bf ? hfx_dense_split(&b->sp, b->dn_scratch, (void *)st)
               : hfx_dense8_split(&b->sp, b->dn_scratch, (void *)st);
@@ -1305,7 +1305,7 @@ static int bt_row_scores(hfx_batch *b, hipStream_t st, void **ev)
                               &sq, b->CH, (void *)st)) ||
         (rc = hfx_rows_scores(b->ctx, mode, bt_items(b), b->scores, b->score_off, b->begin, b->num,
                               b->order, b->dn_bstart, &b->ix->rows, bt_planes(b), qs, &sq, b->CH,
-                              b->sp.d_zmax, (void *)st, ev)))
+                              (void *)st, ev)))
         return rc;
     if (mode != RW_I8X4) return HFX_OK;
     return hfx_xcorr_wide(b->ctx, b->scores, b->score_off, b->begin, b->num, &b->db, &b->sp,

@@ -162,8 +162,8 @@ struct HfxModCands {
      * One word holds the acids' occurrence masks (64 / num_ma bits each) and one
      * their counters; four entries of the slice and eight residues are on their way at
      * a time.  A mask and a test for each acid took 940 of 3,206 us of 10.2 million
-     * candidates; they take 2,800 now.  Occurrences that the masks do not hold (the sixteenth of an acid,
-     * with four acids) are looked up in the slice. */
+     * candidates; they take 2,800 now.  Occurrences that the masks do not hold (the
+     * sixteenth of an acid, with four acids) are looked up in the slice. */
     __device__ __forceinline__ void ladder(const Prep &p, const float *mtab, float *dst,
                                            uint32_t nl) const
     {

@@ -33,9 +33,10 @@ uint32_t hfx_rows_groups(uint32_t x_stride);
 uint32_t hfx_rows_chunk(uint64_t rows, uint32_t cus);
 /* planes [S][RW_PLANES][RW_MAXK] and quanta of the spectra; RW_I8X4 also
  * writes each spectrum's charge level to lvl, or to wide where its digits would
- * lose precision (0 in the other); norms [S], if any: sum and max of |x| */
+ * lose precision (0 in the other); norms [S], if any: sum and max of |x|.  Scores of spectra whose charge is not
+ * generated are set to 0 */
 int hfx_rows_split(int mode, const hfx_spectra *sp, uint8_t *planes, float *qs, uint32_t *lvl,
-                   uint32_t *wide, float2 *norms, void *stream);
+                   uint32_t *wide, float2 *norms, float *scores, const uint64_t *off, void *stream);
 /* writes the rows of the wanted levels (non-null) and tiles (flags
  * [HFX_MAX_CHARGE][ntiles], null: all) */
 int hfx_rows_build(uint32_t cus, const hfx_db *db, const hfx_rows *r, const uint32_t *flags,
@@ -48,13 +49,11 @@ int hfx_rows_blocks(hfx_ctx *ctx, int mode, void *scratch, const uint32_t *order
                     const hfx_spectra *sp, uint32_t CH, void *stream);
 /* flags [HFX_MAX_CHARGE][ntiles]: the tiles those items read */
 int hfx_rows_mark(void *scratch, uint32_t S, uint32_t *flags, uint32_t ntiles, void *stream);
-/* the scores of every item; spectra whose charge in zmax is not generated
- * score 0 (sp's own d_zmax may hide spectra from the items) */
+/* the scores of every item (sp's d_zmax may hide spectra from them) */
 int hfx_rows_scores(hfx_ctx *ctx, int mode, void *scratch, float *d_scores, const uint64_t *d_off,
                     const uint32_t *begin, const uint32_t *num, const uint32_t *order,
                     const uint32_t *bstart, const hfx_rows *r, const uint8_t *planes,
-                    const float *qs, const hfx_spectra *sp, uint32_t CH, const uint32_t *zmax,
-                    void *stream, void **ev);
+                    const float *qs, const hfx_spectra *sp, uint32_t CH, void *stream, void **ev);
 
 /* spectrum order and block cut (hfx_batch.hip) */
 struct hfx_order_bufs {

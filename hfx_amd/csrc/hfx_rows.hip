@@ -84,7 +84,7 @@ __device__ __forceinline__ uint32_t rw_bf16(float f)
 template <int MODE>
 __global__ void __launch_bounds__(256)
     k_rw_split(uint8_t *planes, float *qs, uint32_t *lvl, uint32_t *wide, float2 *norms,
-               hfx_spectra sp)
+               float *scores, const uint64_t *off, hfx_spectra sp)
 {
     constexpr uint32_t NP = RW_PLANES(MODE);
     __shared__ float red[2][256 / HFX_WAVE];
@@ -92,6 +92,9 @@ __global__ void __launch_bounds__(256)
     const uint32_t s = blockIdx.x, tid = threadIdx.x;
     const uint32_t len = min(sp.d_len[s], min(sp.x_stride, (uint32_t)RW_MAXK));
     const float *x = sp.d_x + (size_t)s * sp.x_stride;
+    /* spectra whose fragment charge is not generated score 0 */
+    if (hfx_zeff(sp.d_zmax[s]) == 0)
+        for (uint64_t i = off[s] + tid; i < off[s + 1]; i += 256) scores[i] = 0.0f;
     /* thread t takes the four bins of words t + 256 u (bytes 4 w .. 4 w + 3) */
     constexpr uint32_t NW = RW_MAXK / 4, NU = (NW + 255) / 256;
     float v[NU][4];
@@ -488,30 +491,37 @@ __global__ void __launch_bounds__(RB_THREADS, RB_PER_CU) k_rw_build(RbArgs a)
 /* ------------------------------------------------------------------ */
 
 /* block b: the tiles of its windows' hull, fragment charge levels (bit z),
- * longest row in k-steps, work items (CT tiles each, per level) */
-template <uint32_t NS>
-__global__ void k_rw_blocks(uint32_t *tbeg, uint32_t *tend, uint32_t *binfo, uint32_t *items,
-                            const uint32_t *order, const uint32_t *bstart, const uint32_t *begin,
-                            const uint32_t *num, hfx_spectra sp, uint32_t B, uint32_t CT)
+ * longest row in k-steps, work items (CT tiles each, per level).  Sixteen lanes a
+ * block, a spectrum each (a thread a block read them one after the other: 18 us
+ * for 20,000 spectra, 4.7 now); the first also clears the items' counter. */
+__global__ void __launch_bounds__(256)
+    k_rw_blocks(uint32_t *tbeg, uint32_t *tend, uint32_t *binfo, uint32_t *items, uint32_t *counter,
+                const uint32_t *order, const uint32_t *bstart, const uint32_t *begin,
+                const uint32_t *num, hfx_spectra sp, uint32_t B, uint32_t CT)
 {
-    const uint32_t b = blockIdx.x * blockDim.x + threadIdx.x;
+    const uint32_t b = (blockIdx.x * 256 + threadIdx.x) / 16, g = threadIdx.x & 15u;
+    if (b == 0 && g == 0) *counter = 0;
     if (b >= B) return;
     uint32_t lo = 0xffffffffu, hi = 0, mask = 0, kmax = 0;
-    const uint32_t i0 = bstart[b], i1 = bstart[b + 1];
-    uint32_t sv[NS];
-#pragma unroll
-    for (uint32_t g = 0; g < NS; ++g) sv[g] = i0 + g < i1 ? order[i0 + g] : 0xffffffffu;
-#pragma unroll
-    for (uint32_t g = 0; g < NS; ++g) {
-        const uint32_t s = sv[g];
-        if (s == 0xffffffffu) continue;
+    const uint32_t i = bstart[b] + g;
+    if (i < bstart[b + 1]) {
+        const uint32_t s = order[i];
         const uint32_t z = hfx_zeff(sp.d_zmax[s]), n = num[s], bg = begin[s], ln = sp.d_len[s];
-        if (z == 0 || n == 0) continue;
-        lo = min(lo, bg);
-        hi = max(hi, bg + n);
-        mask |= 1u << z;
-        kmax = max(kmax, min(ln, min(sp.x_stride, (uint32_t)RW_MAXK)));
+        if (z && n) {
+            lo = bg;
+            hi = bg + n;
+            mask = 1u << z;
+            kmax = min(ln, min(sp.x_stride, (uint32_t)RW_MAXK));
+        }
     }
+#pragma unroll
+    for (uint32_t o = 8; o > 0; o >>= 1) {
+        lo = min(lo, (uint32_t)__shfl_xor((int)lo, o, 16));
+        hi = max(hi, (uint32_t)__shfl_xor((int)hi, o, 16));
+        mask |= (uint32_t)__shfl_xor((int)mask, o, 16);
+        kmax = max(kmax, (uint32_t)__shfl_xor((int)kmax, o, 16));
+    }
+    if (g != 0) return;
     const bool any = hi > lo;
     const uint32_t t0 = any ? lo / RW_ROWS : 0u, t1 = any ? (hi + RW_ROWS - 1) / RW_ROWS : 0u;
     if (!any) mask = 0;
@@ -520,8 +530,6 @@ __global__ void k_rw_blocks(uint32_t *tbeg, uint32_t *tend, uint32_t *binfo, uin
     binfo[b] = (kmax + 63u) / 64u | mask << 16;
     items[b] = ((t1 - t0 + CT - 1) / CT) * (uint32_t)__builtin_popcount(mask);
 }
-
-__global__ void k_rw_reset(uint32_t *counter) { *counter = 0; }
 
 __global__ void k_rw_fill(uint32_t *a, uint64_t n, uint32_t v)
 {
@@ -539,15 +547,6 @@ __global__ void k_rw_mark(uint32_t *flags, const uint32_t *tbeg, const uint32_t 
         if ((mask >> l) & 1u)
             for (uint32_t t = tbeg[b] + threadIdx.x; t < tend[b]; t += blockDim.x)
                 flags[(size_t)(l - 1) * ntiles + t] = 1u;
-}
-
-/* spectra whose fragment charge is not generated score 0 */
-__global__ void k_rw_zero_unscored(float *scores, const uint64_t *off, const uint32_t *zmax,
-                                   uint32_t S)
-{
-    const uint32_t s = blockIdx.x;
-    if (s >= S || hfx_zeff(zmax[s]) != 0) return;
-    for (uint64_t i = off[s] + threadIdx.x; i < off[s + 1]; i += blockDim.x) scores[i] = 0.0f;
 }
 
 /* ------------------------------------------------------------------ */
@@ -863,15 +862,15 @@ uint32_t hfx_rows_chunk(uint64_t rows, uint32_t cus)
 }
 
 int hfx_rows_split(int mode, const hfx_spectra *sp, uint8_t *planes, float *qs, uint32_t *lvl,
-                   uint32_t *wide, float2 *norms, void *stream)
+                   uint32_t *wide, float2 *norms, float *scores, const uint64_t *off, void *stream)
 {
     HFX_REQUIRE(sp->x_stride <= RW_MAXK, HFX_ERR_ARG, "rows: spectra of up to %d bins", RW_MAXK);
     if (sp->num_spec == 0) return HFX_OK;
     const dim3 g(sp->num_spec), t(256);
     hipStream_t st = hfx_stream(stream);
-    if (mode == RW_I8X3) hipLaunchKernelGGL(k_rw_split<RW_I8X3>, g, t, 0, st, planes, qs, lvl, wide, norms, *sp);
-    else if (mode == RW_I8X4) hipLaunchKernelGGL(k_rw_split<RW_I8X4>, g, t, 0, st, planes, qs, lvl, wide, norms, *sp);
-    else hipLaunchKernelGGL(k_rw_split<RW_BF16>, g, t, 0, st, planes, qs, lvl, wide, norms, *sp);
+    if (mode == RW_I8X3) hipLaunchKernelGGL(k_rw_split<RW_I8X3>, g, t, 0, st, planes, qs, lvl, wide, norms, scores, off, *sp);
+    else if (mode == RW_I8X4) hipLaunchKernelGGL(k_rw_split<RW_I8X4>, g, t, 0, st, planes, qs, lvl, wide, norms, scores, off, *sp);
+    else hipLaunchKernelGGL(k_rw_split<RW_BF16>, g, t, 0, st, planes, qs, lvl, wide, norms, scores, off, *sp);
     HFX_CHECK_LAUNCH();
     return HFX_OK;
 }
@@ -918,15 +917,11 @@ int hfx_rows_blocks(hfx_ctx *ctx, int mode, void *scratch, const uint32_t *order
     rw_items(scratch, B, &tbeg, &tend, &binfo, &items, &off, &counter);
     hipStream_t st = hfx_stream(stream);
     const uint32_t CT = std::max(CH / RW_ROWS, 1u);
-    if (RW_NS(mode) == 16)
-        hipLaunchKernelGGL(k_rw_blocks<16>, dim3((B + 255) / 256), dim3(256), 0, st, tbeg, tend,
-                           binfo, items, order, bstart, begin, num, *sp, B, CT);
-    else
-        hipLaunchKernelGGL(k_rw_blocks<8>, dim3((B + 255) / 256), dim3(256), 0, st, tbeg, tend,
-                           binfo, items, order, bstart, begin, num, *sp, B, CT);
+    (void)mode;
+    hipLaunchKernelGGL(k_rw_blocks, dim3((B + 15) / 16), dim3(256), 0, st, tbeg, tend, binfo, items,
+                       counter, order, bstart, begin, num, *sp, B, CT);
     int rc = hfx_scan_offsets(ctx, off, items, B, stream);
     if (rc) return rc;
-    hipLaunchKernelGGL(k_rw_reset, dim3(1), dim3(1), 0, st, counter);
     HFX_CHECK_LAUNCH();
     return HFX_OK;
 }
@@ -948,8 +943,7 @@ int hfx_rows_mark(void *scratch, uint32_t S, uint32_t *flags, uint32_t ntiles, v
 int hfx_rows_scores(hfx_ctx *ctx, int mode, void *scratch, float *d_scores, const uint64_t *d_off,
                     const uint32_t *begin, const uint32_t *num, const uint32_t *order,
                     const uint32_t *bstart, const hfx_rows *r, const uint8_t *planes,
-                    const float *qs, const hfx_spectra *sp, uint32_t CH, const uint32_t *zmax,
-                    void *stream, void **ev)
+                    const float *qs, const hfx_spectra *sp, uint32_t CH, void *stream, void **ev)
 {
     const uint32_t S = sp->num_spec;
     uint32_t *tbeg, *tend, *binfo, *items, *counter;
@@ -991,7 +985,6 @@ int hfx_rows_scores(hfx_ctx *ctx, int mode, void *scratch, float *d_scores, cons
     else if (mode == RW_I8X4) hipLaunchKernelGGL(k_rw_mm<RW_I8X4>, g, t, lds, st, a);
     else hipLaunchKernelGGL(k_rw_mm<RW_BF16>, g, t, lds, st, a);
     if (ev) HFX_CHECK_HIP(hipEventRecord((hipEvent_t)ev[1], st));
-    hipLaunchKernelGGL(k_rw_zero_unscored, dim3(S), dim3(256), 0, st, d_scores, d_off, zmax, S);
     HFX_CHECK_LAUNCH();
     return HFX_OK;
 }

@@ -456,7 +456,7 @@ static int xcorr_rows(hfx_ctx *ctx, float *d_scores, const uint64_t *d_off,
     const uint64_t est = max(total / 12, min(total, 2ull * db->num_pep));
     const uint32_t CH = hfx_rows_chunk(est, (uint32_t)hfx_ctx_num_cus(ctx));
     int rc;
-    if ((rc = hfx_rows_split(RW_I8X4, sp, planes, qs, lvl, wide, nullptr, stream)) ||
+    if ((rc = hfx_rows_split(RW_I8X4, sp, planes, qs, lvl, wide, nullptr, d_scores, d_off, stream)) ||
         (rc = hfx_order_spectra(ctx, order, &ob, d_begin, sp->d_zmax, sp->d_mass, S, stream)) ||
         (rc = hfx_cut_blocks(ctx, 16, &cb, order, d_begin, d_num, sp->d_zmax, S, stream)) ||
         (rc = hfx_rows_blocks(ctx, RW_I8X4, items, order, cb.bstart, d_begin, d_num, &sq, CH,
@@ -465,7 +465,7 @@ static int xcorr_rows(hfx_ctx *ctx, float *d_scores, const uint64_t *d_off,
         (rc = hfx_scan_offsets(ctx, (uint64_t *)r.slots, flags, (uint32_t)nf, stream)) ||
         (rc = hfx_rows_build((uint32_t)hfx_ctx_num_cus(ctx), db, &r, flags, stream)) ||
         (rc = hfx_rows_scores(ctx, RW_I8X4, items, d_scores, d_off, d_begin, d_num, order,
-                              cb.bstart, &r, planes, qs, &sq, CH, sp->d_zmax, stream, nullptr)) ||
+                              cb.bstart, &r, planes, qs, &sq, CH, stream, nullptr)) ||
         (rc = hfx_xcorr_wide(ctx, d_scores, d_off, d_begin, d_num, db, sp, wide, stream)))
         return rc;
     *taken = 1;
