@@ -61,6 +61,20 @@ def test_every_way_gives_the_same_ranking(tenv, orc, eps, N, margin):
     assert flagged[-1] > 0 or eps < 10
 
 
+@pytest.mark.parametrize("N", [15, 16, 17])
+def test_exact_windows_by_rounds_and_by_radix(tenv, orc, N):
+    """Windows scored exactly as a whole: up to sixteen places by rounds of the best, more by radix.
+    The two meet here, and the top N is the oracle's on both sides."""
+    pl = tenv["pl"]
+    s = pl.PlainSearch(tenv["ctx"], tenv["db"], tenv["sp"], eps=250.0, topn=N)
+    s.window()
+    s.score()
+    s.t_cnt.zero()
+    s.select_rel(0.5)
+    check(orc, s, tenv["ref"][250.0], N)
+    assert len(s.flagged()) > 0
+
+
 @pytest.mark.parametrize("N", [5, 40])
 def test_scores_with_infinities_keep_their_order(tenv, orc, N):
     """The selection follows the scores' total order: with -inf in most places the finite ones
