@@ -117,6 +117,7 @@ __device__ __forceinline__ uint32_t so_before(const uint32_t *sk, int ja, int jb
     uint32_t rk = 0;
     const uint4 *s4 = (const uint4 *)sk;
     const int a1 = min(jb, max(ja, i0)), a2 = min(jb, max(ja, i0 + HFX_WAVE));
+    #pragma unroll 4
     for (int j = ja / 4; j < a1 / 4; ++j) {
         const uint4 o = s4[j];
         rk += (o.x <= k ? 1u : 0u) + (o.y <= k ? 1u : 0u) + (o.z <= k ? 1u : 0u) +
@@ -129,6 +130,7 @@ __device__ __forceinline__ uint32_t so_before(const uint32_t *sk, int ja, int jb
         rk += (o.z < k || (o.z == k && 4 * j + 2 < i)) ? 1u : 0u;
         rk += (o.w < k || (o.w == k && 4 * j + 3 < i)) ? 1u : 0u;
     }
+    #pragma unroll 4
     for (int j = a2 / 4; j < jb / 4; ++j) {
         const uint4 o = s4[j];
         rk += (o.x < k ? 1u : 0u) + (o.y < k ? 1u : 0u) + (o.z < k ? 1u : 0u) +
@@ -139,11 +141,14 @@ __device__ __forceinline__ uint32_t so_before(const uint32_t *sk, int ja, int jb
 
 /* Up to SO_ONE keys: one launch of one workgroup, each key's place counted
  * against all others (key, then position: stable), four keys an LDS read, the
- * other keys shared out among the waves that a short list leaves over: 7 us
- * for a few hundred keys, where the radix passes' 28 launches took about 100. */
-#define SO_ONE 1024u
-__global__ void __launch_bounds__(SO_ONE) k_sort_one(float *keys, uint32_t *vals, uint32_t n,
-                                                     uint32_t iota, uint32_t init, uint32_t desc)
+ * other keys shared out among the waves that a short list leaves over.  A call
+ * with its synchronisation: 14.8 us for 256 keys, 18.4 for 512, 31.9 for 1024;
+ * by k_sort_rank 16.2, 17.0, 18.2; by radix passes 67. */
+#define SO_ONE 384u
+#define SO_THREADS 1024u
+__global__ void __launch_bounds__(SO_THREADS) k_sort_one(float *keys, uint32_t *vals, uint32_t n,
+                                                         uint32_t iota, uint32_t init,
+                                                         uint32_t desc)
 {
     __shared__ __align__(16) uint32_t sk[SO_ONE];
     __shared__ uint32_t rank[SO_ONE];
@@ -154,10 +159,12 @@ __global__ void __launch_bounds__(SO_ONE) k_sort_one(float *keys, uint32_t *vals
         k = so_key(keys[t], desc);
         v = iota ? init + t : vals[t];
     }
-    sk[t] = k; /* past the end: no key before another */
-    rank[t] = 0;
+    if (t < SO_ONE) {
+        sk[t] = k; /* past the end: no key before another */
+        rank[t] = 0;
+    }
     __syncthreads();
-    const uint32_t parts = SO_ONE / n64, part = t / n64, i = t % n64;
+    const uint32_t parts = SO_THREADS / n64, part = t / n64, i = t % n64;
     if (part < parts) {
         const uint32_t step = ((n64 + parts - 1) / parts + 3u) & ~3u;
         const uint32_t ja = min(part * step, n64), jb = min(ja + step, n64);
@@ -173,33 +180,41 @@ __global__ void __launch_bounds__(SO_ONE) k_sort_one(float *keys, uint32_t *vals
     }
 }
 
-/* Up to SO_RANK keys: the same count, SO_RT keys a workgroup against all of
- * them, into scratch, which a second launch copies back.  The count grows with
- * n^2 and meets the radix passes' twelve launches at about twice this. */
-#define SO_RANK 8192u
-#define SO_RT 256
-__global__ void __launch_bounds__(SO_RT) k_sort_rank(const float *keys, const uint32_t *vals,
-                                                     float *okeys, uint32_t *ovals, uint32_t n,
-                                                     uint32_t iota, uint32_t init, uint32_t desc)
+/* Up to SO_RANK keys: the same count, a workgroup for 64 keys and its sixteen
+ * waves a share of all others each, into scratch, which a second launch copies
+ * back.  The count grows with n^2: 22.9 us for 4,096 keys, 28.9 for 8,192, 40.7
+ * for 16,384, 71 for 24,576; radix passes 67 throughout.  (256 keys a workgroup
+ * of four waves, each against all others: 89 for 4,096, 163 for 8,192.) */
+#define SO_RANK 16384u
+#define SO_CHUNK 8192u
+__global__ void __launch_bounds__(SO_THREADS)
+    k_sort_rank(const float *keys, const uint32_t *vals, float *okeys, uint32_t *ovals, uint32_t n,
+                uint32_t iota, uint32_t init, uint32_t desc)
 {
-    __shared__ __align__(16) uint32_t sk[2048];
-    const uint32_t i = blockIdx.x * SO_RT + threadIdx.x;
+    __shared__ __align__(16) uint32_t sk[SO_CHUNK];
+    __shared__ uint32_t rank[HFX_WAVE];
+    const uint32_t wave = threadIdx.x / HFX_WAVE, i0 = blockIdx.x * HFX_WAVE;
+    const uint32_t i = i0 + hfx_lane();
     const uint32_t k = i < n ? so_key(keys[i], desc) : 0xffffffffu;
+    if (threadIdx.x < HFX_WAVE) rank[threadIdx.x] = 0;
     uint32_t rk = 0;
-    for (uint32_t b = 0; b < n; b += 2048) {
+    for (uint32_t b = 0; b < n; b += SO_CHUNK) {
+        const uint32_t m = (min(n - b, SO_CHUNK) + HFX_WAVE - 1) / HFX_WAVE * HFX_WAVE;
         __syncthreads();
-#pragma unroll
-        for (uint32_t u = 0; u < 2048 / SO_RT; ++u) {
-            const uint32_t j = b + u * SO_RT + threadIdx.x;
-            sk[u * SO_RT + threadIdx.x] = j < n ? so_key(keys[j], desc) : 0xffffffffu;
-        }
+        for (uint32_t j = threadIdx.x; j < m; j += SO_THREADS)
+            sk[j] = b + j < n ? so_key(keys[b + j], desc) : 0xffffffffu;
         __syncthreads();
-        rk += so_before(sk, 0, (int)((min(n - b, 2048u) + 3u) & ~3u),
-                        (int)(i & ~(uint32_t)(HFX_WAVE - 1)) - (int)b, (int)i - (int)b, k);
+        constexpr uint32_t W = SO_THREADS / HFX_WAVE;
+        const uint32_t step = ((m + W - 1) / W + 3u) & ~3u;
+        const uint32_t ja = min(wave * step, m), jb = min(ja + step, m);
+        rk += so_before(sk, (int)ja, (int)jb, (int)i0 - (int)b, (int)i - (int)b, k);
     }
-    if (i < n) {
-        okeys[rk] = so_float(k, desc);
-        ovals[rk] = iota ? init + i : vals[i];
+    if (rk) atomicAdd(&rank[hfx_lane()], rk);
+    __syncthreads();
+    if (wave == 0 && i < n) {
+        const uint32_t r = rank[hfx_lane()];
+        okeys[r] = so_float(k, desc);
+        ovals[r] = iota ? init + i : vals[i];
     }
 }
 __global__ void k_sort_back(const float *k, const uint32_t *v, float *keys, uint32_t *vals,
@@ -402,7 +417,7 @@ static int radix_sort_f32(hfx_ctx *ctx, float *d_keys, uint32_t *d_vals, uint32_
 {
     if (n == 0) return HFX_OK;
     if (n <= SO_ONE) {
-        hipLaunchKernelGGL(k_sort_one, dim3(1), dim3(SO_ONE), 0, st, d_keys, d_vals, n,
+        hipLaunchKernelGGL(k_sort_one, dim3(1), dim3(SO_THREADS), 0, st, d_keys, d_vals, n,
                            (uint32_t)iota, init, desc);
         HFX_CHECK_LAUNCH();
         return HFX_OK;
@@ -415,8 +430,8 @@ static int radix_sort_f32(hfx_ctx *ctx, float *d_keys, uint32_t *d_vals, uint32_
         return rc;
     uint32_t *ka = (uint32_t *)p, *va = ka + n, *kb = va + n, *vb = kb + n, *hist = vb + n;
     if (n <= SO_RANK) {
-        hipLaunchKernelGGL(k_sort_rank, dim3((n + SO_RT - 1) / SO_RT), dim3(SO_RT), 0, st, d_keys,
-                           d_vals, (float *)ka, va, n, (uint32_t)iota, init, desc);
+        hipLaunchKernelGGL(k_sort_rank, dim3((n + HFX_WAVE - 1) / HFX_WAVE), dim3(SO_THREADS), 0, st,
+                           d_keys, d_vals, (float *)ka, va, n, (uint32_t)iota, init, desc);
         hipLaunchKernelGGL(k_sort_back, dim3((n + 255) / 256), dim3(256), 0, st, (float *)ka, va,
                            d_keys, d_vals, n);
         HFX_CHECK_LAUNCH();

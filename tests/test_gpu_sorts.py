@@ -5,7 +5,8 @@ import pytest
 
 pytestmark = pytest.mark.gpu
 
-SIZES = [1, 2, 63, 64, 65, 1023, 1024, 1025, 2049, 8191, 8192, 8193, 12289, 100003]
+SIZES = [1, 2, 63, 64, 65, 383, 384, 385, 1023, 1024, 1025, 2049, 8191, 8192, 8193, 12289, 16384,
+         16385, 100003]
 
 
 def order_key(f):
