@@ -58,9 +58,15 @@
 #define TN_HBINS (1u << TN_HBITS)
 
 /* candidates of a spectrum that its own wave re-scores; the rest of a longer
- * list goes out in tasks of as many */
+ * list goes out in tasks of as many, first to the waves without a spectrum (4
+ * workgroups a CU at least).  Up to TN_FEW spectra half as many.  With eight and
+ * with sixteen, whole top-N: 250 spectra, N = 16: 58 and 79 us; 2,000, N = 16:
+ * 234 and 250, N = 64: 359 and 397, N = 5: 168 and 167; a plain search of 10,000,
+ * N = 10: 2170 and 2088; a BF16 batch of 6,000: 1150 and 1105. */
 #define TN_TASK 16
-#define TN_SPILL ((TN_MAXC - TN_TASK + TN_TASK - 1) / TN_TASK)
+#define TN_TASK_FEW 8
+#define TN_FEW 4096
+#define TN_SPILL ((TN_MAXC - 1) / TN_TASK_FEW)
 
 __device__ __forceinline__ bool before_fx(int64_t fa, uint32_t pa, int64_t fb, uint32_t pb)
 {
@@ -173,6 +179,7 @@ struct TnLists {
     uint32_t *nspill;
     double *tau;     /* [S] the bound, then the exact route's threshold */
     uint32_t *band;  /* [S] band size of flagged spectra */
+    uint32_t task;   /* candidates a task */
 };
 
 template <class Cands>
@@ -518,7 +525,7 @@ __global__ void __launch_bounds__(TN_THREADS)
      * (fmaxf skips a NaN, the sum keeps it) */
     const uint32_t big = xmax < 300.0f && xa == xa ? 0u : TN_BIG;
     for (uint32_t i = tid; i < M; i += TN_THREADS) o.cand[(size_t)s * TN_MAXC + i] = cp[i];
-    const uint32_t ntask = M > TN_TASK ? (M - 1u) / TN_TASK : 0u;
+    const uint32_t ntask = M > o.task ? (M - 1u) / o.task : 0u;
     if (tid == 0) {
         o.mcnt[s] = M | big;
         flag[s] = fl;
@@ -527,7 +534,7 @@ __global__ void __launch_bounds__(TN_THREADS)
     }
     if (ntask) {
         __syncthreads();
-        if (tid < ntask) o.spill[sh_task + tid] = make_uint2(s, (tid + 1u) * TN_TASK);
+        if (tid < ntask) o.spill[sh_task + tid] = make_uint2(s, (tid + 1u) * o.task);
     }
 }
 
@@ -693,7 +700,7 @@ __device__ __forceinline__ void fx_scores(const FxWave &f, uint32_t mstr, const 
     }
 }
 
-/* exact scores of the listed candidates: wave w takes the first TN_TASK of
+/* exact scores of the listed candidates: wave w takes the first o.task of
  * spectrum w, then all waves share the spilled tasks.  fx: [base(s) + i] for
  * candidate i of s's list. */
 template <class Cands>
@@ -709,7 +716,7 @@ __global__ void __launch_bounds__(TN_THREADS)
     __syncthreads();
     auto task = [&](uint32_t s, uint32_t k0) {
         const uint32_t mc = __builtin_amdgcn_readfirstlane(o.mcnt[s]), M = mc & ~TN_BIG;
-        const uint32_t rn = M > k0 ? min(M - k0, (uint32_t)TN_TASK) : 0u;
+        const uint32_t rn = M > k0 ? min(M - k0, o.task) : 0u;
         if (rn == 0) return;
         typename Cands::Prep pr{};
         if (lane < rn) pr = c.prep(s, o.cand[(size_t)s * TN_MAXC + k0 + lane]);
@@ -723,8 +730,9 @@ __global__ void __launch_bounds__(TN_THREADS)
     };
     const uint32_t w = __builtin_amdgcn_readfirstlane(blockIdx.x * TN_WAVES + wave);
     if (w < S) task(w, 0);
-    const uint32_t ns = *o.nspill;
-    for (uint32_t i = w; i < ns; i += gridDim.x * TN_WAVES) {
+    /* the waves without a spectrum first */
+    const uint32_t ns = *o.nspill, W = gridDim.x * TN_WAVES;
+    for (uint32_t i = w < S ? w + (W - S) : w - S; i < ns; i += W) {
         const uint2 t = o.spill[i];
         task(__builtin_amdgcn_readfirstlane(t.x), __builtin_amdgcn_readfirstlane(t.y));
     }
@@ -1263,6 +1271,7 @@ static TxScratch tx_carve(void *p, uint32_t S, uint64_t total)
     x.l.band = x.list + S;
     x.l.mcnt = x.l.band + S;
     x.l.cand = x.l.mcnt + S;
+    x.l.task = S <= TN_FEW ? TN_TASK_FEW : TN_TASK;
     return x;
 }
 static int tx_scratch(hfx_ctx *ctx, void *given, uint32_t S, uint64_t total, void **out)
@@ -1321,8 +1330,8 @@ static int launch_topn(hfx_ctx *ctx, uint32_t *d_top_pos, double *d_top_exact, f
     hipLaunchKernelGGL(k_tx_reset, dim3(1), dim3(1), 0, st, x.counter);
     hipLaunchKernelGGL(k_topn_select<Cands>, dim3(S), dim3(TN_THREADS), 0, st, x.l, d_flag, N,
                        margin, d_scores, c, *sp, rel0, rel1, relq, norms);
-    /* at least a workgroup a CU: the spilled tasks spread over all of them */
-    hipLaunchKernelGGL(k_topn_exact<Cands>, dim3(max(gw, (uint32_t)hfx_ctx_num_cus(ctx))),
+    /* at least four workgroups a CU: the spilled tasks spread over them */
+    hipLaunchKernelGGL(k_topn_exact<Cands>, dim3(max(gw, 4u * (uint32_t)hfx_ctx_num_cus(ctx))),
                        dim3(TN_THREADS), fx_lds_bytes(sp->x_stride), st, x.fxbuf, x.l, c, *sp,
                        xp_map_words(sp->x_stride));
     hipLaunchKernelGGL(k_topn_rank<Cands>, dim3(gw), dim3(TN_THREADS), 0, st, d_top_pos,

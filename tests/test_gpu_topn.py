@@ -22,7 +22,7 @@ def tenv(orc):
     ref = {eps: reference(orc, hdb, x, lens, zmax, mass, 64, eps)[0] for eps in (3.0, 250.0)}
     assert ref[3.0]["num"].min() == 0 and 0 < np.median(ref[3.0]["num"]) < 6144
     assert ref[250.0]["num"].max() > 6144
-    return dict(pl=pl, ctx=ctx, db=db, sp=sp, ref=ref)
+    return dict(pl=pl, ctx=ctx, db=db, sp=sp, ref=ref, rows=(x, lens, zmax, mass))
 
 
 def check(orc, s, ref, N):
@@ -73,6 +73,26 @@ def test_exact_windows_by_rounds_and_by_radix(tenv, orc, N):
     s.select_rel(0.5)
     check(orc, s, tenv["ref"][250.0], N)
     assert len(s.flagged()) > 0
+
+
+@pytest.mark.parametrize("S", [4096, 4097])
+def test_lists_shared_out_whole_and_in_halves(tenv, S):
+    """Many spectra re-score longer runs a wave: each copy of a spectrum has the ranking of the
+    first."""
+    pl = tenv["pl"]
+    which = np.arange(S) % 48
+    sp = Spectra(pl, *(a[which] for a in tenv["rows"]))
+    s = pl.PlainSearch(tenv["ctx"], tenv["db"], sp, eps=3.0, topn=40)
+    s.window()
+    s.score()
+    s.select_rel(1e-3)
+    assert len(s.short()) == 0
+    ref = tenv["ref"][3.0]
+    cnt = pl.host(s.t_cnt, np.uint32, S)
+    pos = pl.host(s.t_pos, np.uint32, S * 40).reshape(S, 40)
+    assert (cnt == np.minimum(ref["num"], 40)[which]).all()
+    for k in range(S):
+        assert pos[k, :cnt[k]].tolist() == ref["top_pos"][which[k], :cnt[k]].tolist(), k
 
 
 @pytest.mark.parametrize("N", [5, 40])
