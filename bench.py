@@ -10,21 +10,24 @@ A step is one pass of the scoring stage over the whole batch with the
 database and the preprocessed spectra resident in HBM: precursor windows ->
 theoretical peaks -> XCorr of every (spectrum, candidate) pair -> per-spectrum
 top-N with exact re-score.  Three forms are timed:
-  plain          hfx_window + hfx_xcorr_sparse + hfx_topn (the drop-in, one
-                 theoretical spectrum per (spectrum, candidate) pair, FP32);
-  batched fp32   hfx_batch_* in its FP32 sparse form (persistent
-                 work-stealing multi-spectrum XCorr over the per-database
-                 peptide ion lists);
-  batched bf16x2 hfx_batch_* in its dense form (blocks of up to eight spectra
-                 contracted with their candidates' theoretical rows on the
-                 MFMA units, BF16 weights x hi+lo BF16 spectra, FP32
-                 accumulation) + top-N with the exact re-score.
+  plain          hfx_window + hfx_xcorr_sparse + hfx_topn (the drop-in: a call
+                 of this size writes the theoretical rows its windows need and
+                 contracts them with blocks of sixteen spectra in 32-bit fixed
+                 point, rounded once to FP32; every step writes them anew);
+  batched fp32   hfx_batch_* in its FP32 form (the same contraction over the
+                 rows the per-database peptide index keeps);
+  batched bf16x2 hfx_batch_* in its BF16 form (blocks of up to eight spectra,
+                 BF16 weights x hi+lo BF16 spectra, FP32 accumulation);
+  batched i8x3   hfx_batch_* in its integer form (blocks of up to sixteen
+                 spectra, int8 weights x three base-256 digits);
+each with its top-N and exact re-score.
 Each batched step runs every per-batch step on the device -- windows,
-spectrum order, block cut and hi/lo rows (dense) or tiles (sparse), scoring,
+spectrum order, block cut, the spectra's digits or hi/lo planes, scoring,
 top-N -- captured once in a hipGraph and replayed.  The per-database peptide
 index (b ladders, ion lists) is built once before the loop and its build
-time is reported beside the step (`db_setup_ms`), as is the one-off plan
-(allocation) time.
+time is reported beside the step (`db_setup_ms`); its theoretical rows are
+added by the first batch that runs on it, before its timed steps; the one-off
+plan (allocation) time is reported too.
 value = scored pairs per second of the batched BF16-split form (whole job,
 one GPU); every form's top-N must equal the plain form's.
 
@@ -375,8 +378,9 @@ def dense_flops(env, res, k_per_pair=4) -> tuple[float, float]:
     """(executed, useful) MFMA operations of one dense pass by the per-pair
     figures of the precision form: executed = k_per_pair K per scored pair
     (BF16 form: 4 K, hi and lo columns over the padded row, K = 2176 bins;
-    integer form: 6 K, three digit contractions), useful = 2 len_s per scored
-    pair (one product per bin of the spectrum)."""
+    integer form: 6 K, three digit contractions; the groups of 256 bins that no
+    peak of a tile reaches are skipped, not subtracted here), useful = 2 len_s
+    per scored pair (one product per bin of the spectrum)."""
     dsp = env["dsp"]
     z = dsp.zmax.astype(np.int64)
     scored = (z <= 4) & (z > 0)
@@ -467,7 +471,7 @@ def main():
         ab = algorithmic_bytes(env, plain_res)
         paths["plain_fp32_sparse"] = dict(
             value=sc * args.steps / el, ms_per_step=el * 1e3 / args.steps, scores_per_step=sc,
-            kernel="k_xcorr_pack", kernel_ms=kern_ms,
+            kernel="k_rw_build + k_rw_mm", kernel_ms=kern_ms,
             kernel_gbs=ab / (kern_ms * 1e-3) / 1e9, algorithmic_bytes=ab,
             flagged_spectra_per_step=flagged)
         log(f"plain: {paths['plain_fp32_sparse']['value']:.3e} scores/s, kernel {kern_ms:.2f} ms")
@@ -497,7 +501,7 @@ def main():
         ab = algorithmic_bytes(env, batch_res)
         paths["batched_fp32_sparse"] = dict(
             value=sc * args.steps / el, ms_per_step=el * 1e3 / args.steps, scores_per_step=sc,
-            kernel="k_batch", kernel_ms=phases["kernel"], phases_ms=phases,
+            kernel="k_rw_mm", kernel_ms=phases["kernel"], phases_ms=phases,
             kernel_gbs=ab / (phases["kernel"] * 1e-3) / 1e9,
             config=dict(G=cfg[0], C=cfg[1], threads=cfg[2]), info=info, plan_ms=plan_ms,
             graph="every per-batch step captured once, replayed per step",
@@ -511,7 +515,7 @@ def main():
         ex, useful = dense_flops(env, dense_res)
         paths["batched_bf16x2_dense"] = dict(
             value=sc * args.steps / el, ms_per_step=el * 1e3 / args.steps, scores_per_step=sc,
-            kernel="k_dense", kernel_ms=phases["kernel"], phases_ms=phases,
+            kernel="k_rw_mm", kernel_ms=phases["kernel"], phases_ms=phases,
             mfma_flops_executed=ex, mfma_flops_useful=useful,
             config=dict(chunk=cfg[1], threads=cfg[2], spectra_per_block_max=8,
                         blocks=info["dense_blocks"]), plan_ms=plan_ms,
@@ -526,7 +530,7 @@ def main():
         ex, useful = dense_flops(env, i8_res, k_per_pair=I8_K)
         paths["batched_i8x3_dense"] = dict(
             value=sc * args.steps / el, ms_per_step=el * 1e3 / args.steps, scores_per_step=sc,
-            kernel="k_dense8", kernel_ms=phases["kernel"], phases_ms=phases,
+            kernel="k_rw_mm", kernel_ms=phases["kernel"], phases_ms=phases,
             mfma_ops_executed=ex, mfma_ops_useful=useful,
             config=dict(chunk=cfg[1], threads=cfg[2], spectra_per_block_max=16,
                         blocks=info["dense_blocks"]), plan_ms=plan_ms,
@@ -551,28 +555,30 @@ def main():
     p = paths[main_key]
     if main_key == "batched_i8x3_dense":
         achieved = p["mfma_ops_executed"] / (p["kernel_ms"] * 1e-3) / 1e12
-        tr = measured_traffic("k_dense8", args.workload)
+        tr = measured_traffic("k_rw_mm_i8x3", args.workload)
         roofline = {"kernel": p["kernel"], "bound": "mfma", "achieved": achieved,
                     "peak": INT8_PEAK_TOPS, "unit": "TOP/s",
                     "frac": achieved / INT8_PEAK_TOPS,
                     "traffic": tr["bytes"] if tr else None,
                     "kernel_ms": p["kernel_ms"], "ops_per_launch": p["mfma_ops_executed"],
                     "ops_rule": f"{I8_K} K per scored pair, K = {DENSE_K} padded bins (three "
-                                "int8 digit contractions, 2 ops a multiply-add)",
+                                "int8 digit contractions, 2 ops a multiply-add); groups of 256 bins "
+                                "past a tile's last peak are skipped, not subtracted",
                     "ops_useful": p["mfma_ops_useful"]}
         if tr:
             roofline["traffic_source"] = tr["source"]
         dtype = "i8x3"
     elif main_key == "batched_bf16x2_dense":
         achieved = p["mfma_flops_executed"] / (p["kernel_ms"] * 1e-3) / 1e12
-        tr = measured_traffic("k_dense", args.workload)
+        tr = measured_traffic("k_rw_mm_bf16x2", args.workload)
         roofline = {"kernel": p["kernel"], "bound": "mfma", "achieved": achieved,
                     "peak": BF16_PEAK_TFLOPS, "unit": "TFLOP/s",
                     "frac": achieved / BF16_PEAK_TFLOPS,
                     "traffic": tr["bytes"] if tr else None,
                     "kernel_ms": p["kernel_ms"], "flops_per_launch": p["mfma_flops_executed"],
                     "flops_rule": f"4 K per scored pair, K = {DENSE_K} padded bins (hi and lo "
-                                  "BF16 columns)",
+                                  "BF16 columns); groups of 256 bins past a tile's last peak "
+                                  "are skipped, not subtracted",
                     "flops_useful": p["mfma_flops_useful"]}
         if tr:
             roofline["traffic_source"] = tr["source"]

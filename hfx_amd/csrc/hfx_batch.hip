@@ -11,7 +11,8 @@
  *      peptide any window touches, for fragment charge levels 1..L (level l =
  *      charges 1..l, max per bin): sorted uint16 entries bin | code << 14
  *      (k_ix_build, one wave per peptide, from the same ladder/bin code as the
- *      plain path);
+ *      plain path), and the rows of 2-bit codes of the same peaks
+ *      (hfx_rows.hip), which every form scores with where memory holds them;
  *   2. sorts the spectra by precursor mass and groups G consecutive spectra
  *      into blocks; a tile is (block, C consecutive candidates of the block's
  *      union window); a persistent kernel pulls tiles from an atomic counter
@@ -19,7 +20,8 @@
  *      the block's G spectra in LDS, streams each candidate's entries once
  *      (coalesced) and gathers every spectrum of the block that holds the
  *      candidate in its window, reducing the G partial sums with one
- *      reduce-scatter butterfly;
+ *      reduce-scatter butterfly (with rows: blocks of up to sixteen ordered
+ *      spectra contracted with the rows of their windows' hull);
  *   3. selects the top N with the exact re-score of hfx_topn (flagged spectra
  *      completed in the same launch sequence, no host round trip).
  * Scores land in the same layout as hfx_xcorr_sparse, so every result is

@@ -31,9 +31,9 @@
  * time went to exact scores with a quarter of the lanes busy, and a spectrum
  * with 200 tied candidates held up a small batch by itself.
  * Now, select + exact + rank: 10,000 spectra, 1120 candidates each, top 10:
- * 127 + 136 + 15 us, against 445 us; 20,000 spectra, top 5: 160 + 148 + 15 us,
+ * 127 + 126 + 15 us, against 445 us; 20,000 spectra, top 5: 157 + 137 + 15 us,
  * against 430 (179 where the selection reads the spectra for their norms); 250
- * spectra: 14 + 39 + 8 us, against 171.  The selection is a chain of short steps,
+ * spectra: 13 + 22 + 7 us, against 171.  The selection is a chain of short steps,
  * half of its waves waiting; the exact scores are bound by their FP64 terms and
  * the maps' LDS atomics.
  */
@@ -47,7 +47,10 @@
 #define TN_MAXC (TN_MAXT + TN_EXT)
 
 /* T at most this: a threshold from the lanes' largest scores, then one
- * collection; above, a radix select */
+ * collection; above, a radix select.  Whole top-N by the first and by radix: 250
+ * spectra, N = 5: 46 and 56 us, 32: 124 and 146, 48: 152 and 162, 64: 169 and
+ * 165; 2,000 spectra, 5: 168 and 184, 32: 325 and 333, 48: 381 and 378, 64: 433
+ * and 423. */
 #define TN_LT 32
 /* scores a thread keeps in registers between its two looks at them: windows of
  * up to 6144 candidates are read once */

@@ -284,14 +284,20 @@ int hfx_scan_offsets(hfx_ctx *ctx, uint64_t *d_off, const uint32_t *d_count, uin
  * for spectrum s and its i-th window candidate (residual-sorted position
  * d_begin[s] + i), d_scores[d_off[s] + i] = sum over the candidate's
  * theoretical bins b < len_s of maxweight(b) * x_s[b], FP32.  `total` is
- * sum_s d_num[s] (findSpecCandsByMass's return value). */
+ * sum_s d_num[s] (findSpecCandsByMass's return value).
+ * Calls large enough for it write each theoretical row once and contract the
+ * rows with the spectra in 32-bit fixed point, rounded once to FP32: nearer the
+ * exact score than the FP32 sums, within the same bound.  Their buffers (the rows,
+ * up to 2.2 GB for 2.7 M peptides; 8.7 KB a spectrum) are kept by the context;
+ * where device memory is short, or the stream is being captured before they
+ * exist, the call sums in FP32 without them. */
 int hfx_xcorr_sparse(hfx_ctx *ctx, float *d_scores, const uint64_t *d_off,
                      const uint32_t *d_begin, const uint32_t *d_num, uint64_t total,
                      const hfx_db *db, const hfx_spectra *sp, void *stream);
 
 /* hfx_xcorr_sparse for callers that cannot allocate device memory (code
  * under hipGraph capture, tight serving loops): no counterpart in the
- * reference.  Same arguments and results as hfx_xcorr_sparse, without the
+ * reference.  Same arguments and bounds as hfx_xcorr_sparse, without the
  * context: the tile table (a few bytes per spectrum) lives in one static
  * device array of the library, so at most HFX_NOALLOC_MAX_SPECTRA spectra per
  * call (larger calls return HFX_ERR_ARG), and no hipMalloc or other
@@ -463,7 +469,8 @@ int hfx_sp_ions(hfx_ctx *ctx, uint32_t *d_nb, uint32_t *d_ny, uint32_t *d_total,
                 const hfx_spectra *sp, int mono, void *stream);
 /* hfx_sp_peaks + hfx_sp_ions over the top N of an unmodified search
  * (hfx_topn layout: [S][N], entries beyond d_top_cnt[s] get zeros), flags in
- * the context's scratch (allocated on first use). */
+ * the context's scratch (allocated on first use; none for rows of up to 3072
+ * bins, whose flags and matches are one kernel). */
 int hfx_sp_ions_topn(hfx_ctx *ctx, uint32_t *d_nb, uint32_t *d_ny, uint32_t *d_total,
                      const uint32_t *d_top_pos, const uint32_t *d_top_cnt,
                      const uint32_t *d_begin, uint32_t N, const hfx_db *db,
@@ -573,6 +580,9 @@ int hfx_format_scan(const hfx_scan_header *hdr, const hfx_match_row *rows, uint3
  *   levels 1..levels (level l = charges 1..l, max weight per bin), bins below
  *   max_len, as sorted uint16 entries bin | code << 14 (the FP32 batched
  *   form's input).
+ * A batch that runs on the index adds the theoretical rows it scores with (a
+ * KiB for each 256 bins of sixteen peptides, per charge level: 1.1 GB a level for
+ * 2.7 M peptides), where the device's memory holds them.
  * The reference has no counterpart: it rebuilds every theoretical spectrum
  * per (spectrum, candidate) pair (Search.hs:177-245).  Synchronises. */
 typedef struct hfx_pepix hfx_pepix;
@@ -616,10 +626,12 @@ int hfx_batch_split(const uint64_t *h_off, uint32_t S, uint32_t N, uint32_t num_
 int hfx_batch_use_index(hfx_batch *b, const hfx_pepix *ix);
 /* One batched search, every per-batch step on the device and without host
  * synchronisation or allocation: windows -> spectrum order (fragment charge
- * level, precursor mass) -> FP32 sparse form: blocks of G spectra,
- * persistent multi-spectrum XCorr over the index's ion lists; dense form:
- * block cut, hi/lo BF16 rows of the spectra, MFMA XCorr over the index's
- * ladders -> top-N with exact re-score. */
+ * level, precursor mass) -> block cut -> the spectra as digits (FP32 form: four
+ * base-256 digits, 32-bit fixed point; integer form: three) or hi and lo BF16 ->
+ * MFMA XCorr over the index's theoretical rows -> top-N with exact re-score.
+ * Without the rows (spectra longer than 2176 bins, no memory for them, a first
+ * run under capture) the FP32 form sums over the index's ion lists, blocks of G
+ * spectra, and the dense forms build the rows of a block from its ladders. */
 int hfx_batch_run(hfx_batch *b, void *stream);
 #define HFX_BATCH_FP32_SPARSE 0u  /* default after hfx_batch_plan */
 #define HFX_BATCH_BF16X2_DENSE 1u /* hfx_xcorr_dense_bf16x2 scores */
