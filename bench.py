@@ -367,7 +367,7 @@ def bench_stats(srch, steps, res):
                            "algorithmic_bytes": fit_bytes,
                            "achieved_gbs": fit_bytes / (fit_ms * 1e-3) / 1e9,
                            "frac_hbm": fit_bytes / (fit_ms * 1e-3) / 1e9 / HBM_PEAK_GBS},
-            "sp_ions": {"kernels": ["k_sp_peaks", "k_sp_topn"], "ms": ions_ms,
+            "sp_ions": {"kernels": ["k_sp_topn"], "ms": ions_ms,
                         "matches": int(res.top_cnt.sum())}}
 
 
