@@ -558,18 +558,19 @@ __global__ void k_ord_rank(uint32_t *order, const uint32_t *tmp, const uint64_t 
  * windows) -- a block spanning a gap in precursor mass would score every
  * candidate in the gap.  A dynamic programme per segment of CUT_SEG order
  * positions (segments are cut independently, which costs about 1% more
- * rows than one programme over the whole order), one row of 16 lanes a
- * segment: lane i holds the window of the (i+1)-th newest position and the
- * best cost of the positions before it.  Each step shifts both by one lane
- * (DPP row_shr:1, the new position entering lane 0), takes the hull of the
- * newest i+1 windows by inclusive row scans (min of starts, max of ends, OR
- * of charge levels) and the best block length by a row minimum of
- * (cost << 4 | i): the shortest block among equal costs, the one a serial
- * scan of lengths 1, 2, ... with strict improvement keeps. */
+ * rows than one programme over the whole order), a wave a segment.  First the
+ * costs of every block, which depend on nothing: sixteen lanes take the newest
+ * 1 .. 16 of j positions, their hulls by inclusive row scans (min of starts, max
+ * of ends, OR of charge levels).  Then the chain of 32 steps, cut to what hangs on
+ * the step before: an addition, a row minimum, a shift by a lane (DPP row_shr:1).
+ * Costs are whole and below 2^43, so exact in FP64, with length / 16 below the
+ * point: the shortest block among equal costs, the one a serial scan of lengths
+ * 1, 2, ... with strict improvement keeps.  11 us, 14.2 with the hulls in the
+ * chain and 64-bit integers. */
 #define CUT_SEG 32
 #define CUT_ROW 16
 #define CUT_WG 256
-#define CUT_SPW (CUT_WG / CUT_ROW) /* segments a workgroup */
+#define CUT_SPW (CUT_WG / HFX_WAVE) /* segments a workgroup */
 
 template <int CTRL>
 __device__ __forceinline__ uint32_t cut_dpp(uint32_t old, uint32_t v)
@@ -577,10 +578,11 @@ __device__ __forceinline__ uint32_t cut_dpp(uint32_t old, uint32_t v)
     return (uint32_t)__builtin_amdgcn_update_dpp((int)old, (int)v, CTRL, 0xf, 0xf, false);
 }
 template <int CTRL>
-__device__ __forceinline__ uint64_t cut_dpp64(uint64_t old, uint64_t v)
+__device__ __forceinline__ double cut_dpp64(double old, double v)
 {
-    return (uint64_t)cut_dpp<CTRL>((uint32_t)(old >> 32), (uint32_t)(v >> 32)) << 32 |
-           cut_dpp<CTRL>((uint32_t)old, (uint32_t)v);
+    return __hiloint2double(
+        (int)cut_dpp<CTRL>((uint32_t)__double2hiint(old), (uint32_t)__double2hiint(v)),
+        (int)cut_dpp<CTRL>((uint32_t)__double2loint(old), (uint32_t)__double2loint(v)));
 }
 
 template <int CUT_NS>
@@ -591,6 +593,7 @@ __global__ void __launch_bounds__(CUT_WG) k_cut_seg(uint32_t *seg_cuts, uint32_t
 {
     static_assert(CUT_NS <= CUT_ROW, "every block length has its lane");
     __shared__ uint32_t lo_s[CUT_SPW * CUT_SEG], hi_s[CUT_SPW * CUT_SEG], lv_s[CUT_SPW * CUT_SEG];
+    __shared__ double cost_s[CUT_SPW][CUT_SEG][CUT_ROW];
     __shared__ uint8_t from_s[CUT_SPW][CUT_SEG + 1];
     const uint32_t base = blockIdx.x * CUT_SPW * CUT_SEG;
     for (uint32_t i = threadIdx.x; i < CUT_SPW * CUT_SEG; i += CUT_WG) {
@@ -609,20 +612,20 @@ __global__ void __launch_bounds__(CUT_WG) k_cut_seg(uint32_t *seg_cuts, uint32_t
         lv_s[i] = lv;
     }
     __syncthreads();
-    const uint32_t r = threadIdx.x / CUT_ROW, i = threadIdx.x % CUT_ROW;
+    const uint32_t r = threadIdx.x / HFX_WAVE, lane = hfx_lane(), i = lane % CUT_ROW;
     const uint32_t seg = blockIdx.x * CUT_SPW + r;
     const uint32_t p0 = seg * CUT_SEG;
-    if (p0 >= S) return; /* the whole row leaves together */
+    if (p0 >= S) return; /* the whole wave leaves together */
     const uint32_t len = min((uint32_t)CUT_SEG, S - p0);
     const uint32_t *lo = lo_s + r * CUT_SEG, *hi = hi_s + r * CUT_SEG, *lv = lv_s + r * CUT_SEG;
     uint8_t *from = from_s[r];
-    uint32_t wlo = 0xffffffffu, whi = 0, wlv = 0;
-    uint64_t bst = i == 0 ? 0ull : ~0ull;
-    for (uint32_t j = 1; j <= len; ++j) {
-        wlo = cut_dpp<0x111>(lo[j - 1], wlo);
-        whi = cut_dpp<0x111>(hi[j - 1], whi);
-        wlv = cut_dpp<0x111>(lv[j - 1], wlv);
-        uint32_t l = wlo, h = whi, v = wlv;
+    /* lane i of a row: the block of the newest i + 1 of j positions, four j a turn */
+#pragma unroll
+    for (uint32_t q = 0; q < CUT_SEG * CUT_ROW / HFX_WAVE; ++q) {
+        const uint32_t j = q * (HFX_WAVE / CUT_ROW) + lane / CUT_ROW + 1;
+        const bool in = i < j;
+        const uint32_t at = in ? j - 1u - i : 0u;
+        uint32_t l = in ? lo[at] : 0xffffffffu, h = in ? hi[at] : 0u, v = in ? lv[at] : 0u;
         l = min(l, cut_dpp<0x111>(0xffffffffu, l));
         h = max(h, cut_dpp<0x111>(0u, h));
         v |= cut_dpp<0x111>(0u, v);
@@ -635,25 +638,30 @@ __global__ void __launch_bounds__(CUT_WG) k_cut_seg(uint32_t *seg_cuts, uint32_t
         l = min(l, cut_dpp<0x118>(0xffffffffu, l));
         h = max(h, cut_dpp<0x118>(0u, h));
         v |= cut_dpp<0x118>(0u, v);
-        /* lane i: the block of the newest i + 1 positions after the best cut
-         * of the ones before (bst, finite for i < j) */
         const uint64_t rows = h > l ? (uint64_t)(h - l) : 0ull;
-        uint64_t key = ~0ull;
-        if (i < (uint32_t)CUT_NS && i < j)
-            key = (bst + rows * (uint64_t)__builtin_popcount(v)) << 4 | i;
-        uint64_t t;
-        t = cut_dpp64<0xB1>(0ull, key);  /* quad_perm [1,0,3,2] */
-        key = t < key ? t : key;
-        t = cut_dpp64<0x4E>(0ull, key);  /* quad_perm [2,3,0,1] */
-        key = t < key ? t : key;
-        t = cut_dpp64<0x141>(0ull, key); /* row_half_mirror */
-        key = t < key ? t : key;
-        t = cut_dpp64<0x140>(0ull, key); /* row_mirror */
-        key = t < key ? t : key;
-        bst = cut_dpp64<0x111>(key >> 4, bst);
-        if (i == 0) from[j] = (uint8_t)(j - 1u - (uint32_t)(key & 15u));
+        cost_s[r][j - 1][i] = i < (uint32_t)CUT_NS && in
+                                  ? (double)(rows * (uint64_t)__builtin_popcount(v)) + 0.0625 * (double)i
+                                  : (double)INFINITY;
     }
-    if (i != 0) return;
+    hfx_wave_sync();
+    /* lane i: the best cost of the positions before that block (finite for i < j) */
+    double bst = i == 0 ? 0.0 : (double)INFINITY;
+#pragma unroll 8
+    for (uint32_t j = 1; j <= len; ++j) {
+        double key = bst + cost_s[r][j - 1][i], t;
+        t = cut_dpp64<0xB1>(0.0, key);  /* quad_perm [1,0,3,2] */
+        key = t < key ? t : key;
+        t = cut_dpp64<0x4E>(0.0, key);  /* quad_perm [2,3,0,1] */
+        key = t < key ? t : key;
+        t = cut_dpp64<0x141>(0.0, key); /* row_half_mirror */
+        key = t < key ? t : key;
+        t = cut_dpp64<0x140>(0.0, key); /* row_mirror */
+        key = t < key ? t : key;
+        const double whole = floor(key);
+        bst = cut_dpp64<0x111>(whole, bst);
+        if (lane == 0) from[j] = (uint8_t)(j - 1u - (uint32_t)((key - whole) * 16.0));
+    }
+    if (lane != 0) return;
     /* block starts, back from the segment's end, then written in order */
     uint32_t cnt = 0;
     for (uint32_t j = len; j > 0; j = from[j]) ++cnt;
