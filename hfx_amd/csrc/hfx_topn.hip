@@ -741,16 +741,86 @@ __global__ void __launch_bounds__(TN_THREADS)
     }
 }
 
+#define TX_CHUNK 256
+/* a flagged spectrum's tiles also number at least its band count / TX_LIVE,
+ * so that the candidates the exact route re-scores spread over the tiles */
+#define TX_LIVE 32
+
+/* the exact route's work: the flagged spectra (in any order), their number, the
+ * first tile of each (off[number] = all tiles) */
+struct TxPlan {
+    uint64_t *off;
+    uint32_t *list, *count;
+};
+
+/* by one workgroup: few spectra are flagged, so the tiles need no table per
+ * spectrum */
+template <class Cands>
+__device__ void tx_plan(TxPlan p, const uint32_t *flag, const uint32_t *band, const Cands &c,
+                        uint32_t S)
+{
+    __shared__ uint32_t nl;
+    __shared__ uint64_t wt[TN_THREADS / HFX_WAVE];
+    const uint32_t lane = hfx_lane(), wave = threadIdx.x / HFX_WAVE;
+    if (threadIdx.x == 0) nl = 0;
+    __syncthreads();
+    for (uint32_t s0 = threadIdx.x; s0 < S; s0 += 8 * TN_THREADS) {
+        uint32_t fv[8];
+#pragma unroll
+        for (uint32_t u = 0; u < 8; ++u) fv[u] = flag[min(s0 + u * TN_THREADS, S - 1u)];
+#pragma unroll
+        for (uint32_t u = 0; u < 8; ++u)
+            if (s0 + u * TN_THREADS < S && fv[u] != 0u)
+                p.list[atomicAdd(&nl, 1u)] = s0 + u * TN_THREADS;
+    }
+    __syncthreads(); /* the list is this workgroup's own: visible to it from here */
+    const uint32_t F = nl;
+    uint64_t nt = 0;
+    for (uint32_t q0 = 0; q0 < F; q0 += TN_THREADS) {
+        const uint32_t q = q0 + threadIdx.x;
+        uint64_t t = 0;
+        if (q < F) {
+            const uint32_t s = p.list[q], n = c.count(s), b = min(band[s], n);
+            t = max((n + TX_CHUNK - 1) / TX_CHUNK, (b + TX_LIVE - 1) / TX_LIVE);
+        }
+        uint64_t x = t;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) {
+            const uint64_t v = __shfl_up(x, o, 64);
+            if (lane >= (uint32_t)o) x += v;
+        }
+        if (lane == HFX_WAVE - 1) wt[wave] = x;
+        __syncthreads();
+        uint64_t to = nt + x - t;
+        for (uint32_t w = 0; w < TN_THREADS / HFX_WAVE; ++w) {
+            if (w < wave) to += wt[w];
+            nt += wt[w];
+        }
+        if (q < F) p.off[q] = to;
+        __syncthreads();
+    }
+    if (threadIdx.x == 0) {
+        p.off[F] = nt;
+        *p.count = F;
+    }
+}
+
 /* the lists in order of (exact desc, position asc): the best N, and for
- * flagged spectra exN - B as the exact route's threshold.  A wave a spectrum. */
+ * flagged spectra exN - B as the exact route's threshold.  A wave a spectrum; the
+ * first workgroup plans the exact route meanwhile, from what the selection left
+ * (its own launch took 2 to 6 us, and the gap). */
 template <class Cands>
 __global__ void __launch_bounds__(TN_THREADS)
     k_topn_rank(uint32_t *top_pos, double *top_exact, float *top_f32, uint32_t *top_cnt,
                 const uint32_t *flag, uint32_t N, const int64_t *fx, TnLists o, const float *scores,
-                Cands c, uint32_t S)
+                Cands c, uint32_t S, TxPlan plan)
 {
     const uint32_t wave = threadIdx.x / HFX_WAVE, lane = hfx_lane();
-    const uint32_t s = blockIdx.x * TN_WAVES + wave;
+    if (blockIdx.x == 0) {
+        tx_plan(plan, flag, o.band, c, S);
+        return;
+    }
+    const uint32_t s = (blockIdx.x - 1u) * TN_WAVES + wave;
     if (s >= S) return;
     const uint32_t M = o.mcnt[s] & ~TN_BIG, n = c.count(s), outn = min(N, n);
     const float *sc = scores + c.base(s);
@@ -808,67 +878,17 @@ __global__ void __launch_bounds__(TN_THREADS)
 /* ------------------------------------------------------------------ */
 
 #define TX_MAXN 64
-#define TX_CHUNK 256
-/* a flagged spectrum's tiles also number at least its band count / TX_LIVE,
- * so that the candidates the exact route re-scores spread over the tiles */
-#define TX_LIVE 32
 /* a wave fetches the metadata of its share of a tile one lane per candidate */
 static_assert(TX_CHUNK / TN_WAVES <= HFX_WAVE && TN_TASK <= HFX_WAVE,
               "one lane per candidate of a wave's share");
 
-/* the flagged spectra (in any order) and the first tile of each (off[their
- * number] = all tiles), by one workgroup: few spectra are flagged, so the tiles
- * need no table per spectrum */
-#define TX_THREADS 1024
+/* the list of the flagged spectra as a launch of its own, where the caller names
+ * them */
 template <class Cands>
-__global__ void __launch_bounds__(TX_THREADS)
-    k_tx_plan(uint64_t *off, uint32_t *list, uint32_t *count, const uint32_t *flag,
-              const uint32_t *band, Cands c, uint32_t S)
+__global__ void __launch_bounds__(TN_THREADS)
+    k_tx_plan(TxPlan p, const uint32_t *flag, const uint32_t *band, Cands c, uint32_t S)
 {
-    __shared__ uint32_t nl;
-    __shared__ uint64_t wt[TX_THREADS / HFX_WAVE];
-    const uint32_t lane = hfx_lane(), wave = threadIdx.x / HFX_WAVE;
-    if (threadIdx.x == 0) nl = 0;
-    __syncthreads();
-    for (uint32_t s0 = threadIdx.x; s0 < S; s0 += 8 * TX_THREADS) {
-        uint32_t fv[8];
-#pragma unroll
-        for (uint32_t u = 0; u < 8; ++u) fv[u] = flag[min(s0 + u * TX_THREADS, S - 1u)];
-#pragma unroll
-        for (uint32_t u = 0; u < 8; ++u)
-            if (s0 + u * TX_THREADS < S && fv[u] != 0u)
-                list[atomicAdd(&nl, 1u)] = s0 + u * TX_THREADS;
-    }
-    __syncthreads(); /* the list is this workgroup's own: visible to it from here */
-    const uint32_t F = nl;
-    uint64_t nt = 0;
-    for (uint32_t q0 = 0; q0 < F; q0 += TX_THREADS) {
-        const uint32_t q = q0 + threadIdx.x;
-        uint64_t t = 0;
-        if (q < F) {
-            const uint32_t s = list[q], n = c.count(s), b = min(band[s], n);
-            t = max((n + TX_CHUNK - 1) / TX_CHUNK, (b + TX_LIVE - 1) / TX_LIVE);
-        }
-        uint64_t x = t;
-#pragma unroll
-        for (int o = 1; o < 64; o <<= 1) {
-            const uint64_t v = __shfl_up(x, o, 64);
-            if (lane >= (uint32_t)o) x += v;
-        }
-        if (lane == HFX_WAVE - 1) wt[wave] = x;
-        __syncthreads();
-        uint64_t to = nt + x - t;
-        for (uint32_t w = 0; w < TX_THREADS / HFX_WAVE; ++w) {
-            if (w < wave) to += wt[w];
-            nt += wt[w];
-        }
-        if (q < F) off[q] = to;
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) {
-        off[F] = nt;
-        *count = F;
-    }
+    tx_plan(p, flag, band, c, S);
 }
 
 __global__ void k_tx_reset(uint32_t *counter)
@@ -1277,6 +1297,7 @@ static TxScratch tx_carve(void *p, uint32_t S, uint64_t total)
     x.l.task = S <= TN_FEW ? TN_TASK_FEW : TN_TASK;
     return x;
 }
+static TxPlan tx_plan_of(const TxScratch &x) { return {x.tile_off, x.list, x.counter + 1}; }
 static int tx_scratch(hfx_ctx *ctx, void *given, uint32_t S, uint64_t total, void **out)
 {
     *out = given;
@@ -1288,7 +1309,7 @@ template <class Cands>
 static int exact_route(hfx_ctx *ctx, uint32_t *d_top_pos, double *d_top_exact, float *d_top_f32,
                        uint32_t *d_top_cnt, uint32_t N, uint32_t *d_flag,
                        const float *d_scores, const Cands &c, uint64_t total,
-                       const hfx_spectra *sp, void *scratch, hipStream_t st)
+                       const hfx_spectra *sp, void *scratch, bool planned, hipStream_t st)
 {
     const uint32_t S = sp->num_spec;
     if (S == 0) return HFX_OK;
@@ -1297,8 +1318,9 @@ static int exact_route(hfx_ctx *ctx, uint32_t *d_top_pos, double *d_top_exact, f
     int rc;
     if ((rc = tx_scratch(ctx, scratch, S, total, &p))) return rc;
     const TxScratch x = tx_carve(p, S, total);
-    hipLaunchKernelGGL(k_tx_plan<Cands>, dim3(1), dim3(TX_THREADS), 0, st, x.tile_off, x.list,
-                       x.counter + 1, d_flag, x.l.band, c, S);
+    if (!planned)
+        hipLaunchKernelGGL(k_tx_plan<Cands>, dim3(1), dim3(TN_THREADS), 0, st, tx_plan_of(x), d_flag,
+                           x.l.band, c, S);
     hipLaunchKernelGGL(k_exact_tiles<Cands>, dim3((uint32_t)hfx_ctx_num_cus(ctx) * 4),
                        dim3(TN_THREADS), fx_lds_bytes(sp->x_stride), st, x.fxbuf, x.tile_off, x.list,
                        x.counter + 1, c, *sp, d_scores, x.l.tau, xp_map_words(sp->x_stride));
@@ -1337,11 +1359,12 @@ static int launch_topn(hfx_ctx *ctx, uint32_t *d_top_pos, double *d_top_exact, f
     hipLaunchKernelGGL(k_topn_exact<Cands>, dim3(max(gw, 4u * (uint32_t)hfx_ctx_num_cus(ctx))),
                        dim3(TN_THREADS), fx_lds_bytes(sp->x_stride), st, x.fxbuf, x.l, c, *sp,
                        xp_map_words(sp->x_stride));
-    hipLaunchKernelGGL(k_topn_rank<Cands>, dim3(gw), dim3(TN_THREADS), 0, st, d_top_pos,
-                       d_top_exact, d_top_f32, d_top_cnt, d_flag, N, x.fxbuf, x.l, d_scores, c, S);
+    hipLaunchKernelGGL(k_topn_rank<Cands>, dim3(gw + 1), dim3(TN_THREADS), 0, st, d_top_pos,
+                       d_top_exact, d_top_f32, d_top_cnt, d_flag, N, x.fxbuf, x.l, d_scores, c, S,
+                       tx_plan_of(x));
     HFX_CHECK_LAUNCH();
     return exact_route(ctx, d_top_pos, d_top_exact, d_top_f32, d_top_cnt, N, d_flag, d_scores, c,
-                       total, sp, p, st);
+                       total, sp, p, true, st);
 }
 
 template <class Cands>
@@ -1365,7 +1388,7 @@ static int launch_topn_exact(hfx_ctx *ctx, uint32_t *d_top_pos, double *d_top_ex
     hipLaunchKernelGGL(k_mark_list, dim3((num_list + 255) / 256), dim3(256), 0, st, flag, x.l.tau,
                        x.l.band, d_list, num_list, S);
     return exact_route(ctx, d_top_pos, d_top_exact, d_top_f32, d_top_cnt, N, flag, d_scores, c,
-                       total, sp, q, st);
+                       total, sp, q, false, st);
 }
 
 /* used by the batched path: the whole top-N on the device */
