@@ -95,6 +95,24 @@ def test_lists_shared_out_whole_and_in_halves(tenv, S):
         assert pos[k, :cnt[k]].tolist() == ref["top_pos"][which[k], :cnt[k]].tolist(), k
 
 
+@pytest.mark.parametrize("S", [255, 700])
+def test_many_spectra_on_the_exact_route(tenv, S):
+    """The list of flagged spectra in one turn of its workgroup and in several."""
+    pl = tenv["pl"]
+    which = np.arange(S) % 48
+    sp = Spectra(pl, *(a[which] for a in tenv["rows"]))
+    s = pl.PlainSearch(tenv["ctx"], tenv["db"], sp, eps=250.0, topn=5)
+    s.window()
+    s.score()
+    s.select_rel(0.5)
+    assert len(s.short()) == 0 and (len(s.flagged()) > 256) == (S == 700)
+    ref = tenv["ref"][250.0]
+    pos = pl.host(s.t_pos, np.uint32, S * 5).reshape(S, 5)
+    for k in range(S):
+        c = min(int(ref["num"][which[k]]), 5)
+        assert pos[k, :c].tolist() == ref["top_pos"][which[k], :c].tolist(), k
+
+
 @pytest.mark.parametrize("N", [5, 40])
 def test_scores_with_infinities_keep_their_order(tenv, orc, N):
     """The selection follows the scores' total order: with -inf in most places the finite ones
