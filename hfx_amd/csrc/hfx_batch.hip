@@ -338,16 +338,114 @@ struct hfx_pepix {
     uint64_t *ent_off;
     uint16_t *ent;
     uint64_t n_ent, n_pos, bytes;
-    /* theoretical rows (hfx_rows.hip), a level at a time when a batch first
-     * needs it; never moved once written.  g_rows_mu guards them. */
-    hfx_rows rows;
+    uint64_t key[2]; /* of the database's contents */
+    struct RowSet *rs; /* its theoretical rows, once a batch has needed them */
 };
-static std::mutex g_rows_mu;
+
+/* The theoretical rows of a database (hfx_rows.hip), one copy for all indexes over
+ * the same contents: 1.57 GB a charge level for 2.7 M peptides.  A level is written
+ * when a batch first needs it and not moved while a batch uses the set; a set
+ * that no batch uses gives its rows back where memory is short (they are written
+ * again when next needed), one that no index holds either is freed.  Two databases are the
+ * same by a 128-bit key of what rows are made from, never by their addresses. */
+struct RowSet {
+    int device;
+    uint32_t num_pep;
+    uint64_t key[2];
+    hfx_rows rows;
+    uint64_t bytes;
+    uint32_t keepers, users; /* indexes, batches */
+};
+static std::mutex g_rows_mu; /* the sets and what they hold */
+static std::vector<RowSet *> g_rowsets;
+
+/* frees a set's rows; called with g_rows_mu held and no batch using it */
+static void rowset_clear(RowSet *rs)
+{
+    (void)hipDeviceSynchronize(); /* work of batches that used it */
+    for (uint8_t *&p : rs->rows.rows) {
+        if (p) (void)hipFree(p);
+        p = nullptr;
+    }
+    if (rs->rows.ng) (void)hipFree(rs->rows.ng);
+    rs->rows.ng = nullptr;
+    rs->bytes = 0;
+}
+
+/* one keeper or user less, g_rows_mu held */
+static void rowset_leave(RowSet *rs, uint32_t RowSet::*count)
+{
+    if (--(rs->*count) || rs->keepers || rs->users) return;
+    rowset_clear(rs);
+    g_rowsets.erase(std::remove(g_rowsets.begin(), g_rowsets.end(), rs), g_rowsets.end());
+    delete rs;
+}
+
+bool hfx_rowsets_release(int device)
+{
+    std::lock_guard<std::mutex> lk(g_rows_mu);
+    bool any = false;
+    for (RowSet *rs : g_rowsets)
+        if (rs->device == device && rs->users == 0 && rs->bytes) {
+            rowset_clear(rs);
+            any = true;
+        }
+    return any;
+}
+
+__global__ void k_ord_fill(uint32_t *a, uint32_t n)
+{
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) a[i] = 0u;
+}
+
+/* A 128-bit key of the peptides in residual order -- residuals, ladder residues --
+ * and the residue masses: two polynomials over each peptide's residues, mixed with its
+ * place and residual (D. Stafford's variant 13 of the 64-bit finaliser) and added
+ * up.  2.7 M peptides are read once, a few tens of us when an index is built. */
+__device__ __forceinline__ uint64_t key_mix(uint64_t x)
+{
+    x = (x ^ (x >> 30)) * 0xbf58476d1ce4e5b9ull;
+    x = (x ^ (x >> 27)) * 0x94d049bb133111ebull;
+    return x ^ (x >> 31);
+}
+__global__ void __launch_bounds__(256) k_db_key(unsigned long long *key, hfx_db db)
+{
+    uint64_t a = 0, b = 0;
+    const uint32_t t = blockIdx.x * 256 + threadIdx.x;
+    if (t < 26) {
+        const uint64_t m = (uint64_t)t << 32 | __float_as_uint(db.d_mass[t]);
+        a = key_mix(m + 0x9e3779b97f4a7c15ull);
+        b = key_mix(m ^ 0xd1b54a32d192ed03ull);
+    }
+    for (uint64_t q = t; q < db.num_pep; q += gridDim.x * 256ull) {
+        const uint32_t pep = db.d_idx_sorted[q];
+        const uint32_t tc = db.d_tc[pep], tn = db.d_tn[pep];
+        const uint32_t n = tn > tc ? tn - tc : 0u;
+        uint64_t x = n, y = ~(uint64_t)n;
+        for (uint32_t j = 0; j < n; ++j) {
+            const uint32_t c = HFX_ACID_IDX(db.d_ions[tc + j]) + 1u;
+            x = x * 0x9e3779b97f4a7c15ull + c;
+            y = y * 0xc2b2ae3d27d4eb4full + c;
+        }
+        const uint64_t at = q << 32 | __float_as_uint(db.d_r[pep]);
+        a += key_mix(key_mix(x) + key_mix(at + 1u));
+        b += key_mix(key_mix(y) ^ key_mix(at ^ 0x5851f42d4c957f2dull));
+    }
+    for (int o = 32; o > 0; o >>= 1) {
+        a += __shfl_xor(a, o, 64);
+        b += __shfl_xor(b, o, 64);
+    }
+    if (hfx_lane() == 0) {
+        atomicAdd(key, (unsigned long long)a);
+        atomicAdd(key + 1, (unsigned long long)b);
+    }
+}
 
 template <class T>
 static int dalloc(T **p, size_t n)
 {
-    hipError_t e = hipMalloc((void **)p, (n ? n : 1) * sizeof(T));
+    hipError_t e = hfx_device_malloc((void **)p, (n ? n : 1) * sizeof(T));
     if (e != hipSuccess) {
         *p = nullptr;
         hfx_set_error("device allocation of %zu bytes failed: %s", n * sizeof(T),
@@ -361,10 +459,11 @@ extern "C" int hfx_pepix_destroy(hfx_pepix *ix)
 {
     if (!ix) return HFX_OK;
     (void)hipDeviceSynchronize();
-    void *ps[] = {ix->lad_mem[0], ix->lad_mem[1], ix->caps,         ix->cnt,
-                  ix->ent_off,    ix->ent,        ix->rows.rows[0], ix->rows.rows[1],
-                  ix->rows.rows[2], ix->rows.rows[3], ix->rows.ng};
-    static_assert(HFX_MAX_CHARGE == 4, "one row buffer a charge level");
+    if (ix->rs) {
+        std::lock_guard<std::mutex> lk(g_rows_mu);
+        rowset_leave(ix->rs, &RowSet::keepers);
+    }
+    void *ps[] = {ix->lad_mem[0], ix->lad_mem[1], ix->caps, ix->cnt, ix->ent_off, ix->ent};
     for (void *p : ps)
         if (p) (void)hipFree(p);
     free(ix);
@@ -390,7 +489,13 @@ extern "C" int hfx_pepix_build(hfx_ctx *ctx, const hfx_db *db, uint32_t forms, u
     hipStream_t st = hfx_stream(stream);
     const uint32_t P = db->num_pep;
     int rc = HFX_OK;
-    if (forms & HFX_PEPIX_LADDER) {
+    unsigned long long *key = nullptr;
+    rc = dalloc(&key, 2);
+    if (!rc && P) {
+        hipLaunchKernelGGL(k_ord_fill, dim3(1), dim3(64), 0, st, (uint32_t *)key, 4u);
+        hipLaunchKernelGGL(k_db_key, dim3(std::min((P + 255) / 256, 4096u)), dim3(256), 0, st, key, *db);
+    }
+    if (!rc && (forms & HFX_PEPIX_LADDER)) {
         rc = hfx_dense_ladder_build(ctx, db, 0, P, 1, &ix->lad, ix->lad_mem, stream);
         if (!rc) {
             ix->n_pos = 0;
@@ -437,10 +542,15 @@ extern "C" int hfx_pepix_build(hfx_ctx *ctx, const hfx_db *db, uint32_t forms, u
         hfx_set_error("hfx_pepix_build: kernel launch failed");
         rc = HFX_ERR_HIP;
     }
-    if (!rc && hipStreamSynchronize(st) != hipSuccess) {
+    if (!rc && P && hipMemcpyAsync(ix->key, key, 16, hipMemcpyDeviceToHost, st) != hipSuccess) {
+        hfx_set_error("hfx_pepix_build: reading the key failed");
+        rc = HFX_ERR_HIP;
+    }
+    if (hipStreamSynchronize(st) != hipSuccess && !rc) {
         hfx_set_error("hfx_pepix_build: synchronize failed");
         rc = HFX_ERR_HIP;
     }
+    if (key) (void)hipFree(key);
     if (rc) {
         hfx_pepix_destroy(ix);
         return rc;
@@ -449,50 +559,68 @@ extern "C" int hfx_pepix_build(hfx_ctx *ctx, const hfx_db *db, uint32_t forms, u
     return HFX_OK;
 }
 
-/* The index's rows of charge levels 1..L, written now where they are missing
- * (waits for the stream then): false when a quarter of the free memory does
- * not hold them, and the batch keeps the ladder or ion-list kernels.  The rows
- * of a level take RW_G KiB for sixteen peptides: 1.57 GB for 2.7 M. */
-static bool pepix_need_rows(hfx_pepix *ix, uint32_t L, uint32_t cus, hipStream_t st)
+/* The rows of charge levels 1..L of the index's database, for one more batch
+ * (rowset_leave(.., &RowSet::users) when it is done): written now where they are
+ * missing (waits for the stream then).  Null when a quarter of the free memory does
+ * not hold them: the batch keeps the ladder or ion-list kernels. */
+static RowSet *pepix_use_rows(hfx_pepix *ix, uint32_t L, uint32_t cus, hipStream_t st, hfx_rows *out)
 {
     std::lock_guard<std::mutex> lk(g_rows_mu);
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess) return nullptr;
+    if (!ix->rs) {
+        for (RowSet *rs : g_rowsets)
+            if (rs->device == dev && rs->num_pep == ix->db.num_pep && rs->key[0] == ix->key[0] &&
+                rs->key[1] == ix->key[1])
+                ix->rs = rs;
+        if (!ix->rs) {
+            ix->rs = new RowSet{dev, ix->db.num_pep, {ix->key[0], ix->key[1]}, {}, 0, 0, 0};
+            g_rowsets.push_back(ix->rs);
+        }
+        ++ix->rs->keepers;
+    }
+    RowSet *rs = ix->rs;
     const uint32_t nt = hfx_rows_tiles(ix->db.num_pep);
     const uint64_t level = std::max<uint64_t>((uint64_t)nt * RW_G * 1024, 256);
     hfx_rows want{};
     want.ntiles = nt;
     want.G = RW_G;
     uint64_t need = 0;
-    for (uint32_t l = 0; l < L; ++l) need += ix->rows.rows[l] ? 0 : level;
-    if (need == 0) return true;
-    size_t fr = 0, tot = 0;
-    bool ok = hipMemGetInfo(&fr, &tot) == hipSuccess && need <= fr / 4;
-    if (ok && !ix->rows.ng) ok = hipMalloc((void **)&ix->rows.ng, nt + 4ull) == hipSuccess;
-    for (uint32_t l = 0; l < L && ok; ++l)
-        if (!ix->rows.rows[l]) ok = hipMalloc((void **)&want.rows[l], level) == hipSuccess;
-    want.ng = ix->rows.ng;
-    ok = ok && hfx_rows_build(cus, &ix->db, &want, nullptr, (void *)st) == HFX_OK &&
-         hipStreamSynchronize(st) == hipSuccess;
-    for (uint32_t l = 0; l < HFX_MAX_CHARGE; ++l) {
-        if (!want.rows[l]) continue;
-        if (!ok) {
-            (void)hipFree(want.rows[l]);
-            continue;
+    for (uint32_t l = 0; l < L; ++l) need += rs->rows.rows[l] ? 0 : level;
+    if (need) {
+        size_t fr = 0, tot = 0;
+        bool ok = hipMemGetInfo(&fr, &tot) == hipSuccess && need <= fr / 4;
+        if (ok && !rs->rows.ng) ok = hipMalloc((void **)&rs->rows.ng, nt + 4ull) == hipSuccess;
+        for (uint32_t l = 0; l < L && ok; ++l)
+            if (!rs->rows.rows[l]) ok = hipMalloc((void **)&want.rows[l], level) == hipSuccess;
+        want.ng = rs->rows.ng;
+        ok = ok && hfx_rows_build(cus, &ix->db, &want, nullptr, (void *)st) == HFX_OK &&
+             hipStreamSynchronize(st) == hipSuccess;
+        for (uint32_t l = 0; l < HFX_MAX_CHARGE; ++l) {
+            if (!want.rows[l]) continue;
+            if (!ok) {
+                (void)hipFree(want.rows[l]);
+                continue;
+            }
+            rs->rows.rows[l] = want.rows[l];
+            rs->bytes += level;
         }
-        ix->rows.rows[l] = want.rows[l];
-        ix->bytes += level;
+        (void)hipGetLastError();
+        if (!ok) return nullptr;
+        rs->rows.ntiles = nt;
+        rs->rows.G = RW_G;
     }
-    (void)hipGetLastError();
-    if (!ok) return false;
-    ix->rows.ntiles = nt;
-    ix->rows.G = RW_G;
-    return true;
+    ++rs->users;
+    *out = rs->rows;
+    return rs;
 }
 
 extern "C" int hfx_pepix_info(const hfx_pepix *ix, uint64_t *info /*[6]*/)
 {
     HFX_REQUIRE(ix && info, HFX_ERR_ARG, "hfx_pepix_info: null argument");
     info[0] = ix->forms; info[1] = ix->L; info[2] = ix->lcap; info[3] = ix->n_pos;
-    info[4] = ix->n_ent; info[5] = ix->bytes;
+    std::lock_guard<std::mutex> lk(g_rows_mu);
+    info[4] = ix->n_ent; info[5] = ix->bytes + (ix->rs ? ix->rs->bytes : 0);
     return HFX_OK;
 }
 
@@ -504,12 +632,6 @@ extern "C" int hfx_pepix_info(const hfx_pepix *ix, uint64_t *info /*[6]*/)
  * bucket = level * nbz + (window begin >> sh) -- the window's first
  * residual-sorted position is a monotone function of the precursor mass --
  * counted, scattered, then ranked inside each bucket by (mass, index). */
-__global__ void k_ord_fill(uint32_t *a, uint32_t n)
-{
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) a[i] = 0u;
-}
-
 __device__ __forceinline__ uint32_t ord_bucket(uint32_t s, const uint32_t *begin,
                                                const uint32_t *zmax, uint32_t sh, uint32_t nbz)
 {
@@ -769,14 +891,28 @@ struct hfx_batch {
     uint64_t *cut_off;
     uint32_t nseg;
     bool dense_set;      /* a dense form was chosen since the plan */
-    bool rows_tried, use_rows; /* scores come from the index's rows */
+    bool rows_tried, use_rows; /* scores come from the database's rows */
+    RowSet *rs;                /* the set they are in, and what this batch reads of it */
+    hfx_rows rows;
     uint32_t *rw_small;  /* rows: [S] sum and max of |x|, [3][S] quanta, levels, wide marks */
     hipGraph_t graph;
     hipGraphExec_t exec;
 };
 
+/* the rows are decided anew at the next run */
+static void bt_rows_drop(hfx_batch *b)
+{
+    if (b->rs) {
+        std::lock_guard<std::mutex> lk(g_rows_mu);
+        rowset_leave(b->rs, &RowSet::users);
+    }
+    b->rs = nullptr;
+    b->rows_tried = b->use_rows = false;
+}
+
 static void bt_free(hfx_batch *b)
 {
+    bt_rows_drop(b);
     void *ps[] = {b->begin,    b->num,       b->order,     b->ubeg,      b->uend,
                   b->ntiles,   b->counter,   b->score_off, b->tile_off,  b->scores,
                   b->top_pos,  b->top_cnt,   b->flag,      b->top_exact, b->top_f32,
@@ -822,7 +958,7 @@ extern "C" int hfx_batch_use_index(hfx_batch *b, const hfx_pepix *ix)
                     (ix->db.d_idx_sorted == b->db.d_idx_sorted && ix->db.num_pep == b->db.num_pep),
                 HFX_ERR_ARG, "hfx_batch_use_index: the index belongs to another database");
     b->ix = ix;
-    b->rows_tried = b->use_rows = false;
+    bt_rows_drop(b);
     if (b->exec) {
         (void)hipGraphExecDestroy(b->exec);
         b->exec = nullptr;
@@ -968,7 +1104,7 @@ static int bt_need_index(hfx_batch *b, hipStream_t st)
     if (b->own) hfx_pepix_destroy(b->own);
     b->own = nx;
     b->ix = nx;
-    b->rows_tried = b->use_rows = false;
+    bt_rows_drop(b);
     return HFX_OK;
 }
 
@@ -989,9 +1125,13 @@ static int bt_ready(hfx_batch *b, hipStream_t st)
     size_t fr = 0, tot = 0;
     HFX_CHECK_HIP(hipMemGetInfo(&fr, &tot));
     if (!b->dn_scratch && (uint64_t)b->S * 16384 > fr / 4) return HFX_OK;
-    if (!pepix_need_rows(const_cast<hfx_pepix *>(b->ix), b->L, (uint32_t)hfx_ctx_num_cus(b->ctx), st)) return HFX_OK;
+    b->rs = pepix_use_rows(const_cast<hfx_pepix *>(b->ix), b->L, (uint32_t)hfx_ctx_num_cus(b->ctx),
+                           st, &b->rows);
+    if (!b->rs) return HFX_OK;
     if (bt_dense_alloc(b) || (!b->rw_small && dalloc(&b->rw_small, 5 * (size_t)b->S))) {
         (void)hipGetLastError();
+        bt_rows_drop(b);
+        b->rows_tried = true;
         return HFX_OK;
     }
     b->use_rows = true;
@@ -1123,6 +1263,7 @@ extern "C" int hfx_batch_plan(hfx_batch *b, const hfx_db *db, const hfx_spectra 
         size_t fr = 0, tot = 0;
         HFX_CHECK_HIP(hipMemGetInfo(&fr, &tot));
         const uint64_t need = bt_bytes(S, b->total, N, db->num_pep, HFX_BATCH_FP32_SPARSE);
+        if (need > fr && hfx_spare_release()) HFX_CHECK_HIP(hipMemGetInfo(&fr, &tot));
         HFX_REQUIRE(need <= fr, HFX_ERR_NOMEM,
                     "hfx_batch_plan: %u spectra with %llu scores need %llu device bytes, %zu free "
                     "(split them with hfx_batch_split)",
@@ -1314,7 +1455,7 @@ static int bt_row_scores(hfx_batch *b, hipStream_t st, void **ev)
     if ((rc = hfx_rows_blocks(b->ctx, mode, bt_items(b), b->order, b->dn_bstart, b->begin, b->num,
                               &sq, b->CH, (void *)st)) ||
         (rc = hfx_rows_scores(b->ctx, mode, bt_items(b), b->scores, b->score_off, b->begin, b->num,
-                              b->order, b->dn_bstart, &b->ix->rows, bt_planes(b), qs, &sq, b->CH,
+                              b->order, b->dn_bstart, &b->rows, bt_planes(b), qs, &sq, b->CH,
                               (void *)st, ev)))
         return rc;
     if (mode != RW_I8X4) return HFX_OK;

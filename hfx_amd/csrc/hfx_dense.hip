@@ -1163,7 +1163,7 @@ int hfx_dense_ladder_build(hfx_ctx *ctx, const hfx_db *db, uint32_t q0, uint32_t
     void *m = nullptr;
     int rc;
     if (own) {
-        HFX_CHECK_HIP(hipMalloc(&m, meta));
+        HFX_CHECK_HIP(hfx_device_malloc((void **)&m, meta));
         mem[0] = m;
     } else if ((rc = hfx_ctx_scratch(ctx, HFX_SLOT_LADDER, meta, &m))) {
         return rc;
@@ -1181,7 +1181,7 @@ int hfx_dense_ladder_build(hfx_ctx *ctx, const hfx_db *db, uint32_t q0, uint32_t
     const size_t pb = (size_t)std::max<uint64_t>(total, 1) * sizeof(hfx_dn_pos);
     void *pp = nullptr;
     if (own) {
-        HFX_CHECK_HIP(hipMalloc(&pp, pb));
+        HFX_CHECK_HIP(hfx_device_malloc((void **)&pp, pb));
         mem[1] = pp;
     } else if ((rc = hfx_ctx_scratch(ctx, HFX_SLOT_LADDER2, pb, &pp))) {
         return rc;

@@ -12,7 +12,9 @@
 #include <stdlib.h>
 #include <string.h>
 
+#include <algorithm>
 #include <mutex>
+#include <vector>
 
 static thread_local char g_err[1024] = "";
 
@@ -33,7 +35,12 @@ struct hfx_ctx {
     size_t scratch_bytes[HFX_SCRATCH_SLOTS];
     void *pinned;
     size_t pinned_bytes;
+    uint32_t spare_users; /* calls that hold spare slots now; g_ctx_mu */
 };
+
+/* the contexts there are, and their spare_users */
+static std::mutex g_ctx_mu;
+static std::vector<hfx_ctx *> g_ctxs;
 
 extern "C" int hfx_ctx_create(int device, hfx_ctx **out)
 {
@@ -45,6 +52,10 @@ extern "C" int hfx_ctx_create(int device, hfx_ctx **out)
     HFX_REQUIRE(c != nullptr, HFX_ERR_NOMEM, "hfx_ctx_create: out of host memory");
     c->device = device;
     c->num_cus = prop.multiProcessorCount;
+    {
+        std::lock_guard<std::mutex> lk(g_ctx_mu);
+        g_ctxs.push_back(c);
+    }
     *out = c;
     return HFX_OK;
 }
@@ -52,6 +63,10 @@ extern "C" int hfx_ctx_create(int device, hfx_ctx **out)
 extern "C" int hfx_ctx_destroy(hfx_ctx *ctx)
 {
     if (!ctx) return HFX_OK;
+    {
+        std::lock_guard<std::mutex> lk(g_ctx_mu);
+        g_ctxs.erase(std::remove(g_ctxs.begin(), g_ctxs.end(), ctx), g_ctxs.end());
+    }
     for (int i = 0; i < HFX_SCRATCH_SLOTS; ++i)
         if (ctx->scratch[i]) (void)hipFree(ctx->scratch[i]);
     if (ctx->pinned) (void)hipHostFree(ctx->pinned);
@@ -72,7 +87,7 @@ int hfx_ctx_scratch(hfx_ctx *ctx, int slot, size_t bytes, void **out)
         }
         size_t sz = bytes + bytes / 4;
         sz = (sz + 255) & ~(size_t)255;
-        hipError_t e = hipMalloc(&ctx->scratch[slot], sz);
+        hipError_t e = hfx_device_malloc(&ctx->scratch[slot], sz);
         if (e != hipSuccess) {
             ctx->scratch[slot] = nullptr;
             hfx_set_error("scratch allocation of %zu bytes failed: %s", sz, hipGetErrorString(e));
@@ -95,14 +110,61 @@ void *hfx_ctx_scratch_spare(hfx_ctx *ctx, int slot, size_t bytes, void *stream)
         (void)hipGetLastError();
         return nullptr;
     }
-    const size_t sz = bytes + bytes / 4 + 256; /* what hfx_ctx_scratch allocates */
-    if (sz > tot / 8 || sz > (fr + ctx->scratch_bytes[slot]) / 2) return nullptr;
-    void *p = nullptr;
-    if (hfx_ctx_scratch(ctx, slot, bytes, &p) != HFX_OK) {
+    if (bytes > tot / 8 || bytes > (fr + ctx->scratch_bytes[slot]) / 2) return nullptr;
+    if (ctx->scratch[slot]) {
+        if (hipDeviceSynchronize() != hipSuccess || hipFree(ctx->scratch[slot]) != hipSuccess) {
+            (void)hipGetLastError();
+            return nullptr;
+        }
+        ctx->scratch[slot] = nullptr;
+        ctx->scratch_bytes[slot] = 0;
+    }
+    if (hipMalloc(&ctx->scratch[slot], bytes) != hipSuccess) {
+        ctx->scratch[slot] = nullptr;
         (void)hipGetLastError();
         return nullptr;
     }
-    return p;
+    ctx->scratch_bytes[slot] = bytes;
+    return ctx->scratch[slot];
+}
+
+void hfx_ctx_spare_begin(hfx_ctx *ctx)
+{
+    std::lock_guard<std::mutex> lk(g_ctx_mu);
+    ++ctx->spare_users;
+}
+void hfx_ctx_spare_end(hfx_ctx *ctx)
+{
+    std::lock_guard<std::mutex> lk(g_ctx_mu);
+    --ctx->spare_users;
+}
+
+bool hfx_spare_release(void)
+{
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess) return false;
+    bool any = hfx_rowsets_release(dev);
+    std::lock_guard<std::mutex> lk(g_ctx_mu);
+    for (hfx_ctx *c : g_ctxs) {
+        if (c->device != dev || c->spare_users) continue;
+        for (int slot : {HFX_SLOT_ROWS, HFX_SLOT_ROWS2}) {
+            if (!c->scratch[slot]) continue;
+            (void)hipDeviceSynchronize(); /* work launched with it */
+            (void)hipFree(c->scratch[slot]);
+            c->scratch[slot] = nullptr;
+            c->scratch_bytes[slot] = 0;
+            any = true;
+        }
+    }
+    return any;
+}
+
+hipError_t hfx_device_malloc(void **p, size_t bytes)
+{
+    hipError_t e = hipMalloc(p, bytes);
+    if (e != hipErrorOutOfMemory) return e;
+    (void)hipGetLastError();
+    return hfx_spare_release() ? hipMalloc(p, bytes) : e;
 }
 
 int hfx_ctx_pinned(hfx_ctx *ctx, size_t bytes, void **out)
@@ -141,7 +203,7 @@ hfx_ctx *hfx_default_ctx(void)
 extern "C" int hfx_malloc(void **d_ptr, size_t bytes)
 {
     HFX_REQUIRE(d_ptr != nullptr, HFX_ERR_ARG, "hfx_malloc: null out");
-    hipError_t e = hipMalloc(d_ptr, bytes ? bytes : 1);
+    hipError_t e = hfx_device_malloc(d_ptr, bytes ? bytes : 1);
     if (e != hipSuccess) {
         hfx_set_error("hfx_malloc(%zu): %s", bytes, hipGetErrorString(e));
         return HFX_ERR_NOMEM;

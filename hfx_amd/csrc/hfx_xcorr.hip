@@ -408,6 +408,12 @@ static int xcorr_rows(hfx_ctx *ctx, float *d_scores, const uint64_t *d_off,
                       const hfx_db *db, const hfx_spectra *sp, void *stream, int *taken)
 {
     *taken = 0;
+    /* the buffers are this call's until its work is launched */
+    struct Spare {
+        hfx_ctx *c;
+        explicit Spare(hfx_ctx *ctx) : c(ctx) { hfx_ctx_spare_begin(c); }
+        ~Spare() { hfx_ctx_spare_end(c); }
+    } spare(ctx);
     const uint32_t S = sp->num_spec;
     const uint32_t nt = hfx_rows_tiles(db->num_pep), G = hfx_rows_groups(sp->x_stride);
     if (!xr_pays(total, nt) || sp->x_stride > RW_MAXK || db->num_pep == 0) return HFX_OK;
