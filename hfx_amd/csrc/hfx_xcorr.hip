@@ -67,27 +67,29 @@ static size_t xp_lds_bytes(uint32_t xstr)
 }
 
 /* claims the peaks of one position (clearing them) and adds weight * x of
- * every nibble it receives (clamped peaks sit on zero spectrum values) */
-__device__ __forceinline__ float xp_claim(const XpPeaks &pk, const float *xsm, float acc)
+ * every nibble it receives (clamped peaks sit on zero spectrum values), those of
+ * the b ion's side and of the y ion's to sums of their own: shorter sums round
+ * less */
+__device__ __forceinline__ void xp_claim(const XpPeaks &pk, const float *xsm, float (&acc)[2])
 {
 #pragma unroll
     for (int i = 0; i < 6; ++i) {
         const uint32_t sh = pk.sh[i];
+        float &s = acc[i >= 4];
         if (i == 1 || i == 4) {
             const uint64_t t = (uint64_t)0xfffu << sh;
             const uint32_t o0 = atomicAnd(pk.w[i], ~(uint32_t)t);
             const uint32_t o1 = atomicAnd(pk.w[i] + 1, ~(uint32_t)(t >> 32));
             const uint32_t f = (uint32_t)(((uint64_t)o1 << 32 | o0) >> sh);
             const float *xv = xsm + pk.u[i];
-            acc = __builtin_fmaf(xp_weight(f & 15u), xv[0], acc);
-            acc = __builtin_fmaf(xp_weight((f >> 4) & 15u), xv[1], acc);
-            acc = __builtin_fmaf(xp_weight((f >> 8) & 15u), xv[2], acc);
+            s = __builtin_fmaf(xp_weight(f & 15u), xv[0], s);
+            s = __builtin_fmaf(xp_weight((f >> 4) & 15u), xv[1], s);
+            s = __builtin_fmaf(xp_weight((f >> 8) & 15u), xv[2], s);
         } else {
             const uint32_t old = atomicAnd(pk.w[i], ~(0xfu << sh));
-            acc = __builtin_fmaf(xp_weight((old >> sh) & 15u), xsm[pk.u[i]], acc);
+            s = __builtin_fmaf(xp_weight((old >> sh) & 15u), xsm[pk.u[i]], s);
         }
     }
-    return acc;
 }
 
 /* the value of the lane before (0 in lane 0) */
@@ -141,7 +143,7 @@ __device__ __forceinline__ void xp_pack(uint32_t *maps, uint32_t mstr, const flo
     /* charges 1..Z: the bins of each (and, for Z <= 2, their words and
      * shifts) kept in registers from the OR pass to the claim pass */
     uint32_t xz[Z][6];
-    float acc = 0.0f;
+    float acc[2] = {0.0f, 0.0f};
     if constexpr (Z <= 2) {
         XpPeaks pks[Z];
         if (act) {
@@ -154,7 +156,7 @@ __device__ __forceinline__ void xp_pack(uint32_t *maps, uint32_t mstr, const flo
         hfx_wave_sync();
         if (act) {
 #pragma unroll
-            for (int z = 0; z < Z; ++z) acc = xp_claim(pks[z], xsm, acc);
+            for (int z = 0; z < Z; ++z) xp_claim(pks[z], xsm, acc);
         }
     } else {
         if (act) {
@@ -175,11 +177,11 @@ __device__ __forceinline__ void xp_pack(uint32_t *maps, uint32_t mstr, const flo
             for (int z = 0; z < Z; ++z) {
                 XpPeaks pk;
                 xp_locate(rowm, xz[z], pk);
-                acc = xp_claim(pk, xsm, acc);
+                xp_claim(pk, xsm, acc);
             }
         }
     }
-    const float sc = xp_segsum(acc, kpos, lane);
+    const float sc = xp_segsum(acc[0] + acc[1], kpos, lane);
     hfx_wave_sync();
     /* the last lane of each candidate holds its score; a candidate without
      * positions scores 0 */
