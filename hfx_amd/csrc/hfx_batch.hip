@@ -794,9 +794,11 @@ __global__ void __launch_bounds__(CUT_WG) k_cut_seg(uint32_t *seg_cuts, uint32_t
 
 /* bstart[0 .. nb) = the segments' block starts in order, bstart[nb .. cap]
  * = S (empty blocks), nb = seg_off[nseg] */
-__global__ void k_cut_place(uint32_t *bstart, const uint32_t *seg_cuts, const uint32_t *seg_n,
+/* also clears a word for what follows, if asked to */
+__global__ void k_cut_place(uint32_t *clear, uint32_t *bstart, const uint32_t *seg_cuts, const uint32_t *seg_n,
                             const uint64_t *seg_off, uint32_t nseg, uint32_t cap, uint32_t S)
 {
+    if (clear && blockIdx.x == 0 && threadIdx.x == 0) *clear = 0;
     const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
     const uint32_t seg = t / CUT_SEG, i = t % CUT_SEG;
     if (seg < nseg && i < seg_n[seg]) bstart[seg_off[seg] + i] = seg_cuts[t];
@@ -850,7 +852,7 @@ int hfx_cut_blocks(hfx_ctx *ctx, uint32_t ns, const hfx_cut_bufs *c, const uint3
     int rc;
     if ((rc = hfx_scan_offsets(ctx, c->off, c->n, nseg, stream))) return rc;
     const uint32_t nt = std::max(nseg * CUT_SEG, S + 1);
-    hipLaunchKernelGGL(k_cut_place, dim3((nt + 255) / 256), dim3(256), 0, st, c->bstart, c->seg,
+    hipLaunchKernelGGL(k_cut_place, dim3((nt + 255) / 256), dim3(256), 0, st, c->clear, c->bstart, c->seg,
                        c->n, c->off, nseg, S, S);
     HFX_CHECK_LAUNCH();
     return HFX_OK;
@@ -894,7 +896,8 @@ struct hfx_batch {
     bool rows_tried, use_rows; /* scores come from the database's rows */
     RowSet *rs;                /* the set they are in, and what this batch reads of it */
     hfx_rows rows;
-    uint32_t *rw_small;  /* rows: [S] sum and max of |x|, [3][S] quanta, levels, wide marks */
+    uint32_t have;             /* the highest charge level of those rows */
+    uint32_t *rw_small;  /* rows: [S] sum and max of |x|, [S] quanta, [S] levels, the rest's list */
     hipGraph_t graph;
     hipGraphExec_t exec;
 };
@@ -1128,12 +1131,13 @@ static int bt_ready(hfx_batch *b, hipStream_t st)
     b->rs = pepix_use_rows(const_cast<hfx_pepix *>(b->ix), b->L, (uint32_t)hfx_ctx_num_cus(b->ctx),
                            st, &b->rows);
     if (!b->rs) return HFX_OK;
-    if (bt_dense_alloc(b) || (!b->rw_small && dalloc(&b->rw_small, 5 * (size_t)b->S))) {
+    if (bt_dense_alloc(b) || (!b->rw_small && dalloc(&b->rw_small, 5 * (size_t)b->S + 1))) {
         (void)hipGetLastError();
         bt_rows_drop(b);
         b->rows_tried = true;
         return HFX_OK;
     }
+    for (b->have = 0; b->have < HFX_MAX_CHARGE && b->rows.rows[b->have];) ++b->have;
     b->use_rows = true;
     return HFX_OK;
 }
@@ -1364,11 +1368,14 @@ static int bt_mode(const hfx_batch *b)
                                                     : RW_I8X4;
 }
 /* dn_scratch as the rows route carves it: planes | item bookkeeping; norms,
- * quanta, levels and wide marks in rw_small */
+ * quanta, levels and the list of the rest in rw_small */
 static float2 *bt_norms(const hfx_batch *b) { return (float2 *)b->rw_small; }
 static float *bt_quanta(const hfx_batch *b) { return (float *)(b->rw_small + 2 * (size_t)b->S); }
 static uint32_t *bt_levels(const hfx_batch *b) { return b->rw_small + 3 * (size_t)b->S; }
-static uint32_t *bt_wide(const hfx_batch *b) { return b->rw_small + 4 * (size_t)b->S; }
+static hfx_rest bt_rest(const hfx_batch *b)
+{
+    return {b->rw_small + 4 * (size_t)b->S, b->rw_small + 5 * (size_t)b->S};
+}
 static uint8_t *bt_planes(const hfx_batch *b) { return b->dn_scratch; }
 static void *bt_items(const hfx_batch *b)
 {
@@ -1380,14 +1387,15 @@ static void *bt_items(const hfx_batch *b)
 static int bt_dense_prep(hfx_batch *b, hipStream_t st)
 {
     const bool bf = b->precision == HFX_BATCH_BF16X2_DENSE;
-    const hfx_cut_bufs c{b->cut_seg, b->cut_n, b->cut_off, b->dn_bstart};
+    const hfx_rest rest = bt_rest(b);
+    const hfx_cut_bufs c{b->cut_seg, b->cut_n, b->cut_off, b->dn_bstart, b->use_rows ? rest.count : nullptr};
     int rc;
     if ((rc = hfx_cut_blocks(b->ctx, bf ? 8u : 16u, &c, b->order, b->begin, b->num, b->sp.d_zmax,
                              b->S, (void *)st)))
         return rc;
     if (b->use_rows) {
-        return hfx_rows_split(bt_mode(b), &b->sp, bt_planes(b), bt_quanta(b), bt_levels(b),
-                              bt_wide(b), bt_norms(b), b->scores, b->score_off, (void *)st);
+        return hfx_rows_split(bt_mode(b), &b->sp, bt_planes(b), bt_quanta(b), bt_levels(b), &rest,
+                              b->have, bt_norms(b), b->scores, b->score_off, (void *)st);
     }
     return bf ? hfx_dense_split(&b->sp, b->dn_scratch, (void *)st)
               : hfx_dense8_split(&b->sp, b->dn_scratch, (void *)st);
@@ -1443,24 +1451,26 @@ static int bt_score(hfx_batch *b, hipStream_t st, void **ev)
     return HFX_OK;
 }
 
-/* scores from the index's rows, in the current precision */
+/* scores from the database's rows, in the current precision; the spectra that these do
+ * not serve -- a charge above those the plan's spectra had, or, in the FP32 form, values
+ * that the digits do not hold -- by sums within the form's bound */
 static int bt_row_scores(hfx_batch *b, hipStream_t st, void **ev)
 {
     if (b->total == 0) return HFX_OK;
     const int mode = bt_mode(b);
     const float *qs = bt_quanta(b);
     hfx_spectra sq = b->sp;
-    if (mode == RW_I8X4) sq.d_zmax = bt_levels(b); /* wide spectra hidden */
+    sq.d_zmax = bt_levels(b); /* the rest hidden */
+    const hfx_rest rest = bt_rest(b);
     int rc;
-    if ((rc = hfx_rows_blocks(b->ctx, mode, bt_items(b), b->order, b->dn_bstart, b->begin, b->num,
-                              &sq, b->CH, (void *)st)) ||
+    if ((rc = hfx_rows_blocks(b->ctx, bt_items(b), b->order, b->dn_bstart, b->begin, b->num, &sq,
+                              b->CH, (void *)st)) ||
         (rc = hfx_rows_scores(b->ctx, mode, bt_items(b), b->scores, b->score_off, b->begin, b->num,
                               b->order, b->dn_bstart, &b->rows, bt_planes(b), qs, &sq, b->CH,
                               (void *)st, ev)))
         return rc;
-    if (mode != RW_I8X4) return HFX_OK;
-    return hfx_xcorr_wide(b->ctx, b->scores, b->score_off, b->begin, b->num, &b->db, &b->sp,
-                          bt_wide(b), (void *)st);
+    return hfx_xcorr_rest(b->ctx, b->scores, b->score_off, b->begin, b->num, &b->db, &b->sp, &rest,
+                          mode != RW_I8X4, (void *)st);
 }
 
 /* ev (optional): events recorded around the scoring kernel itself */

@@ -173,11 +173,13 @@ int hfx_dense8_scores(hfx_ctx *ctx, float *d_scores, const uint64_t *d_off,
                       const uint32_t *d_bstart, uint32_t nblocks, const hfx_dn_ladder *lad,
                       const hfx_spectra *sp, uint32_t CH, void *scratch, int presplit,
                       void *stream, void **ev);
-/* FP32 scores of the unmodified candidates of the spectra with wide[s] != 0
- * (hfx_xcorr_sparse's kernel, no scratch) */
-int hfx_xcorr_wide(hfx_ctx *ctx, float *d_scores, const uint64_t *d_off, const uint32_t *d_begin,
+/* scores of the unmodified candidates of the listed spectra, without rows or
+ * scratch: the FP32 sums of hfx_xcorr_sparse's packed kernel, or sums in FP64
+ * rounded once to FP32 (within every form's bound) */
+struct hfx_rest;
+int hfx_xcorr_rest(hfx_ctx *ctx, float *d_scores, const uint64_t *d_off, const uint32_t *d_begin,
                    const uint32_t *d_num, const hfx_db *db, const hfx_spectra *sp,
-                   const uint32_t *wide, void *stream);
+                   const hfx_rest *rest, int fp64, void *stream);
 /* ev (optional): two hipEvent_t recorded right before and after the
  * contraction kernel itself */
 int hfx_dense_scores(hfx_ctx *ctx, float *d_scores, const uint64_t *d_off, const uint32_t *d_begin,
@@ -345,13 +347,14 @@ __device__ __forceinline__ void hfx_wave_peaks_z(uint32_t *map, uint32_t n, floa
     }
 }
 
-/* Dot of the map with the LDS spectrum, FP32, clearing the map as it goes.
- * Lane l scans words l, l+64, ... (conflict-free), bins ascending. */
-__device__ __forceinline__ float hfx_wave_dot_f32(uint32_t *map, const float *xs, uint32_t len)
+/* Dot of the map with the LDS spectrum in A (float or double), clearing the map as
+ * it goes.  Lane l scans words l, l+64, ... (conflict-free), bins ascending. */
+template <class A>
+__device__ __forceinline__ A hfx_wave_dot(uint32_t *map, const float *xs, uint32_t len)
 {
     const uint32_t lane = hfx_lane();
     const uint32_t nw = (len + 7) >> 3;
-    float acc = 0.0f;
+    A acc = 0;
     for (uint32_t w = lane; w < nw; w += HFX_WAVE) {
         uint32_t word = map[w];
         if (word) {
@@ -360,38 +363,13 @@ __device__ __forceinline__ float hfx_wave_dot_f32(uint32_t *map, const float *xs
                 uint32_t sh = __builtin_ctz(word) & ~3u;
                 uint32_t nib = (word >> sh) & 0xFu;
                 word &= ~(0xFu << sh);
-                acc = acc + hfx_code_weight(nib) * xs[(w << 3) + (sh >> 2)];
+                acc = acc + (A)hfx_code_weight(nib) * (A)xs[(w << 3) + (sh >> 2)];
             }
         }
     }
-    return hfx_wave_sum_f32(acc);
-}
-
-/* FP32 and exact dots of the map in one pass, clearing it. */
-__device__ __forceinline__ void hfx_wave_dot_both(uint32_t *map, const float *xs, uint32_t len,
-                                                  float *f32_out, int64_t *fx_out)
-{
-    const uint32_t lane = hfx_lane();
-    const uint32_t nw = (len + 7) >> 3;
-    float acc = 0.0f;
-    int64_t fx = 0;
-    for (uint32_t w = lane; w < nw; w += HFX_WAVE) {
-        uint32_t word = map[w];
-        if (word) {
-            map[w] = 0;
-            while (word) {
-                uint32_t sh = __builtin_ctz(word) & ~3u;
-                uint32_t nib = (word >> sh) & 0xFu;
-                word &= ~(0xFu << sh);
-                const float wt = hfx_code_weight(nib);
-                const float xv = xs[(w << 3) + (sh >> 2)];
-                acc = acc + wt * xv;
-                fx += hfx_fx_term(wt, xv);
-            }
-        }
-    }
-    *f32_out = hfx_wave_sum_f32(acc);
-    *fx_out = hfx_wave_sum_i64(fx);
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) acc += __shfl_xor(acc, o, 64);
+    return acc;
 }
 
 /* Exact (fixed-point) dot of the map with the LDS spectrum, clearing it. */

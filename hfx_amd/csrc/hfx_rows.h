@@ -31,12 +31,18 @@ struct hfx_rows {
 uint32_t hfx_rows_tiles(uint32_t num_pep);
 uint32_t hfx_rows_groups(uint32_t x_stride);
 uint32_t hfx_rows_chunk(uint64_t rows, uint32_t cus);
-/* planes [S][RW_PLANES][RW_MAXK] and quanta of the spectra; RW_I8X4 also
- * writes each spectrum's charge level to lvl, or to wide where its digits would
- * lose precision (0 in the other); norms [S], if any: sum and max of |x|.  Scores of spectra whose charge is not
+/* spectra that are scored without rows (hfx_xcorr_rest), in any order */
+struct hfx_rest {
+    uint32_t *list, *count; /* [S]; cleared before hfx_rows_split (hfx_cut_bufs) */
+};
+/* planes [S][RW_PLANES][RW_MAXK] and quanta of the spectra, and the charge level of
+ * each, 0 for those put on the list `rest`: charges above `have`, the highest level
+ * there are rows for; in RW_I8X4 spectra whose digits would lose precision.  norms
+ * [S], if any: sum and max of |x|.  The num[s] scores of spectra whose charge is not
  * generated are set to 0 */
 int hfx_rows_split(int mode, const hfx_spectra *sp, uint8_t *planes, float *qs, uint32_t *lvl,
-                   uint32_t *wide, float2 *norms, float *scores, const uint64_t *off, void *stream);
+                   const hfx_rest *rest, uint32_t have, float2 *norms, float *scores,
+                   const uint64_t *off, void *stream);
 /* writes the rows of the wanted levels (non-null) and tiles (flags
  * [HFX_MAX_CHARGE][ntiles], null: all) */
 int hfx_rows_build(uint32_t cus, const hfx_db *db, const hfx_rows *r, const uint32_t *flags,
@@ -44,9 +50,9 @@ int hfx_rows_build(uint32_t cus, const hfx_db *db, const hfx_rows *r, const uint
 /* work items of the blocks bstart (num_spec + 1 entries, empty blocks at the
  * end) of CH candidates each, in scratch of hfx_rows_items_bytes(num_spec) */
 size_t hfx_rows_items_bytes(uint32_t S);
-int hfx_rows_blocks(hfx_ctx *ctx, int mode, void *scratch, const uint32_t *order,
-                    const uint32_t *bstart, const uint32_t *begin, const uint32_t *num,
-                    const hfx_spectra *sp, uint32_t CH, void *stream);
+int hfx_rows_blocks(hfx_ctx *ctx, void *scratch, const uint32_t *order, const uint32_t *bstart,
+                    const uint32_t *begin, const uint32_t *num, const hfx_spectra *sp, uint32_t CH,
+                    void *stream);
 /* flags [HFX_MAX_CHARGE][ntiles]: the tiles those items read */
 int hfx_rows_mark(void *scratch, uint32_t S, uint32_t *flags, uint32_t ntiles, void *stream);
 /* the scores of every item (sp's d_zmax may hide spectra from them) */
@@ -70,6 +76,7 @@ struct hfx_cut_bufs {
     uint32_t *seg, *n; /* [hfx_cut_segs(S) * 32], [hfx_cut_segs(S)] */
     uint64_t *off;     /* [hfx_cut_segs(S) + 1] */
     uint32_t *bstart;  /* [S + 1] */
+    uint32_t *clear;   /* a word cleared on the way, if any */
 };
 uint32_t hfx_cut_segs(uint32_t S);
 /* blocks of at most ns (8 or 16) consecutive ordered spectra */

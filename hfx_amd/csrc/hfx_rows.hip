@@ -79,12 +79,14 @@ __device__ __forceinline__ uint32_t rw_bf16(float f)
 /* planes[s][plane][RW_MAXK]: byte 64 ks + 16 kg + j of a digit plane is the
  * digit of bin 64 ks + rw_bin_of(kg, j); the BF16 planes (hi of bytes j < 8,
  * hi of j >= 8, lo, lo) hold eight BF16 in the 16 bytes of a k-group.
- * qs[s] = 2^-k.  norms (if any): sum and max of |x|.  lvl (RW_I8X4): the fragment charge of the spectra the digits
- * serve, 0 for wide ones (their charge goes to wide[s] instead). */
+ * qs[s] = 2^-k.  norms (if any): sum and max of |x|.  A spectrum whose charge has no
+ * rows (above `have`; a later one than those a batch was planned with) or, in the
+ * FP32 form, one that the digits do not serve goes to the list `rest`, and its
+ * lvl[s] is 0; the others' lvl[s] is their fragment charge. */
 template <int MODE>
 __global__ void __launch_bounds__(256)
-    k_rw_split(uint8_t *planes, float *qs, uint32_t *lvl, uint32_t *wide, float2 *norms,
-               float *scores, const uint64_t *off, hfx_spectra sp)
+    k_rw_split(uint8_t *planes, float *qs, uint32_t *lvl, hfx_rest rest, uint32_t have,
+               float2 *norms, float *scores, const uint64_t *off, hfx_spectra sp)
 {
     constexpr uint32_t NP = RW_PLANES(MODE);
     __shared__ float red[2][256 / HFX_WAVE];
@@ -93,7 +95,8 @@ __global__ void __launch_bounds__(256)
     const uint32_t len = min(sp.d_len[s], min(sp.x_stride, (uint32_t)RW_MAXK));
     const float *x = sp.d_x + (size_t)s * sp.x_stride;
     /* spectra whose fragment charge is not generated score 0 */
-    if (hfx_zeff(sp.d_zmax[s]) == 0)
+    const uint32_t z = hfx_zeff(sp.d_zmax[s]);
+    if (z == 0)
         for (uint64_t i = off[s] + tid; i < off[s + 1]; i += 256) scores[i] = 0.0f;
     /* thread t takes the four bins of words t + 256 u (bytes 4 w .. 4 w + 3) */
     constexpr uint32_t NW = RW_MAXK / 4, NU = (NW + 255) / 256;
@@ -128,6 +131,12 @@ __global__ void __launch_bounds__(256)
     m = fmaxf(fmaxf(red[0][0], red[0][1]), fmaxf(red[0][2], red[0][3]));
     x1 = red[1][0] + red[1][1] + red[1][2] + red[1][3];
     if (tid == 0 && norms) norms[s] = make_float2(x1, m);
+    const bool out = z > have || (MODE == RW_I8X4 && (bad || !(x1 >= m * (float)len * (1.0f / 4096.0f))));
+    if (tid == 0) {
+        lvl[s] = out ? 0u : z;
+        if (out && z) rest.list[atomicAdd(rest.count, 1u)] = s;
+    }
+    if (out) return; /* its planes are read into no score */
     uint8_t *o = planes + (size_t)s * NP * RW_MAXK;
     if constexpr (MODE == RW_BF16) {
 #pragma unroll
@@ -153,9 +162,8 @@ __global__ void __launch_bounds__(256)
      * the largest value the digits reach; at most 126 */
     constexpr int B = MODE == RW_I8X4 ? 31 : 23;
     constexpr float XMAX = MODE == RW_I8X4 ? 2139062143.0f : 8355711.0f;
-    const bool w4 = MODE == RW_I8X4 && (bad || !(x1 >= m * (float)len * (1.0f / 4096.0f)));
     int k = 0;
-    if (m > 0.0f && !w4) {
+    if (m > 0.0f) {
         const int e = (int)((__float_as_uint(m) >> 23) & 255u) - 127;
         k = B - 1 - e;
         if (k > 126) k = 126;
@@ -163,15 +171,7 @@ __global__ void __launch_bounds__(256)
         else if (ldexpf(m, k) >= XMAX && (MODE == RW_I8X4 || ldexpf(m, k) > XMAX)) --k;
     }
     const float sc = ldexpf(1.0f, k);
-    if (tid == 0) {
-        qs[s] = ldexpf(1.0f, -k);
-        if constexpr (MODE == RW_I8X4) {
-            const uint32_t z = hfx_zeff(sp.d_zmax[s]);
-            lvl[s] = w4 ? 0u : z;
-            wide[s] = w4 ? z : 0u;
-        }
-    }
-    if (w4) return; /* its planes are never read into a score */
+    if (tid == 0) qs[s] = ldexpf(1.0f, -k);
 #pragma unroll
     for (uint32_t u = 0; u < NU; ++u) {
         const uint32_t t = tid + 256 * u;
@@ -862,15 +862,17 @@ uint32_t hfx_rows_chunk(uint64_t rows, uint32_t cus)
 }
 
 int hfx_rows_split(int mode, const hfx_spectra *sp, uint8_t *planes, float *qs, uint32_t *lvl,
-                   uint32_t *wide, float2 *norms, float *scores, const uint64_t *off, void *stream)
+                   const hfx_rest *rest, uint32_t have, float2 *norms, float *scores,
+                   const uint64_t *off, void *stream)
 {
     HFX_REQUIRE(sp->x_stride <= RW_MAXK, HFX_ERR_ARG, "rows: spectra of up to %d bins", RW_MAXK);
     if (sp->num_spec == 0) return HFX_OK;
     const dim3 g(sp->num_spec), t(256);
     hipStream_t st = hfx_stream(stream);
-    if (mode == RW_I8X3) hipLaunchKernelGGL(k_rw_split<RW_I8X3>, g, t, 0, st, planes, qs, lvl, wide, norms, scores, off, *sp);
-    else if (mode == RW_I8X4) hipLaunchKernelGGL(k_rw_split<RW_I8X4>, g, t, 0, st, planes, qs, lvl, wide, norms, scores, off, *sp);
-    else hipLaunchKernelGGL(k_rw_split<RW_BF16>, g, t, 0, st, planes, qs, lvl, wide, norms, scores, off, *sp);
+    const auto kernel = mode == RW_I8X3   ? k_rw_split<RW_I8X3>
+                        : mode == RW_I8X4 ? k_rw_split<RW_I8X4>
+                                          : k_rw_split<RW_BF16>;
+    hipLaunchKernelGGL(kernel, g, t, 0, st, planes, qs, lvl, *rest, have, norms, scores, off, *sp);
     HFX_CHECK_LAUNCH();
     return HFX_OK;
 }
@@ -907,9 +909,9 @@ static void rw_items(void *p, uint32_t S, uint32_t **tbeg, uint32_t **tend, uint
     *counter = *items + S;
 }
 
-int hfx_rows_blocks(hfx_ctx *ctx, int mode, void *scratch, const uint32_t *order,
-                    const uint32_t *bstart, const uint32_t *begin, const uint32_t *num,
-                    const hfx_spectra *sp, uint32_t CH, void *stream)
+int hfx_rows_blocks(hfx_ctx *ctx, void *scratch, const uint32_t *order, const uint32_t *bstart,
+                    const uint32_t *begin, const uint32_t *num, const hfx_spectra *sp, uint32_t CH,
+                    void *stream)
 {
     const uint32_t B = sp->num_spec;
     uint32_t *tbeg, *tend, *binfo, *items, *counter;
@@ -917,7 +919,6 @@ int hfx_rows_blocks(hfx_ctx *ctx, int mode, void *scratch, const uint32_t *order
     rw_items(scratch, B, &tbeg, &tend, &binfo, &items, &off, &counter);
     hipStream_t st = hfx_stream(stream);
     const uint32_t CT = std::max(CH / RW_ROWS, 1u);
-    (void)mode;
     hipLaunchKernelGGL(k_rw_blocks, dim3((B + 15) / 16), dim3(256), 0, st, tbeg, tend, binfo, items,
                        counter, order, bstart, begin, num, *sp, B, CT);
     int rc = hfx_scan_offsets(ctx, off, items, B, stream);

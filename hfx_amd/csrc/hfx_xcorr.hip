@@ -70,24 +70,29 @@ static size_t xp_lds_bytes(uint32_t xstr)
  * every nibble it receives (clamped peaks sit on zero spectrum values), those of
  * the b ion's side and of the y ion's to sums of their own: shorter sums round
  * less */
-__device__ __forceinline__ void xp_claim(const XpPeaks &pk, const float *xsm, float (&acc)[2])
+template <class A>
+__device__ __forceinline__ void xp_claim(const XpPeaks &pk, const float *xsm, A (&acc)[2])
 {
+    auto add = [](uint32_t nib, float x, A &sum) {
+        if constexpr (sizeof(A) == 8) sum = __builtin_fma((double)xp_weight(nib), (double)x, sum);
+        else sum = __builtin_fmaf(xp_weight(nib), x, sum);
+    };
 #pragma unroll
     for (int i = 0; i < 6; ++i) {
         const uint32_t sh = pk.sh[i];
-        float &s = acc[i >= 4];
+        A &s = acc[i >= 4];
         if (i == 1 || i == 4) {
             const uint64_t t = (uint64_t)0xfffu << sh;
             const uint32_t o0 = atomicAnd(pk.w[i], ~(uint32_t)t);
             const uint32_t o1 = atomicAnd(pk.w[i] + 1, ~(uint32_t)(t >> 32));
             const uint32_t f = (uint32_t)(((uint64_t)o1 << 32 | o0) >> sh);
             const float *xv = xsm + pk.u[i];
-            s = __builtin_fmaf(xp_weight(f & 15u), xv[0], s);
-            s = __builtin_fmaf(xp_weight((f >> 4) & 15u), xv[1], s);
-            s = __builtin_fmaf(xp_weight((f >> 8) & 15u), xv[2], s);
+            add(f & 15u, xv[0], s);
+            add((f >> 4) & 15u, xv[1], s);
+            add((f >> 8) & 15u, xv[2], s);
         } else {
             const uint32_t old = atomicAnd(pk.w[i], ~(0xfu << sh));
-            s = __builtin_fmaf(xp_weight((old >> sh) & 15u), xsm[pk.u[i]], s);
+            add((old >> sh) & 15u, xsm[pk.u[i]], s);
         }
     }
 }
@@ -99,30 +104,51 @@ __device__ __forceinline__ float xp_prev(float v)
                                                                  0x138 /* wave_shr:1 */, 0xf, 0xf, false));
 }
 
+__device__ __forceinline__ double xp_prev(double v)
+{
+    const uint64_t u = (uint64_t)__double_as_longlong(v);
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)u, 0x138, 0xf, 0xf, false);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(u >> 32), 0x138, 0xf, 0xf, false);
+    return __longlong_as_double((long long)((uint64_t)hi << 32 | lo));
+}
+/* lane l's value, l a lane's own (any, where l is not one) */
+__device__ __forceinline__ float xp_from(float v, uint32_t l)
+{
+    return __uint_as_float((uint32_t)__builtin_amdgcn_ds_bpermute((int)(l << 2), (int)__float_as_uint(v)));
+}
+__device__ __forceinline__ double xp_from(double v, uint32_t l)
+{
+    const uint64_t u = (uint64_t)__double_as_longlong(v);
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_ds_bpermute((int)(l << 2), (int)(uint32_t)u);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_ds_bpermute((int)(l << 2), (int)(uint32_t)(u >> 32));
+    return __longlong_as_double((long long)((uint64_t)hi << 32 | lo));
+}
+
 /* Inclusive segmented sum over the wave: lane l ends with the sum of the lanes of
  * its segment from the segment's first lane (kpos = 0) to l, by doubling steps
  * taken where kpos reaches back that far: the order of the additions is that of the
  * candidate's positions alone, so that a score has the same bits wherever its
  * candidate lies in a pack. */
-__device__ __forceinline__ float xp_segsum(float v, uint32_t kpos, uint32_t lane)
+template <class A>
+__device__ __forceinline__ A xp_segsum(A v, uint32_t kpos, uint32_t lane)
 {
 #pragma unroll
     for (uint32_t o = 1; o < HFX_WAVE; o <<= 1) {
-        float t = v;
+        A t = v;
         if (o <= 4) {
 #pragma unroll
             for (uint32_t i = 0; i < o; ++i) t = xp_prev(t);
         } else {
-            t = __uint_as_float((uint32_t)__builtin_amdgcn_ds_bpermute((int)((lane - o) << 2),
-                                                                       (int)__float_as_uint(v)));
+            t = xp_from(v, lane - o);
         }
         v = kpos >= o ? v + t : v;
     }
     return v;
 }
 
-/* one pack at fragment charges 1..Z; the candidates' b ladders are in lb */
-template <int Z>
+/* one pack at fragment charges 1..Z; the candidates' b ladders are in lb; sums in
+ * A (float, or double rounded once) */
+template <int Z, class A>
 __device__ __forceinline__ void xp_pack(uint32_t *maps, uint32_t mstr, const float *xs,
                                         const float *lb, uint32_t len, const XpPack pk,
                                         float *out)
@@ -143,7 +169,7 @@ __device__ __forceinline__ void xp_pack(uint32_t *maps, uint32_t mstr, const flo
     /* charges 1..Z: the bins of each (and, for Z <= 2, their words and
      * shifts) kept in registers from the OR pass to the claim pass */
     uint32_t xz[Z][6];
-    float acc[2] = {0.0f, 0.0f};
+    A acc[2] = {0, 0};
     if constexpr (Z <= 2) {
         XpPeaks pks[Z];
         if (act) {
@@ -181,7 +207,7 @@ __device__ __forceinline__ void xp_pack(uint32_t *maps, uint32_t mstr, const flo
             }
         }
     }
-    const float sc = xp_segsum(acc[0] + acc[1], kpos, lane);
+    const float sc = (float)xp_segsum(acc[0] + acc[1], kpos, lane);
     hfx_wave_sync();
     /* the last lane of each candidate holds its score; a candidate without
      * positions scores 0 */
@@ -196,7 +222,7 @@ __device__ __forceinline__ void xp_pack(uint32_t *maps, uint32_t mstr, const flo
 
 /* the tile of spectrum s from its candidate `first` on; every thread of the
  * workgroup calls it */
-template <class Cands>
+template <class A, class Cands>
 __device__ __forceinline__ void xp_tile(float *xp_lds, float *mtab, float *scores, const Cands &c,
                                         const hfx_spectra &sp, uint32_t mstr, uint32_t s,
                                         uint32_t first, uint32_t chunk)
@@ -256,7 +282,7 @@ __device__ __forceinline__ void xp_tile(float *xp_lds, float *mtab, float *score
                 const typename Cands::Prep qq = Cands::take(pr, p);
                 c.peaks_prep(maps + XP_PAD / 8, mtab, qq, len, zeff);
                 hfx_wave_sync();
-                const float sc = hfx_wave_dot_f32(maps + XP_PAD / 8, xs, len);
+                const float sc = (float)hfx_wave_dot<A>(maps + XP_PAD / 8, xs, len);
                 hfx_wave_sync();
                 if (lane == 0) out[p] = sc;
                 ++p;
@@ -264,10 +290,10 @@ __device__ __forceinline__ void xp_tile(float *xp_lds, float *mtab, float *score
             }
             const XpPack pk = xp_form(p, q, pr.n, pr.r, pofs, base);
             switch (zeff) {
-            case 1: xp_pack<1>(maps, mstr, xs, lb, len, pk, out + p); break;
-            case 2: xp_pack<2>(maps, mstr, xs, lb, len, pk, out + p); break;
-            case 3: xp_pack<3>(maps, mstr, xs, lb, len, pk, out + p); break;
-            default: xp_pack<4>(maps, mstr, xs, lb, len, pk, out + p); break;
+            case 1: xp_pack<1, A>(maps, mstr, xs, lb, len, pk, out + p); break;
+            case 2: xp_pack<2, A>(maps, mstr, xs, lb, len, pk, out + p); break;
+            case 3: xp_pack<3, A>(maps, mstr, xs, lb, len, pk, out + p); break;
+            default: xp_pack<4, A>(maps, mstr, xs, lb, len, pk, out + p); break;
             }
             p += pk.K;
         }
@@ -286,36 +312,29 @@ __global__ void __launch_bounds__(XP_THREADS)
     const uint64_t t = blockIdx.x;
     if (t >= tile_off[S]) return;
     const uint32_t s = find_segment(tile_off, S, t);
-    xp_tile(xp_lds, mtab, scores, c, sp, mstr, s, (uint32_t)(t - tile_off[s]) * chunk, chunk);
+    xp_tile<float>(xp_lds, mtab, scores, c, sp, mstr, s, (uint32_t)(t - tile_off[s]) * chunk, chunk);
 }
 
-/* The spectra marked in wide (seldom any), a workgroup each at a time: the
- * workgroups look at XP_THREADS spectra a step and walk the tiles of those
- * marked. */
+/* The spectra that have no rows, or not in their form (seldom any: then a launch that
+ * reads one word): persistent workgroups take every G-th of their tiles, of XR_CHUNK
+ * candidates, so that one spectrum's window is spread over the chip. */
+#define XR_CHUNK 32
+template <class A>
 __global__ void __launch_bounds__(XP_THREADS)
-    k_xcorr_wide(float *scores, HfxPlainCands c, hfx_spectra sp, const uint32_t *wide,
-                 uint32_t mstr)
+    k_xcorr_rest(float *scores, HfxPlainCands c, hfx_spectra sp, hfx_rest rest, uint32_t mstr)
 {
     extern __shared__ __align__(16) float xp_lds[];
     __shared__ float mtab[HFX_MTAB];
-    __shared__ uint64_t marked[XP_WAVES];
-    const uint32_t S = sp.num_spec, G = gridDim.x;
-    /* this workgroup's spectra are blockIdx.x + k G, k = 0, 1, ... */
-    for (uint64_t k0 = 0; blockIdx.x + k0 * G < S; k0 += XP_THREADS) {
-        const uint64_t mine = blockIdx.x + (k0 + threadIdx.x) * G;
-        const uint64_t bal = __ballot(mine < S && wide[mine] != 0u);
-        if (hfx_lane() == 0) marked[threadIdx.x / HFX_WAVE] = bal;
-        __syncthreads();
-        for (uint32_t w = 0; w < XP_WAVES; ++w)
-            for (uint64_t m = marked[w]; m; m &= m - 1ull) {
-                const uint32_t s = (uint32_t)(blockIdx.x + (k0 + w * HFX_WAVE +
-                                                            (uint32_t)__builtin_ctzll(m)) * G);
-                for (uint32_t f = 0; f < c.count(s); f += XP_CHUNK) {
-                    xp_tile(xp_lds, mtab, scores, c, sp, mstr, s, f, XP_CHUNK);
-                    __syncthreads(); /* its LDS is staged anew */
-                }
-            }
-        __syncthreads();
+    const uint32_t F = *rest.count;
+    uint64_t at = blockIdx.x; /* of the tiles from the j-th spectrum on */
+    for (uint32_t j = 0; j < F; ++j) {
+        const uint32_t s = rest.list[j];
+        const uint32_t nt = c.count(s) / XR_CHUNK + (c.count(s) % XR_CHUNK ? 1u : 0u);
+        for (; at < nt; at += gridDim.x) {
+            xp_tile<A>(xp_lds, mtab, scores, c, sp, mstr, s, (uint32_t)at * XR_CHUNK, XR_CHUNK);
+            __syncthreads(); /* its LDS is staged anew */
+        }
+        at -= nt;
     }
 }
 
@@ -368,16 +387,16 @@ static int launch_xcorr(void *scratch, float *d_scores, const Cands &c, uint64_t
     return HFX_OK;
 }
 
-int hfx_xcorr_wide(hfx_ctx *ctx, float *d_scores, const uint64_t *d_off, const uint32_t *d_begin,
+int hfx_xcorr_rest(hfx_ctx *ctx, float *d_scores, const uint64_t *d_off, const uint32_t *d_begin,
                    const uint32_t *d_num, const hfx_db *db, const hfx_spectra *sp,
-                   const uint32_t *wide, void *stream)
+                   const hfx_rest *rest, int fp64, void *stream)
 {
-    const uint32_t S = sp->num_spec;
-    if (S == 0) return HFX_OK;
+    if (sp->num_spec == 0) return HFX_OK;
     HfxPlainCands c{*db, d_begin, d_num, d_off};
-    hipLaunchKernelGGL(k_xcorr_wide, dim3(min(S, (uint32_t)hfx_ctx_num_cus(ctx) * 4u)),
-                       dim3(XP_THREADS), xp_lds_bytes(sp->x_stride), hfx_stream(stream), d_scores, c,
-                       *sp, wide, xp_map_words(sp->x_stride));
+    hipLaunchKernelGGL(fp64 ? k_xcorr_rest<double> : k_xcorr_rest<float>,
+                       dim3((uint32_t)hfx_ctx_num_cus(ctx) * 4u), dim3(XP_THREADS),
+                       xp_lds_bytes(sp->x_stride), hfx_stream(stream), d_scores, c, *sp, *rest,
+                       xp_map_words(sp->x_stride));
     HFX_CHECK_LAUNCH();
     return HFX_OK;
 }
@@ -428,7 +447,7 @@ static int xcorr_rows(hfx_ctx *ctx, float *d_scores, const uint64_t *d_off,
     const uint32_t nseg = hfx_cut_segs(S);
     auto al = [](uint64_t n) { return (n + 255) & ~(uint64_t)255; };
     const uint64_t sizes[] = {
-        al((uint64_t)S * RW_PLANES(RW_I8X4) * RW_MAXK), al(4ull * S), al(4ull * S), al(4ull * S),
+        al((uint64_t)S * RW_PLANES(RW_I8X4) * RW_MAXK), al(4ull * S), al(4ull * S), al(4ull * S + 4),
         al(4ull * S), al(4ull * ob.nb), al(4ull * S), al(8ull * ob.nb + 8), al(4ull * nseg * 32),
         al(4ull * nseg), al(8ull * nseg + 8), al(4ull * S + 4), al(hfx_rows_items_bytes(S)),
         al(4 * nf), al(8 * nf + 8), al(nt + 4ull)};
@@ -445,12 +464,13 @@ static int xcorr_rows(hfx_ctx *ctx, float *d_scores, const uint64_t *d_off,
     }
     uint8_t *planes = part[0];
     float *qs = (float *)part[1];
-    uint32_t *lvl = (uint32_t *)part[2], *wide = (uint32_t *)part[3], *order = (uint32_t *)part[4];
+    uint32_t *lvl = (uint32_t *)part[2], *order = (uint32_t *)part[4];
+    const hfx_rest rest{(uint32_t *)part[3], (uint32_t *)part[3] + S};
     ob.cnt = (uint32_t *)part[5];
     ob.tmp = (uint32_t *)part[6];
     ob.off = (uint64_t *)part[7];
     const hfx_cut_bufs cb{(uint32_t *)part[8], (uint32_t *)part[9], (uint64_t *)part[10],
-                          (uint32_t *)part[11]};
+                          (uint32_t *)part[11], rest.count};
     void *items = part[12];
     uint32_t *flags = (uint32_t *)part[13];
     hfx_rows r{};
@@ -460,21 +480,21 @@ static int xcorr_rows(hfx_ctx *ctx, float *d_scores, const uint64_t *d_off,
     r.G = G;
     for (int l = 0; l < HFX_MAX_CHARGE; ++l) r.rows[l] = rows;
     hfx_spectra sq = *sp;
-    sq.d_zmax = lvl; /* wide spectra hidden from the items */
+    sq.d_zmax = lvl; /* the rest hidden from the items */
     const uint64_t est = max(total / 12, min(total, 2ull * db->num_pep));
     const uint32_t CH = hfx_rows_chunk(est, (uint32_t)hfx_ctx_num_cus(ctx));
     int rc;
-    if ((rc = hfx_rows_split(RW_I8X4, sp, planes, qs, lvl, wide, nullptr, d_scores, d_off, stream)) ||
-        (rc = hfx_order_spectra(ctx, order, &ob, d_begin, sp->d_zmax, sp->d_mass, S, stream)) ||
+    if ((rc = hfx_order_spectra(ctx, order, &ob, d_begin, sp->d_zmax, sp->d_mass, S, stream)) ||
         (rc = hfx_cut_blocks(ctx, 16, &cb, order, d_begin, d_num, sp->d_zmax, S, stream)) ||
-        (rc = hfx_rows_blocks(ctx, RW_I8X4, items, order, cb.bstart, d_begin, d_num, &sq, CH,
-                              stream)) ||
+        (rc = hfx_rows_split(RW_I8X4, sp, planes, qs, lvl, &rest, HFX_MAX_CHARGE, nullptr, d_scores,
+                             d_off, stream)) ||
+        (rc = hfx_rows_blocks(ctx, items, order, cb.bstart, d_begin, d_num, &sq, CH, stream)) ||
         (rc = hfx_rows_mark(items, S, flags, nt, stream)) ||
         (rc = hfx_scan_offsets(ctx, (uint64_t *)r.slots, flags, (uint32_t)nf, stream)) ||
         (rc = hfx_rows_build((uint32_t)hfx_ctx_num_cus(ctx), db, &r, flags, stream)) ||
         (rc = hfx_rows_scores(ctx, RW_I8X4, items, d_scores, d_off, d_begin, d_num, order,
                               cb.bstart, &r, planes, qs, &sq, CH, stream, nullptr)) ||
-        (rc = hfx_xcorr_wide(ctx, d_scores, d_off, d_begin, d_num, db, sp, wide, stream)))
+        (rc = hfx_xcorr_rest(ctx, d_scores, d_off, d_begin, d_num, db, sp, &rest, 0, stream)))
         return rc;
     *taken = 1;
     return HFX_OK;
