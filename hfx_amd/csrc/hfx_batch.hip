@@ -1395,7 +1395,7 @@ static int bt_dense_prep(hfx_batch *b, hipStream_t st)
         return rc;
     if (b->use_rows) {
         return hfx_rows_split(bt_mode(b), &b->sp, bt_planes(b), bt_quanta(b), bt_levels(b), &rest,
-                              b->have, bt_norms(b), b->scores, b->score_off, (void *)st);
+                              b->have, bt_norms(b), b->scores, b->score_off, b->num, (void *)st);
     }
     return bf ? hfx_dense_split(&b->sp, b->dn_scratch, (void *)st)
               : hfx_dense8_split(&b->sp, b->dn_scratch, (void *)st);

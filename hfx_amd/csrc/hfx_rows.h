@@ -39,10 +39,10 @@ struct hfx_rest {
  * each, 0 for those put on the list `rest`: charges above `have`, the highest level
  * there are rows for; in RW_I8X4 spectra whose digits would lose precision.  norms
  * [S], if any: sum and max of |x|.  The num[s] scores of spectra whose charge is not
- * generated are set to 0 */
+ * generated are set to 0, and nothing between one spectrum's scores and the next's */
 int hfx_rows_split(int mode, const hfx_spectra *sp, uint8_t *planes, float *qs, uint32_t *lvl,
                    const hfx_rest *rest, uint32_t have, float2 *norms, float *scores,
-                   const uint64_t *off, void *stream);
+                   const uint64_t *off, const uint32_t *num, void *stream);
 /* writes the rows of the wanted levels (non-null) and tiles (flags
  * [HFX_MAX_CHARGE][ntiles], null: all) */
 int hfx_rows_build(uint32_t cus, const hfx_db *db, const hfx_rows *r, const uint32_t *flags,

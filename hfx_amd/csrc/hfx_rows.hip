@@ -86,7 +86,8 @@ __device__ __forceinline__ uint32_t rw_bf16(float f)
 template <int MODE>
 __global__ void __launch_bounds__(256)
     k_rw_split(uint8_t *planes, float *qs, uint32_t *lvl, hfx_rest rest, uint32_t have,
-               float2 *norms, float *scores, const uint64_t *off, hfx_spectra sp)
+               float2 *norms, float *scores, const uint64_t *off, const uint32_t *num,
+               hfx_spectra sp)
 {
     constexpr uint32_t NP = RW_PLANES(MODE);
     __shared__ float red[2][256 / HFX_WAVE];
@@ -97,7 +98,7 @@ __global__ void __launch_bounds__(256)
     /* spectra whose fragment charge is not generated score 0 */
     const uint32_t z = hfx_zeff(sp.d_zmax[s]);
     if (z == 0)
-        for (uint64_t i = off[s] + tid; i < off[s + 1]; i += 256) scores[i] = 0.0f;
+        for (uint32_t i = tid; i < num[s]; i += 256) scores[off[s] + i] = 0.0f;
     /* thread t takes the four bins of words t + 256 u (bytes 4 w .. 4 w + 3) */
     constexpr uint32_t NW = RW_MAXK / 4, NU = (NW + 255) / 256;
     float v[NU][4];
@@ -863,7 +864,7 @@ uint32_t hfx_rows_chunk(uint64_t rows, uint32_t cus)
 
 int hfx_rows_split(int mode, const hfx_spectra *sp, uint8_t *planes, float *qs, uint32_t *lvl,
                    const hfx_rest *rest, uint32_t have, float2 *norms, float *scores,
-                   const uint64_t *off, void *stream)
+                   const uint64_t *off, const uint32_t *num, void *stream)
 {
     HFX_REQUIRE(sp->x_stride <= RW_MAXK, HFX_ERR_ARG, "rows: spectra of up to %d bins", RW_MAXK);
     if (sp->num_spec == 0) return HFX_OK;
@@ -872,7 +873,7 @@ int hfx_rows_split(int mode, const hfx_spectra *sp, uint8_t *planes, float *qs, 
     const auto kernel = mode == RW_I8X3   ? k_rw_split<RW_I8X3>
                         : mode == RW_I8X4 ? k_rw_split<RW_I8X4>
                                           : k_rw_split<RW_BF16>;
-    hipLaunchKernelGGL(kernel, g, t, 0, st, planes, qs, lvl, *rest, have, norms, scores, off, *sp);
+    hipLaunchKernelGGL(kernel, g, t, 0, st, planes, qs, lvl, *rest, have, norms, scores, off, num, *sp);
     HFX_CHECK_LAUNCH();
     return HFX_OK;
 }
