@@ -631,11 +631,14 @@ extern "C" int hfx_pepix_info(const hfx_pepix *ix, uint64_t *info /*[6]*/)
 /* Spectra are ordered by (fragment charge level, precursor mass, index):
  * bucket = level * nbz + (window begin >> sh) -- the window's first
  * residual-sorted position is a monotone function of the precursor mass --
- * counted, scattered, then ranked inside each bucket by (mass, index). */
+ * counted, scattered, then ranked inside each bucket by (mass, index).  Without
+ * masses the window's begin takes their place.  Any input gives a permutation: the
+ * begin of an empty window, which nothing else reads, may be anything, and masses
+ * that are NaN come last. */
 __device__ __forceinline__ uint32_t ord_bucket(uint32_t s, const uint32_t *begin,
                                                const uint32_t *zmax, uint32_t sh, uint32_t nbz)
 {
-    return hfx_zeff(zmax[s]) * nbz + (begin[s] >> sh);
+    return hfx_zeff(zmax[s]) * nbz + min(begin[s] >> sh, nbz - 1u);
 }
 
 __global__ void k_ord_count(uint32_t *cnt, const uint32_t *begin, const uint32_t *zmax, uint32_t S,
@@ -665,12 +668,16 @@ __global__ void k_ord_rank(uint32_t *order, const uint32_t *tmp, const uint64_t 
     const uint32_t s = tmp[i];
     const uint32_t k = ord_bucket(s, begin, zmax, sh, nbz);
     const uint32_t a = (uint32_t)boff[k], e = (uint32_t)boff[k + 1];
-    const float ms = mass[s];
+    auto key = [&](uint32_t t) {
+        if (!mass) return begin[t];
+        const float m = mass[t] + 0.0f; /* -0 as 0 */
+        return m == m ? hfx_f2key(m) : 0xffffffffu;
+    };
+    const uint32_t ks = key(s);
     uint32_t rank = 0;
     for (uint32_t j = a; j < e; ++j) {
-        const uint32_t t = tmp[j];
-        const float mt = mass[t];
-        rank += (mt < ms || (mt == ms && t < s)) ? 1u : 0u;
+        const uint32_t t = tmp[j], kt = key(t);
+        rank += (kt < ks || (kt == ks && t < s)) ? 1u : 0u;
     }
     order[a + rank] = s;
 }

@@ -68,7 +68,8 @@ struct hfx_order_bufs {
     uint64_t *off;        /* [nb + 1] */
 };
 void hfx_order_shape(uint32_t S, uint32_t num_pep, hfx_order_bufs *o);
-/* order: (fragment charge level, precursor mass, index) */
+/* order: (fragment charge level, precursor mass, or window begin where mass is
+ * null, index); a permutation whatever begin and mass hold */
 int hfx_order_spectra(hfx_ctx *ctx, uint32_t *order, const hfx_order_bufs *o,
                       const uint32_t *begin, const uint32_t *zmax, const float *mass, uint32_t S,
                       void *stream);

@@ -484,7 +484,7 @@ static int xcorr_rows(hfx_ctx *ctx, float *d_scores, const uint64_t *d_off,
     const uint64_t est = max(total / 12, min(total, 2ull * db->num_pep));
     const uint32_t CH = hfx_rows_chunk(est, (uint32_t)hfx_ctx_num_cus(ctx));
     int rc;
-    if ((rc = hfx_order_spectra(ctx, order, &ob, d_begin, sp->d_zmax, sp->d_mass, S, stream)) ||
+    if ((rc = hfx_order_spectra(ctx, order, &ob, d_begin, sp->d_zmax, nullptr, S, stream)) ||
         (rc = hfx_cut_blocks(ctx, 16, &cb, order, d_begin, d_num, sp->d_zmax, S, stream)) ||
         (rc = hfx_rows_split(RW_I8X4, sp, planes, qs, lvl, &rest, HFX_MAX_CHARGE, nullptr, d_scores,
                              d_off, d_num, stream)) ||

@@ -22,7 +22,7 @@ def search(orc):
     return hdb, x, lens, zmax, mass, ref, exact, scale
 
 
-@pytest.mark.parametrize("what", ["gaps"])
+@pytest.mark.parametrize("what", ["no masses", "any begin", "gaps"])
 def test_sparse_through_rows_reads_only_what_it_is_given(search, what):
     from hfx_amd import HfxSpectra, check as ok, lib
     from hfx_amd import pipeline as pl
@@ -52,3 +52,24 @@ def test_sparse_through_rows_reads_only_what_it_is_given(search, what):
     rest = np.ones(len(got), bool)
     rest[mine] = False
     assert (got[rest] == 12345.0).all()
+
+
+def test_batch_with_masses_that_are_not_numbers(search, orc):
+    from hfx_amd import pipeline as pl
+
+    hdb, x, lens, zmax, mass, *_ = search
+    x, lens, zmax, mass = x[:200], lens[:200], zmax[:200], mass[:200].copy()
+    bs = {}
+    for name, odd in (("nan", np.nan), ("empty", -5000.0)):
+        mass[::3] = odd
+        b = bs[name] = pl.BatchSearch(pl.Ctx(0), pl.DeviceDB(hdb), Spectra(pl, x, lens, zmax, mass), 3.0, 5)
+        b.run()
+        assert sorted(b.order()) == list(range(200))
+    # every window but those of NaN, whose two bounds are where the search leaves them
+    ref, exact, scale = reference(orc, hdb, x, lens, zmax, mass, 5)
+    check(orc, bs["empty"].results(keep_scores=True), ref, exact, scale, x, *FORMS["fp32"])
+    got, want = bs["nan"].results(), bs["empty"].results()
+    keep = np.arange(200) % 3 != 0
+    for a, b in ((got.top_pos, want.top_pos), (got.top_exact, want.top_exact)):
+        live = keep[:, None] & (np.arange(5) < want.top_cnt[:, None])
+        assert (a[live] == b[live]).all()
