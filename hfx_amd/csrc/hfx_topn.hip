@@ -706,8 +706,7 @@ __device__ __forceinline__ void fx_scores(const FxWave &f, uint32_t mstr, const 
 }
 
 /* exact scores of the listed candidates: wave w takes the first o.task of
- * spectrum w, then all waves share the spilled tasks.  fx: [base(s) + i] for
- * candidate i of s's list. */
+ * spectrum w, then all waves share the spilled tasks.  fx: [s][TN_MAXC]. */
 template <class Cands>
 __global__ void __launch_bounds__(TN_THREADS)
     k_topn_exact(int64_t *fx, TnLists o, Cands c, hfx_spectra sp, uint32_t mstr)
@@ -726,7 +725,7 @@ __global__ void __launch_bounds__(TN_THREADS)
         typename Cands::Prep pr{};
         if (lane < rn) pr = c.prep(s, o.cand[(size_t)s * TN_MAXC + k0 + lane]);
         const uint32_t len = min(sp.d_len[s], min(sp.x_stride, (uint32_t)HFX_MAX_LEN));
-        int64_t *out = fx + c.base(s) + k0;
+        int64_t *out = fx + (size_t)s * TN_MAXC + k0;
         const float *x = sp.d_x + (size_t)s * sp.x_stride;
         const uint32_t zeff = c.zeff(sp.d_zmax[s]);
         auto emit = [&](uint32_t i, int64_t v) { out[i] = v; };
@@ -749,9 +748,10 @@ __global__ void __launch_bounds__(TN_THREADS)
 #define TX_LIVE 32
 
 /* the exact route's work: the flagged spectra (in any order), their number, the
- * first tile of each (off[number] = all tiles) */
+ * first tile of each (off[number] = all tiles), and the place of each one's exact
+ * scores (a sum of window sizes, wherever the spectra's own scores lie) */
 struct TxPlan {
-    uint64_t *off;
+    uint64_t *off, *at;
     uint32_t *list, *count;
 };
 
@@ -762,7 +762,7 @@ __device__ void tx_plan(TxPlan p, const uint32_t *flag, const uint32_t *band, co
                         uint32_t S)
 {
     __shared__ uint32_t nl;
-    __shared__ uint64_t wt[TN_THREADS / HFX_WAVE];
+    __shared__ uint64_t wt[TN_THREADS / HFX_WAVE], wa[TN_THREADS / HFX_WAVE];
     const uint32_t lane = hfx_lane(), wave = threadIdx.x / HFX_WAVE;
     if (threadIdx.x == 0) nl = 0;
     __syncthreads();
@@ -777,28 +777,42 @@ __device__ void tx_plan(TxPlan p, const uint32_t *flag, const uint32_t *band, co
     }
     __syncthreads(); /* the list is this workgroup's own: visible to it from here */
     const uint32_t F = nl;
-    uint64_t nt = 0;
+    uint64_t nt = 0, na = 0;
     for (uint32_t q0 = 0; q0 < F; q0 += TN_THREADS) {
         const uint32_t q = q0 + threadIdx.x;
-        uint64_t t = 0;
+        uint64_t t = 0, n = 0;
         if (q < F) {
-            const uint32_t s = p.list[q], n = c.count(s), b = min(band[s], n);
-            t = max((n + TX_CHUNK - 1) / TX_CHUNK, (b + TX_LIVE - 1) / TX_LIVE);
+            const uint32_t s = p.list[q], b = min(band[s], c.count(s));
+            n = c.count(s);
+            t = max((n + TX_CHUNK - 1) / TX_CHUNK, ((uint64_t)b + TX_LIVE - 1) / TX_LIVE);
         }
-        uint64_t x = t;
+        uint64_t x = t, y = n;
 #pragma unroll
         for (int o = 1; o < 64; o <<= 1) {
-            const uint64_t v = __shfl_up(x, o, 64);
-            if (lane >= (uint32_t)o) x += v;
+            const uint64_t v = __shfl_up(x, o, 64), u = __shfl_up(y, o, 64);
+            if (lane >= (uint32_t)o) {
+                x += v;
+                y += u;
+            }
         }
-        if (lane == HFX_WAVE - 1) wt[wave] = x;
+        if (lane == HFX_WAVE - 1) {
+            wt[wave] = x;
+            wa[wave] = y;
+        }
         __syncthreads();
-        uint64_t to = nt + x - t;
+        uint64_t to = nt + x - t, at = na + y - n;
         for (uint32_t w = 0; w < TN_THREADS / HFX_WAVE; ++w) {
-            if (w < wave) to += wt[w];
+            if (w < wave) {
+                to += wt[w];
+                at += wa[w];
+            }
             nt += wt[w];
+            na += wa[w];
         }
-        if (q < F) p.off[q] = to;
+        if (q < F) {
+            p.off[q] = to;
+            p.at[q] = at;
+        }
         __syncthreads();
     }
     if (threadIdx.x == 0) {
@@ -827,7 +841,7 @@ __global__ void __launch_bounds__(TN_THREADS)
     const uint32_t M = o.mcnt[s] & ~TN_BIG, n = c.count(s), outn = min(N, n);
     const float *sc = scores + c.base(s);
     const bool fl = M && flag[s] != 0u;
-    const int64_t *f = fx + c.base(s);
+    const int64_t *f = fx + (size_t)s * TN_MAXC;
     const uint32_t *p = o.cand + (size_t)s * TN_MAXC;
     auto put = [&](uint32_t rk, uint64_t k, uint32_t pos) {
         const double v = (double)(int64_t)(k ^ 0x8000000000000000ull) * (1.0 / HFX_FX_SCALE);
@@ -922,8 +936,8 @@ __global__ void k_mark_list(uint32_t *flag, double *tau, uint32_t *band, const u
  * spread over the tiles. */
 template <class Cands>
 __global__ void __launch_bounds__(TN_THREADS)
-    k_exact_tiles(int64_t *fxbuf, const uint64_t *tile_off, const uint32_t *list,
-                  const uint32_t *count, Cands c, hfx_spectra sp, const float *scores,
+    k_exact_tiles(int64_t *fxbuf, const uint64_t *tile_off, const uint64_t *fx_at,
+                  const uint32_t *list, const uint32_t *count, Cands c, hfx_spectra sp, const float *scores,
                   const double *tau, uint32_t mstr)
 {
     extern __shared__ __align__(16) unsigned char tn_dyn[];
@@ -954,13 +968,14 @@ __global__ void __launch_bounds__(TN_THREADS)
          * cannot reach the top N (its exact score is below the N-th exact
          * score): it keeps the smallest key, stored by its own lane.  The
          * others are moved to the first lanes and re-scored. */
-        const uint64_t tb = c.base(s);
+        const float *sc = scores + c.base(s);
+        int64_t *fx = fxbuf + fx_at[lo];
         const uint64_t mi64 = k + (uint64_t)nt * (wave + TN_WAVES * lane);
         const uint32_t mi = (uint32_t)mi64;
         bool live = false;
         if (wave + TN_WAVES * lane < TX_CHUNK && mi64 < n) {
-            live = !((double)scores[tb + mi] < ts);
-            if (!live) fxbuf[tb + mi] = INT64_MIN;
+            live = !((double)sc[mi] < ts);
+            if (!live) fx[mi] = INT64_MIN;
         }
         const uint64_t lm = __ballot(live);
         const uint32_t rn = (uint32_t)__builtin_popcountll(lm);
@@ -974,7 +989,7 @@ __global__ void __launch_bounds__(TN_THREADS)
         }
         fx_scores<true>(f, mstr, mtab, sp.d_x + (size_t)s * sp.x_stride, len,
                         c.zeff(sp.d_zmax[s]), c, pr, rn,
-                        [&](uint32_t i, int64_t v) { fxbuf[tb + lpos[wave][i]] = v; });
+                        [&](uint32_t i, int64_t v) { fx[lpos[wave][i]] = v; });
         hfx_wave_sync();
     }
 }
@@ -1006,7 +1021,7 @@ template <class Cands>
 __global__ void __launch_bounds__(FX_THREADS)
     k_topn_fx(uint32_t *top_pos, double *top_exact, float *top_f32, uint32_t *top_cnt,
               uint32_t *flag, uint32_t N, const uint32_t *list, const uint32_t *list_cnt,
-              const int64_t *fxbuf, const float *scores, Cands c)
+              const int64_t *fxbuf, const uint64_t *fx_at, const float *scores, Cands c)
 {
     __shared__ uint64_t lk[FX_CAP];
     __shared__ uint32_t lp[FX_CAP];
@@ -1022,7 +1037,7 @@ __global__ void __launch_bounds__(FX_THREADS)
     for (uint32_t q = blockIdx.x; q < F; q += gridDim.x) {
         const uint32_t s = list[q];
         const uint32_t n = c.count(s);
-        const int64_t *fx = fxbuf + c.base(s);
+        const int64_t *fx = fxbuf + fx_at[q];
         const float *sc = scores + c.base(s);
         uint32_t want = min(N, n);
         if (want == 0) {
@@ -1269,17 +1284,19 @@ __global__ void __launch_bounds__(FX_THREADS)
 /* ------------------------------------------------------------------ */
 
 /* scratch of a call:
- * fxbuf[total] | tile_off[S+1] | tau[S] | spill[S * TN_SPILL] | counters (256 B) |
- * list[S] | band[S] | mcnt[S] | cand[S][TN_MAXC] */
+ * fxbuf[total] | tile_off[S+1] | fx_at[S] | tau[S] | lfx[S][TN_MAXC] |
+ * spill[S * TN_SPILL] | counters (256 B) | list[S] | band[S] | mcnt[S] |
+ * cand[S][TN_MAXC].  No place follows the caller's score offsets, which may start
+ * anywhere and leave room between the spectra. */
 size_t hfx_topn_scratch_bytes(uint32_t S, uint64_t total)
 {
-    return total * 8 + ((size_t)S + 1) * 8 + (size_t)S * (8 + 8 * TN_SPILL) + 256 +
+    return total * 8 + ((size_t)S + 1) * 8 + (size_t)S * (16 + 8 * TN_MAXC + 8 * TN_SPILL) + 256 +
            (size_t)S * 4 * (3 + TN_MAXC);
 }
 
 struct TxScratch {
-    int64_t *fxbuf;
-    uint64_t *tile_off;
+    int64_t *fxbuf, *lfx;
+    uint64_t *tile_off, *fx_at;
     uint32_t *counter, *list; /* counter: spilled tasks, flagged spectra */
     TnLists l;
 };
@@ -1288,8 +1305,10 @@ static TxScratch tx_carve(void *p, uint32_t S, uint64_t total)
     TxScratch x;
     x.fxbuf = (int64_t *)p;
     x.tile_off = (uint64_t *)(x.fxbuf + total);
-    x.l.tau = (double *)(x.tile_off + S + 1);
-    x.l.spill = (uint2 *)(x.l.tau + S);
+    x.fx_at = x.tile_off + S + 1;
+    x.l.tau = (double *)(x.fx_at + S);
+    x.lfx = (int64_t *)(x.l.tau + S);
+    x.l.spill = (uint2 *)(x.lfx + (size_t)S * TN_MAXC);
     x.counter = (uint32_t *)(x.l.spill + (size_t)S * TN_SPILL);
     x.l.nspill = x.counter;
     x.list = x.counter + 64;
@@ -1299,7 +1318,7 @@ static TxScratch tx_carve(void *p, uint32_t S, uint64_t total)
     x.l.task = S <= TN_FEW ? TN_TASK_FEW : TN_TASK;
     return x;
 }
-static TxPlan tx_plan_of(const TxScratch &x) { return {x.tile_off, x.list, x.counter + 1}; }
+static TxPlan tx_plan_of(const TxScratch &x) { return {x.tile_off, x.fx_at, x.list, x.counter + 1}; }
 static int tx_scratch(hfx_ctx *ctx, void *given, uint32_t S, uint64_t total, void **out)
 {
     *out = given;
@@ -1324,11 +1343,11 @@ static int exact_route(hfx_ctx *ctx, uint32_t *d_top_pos, double *d_top_exact, f
         hipLaunchKernelGGL(k_tx_plan<Cands>, dim3(1), dim3(TN_THREADS), 0, st, tx_plan_of(x), d_flag,
                            x.l.band, c, S);
     hipLaunchKernelGGL(k_exact_tiles<Cands>, dim3((uint32_t)hfx_ctx_num_cus(ctx) * 4),
-                       dim3(TN_THREADS), fx_lds_bytes(sp->x_stride), st, x.fxbuf, x.tile_off, x.list,
-                       x.counter + 1, c, *sp, d_scores, x.l.tau, xp_map_words(sp->x_stride));
+                       dim3(TN_THREADS), fx_lds_bytes(sp->x_stride), st, x.fxbuf, x.tile_off, x.fx_at,
+                       x.list, x.counter + 1, c, *sp, d_scores, x.l.tau, xp_map_words(sp->x_stride));
     hipLaunchKernelGGL(k_topn_fx<Cands>, dim3(min(S, (uint32_t)hfx_ctx_num_cus(ctx))),
                        dim3(FX_THREADS), 0, st, d_top_pos, d_top_exact, d_top_f32, d_top_cnt,
-                       d_flag, N, x.list, x.counter + 1, x.fxbuf, d_scores, c);
+                       d_flag, N, x.list, x.counter + 1, x.fxbuf, x.fx_at, d_scores, c);
     HFX_CHECK_LAUNCH();
     return HFX_OK;
 }
@@ -1359,10 +1378,10 @@ static int launch_topn(hfx_ctx *ctx, uint32_t *d_top_pos, double *d_top_exact, f
                        margin, d_scores, c, *sp, rel0, rel1, relq, norms);
     /* at least four workgroups a CU: the spilled tasks spread over them */
     hipLaunchKernelGGL(k_topn_exact<Cands>, dim3(max(gw, 4u * (uint32_t)hfx_ctx_num_cus(ctx))),
-                       dim3(TN_THREADS), fx_lds_bytes(sp->x_stride), st, x.fxbuf, x.l, c, *sp,
+                       dim3(TN_THREADS), fx_lds_bytes(sp->x_stride), st, x.lfx, x.l, c, *sp,
                        xp_map_words(sp->x_stride));
     hipLaunchKernelGGL(k_topn_rank<Cands>, dim3(gw + 1), dim3(TN_THREADS), 0, st, d_top_pos,
-                       d_top_exact, d_top_f32, d_top_cnt, d_flag, N, x.fxbuf, x.l, d_scores, c, S,
+                       d_top_exact, d_top_f32, d_top_cnt, d_flag, N, x.lfx, x.l, d_scores, c, S,
                        tx_plan_of(x));
     HFX_CHECK_LAUNCH();
     return exact_route(ctx, d_top_pos, d_top_exact, d_top_f32, d_top_cnt, N, d_flag, d_scores, c,
