@@ -1294,6 +1294,9 @@ size_t hfx_topn_scratch_bytes(uint32_t S, uint64_t total)
            (size_t)S * 4 * (3 + TN_MAXC);
 }
 
+/* the bins of a row that are read, whatever its stride */
+static uint32_t tn_bins(const hfx_spectra *sp) { return min(sp->x_stride, (uint32_t)HFX_MAX_LEN); }
+
 struct TxScratch {
     int64_t *fxbuf, *lfx;
     uint64_t *tile_off, *fx_at;
@@ -1343,8 +1346,8 @@ static int exact_route(hfx_ctx *ctx, uint32_t *d_top_pos, double *d_top_exact, f
         hipLaunchKernelGGL(k_tx_plan<Cands>, dim3(1), dim3(TN_THREADS), 0, st, tx_plan_of(x), d_flag,
                            x.l.band, c, S);
     hipLaunchKernelGGL(k_exact_tiles<Cands>, dim3((uint32_t)hfx_ctx_num_cus(ctx) * 4),
-                       dim3(TN_THREADS), fx_lds_bytes(sp->x_stride), st, x.fxbuf, x.tile_off, x.fx_at,
-                       x.list, x.counter + 1, c, *sp, d_scores, x.l.tau, xp_map_words(sp->x_stride));
+                       dim3(TN_THREADS), fx_lds_bytes(tn_bins(sp)), st, x.fxbuf, x.tile_off, x.fx_at,
+                       x.list, x.counter + 1, c, *sp, d_scores, x.l.tau, xp_map_words(tn_bins(sp)));
     hipLaunchKernelGGL(k_topn_fx<Cands>, dim3(min(S, (uint32_t)hfx_ctx_num_cus(ctx))),
                        dim3(FX_THREADS), 0, st, d_top_pos, d_top_exact, d_top_f32, d_top_cnt,
                        d_flag, N, x.list, x.counter + 1, x.fxbuf, x.fx_at, d_scores, c);
@@ -1378,8 +1381,8 @@ static int launch_topn(hfx_ctx *ctx, uint32_t *d_top_pos, double *d_top_exact, f
                        margin, d_scores, c, *sp, rel0, rel1, relq, norms);
     /* at least four workgroups a CU: the spilled tasks spread over them */
     hipLaunchKernelGGL(k_topn_exact<Cands>, dim3(max(gw, 4u * (uint32_t)hfx_ctx_num_cus(ctx))),
-                       dim3(TN_THREADS), fx_lds_bytes(sp->x_stride), st, x.lfx, x.l, c, *sp,
-                       xp_map_words(sp->x_stride));
+                       dim3(TN_THREADS), fx_lds_bytes(tn_bins(sp)), st, x.lfx, x.l, c, *sp,
+                       xp_map_words(tn_bins(sp)));
     hipLaunchKernelGGL(k_topn_rank<Cands>, dim3(gw + 1), dim3(TN_THREADS), 0, st, d_top_pos,
                        d_top_exact, d_top_f32, d_top_cnt, d_flag, N, x.lfx, x.l, d_scores, c, S,
                        tx_plan_of(x));

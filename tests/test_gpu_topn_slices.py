@@ -1,5 +1,5 @@
 """hfx_topn over part of the spectra of a search, whose scores start past the first and leave room
-between the spectra."""
+between the spectra, and over rows whose stride passes the longest spectrum."""
 import ctypes as C
 
 import numpy as np
@@ -66,3 +66,15 @@ def test_part_of_a_search(env, orc, gap, rel0):
                    int(ref["num"][a:b].sum()), rel0)
         same(orc, got, ref, a, b)
         assert rel0 < 0.1 or b - a == 1 or got[3].any()   # some took the exact route
+
+
+def test_rows_of_a_longer_stride(env, orc):
+    pl, ctx, db, (x, lens, zmax, mass), ref, scores = env
+    long = np.zeros((len(x), 9000), np.float32)
+    long[:, :x.shape[1]] = x
+    sp = Spectra(pl, long, lens, zmax, mass)
+    t = [pl.dev(v) for v in (scores, ref["off"].astype(np.uint64), ref["begin"].astype(np.uint32),
+                             ref["num"].astype(np.uint32))]
+    for rel0 in (80 * 2.0**-24, 0.5):
+        got = topn(pl, ctx, db, sp.desc, len(x), [b.p for b in t], len(scores), rel0)
+        same(orc, got, ref, 0, len(x))
