@@ -904,6 +904,7 @@ struct hfx_batch {
     RowSet *rs;                /* the set they are in, and what this batch reads of it */
     hfx_rows rows;
     uint32_t have;             /* the highest charge level of those rows */
+    uint8_t *rw_planes;  /* rows, FP32 form: six digits of every spectrum | item bookkeeping */
     uint32_t *rw_small;  /* rows: [S] sum and max of |x|, [S] quanta, [S] levels, the rest's list */
     hipGraph_t graph;
     hipGraphExec_t exec;
@@ -927,7 +928,8 @@ static void bt_free(hfx_batch *b)
                   b->ntiles,   b->counter,   b->score_off, b->tile_off,  b->scores,
                   b->top_pos,  b->top_cnt,   b->flag,      b->top_exact, b->top_f32,
                   b->tx_scratch, b->ord_cnt, b->ord_tmp,   b->ord_off,   b->dn_scratch,
-                  b->dn_bstart, b->cut_seg,  b->cut_n,     b->cut_off,   b->rw_small};
+                  b->dn_bstart, b->cut_seg,  b->cut_n,     b->cut_off,   b->rw_small,
+                  b->rw_planes};
     for (void *p : ps)
         if (p) (void)hipFree(p);
     if (b->exec) (void)hipGraphExecDestroy(b->exec);
@@ -1118,15 +1120,29 @@ static int bt_need_index(hfx_batch *b, hipStream_t st)
     return HFX_OK;
 }
 
+static int bt_cut_alloc(hfx_batch *b);
 static int bt_dense_alloc(hfx_batch *b);
+/* the FP32 form's planes and work items */
+static size_t bt_planes_bytes(uint32_t S)
+{
+    return (size_t)S * RW_PLANES(RW_I8X6) * RW_MAXK + hfx_rows_items_bytes(S);
+}
 
-/* the index, and its rows where they fit (decided once a plan or index, never
+/* the current form's own buffers of the rows route are there */
+static bool bt_rows_bufs(const hfx_batch *b)
+{
+    return b->rw_small && (bt_is_dense(b->precision) ? b->dn_scratch : b->rw_planes);
+}
+/* the next scores come from rows */
+static bool bt_rows(const hfx_batch *b) { return b->use_rows && bt_rows_bufs(b); }
+
+/* the index, and its rows where they fit (decided once a plan, index and form, never
  * under capture: a batch captured by its caller without a run before it keeps
  * the other kernels) */
 static int bt_ready(hfx_batch *b, hipStream_t st)
 {
     int rc = bt_need_index(b, st);
-    if (rc || b->rows_tried || b->S == 0) return rc;
+    if (rc || b->S == 0 || (b->rows_tried && (!b->use_rows || bt_rows_bufs(b)))) return rc;
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
     HFX_CHECK_HIP(hipStreamIsCapturing(st, &cs));
     if (cs != hipStreamCaptureStatusNone) return HFX_OK;
@@ -1134,11 +1150,17 @@ static int bt_ready(hfx_batch *b, hipStream_t st)
     if (b->sp.x_stride > RW_MAXK || b->db.num_pep == 0) return HFX_OK;
     size_t fr = 0, tot = 0;
     HFX_CHECK_HIP(hipMemGetInfo(&fr, &tot));
-    if (!b->dn_scratch && (uint64_t)b->S * 16384 > fr / 4) return HFX_OK;
-    b->rs = pepix_use_rows(const_cast<hfx_pepix *>(b->ix), b->L, (uint32_t)hfx_ctx_num_cus(b->ctx),
+    if (!bt_rows_bufs(b) && (uint64_t)b->S * 16384 > fr / 4) {
+        bt_rows_drop(b);
+        b->rows_tried = true;
+        return HFX_OK;
+    }
+    if (!b->rs) b->rs = pepix_use_rows(const_cast<hfx_pepix *>(b->ix), b->L, (uint32_t)hfx_ctx_num_cus(b->ctx),
                            st, &b->rows);
     if (!b->rs) return HFX_OK;
-    if (bt_dense_alloc(b) || (!b->rw_small && dalloc(&b->rw_small, 5 * (size_t)b->S + 1))) {
+    if (bt_cut_alloc(b) || (!b->rw_small && dalloc(&b->rw_small, 5 * (size_t)b->S + 1)) ||
+        (bt_is_dense(b->precision) ? bt_dense_alloc(b)
+                                   : !b->rw_planes && dalloc(&b->rw_planes, bt_planes_bytes(b->S)))) {
         (void)hipGetLastError();
         bt_rows_drop(b);
         b->rows_tried = true;
@@ -1333,19 +1355,26 @@ extern "C" int hfx_batch_plan_ix(hfx_batch *b, const hfx_pepix *ix, const hfx_sp
     return hfx_batch_plan(b, &ix->db, sp, eps, N, margin, stream);
 }
 
+/* the block cut's buffers */
+static int bt_cut_alloc(hfx_batch *b)
+{
+    int rc;
+    b->nseg = (b->S + CUT_SEG - 1) / CUT_SEG;
+    if ((!b->dn_bstart && (rc = dalloc(&b->dn_bstart, (size_t)b->S + 1))) ||
+        (!b->cut_seg && (rc = dalloc(&b->cut_seg, (size_t)b->nseg * CUT_SEG))) ||
+        (!b->cut_n && (rc = dalloc(&b->cut_n, b->nseg))) ||
+        (!b->cut_off && (rc = dalloc(&b->cut_off, (size_t)b->nseg + 1))))
+        return rc;
+    return HFX_OK;
+}
+
 /* the dense form's per-batch buffers (hi/lo rows of every spectrum, block
  * bookkeeping), allocated when the form is first chosen */
 static int bt_dense_alloc(hfx_batch *b)
 {
-    if (b->dn_scratch) return HFX_OK;
-    int rc;
-    b->nseg = (b->S + CUT_SEG - 1) / CUT_SEG;
-    if ((rc = dalloc(&b->dn_scratch, bt_dense_scratch(b->S))) ||
-        (rc = dalloc(&b->dn_bstart, (size_t)b->S + 1)) ||
-        (rc = dalloc(&b->cut_seg, (size_t)b->nseg * CUT_SEG)) || (rc = dalloc(&b->cut_n, b->nseg)) ||
-        (rc = dalloc(&b->cut_off, (size_t)b->nseg + 1)))
-        return rc;
-    return HFX_OK;
+    const int rc = bt_cut_alloc(b);
+    if (rc || b->dn_scratch) return rc;
+    return dalloc(&b->dn_scratch, bt_dense_scratch(b->S));
 }
 
 /* ---- the phases of one batched search ---- */
@@ -1372,10 +1401,10 @@ static int bt_mode(const hfx_batch *b)
 {
     return b->precision == HFX_BATCH_I8X3_DENSE     ? RW_I8X3
            : b->precision == HFX_BATCH_BF16X2_DENSE ? RW_BF16
-                                                    : RW_I8X4;
+                                                    : RW_I8X6;
 }
-/* dn_scratch as the rows route carves it: planes | item bookkeeping; norms,
- * quanta, levels and the list of the rest in rw_small */
+/* dn_scratch (dense forms) or rw_planes as the rows route carves them: planes | item
+ * bookkeeping; norms, quanta, levels and the list of the rest in rw_small */
 static float2 *bt_norms(const hfx_batch *b) { return (float2 *)b->rw_small; }
 static float *bt_quanta(const hfx_batch *b) { return (float *)(b->rw_small + 2 * (size_t)b->S); }
 static uint32_t *bt_levels(const hfx_batch *b) { return b->rw_small + 3 * (size_t)b->S; }
@@ -1383,29 +1412,32 @@ static hfx_rest bt_rest(const hfx_batch *b)
 {
     return {b->rw_small + 4 * (size_t)b->S, b->rw_small + 5 * (size_t)b->S};
 }
-static uint8_t *bt_planes(const hfx_batch *b) { return b->dn_scratch; }
+static uint8_t *bt_planes(const hfx_batch *b)
+{
+    return bt_is_dense(b->precision) ? b->dn_scratch : b->rw_planes;
+}
 static void *bt_items(const hfx_batch *b)
 {
-    return b->dn_scratch + (size_t)b->S * 4 * RW_MAXK;
+    return bt_planes(b) + (size_t)b->S * (bt_is_dense(b->precision) ? 4 : RW_PLANES(RW_I8X6)) * RW_MAXK;
 }
 
-/* blocks (segment DP; eight spectra a block in the BF16 form, sixteen in the
+/* blocks (segment DP; sixteen spectra a block in the integer form, eight in the
  * others) and the spectra's hi/lo rows or digits */
 static int bt_dense_prep(hfx_batch *b, hipStream_t st)
 {
-    const bool bf = b->precision == HFX_BATCH_BF16X2_DENSE;
+    const bool i8 = b->precision == HFX_BATCH_I8X3_DENSE;
     const hfx_rest rest = bt_rest(b);
-    const hfx_cut_bufs c{b->cut_seg, b->cut_n, b->cut_off, b->dn_bstart, b->use_rows ? rest.count : nullptr};
+    const hfx_cut_bufs c{b->cut_seg, b->cut_n, b->cut_off, b->dn_bstart, bt_rows(b) ? rest.count : nullptr};
     int rc;
-    if ((rc = hfx_cut_blocks(b->ctx, bf ? 8u : 16u, &c, b->order, b->begin, b->num, b->sp.d_zmax,
+    if ((rc = hfx_cut_blocks(b->ctx, i8 ? 16u : 8u, &c, b->order, b->begin, b->num, b->sp.d_zmax,
                              b->S, (void *)st)))
         return rc;
-    if (b->use_rows) {
+    if (bt_rows(b)) {
         return hfx_rows_split(bt_mode(b), &b->sp, bt_planes(b), bt_quanta(b), bt_levels(b), &rest,
                               b->have, bt_norms(b), b->scores, b->score_off, b->num, (void *)st);
     }
-    return bf ? hfx_dense_split(&b->sp, b->dn_scratch, (void *)st)
-              : hfx_dense8_split(&b->sp, b->dn_scratch, (void *)st);
+    return i8 ? hfx_dense8_split(&b->sp, b->dn_scratch, (void *)st)
+              : hfx_dense_split(&b->sp, b->dn_scratch, (void *)st);
 }
 
 /* blocks of G spectra in order + tiles for the current (G, C) */
@@ -1422,7 +1454,7 @@ static int bt_prep(hfx_batch *b, hipStream_t st)
 {
     int rc;
     if ((rc = bt_order(b, st))) return rc;
-    if (b->use_rows || bt_is_dense(b->precision)) return bt_dense_prep(b, st);
+    if (bt_rows(b) || bt_is_dense(b->precision)) return bt_dense_prep(b, st);
     return bt_tiles(b, st);
 }
 
@@ -1477,13 +1509,13 @@ static int bt_row_scores(hfx_batch *b, hipStream_t st, void **ev)
                               (void *)st, ev)))
         return rc;
     return hfx_xcorr_rest(b->ctx, b->scores, b->score_off, b->begin, b->num, &b->db, &b->sp, &rest,
-                          mode != RW_I8X4, (void *)st);
+                          mode != RW_I8X6, (void *)st);
 }
 
 /* ev (optional): events recorded around the scoring kernel itself */
 static int bt_scores(hfx_batch *b, hipStream_t st, void **ev = nullptr)
 {
-    if (b->use_rows) return bt_row_scores(b, st, ev);
+    if (bt_rows(b)) return bt_row_scores(b, st, ev);
     if (b->precision == HFX_BATCH_I8X3_DENSE) {
         if (b->total == 0) return HFX_OK;
         return hfx_dense8_scores(b->ctx, b->scores, b->score_off, b->begin, b->num, b->order,
@@ -1517,7 +1549,7 @@ static int bt_topn(hfx_batch *b, hipStream_t st)
     return hfx_topn_device(b->ctx, b->top_pos, b->top_exact, b->top_f32, b->top_cnt, b->flag,
                            b->N, b->margin, b->scores, b->score_off, b->total, b->begin, b->num,
                            &b->db, &b->sp, rel0, 0.0f, i8 ? BT_RELQ_I8 : 0.0f,
-                           b->use_rows ? bt_norms(b) : nullptr, b->tx_scratch, (void *)st);
+                           bt_rows(b) ? bt_norms(b) : nullptr, b->tx_scratch, (void *)st);
 }
 
 extern "C" int hfx_batch_run(hfx_batch *b, void *stream)
@@ -1697,7 +1729,7 @@ extern "C" int hfx_batch_time(hfx_batch *b, void *stream, float *ms)
     HFX_CHECK_HIP(hipEventRecord(ev[1], st));
     if (!rc) rc = bt_prep(b, st);
     HFX_CHECK_HIP(hipEventRecord(ev[2], st));
-    const bool scored = b->total != 0 && (b->use_rows || bt_is_dense(b->precision) || b->B != 0);
+    const bool scored = b->total != 0 && (bt_rows(b) || bt_is_dense(b->precision) || b->B != 0);
     if (!rc) rc = bt_scores(b, st, kev);
     HFX_CHECK_HIP(hipEventRecord(ev[3], st));
     if (!rc) rc = bt_topn(b, st);

@@ -12,10 +12,10 @@
 
 /* precision forms: planes of a spectrum, spectra a block */
 #define RW_I8X3 0
-#define RW_I8X4 1
+#define RW_I8X6 1
 #define RW_BF16 2
-#define RW_PLANES(mode) ((mode) == RW_I8X3 ? 3 : 4)
-#define RW_NS(mode) ((mode) == RW_BF16 ? 8u : 16u)
+#define RW_PLANES(mode) ((mode) == RW_I8X3 ? 3 : (mode) == RW_I8X6 ? 6 : 4)
+#define RW_NS(mode) ((mode) == RW_I8X3 ? 16u : 8u)
 
 /* rows[l - 1]: charge level l's tiles of G KiB each, or null; slots: tile t of
  * level l at place slots[(l - 1) ntiles + t] of rows[l - 1] (null: place t);
@@ -37,7 +37,7 @@ struct hfx_rest {
 };
 /* planes [S][RW_PLANES][RW_MAXK] and quanta of the spectra, and the charge level of
  * each, 0 for those put on the list `rest`: charges above `have`, the highest level
- * there are rows for; in RW_I8X4 spectra whose digits would lose precision.  norms
+ * there are rows for; in RW_I8X6 spectra with a value that six digits do not hold.  norms
  * [S], if any: sum and max of |x|.  The num[s] scores of spectra whose charge is not
  * generated are set to 0, and nothing between one spectrum's scores and the next's */
 int hfx_rows_split(int mode, const hfx_spectra *sp, uint8_t *planes, float *qs, uint32_t *lvl,

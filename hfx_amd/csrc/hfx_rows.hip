@@ -24,19 +24,19 @@
  * Spectra.  Precision forms (see hfx_dense.hip for their bounds):
  *   RW_I8X3  three balanced base-256 digits of X = rint(x 2^k),
  *            max|x| 2^k <= 8355711; a block is sixteen spectra;
- *   RW_I8X4  four digits, max|x| 2^k <= 2139062143: 32-bit fixed point, for the
- *            FP32 forms.  |score - exact| <= max|x| 2^-31 sum w + 2^-24 |score|,
- *            which is below the rounding of the FP32 sums it replaces while
- *            mean|x| >= max|x| 2^-12 (the sum of T products of mean w mean|x|
- *            rounds to about 2^-25 T w mean|x|, the digits err by
- *            sqrt(T) w max|x| 2^-31).  A spectrum beyond that, or with a value
- *            that is not finite, is marked wide and keeps the FP32 kernel;
+ *   RW_I8X6  six digits, max|x| in [2^45, 2^46) of the last one's unit, for the FP32
+ *            forms: they hold every FP32 value from max|x| 2^-22 up with all of
+ *            its 24 bits, so that the sums are exact and a score is rounded once.  A
+ *            spectrum with a value that they do not hold (smaller, and not a
+ *            multiple of the unit; or not finite) keeps the packed kernel.  A column of the
+ *            matrix instructions is half a spectrum's digits, a block eight
+ *            spectra;
  *   RW_BF16  hi and lo BF16 of eight spectra, FP32 accumulation.
  *
  * Scoring kernels, 20,000 proteins (2.7 M peptides), before (rows written per
  * block into LDS, or per pair) and after: three digits, 20,000 spectra 1,978 ->
  * 864 us; BF16, 6,000 spectra 1,937 -> 773 us; FP32 batched, 4,000 spectra
- * 10,114 -> 547 us.  Writing two levels' rows of the database takes 0.87 ms,
+ * 10,114 -> 570 us.  Writing two levels' rows of the database takes 0.87 ms,
  * once.
  */
 #include "hfx_cand.h"
@@ -76,8 +76,8 @@ __device__ __forceinline__ uint32_t rw_bf16(float f)
     return (u + 0x7fffu + ((u >> 16) & 1u)) >> 16;
 }
 
-/* planes[s][plane][RW_MAXK]: byte 64 ks + 16 kg + j of a digit plane is the
- * digit of bin 64 ks + rw_bin_of(kg, j); the BF16 planes (hi of bytes j < 8,
+/* planes[s][plane][RW_MAXK]: byte 64 ks + 16 kg + j of a digit plane (the lowest
+ * digit first) is the digit of bin 64 ks + rw_bin_of(kg, j); the BF16 planes (hi of bytes j < 8,
  * hi of j >= 8, lo, lo) hold eight BF16 in the 16 bytes of a k-group.
  * qs[s] = 2^-k.  norms (if any): sum and max of |x|.  A spectrum whose charge has no
  * rows (above `have`; a later one than those a batch was planned with) or, in the
@@ -132,7 +132,24 @@ __global__ void __launch_bounds__(256)
     m = fmaxf(fmaxf(red[0][0], red[0][1]), fmaxf(red[0][2], red[0][3]));
     x1 = red[1][0] + red[1][1] + red[1][2] + red[1][3];
     if (tid == 0 && norms) norms[s] = make_float2(x1, m);
-    const bool out = z > have || (MODE == RW_I8X4 && (bad || !(x1 >= m * (float)len * (1.0f / 4096.0f))));
+    bool out = z > have;
+    /* RW_I8X6, k: m 2^k in [2^45, 2^46), at most 126 */
+    [[maybe_unused]] double sc6 = 1.0;
+    if constexpr (MODE == RW_I8X6) {
+        int k = 0;
+        if (m > 0.0f && !bad) k = min(45 - ((int)((__float_as_uint(m) >> 23) & 255u) - 127), 126);
+        sc6 = ldexp(1.0, k);
+        if (tid == 0) qs[s] = ldexpf(1.0f, -k);
+        bool lost = bad != 0;
+#pragma unroll
+        for (uint32_t u = 0; u < NU; ++u)
+#pragma unroll
+            for (uint32_t i = 0; i < 4; ++i) {
+                const double d = (double)v[u][i] * sc6;
+                lost |= !(rint(d) == d);
+            }
+        out |= __syncthreads_or(lost) != 0;
+    }
     if (tid == 0) {
         lvl[s] = out ? 0u : z;
         if (out && z) rest.list[atomicAdd(rest.count, 1u)] = s;
@@ -159,20 +176,21 @@ __global__ void __launch_bounds__(256)
         }
         return;
     }
-    /* k: m 2^k in [2^(B-1), 2^B) from m's exponent, one less where that passes
+    /* RW_I8X3, k: m 2^k in [2^22, 2^23) from m's exponent, one less where that passes
      * the largest value the digits reach; at most 126 */
-    constexpr int B = MODE == RW_I8X4 ? 31 : 23;
-    constexpr float XMAX = MODE == RW_I8X4 ? 2139062143.0f : 8355711.0f;
-    int k = 0;
-    if (m > 0.0f) {
-        const int e = (int)((__float_as_uint(m) >> 23) & 255u) - 127;
-        k = B - 1 - e;
-        if (k > 126) k = 126;
-        /* XMAX of four digits rounds up to 2139062144, one past their largest */
-        else if (ldexpf(m, k) >= XMAX && (MODE == RW_I8X4 || ldexpf(m, k) > XMAX)) --k;
+    [[maybe_unused]] float sc = 1.0f;
+    if constexpr (MODE == RW_I8X3) {
+        int k = 0;
+        if (m > 0.0f) {
+            const int e = (int)((__float_as_uint(m) >> 23) & 255u) - 127;
+            k = 22 - e;
+            if (k > 126) k = 126;
+            else if (ldexpf(m, k) > 8355711.0f) --k;
+        }
+        sc = ldexpf(1.0f, k);
+        if (tid == 0) qs[s] = ldexpf(1.0f, -k);
     }
-    const float sc = ldexpf(1.0f, k);
-    if (tid == 0) qs[s] = ldexpf(1.0f, -k);
+    using X_t = std::conditional_t<MODE == RW_I8X6, int64_t, int32_t>;
 #pragma unroll
     for (uint32_t u = 0; u < NU; ++u) {
         const uint32_t t = tid + 256 * u;
@@ -182,10 +200,12 @@ __global__ void __launch_bounds__(256)
         for (uint32_t d = 0; d < NP; ++d) w[d] = 0u;
 #pragma unroll
         for (uint32_t i = 0; i < 4; ++i) {
-            int32_t X = (int32_t)rintf(v[u][i] * sc);
+            X_t X;
+            if constexpr (MODE == RW_I8X6) X = (int64_t)((double)v[u][i] * sc6);
+            else X = (int32_t)rintf(v[u][i] * sc);
 #pragma unroll
             for (uint32_t d = 0; d < NP; ++d) {
-                const int32_t g = d + 1 < NP ? ((X + 128) & 255) - 128 : X;
+                const int32_t g = d + 1 < NP ? (((int32_t)X + 128) & 255) - 128 : (int32_t)X;
                 w[d] |= (uint32_t)(g & 255) << (8 * i);
                 X = (X - g) >> 8;
             }
@@ -575,6 +595,15 @@ struct RmArgs {
     hfx_spectra sp;
 };
 
+/* an even lane: the next lane's value */
+__device__ __forceinline__ double rm_next(double h)
+{
+    const uint64_t u = (uint64_t)__double_as_longlong(h);
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)u, 0xb1, 0xf, 0xf, false);
+    const uint32_t hi = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)(uint32_t)(u >> 32), 0xb1, 0xf, 0xf, false);
+    return __longlong_as_double((long long)((uint64_t)hi << 32 | lo));
+}
+
 /* Persistent workgroups of twelve waves over (block, level, CT tiles).  The
  * block's planes stay in LDS, laid out so that a fragment read is one
  * contiguous KiB ([k-step][plane][lane]); each wave contracts four tiles at a
@@ -586,15 +615,20 @@ struct RmArgs {
  * the cycles, with rows from cache as well, and interleaving them by hand
  * changes nothing.  So what is not a lookup was taken out of the loop (copies of
  * the codes, per-lane addresses, FP64 folds) and a third wave a SIMD fills its
- * waits: three digits, 20,000 spectra 963 -> 881 (the wave) -> 864 us; four, a
- * plain search of 10,000, 840 -> 767 -> 757; BF16 850 -> 812 -> 773.  Sixteen
+ * waits: three digits, 20,000 spectra 963 -> 881 (the wave) -> 864 us; BF16 850 ->
+ * 812 -> 773.  Six digits take three matrix instructions a k-step of four tiles as
+ * well, for half as many spectra: a plain search of 10,000 866 us, a batch of 4,000
+ * 570 (four digits and sixteen spectra, which rounded the FP32 values below
+ * max|x| / 128, 757 and 547).  Sixteen
  * waves spill (983 us, three digits); three groups of codes on their way, also
  * across tiles, cost more scalar work than they hide (1,134). */
 template <int MODE>
 __global__ void __launch_bounds__(RM_THREADS, 3) k_rw_mm(RmArgs a)
 {
-    constexpr uint32_t NP = MODE == RW_BF16 ? 2 : RW_PLANES(MODE); /* planes in LDS */
+    constexpr uint32_t NP = MODE == RW_BF16 ? 2 : 3; /* planes in LDS */
     constexpr uint32_t NS = RW_NS(MODE);
+    /* a column is half of a spectrum: its high or low digits, its hi or lo */
+    constexpr bool HALF = MODE != RW_I8X3;
     extern __shared__ __align__(16) uint8_t rm_lds[];
     rw_u32x4 *Bl = (rw_u32x4 *)rm_lds; /* [k-step][plane][64 lanes] */
     __shared__ uint32_t m_s[16], m_beg[16], m_end[16], m_z[16];
@@ -604,7 +638,7 @@ __global__ void __launch_bounds__(RM_THREADS, 3) k_rw_mm(RmArgs a)
     const uint32_t tid = threadIdx.x, lane = hfx_lane();
     const uint32_t wave = __builtin_amdgcn_readfirstlane(tid / HFX_WAVE);
     const uint32_t col = lane & 15u, kg = lane >> 4;
-    const uint32_t g_of = MODE == RW_BF16 ? col >> 1 : col; /* spectrum of this lane's column */
+    const uint32_t g_of = HALF ? col >> 1 : col; /* spectrum of this lane's column */
     const uint32_t nitems = (uint32_t)rw_sload(a.item_off, a.B);
     uint32_t cur = 0xffffffffu;
     if (tid == 0) sh_t[0] = atomicAdd(a.counter, 1u);
@@ -656,7 +690,9 @@ __global__ void __launch_bounds__(RM_THREADS, 3) k_rw_mm(RmArgs a)
                     const uint32_t s = m_s[g_of];
                     val[u] = rw_u32x4{0u, 0u, 0u, 0u};
                     if (i < nv && s != 0xffffffffu) {
-                        const uint32_t pl = MODE == RW_BF16 ? (col & 1u) * 2u + d : d;
+                        const uint32_t pl = MODE == RW_BF16   ? (col & 1u) * 2u + d
+                                            : MODE == RW_I8X6 ? (col & 1u ? d : 3u + d)
+                                                              : d;
                         val[u] = *(const rw_u32x4 *)(a.planes +
                                                      ((size_t)s * RW_PLANES(MODE) + pl) * RW_MAXK +
                                                      ks * 64u + kg * 16u);
@@ -682,7 +718,7 @@ __global__ void __launch_bounds__(RM_THREADS, 3) k_rw_mm(RmArgs a)
                             : lvl == 3 ? a.rows[2] : a.rows[3];
         const uint64_t *slots = a.slots ? a.slots + (size_t)(lvl - 1u) * a.ntiles : nullptr;
         const uint32_t beg = m_beg[g_of], end = m_end[g_of];
-        const bool mine = m_z[g_of] == lvl && (MODE != RW_BF16 || (col & 1u) == 0u);
+        const bool mine = m_z[g_of] == lvl && (!HALF || (col & 1u) == 0u);
         const float qf = MODE == RW_BF16 ? 0.0f : m_q[g_of];
         float *const out = a.scores + m_off[g_of];
         const size_t tile_bytes = (size_t)a.G * 1024u;
@@ -818,9 +854,11 @@ __global__ void __launch_bounds__(RM_THREADS, 3) k_rw_mm(RmArgs a)
                         }
                     }
                 });
-                /* Digit sums are below 50 * 128 * RW_MAXK < 2^23.8.  Carries go up
-                 * until the highest digit is followed by 16 or 24 bits; both parts
-                 * are exact in FP32, and the fused sum rounds once. */
+                /* Digit sums are below 50 * 128 * RW_MAXK < 2^23.8.  Carries go up until
+                 * the highest digit is followed by 16 bits.  Three digits: both parts
+                 * are exact in FP32, and the fused sum rounds once.  Six: each half is
+                 * exact in FP64, the odd column's (the low one) is fetched, and the
+                 * fused sum is rounded to FP32. */
 #pragma unroll
                 for (uint32_t k = 0; k < RM_T; ++k) {
                     const uint32_t t = u0 + k;
@@ -833,8 +871,13 @@ __global__ void __launch_bounds__(RM_THREADS, 3) k_rw_mm(RmArgs a)
                             low |= ((uint32_t)top & 255u) << (8 * (d - 1));
                             top = acc[k][d][i] + (top >> 8);
                         }
-                        const float v = __builtin_fmaf((float)top, (float)(1u << (8 * (NP - 1))),
-                                                       (float)low) * qf;
+                        float v;
+                        if constexpr (MODE == RW_I8X6) {
+                            const double h = __builtin_fma((double)top, 65536.0, (double)low);
+                            v = (float)__builtin_fma(h, 16777216.0, rm_next(h)) * qf;
+                        } else {
+                            v = __builtin_fmaf((float)top, 65536.0f, (float)low) * qf;
+                        }
                         const uint32_t p = t * RW_ROWS + 4u * kg + i;
                         if (mine && t < c1 && beg <= p && p < end) out[p - beg] = v;
                     }
@@ -871,7 +914,7 @@ int hfx_rows_split(int mode, const hfx_spectra *sp, uint8_t *planes, float *qs, 
     const dim3 g(sp->num_spec), t(256);
     hipStream_t st = hfx_stream(stream);
     const auto kernel = mode == RW_I8X3   ? k_rw_split<RW_I8X3>
-                        : mode == RW_I8X4 ? k_rw_split<RW_I8X4>
+                        : mode == RW_I8X6 ? k_rw_split<RW_I8X6>
                                           : k_rw_split<RW_BF16>;
     hipLaunchKernelGGL(kernel, g, t, 0, st, planes, qs, lvl, *rest, have, norms, scores, off, num, *sp);
     HFX_CHECK_LAUNCH();
@@ -974,17 +1017,16 @@ int hfx_rows_scores(hfx_ctx *ctx, int mode, void *scratch, float *d_scores, cons
     a.ntiles = r->ntiles;
     a.G = r->G;
     a.sp = *sp;
-    const uint32_t np = mode == RW_BF16 ? 2u : (uint32_t)RW_PLANES(mode);
-    const uint32_t lds = RW_NKS * np * 1024u;
+    const uint32_t lds = RW_NKS * (mode == RW_BF16 ? 2u : 3u) * 1024u;
     const uint32_t per_cu = lds * 2 <= 156u * 1024u ? 2u : 1u;
     const dim3 g((uint32_t)hfx_ctx_num_cus(ctx) * per_cu), t(RM_THREADS);
     const void *fn = mode == RW_I8X3   ? (const void *)k_rw_mm<RW_I8X3>
-                     : mode == RW_I8X4 ? (const void *)k_rw_mm<RW_I8X4>
+                     : mode == RW_I8X6 ? (const void *)k_rw_mm<RW_I8X6>
                                        : (const void *)k_rw_mm<RW_BF16>;
     HFX_CHECK_HIP(hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     if (ev) HFX_CHECK_HIP(hipEventRecord((hipEvent_t)ev[0], st));
     if (mode == RW_I8X3) hipLaunchKernelGGL(k_rw_mm<RW_I8X3>, g, t, lds, st, a);
-    else if (mode == RW_I8X4) hipLaunchKernelGGL(k_rw_mm<RW_I8X4>, g, t, lds, st, a);
+    else if (mode == RW_I8X6) hipLaunchKernelGGL(k_rw_mm<RW_I8X6>, g, t, lds, st, a);
     else hipLaunchKernelGGL(k_rw_mm<RW_BF16>, g, t, lds, st, a);
     if (ev) HFX_CHECK_HIP(hipEventRecord((hipEvent_t)ev[1], st));
     HFX_CHECK_LAUNCH();

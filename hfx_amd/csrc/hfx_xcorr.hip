@@ -406,7 +406,7 @@ int hfx_xcorr_rest(hfx_ctx *ctx, float *d_scores, const uint64_t *d_off, const u
 /* ------------------------------------------------------------------ */
 
 /* hfx_xcorr_sparse writes each candidate's theoretical row once and contracts the
- * rows with blocks of sixteen spectra (hfx_rows.hip, 32-bit fixed point) instead
+ * rows with blocks of eight spectra (hfx_rows.hip, fixed point that holds them) instead
  * of building a row per pair, where that is quicker.  In ns: a pair costs 230 ps
  * to score by itself, 30 through its row; the rows' dozen launches 80,000 more
  * than the packed kernel's three; a tile of the database 1/3 to look at and, if a
@@ -447,7 +447,7 @@ static int xcorr_rows(hfx_ctx *ctx, float *d_scores, const uint64_t *d_off,
     const uint32_t nseg = hfx_cut_segs(S);
     auto al = [](uint64_t n) { return (n + 255) & ~(uint64_t)255; };
     const uint64_t sizes[] = {
-        al((uint64_t)S * RW_PLANES(RW_I8X4) * RW_MAXK), al(4ull * S), al(4ull * S), al(4ull * S + 4),
+        al((uint64_t)S * RW_PLANES(RW_I8X6) * RW_MAXK), al(4ull * S), al(4ull * S), al(4ull * S + 4),
         al(4ull * S), al(4ull * ob.nb), al(4ull * S), al(8ull * ob.nb + 8), al(4ull * nseg * 32),
         al(4ull * nseg), al(8ull * nseg + 8), al(4ull * S + 4), al(hfx_rows_items_bytes(S)),
         al(4 * nf), al(8 * nf + 8), al(nt + 4ull)};
@@ -485,14 +485,14 @@ static int xcorr_rows(hfx_ctx *ctx, float *d_scores, const uint64_t *d_off,
     const uint32_t CH = hfx_rows_chunk(est, (uint32_t)hfx_ctx_num_cus(ctx));
     int rc;
     if ((rc = hfx_order_spectra(ctx, order, &ob, d_begin, sp->d_zmax, nullptr, S, stream)) ||
-        (rc = hfx_cut_blocks(ctx, 16, &cb, order, d_begin, d_num, sp->d_zmax, S, stream)) ||
-        (rc = hfx_rows_split(RW_I8X4, sp, planes, qs, lvl, &rest, HFX_MAX_CHARGE, nullptr, d_scores,
+        (rc = hfx_cut_blocks(ctx, RW_NS(RW_I8X6), &cb, order, d_begin, d_num, sp->d_zmax, S, stream)) ||
+        (rc = hfx_rows_split(RW_I8X6, sp, planes, qs, lvl, &rest, HFX_MAX_CHARGE, nullptr, d_scores,
                              d_off, d_num, stream)) ||
         (rc = hfx_rows_blocks(ctx, items, order, cb.bstart, d_begin, d_num, &sq, CH, stream)) ||
         (rc = hfx_rows_mark(items, S, flags, nt, stream)) ||
         (rc = hfx_scan_offsets(ctx, (uint64_t *)r.slots, flags, (uint32_t)nf, stream)) ||
         (rc = hfx_rows_build((uint32_t)hfx_ctx_num_cus(ctx), db, &r, flags, stream)) ||
-        (rc = hfx_rows_scores(ctx, RW_I8X4, items, d_scores, d_off, d_begin, d_num, order,
+        (rc = hfx_rows_scores(ctx, RW_I8X6, items, d_scores, d_off, d_begin, d_num, order,
                               cb.bstart, &r, planes, qs, &sq, CH, stream, nullptr)) ||
         (rc = hfx_xcorr_rest(ctx, d_scores, d_off, d_begin, d_num, db, sp, &rest, 0, stream)))
         return rc;

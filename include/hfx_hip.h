@@ -286,11 +286,15 @@ int hfx_scan_offsets(hfx_ctx *ctx, uint64_t *d_off, const uint32_t *d_count, uin
  * theoretical bins b < len_s of maxweight(b) * x_s[b], FP32.  `total` is
  * sum_s d_num[s] (findSpecCandsByMass's return value).
  * Calls large enough for it write each theoretical row once and contract the
- * rows with the spectra in 32-bit fixed point, rounded once to FP32: nearer the
- * exact score than the FP32 sums, within the same bound.  Their buffers (the rows,
- * up to 2.2 GB for 2.7 M peptides; 8.7 KB a spectrum) are kept by the context;
- * where device memory is short, or the stream is being captured before they
- * exist, the call sums in FP32 without them. */
+ * rows with the spectra in fixed point that holds their values, exact sums rounded
+ * once to FP32 (spectra whose values span more than 2^22, or are not finite, are
+ * summed in FP32): nearer the exact score than the FP32 sums, within the same
+ * bound, and the same but for that rounding.  Their buffers (room for the rows of
+ * four charge levels, 1.6 GB each for 2.7 M peptides, or for as many as the pairs
+ * can need; 13 KB a spectrum) are kept by the context and given back where an
+ * allocation of this library finds memory short.  Where it is short already, or the
+ * stream is being captured before they exist, the call sums in FP32 without them, so
+ * that two calls may differ in the last bit. */
 int hfx_xcorr_sparse(hfx_ctx *ctx, float *d_scores, const uint64_t *d_off,
                      const uint32_t *d_begin, const uint32_t *d_num, uint64_t total,
                      const hfx_db *db, const hfx_spectra *sp, void *stream);
@@ -626,8 +630,8 @@ int hfx_batch_split(const uint64_t *h_off, uint32_t S, uint32_t N, uint32_t num_
 int hfx_batch_use_index(hfx_batch *b, const hfx_pepix *ix);
 /* One batched search, every per-batch step on the device and without host
  * synchronisation or allocation: windows -> spectrum order (fragment charge
- * level, precursor mass) -> block cut -> the spectra as digits (FP32 form: four
- * base-256 digits, 32-bit fixed point; integer form: three) or hi and lo BF16 ->
+ * level, precursor mass) -> block cut -> the spectra as digits (FP32 form: six
+ * base-256 digits, which hold its values; integer form: three) or hi and lo BF16 ->
  * MFMA XCorr over the index's theoretical rows -> top-N with exact re-score.
  * Without the rows (spectra longer than 2176 bins, no memory for them, a first
  * run under capture) the FP32 form sums over the index's ion lists, blocks of G
