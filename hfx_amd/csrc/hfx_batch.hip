@@ -355,9 +355,10 @@ struct RowSet {
     hfx_rows rows;
     uint64_t bytes;
     uint32_t keepers, users; /* indexes, batches */
+    RowSet *next;
 };
 static std::mutex g_rows_mu; /* the sets and what they hold */
-static std::vector<RowSet *> g_rowsets;
+static RowSet *g_rowsets;
 
 /* frees a set's rows; called with g_rows_mu held and no batch using it */
 static void rowset_clear(RowSet *rs)
@@ -377,15 +378,17 @@ static void rowset_leave(RowSet *rs, uint32_t RowSet::*count)
 {
     if (--(rs->*count) || rs->keepers || rs->users) return;
     rowset_clear(rs);
-    g_rowsets.erase(std::remove(g_rowsets.begin(), g_rowsets.end(), rs), g_rowsets.end());
-    delete rs;
+    RowSet **at = &g_rowsets;
+    while (*at != rs) at = &(*at)->next;
+    *at = rs->next;
+    free(rs);
 }
 
 bool hfx_rowsets_release(int device)
 {
     std::lock_guard<std::mutex> lk(g_rows_mu);
     bool any = false;
-    for (RowSet *rs : g_rowsets)
+    for (RowSet *rs = g_rowsets; rs; rs = rs->next)
         if (rs->device == device && rs->users == 0 && rs->bytes) {
             rowset_clear(rs);
             any = true;
@@ -399,47 +402,80 @@ __global__ void k_ord_fill(uint32_t *a, uint32_t n)
     if (i < n) a[i] = 0u;
 }
 
-/* A 128-bit key of the peptides in residual order -- residuals, ladder residues --
- * and the residue masses: two polynomials over each peptide's residues, mixed with its
- * place and residual (D. Stafford's variant 13 of the 64-bit finaliser) and added
- * up.  2.7 M peptides are read once, a few tens of us when an index is built. */
+/* A 128-bit key of what rows are made from: residuals, ladder bounds and residual
+ * order of the peptides, the residues up to the last ladder's end (mod bits aside) and
+ * the residue masses, each value mixed with its place (D. Stafford's variant 13 of the
+ * 64-bit finaliser) and added up.  key[2]: the last ladder's end, which the residues
+ * are read up to by the second kernel.  The 52 MB of 2.7 M peptides, read in order, take
+ * 70 us; an atomic a wave, not one a workgroup, 500. */
 __device__ __forceinline__ uint64_t key_mix(uint64_t x)
 {
     x = (x ^ (x >> 30)) * 0xbf58476d1ce4e5b9ull;
     x = (x ^ (x >> 27)) * 0x94d049bb133111ebull;
     return x ^ (x >> 31);
 }
-__global__ void __launch_bounds__(256) k_db_key(unsigned long long *key, hfx_db db)
-{
+struct KeySum {
     uint64_t a = 0, b = 0;
-    const uint32_t t = blockIdx.x * 256 + threadIdx.x;
-    if (t < 26) {
-        const uint64_t m = (uint64_t)t << 32 | __float_as_uint(db.d_mass[t]);
-        a = key_mix(m + 0x9e3779b97f4a7c15ull);
-        b = key_mix(m ^ 0xd1b54a32d192ed03ull);
+    __device__ __forceinline__ void add(uint32_t array, uint64_t i, uint32_t v)
+    {
+        const uint64_t at = (i << 32 | v) + (uint64_t)(array + 1u) * 0x9e3779b97f4a7c15ull;
+        a += key_mix(at);
+        b += key_mix(at ^ 0xd1b54a32d192ed03ull);
     }
-    for (uint64_t q = t; q < db.num_pep; q += gridDim.x * 256ull) {
-        const uint32_t pep = db.d_idx_sorted[q];
-        const uint32_t tc = db.d_tc[pep], tn = db.d_tn[pep];
-        const uint32_t n = tn > tc ? tn - tc : 0u;
-        uint64_t x = n, y = ~(uint64_t)n;
-        for (uint32_t j = 0; j < n; ++j) {
-            const uint32_t c = HFX_ACID_IDX(db.d_ions[tc + j]) + 1u;
-            x = x * 0x9e3779b97f4a7c15ull + c;
-            y = y * 0xc2b2ae3d27d4eb4full + c;
+    /* by every thread of a workgroup, which adds once: atomics on one word queue */
+    __device__ __forceinline__ void to(unsigned long long *key)
+    {
+        __shared__ unsigned long long sum[2];
+        if (threadIdx.x < 2) sum[threadIdx.x] = 0;
+        for (int o = 32; o > 0; o >>= 1) {
+            a += __shfl_xor(a, o, 64);
+            b += __shfl_xor(b, o, 64);
         }
-        const uint64_t at = q << 32 | __float_as_uint(db.d_r[pep]);
-        a += key_mix(key_mix(x) + key_mix(at + 1u));
-        b += key_mix(key_mix(y) ^ key_mix(at ^ 0x5851f42d4c957f2dull));
+        __syncthreads();
+        if (hfx_lane() == 0) {
+            atomicAdd(&sum[0], (unsigned long long)a);
+            atomicAdd(&sum[1], (unsigned long long)b);
+        }
+        __syncthreads();
+        if (threadIdx.x < 2) atomicAdd(key + threadIdx.x, sum[threadIdx.x]);
     }
-    for (int o = 32; o > 0; o >>= 1) {
-        a += __shfl_xor(a, o, 64);
-        b += __shfl_xor(b, o, 64);
+};
+__global__ void __launch_bounds__(256) k_db_key_peptides(unsigned long long *key, hfx_db db)
+{
+    KeySum k;
+    uint32_t end = 0;
+    const uint32_t t = blockIdx.x * 256 + threadIdx.x;
+    if (t < 26) k.add(0, t, __float_as_uint(db.d_mass[t]));
+    for (uint64_t p = t; p < db.num_pep; p += gridDim.x * 256ull) {
+        const uint32_t tn = db.d_tn[p];
+        k.add(1, p, __float_as_uint(db.d_r[p]));
+        k.add(2, p, db.d_tc[p]);
+        k.add(3, p, tn);
+        k.add(4, p, db.d_idx_sorted[p]);
+        end = max(end, tn);
     }
-    if (hfx_lane() == 0) {
-        atomicAdd(key, (unsigned long long)a);
-        atomicAdd(key + 1, (unsigned long long)b);
+    for (int o = 32; o > 0; o >>= 1) end = max(end, (uint32_t)__shfl_xor((int)end, o, 64));
+    if (hfx_lane() == 0 && end) atomicMax(key + 2, (unsigned long long)end);
+    k.to(key);
+}
+__global__ void __launch_bounds__(256) k_db_key_residues(unsigned long long *key, hfx_db db)
+{
+    KeySum k;
+    const uint64_t n = key[2];
+    /* four residues a step, those before the first multiple of four on their own */
+    const uint64_t head = min(n, (uint64_t)(-(uintptr_t)db.d_ions & 3u)), words = (n - head) / 4;
+    const uint32_t t = blockIdx.x * 256 + threadIdx.x;
+    /* (a residue's own place and code: the same sum wherever the words lie) */
+    auto one = [&](uint64_t i, uint32_t c) { k.add(5, i, HFX_ACID_IDX(c)); };
+    for (uint64_t w = t; w < words; w += gridDim.x * 256ull) {
+        const uint32_t v = *(const uint32_t *)(db.d_ions + head + 4 * w);
+#pragma unroll
+        for (uint32_t j = 0; j < 4; ++j) one(head + 4 * w + j, v >> (8 * j));
     }
+    const uint64_t tail = head + 4 * words;
+    if (t < head) one(t, db.d_ions[t]);
+    if (t < n - tail) one(tail + t, db.d_ions[tail + t]);
+    k.to(key);
 }
 
 template <class T>
@@ -490,10 +526,12 @@ extern "C" int hfx_pepix_build(hfx_ctx *ctx, const hfx_db *db, uint32_t forms, u
     const uint32_t P = db->num_pep;
     int rc = HFX_OK;
     unsigned long long *key = nullptr;
-    rc = dalloc(&key, 2);
+    rc = dalloc(&key, 3);
     if (!rc && P) {
-        hipLaunchKernelGGL(k_ord_fill, dim3(1), dim3(64), 0, st, (uint32_t *)key, 4u);
-        hipLaunchKernelGGL(k_db_key, dim3(std::min((P + 255) / 256, 4096u)), dim3(256), 0, st, key, *db);
+        hipLaunchKernelGGL(k_ord_fill, dim3(1), dim3(64), 0, st, (uint32_t *)key, 6u);
+        const dim3 g(std::min((P + 255) / 256, 512u));
+        hipLaunchKernelGGL(k_db_key_peptides, g, dim3(256), 0, st, key, *db);
+        hipLaunchKernelGGL(k_db_key_residues, g, dim3(256), 0, st, key, *db);
     }
     if (!rc && (forms & HFX_PEPIX_LADDER)) {
         rc = hfx_dense_ladder_build(ctx, db, 0, P, 1, &ix->lad, ix->lad_mem, stream);
@@ -569,13 +607,19 @@ static RowSet *pepix_use_rows(hfx_pepix *ix, uint32_t L, uint32_t cus, hipStream
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess) return nullptr;
     if (!ix->rs) {
-        for (RowSet *rs : g_rowsets)
+        for (RowSet *rs = g_rowsets; rs; rs = rs->next)
             if (rs->device == dev && rs->num_pep == ix->db.num_pep && rs->key[0] == ix->key[0] &&
                 rs->key[1] == ix->key[1])
                 ix->rs = rs;
         if (!ix->rs) {
-            ix->rs = new RowSet{dev, ix->db.num_pep, {ix->key[0], ix->key[1]}, {}, 0, 0, 0};
-            g_rowsets.push_back(ix->rs);
+            ix->rs = (RowSet *)calloc(1, sizeof(RowSet));
+            if (!ix->rs) return nullptr;
+            ix->rs->device = dev;
+            ix->rs->num_pep = ix->db.num_pep;
+            ix->rs->key[0] = ix->key[0];
+            ix->rs->key[1] = ix->key[1];
+            ix->rs->next = g_rowsets;
+            g_rowsets = ix->rs;
         }
         ++ix->rs->keepers;
     }

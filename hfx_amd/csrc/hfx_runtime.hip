@@ -12,9 +12,7 @@
 #include <stdlib.h>
 #include <string.h>
 
-#include <algorithm>
 #include <mutex>
-#include <vector>
 
 static thread_local char g_err[1024] = "";
 
@@ -36,11 +34,12 @@ struct hfx_ctx {
     void *pinned;
     size_t pinned_bytes;
     uint32_t spare_users; /* calls that hold spare slots now; g_ctx_mu */
+    hfx_ctx *next;        /* of all contexts; g_ctx_mu */
 };
 
 /* the contexts there are, and their spare_users */
 static std::mutex g_ctx_mu;
-static std::vector<hfx_ctx *> g_ctxs;
+static hfx_ctx *g_ctxs;
 
 extern "C" int hfx_ctx_create(int device, hfx_ctx **out)
 {
@@ -54,7 +53,8 @@ extern "C" int hfx_ctx_create(int device, hfx_ctx **out)
     c->num_cus = prop.multiProcessorCount;
     {
         std::lock_guard<std::mutex> lk(g_ctx_mu);
-        g_ctxs.push_back(c);
+        c->next = g_ctxs;
+        g_ctxs = c;
     }
     *out = c;
     return HFX_OK;
@@ -65,7 +65,9 @@ extern "C" int hfx_ctx_destroy(hfx_ctx *ctx)
     if (!ctx) return HFX_OK;
     {
         std::lock_guard<std::mutex> lk(g_ctx_mu);
-        g_ctxs.erase(std::remove(g_ctxs.begin(), g_ctxs.end(), ctx), g_ctxs.end());
+        hfx_ctx **at = &g_ctxs;
+        while (*at && *at != ctx) at = &(*at)->next;
+        if (*at) *at = ctx->next;
     }
     for (int i = 0; i < HFX_SCRATCH_SLOTS; ++i)
         if (ctx->scratch[i]) (void)hipFree(ctx->scratch[i]);
@@ -145,7 +147,7 @@ bool hfx_spare_release(void)
     if (hipGetDevice(&dev) != hipSuccess) return false;
     bool any = hfx_rowsets_release(dev);
     std::lock_guard<std::mutex> lk(g_ctx_mu);
-    for (hfx_ctx *c : g_ctxs) {
+    for (hfx_ctx *c = g_ctxs; c; c = c->next) {
         if (c->device != dev || c->spare_users) continue;
         for (int slot : {HFX_SLOT_ROWS, HFX_SLOT_ROWS2}) {
             if (!c->scratch[slot]) continue;
