@@ -1223,11 +1223,13 @@ static int bt_ready_attached(hfx_batch *b, hipStream_t st)
     return bt_ready(b, st);
 }
 
-/* Device bytes hfx_batch_plan allocates for S spectra with `total` scored
- * pairs (the precision form's own buffers included, the per-database index
- * not): the same sums as the allocations below. */
+/* Device bytes a batch allocates for S spectra with `total` scored pairs (the
+ * precision form's own buffers included, the per-database index and rows not):
+ * the same sums as the allocations.  rows: with what it takes to score through
+ * rows, which it does without where memory is short; the FP32 form's is counted
+ * for the others too, as a plan starts in that form. */
 static uint64_t bt_bytes(uint32_t S, uint64_t total, uint32_t N, uint32_t num_pep,
-                         uint32_t precision)
+                         uint32_t precision, bool rows = true)
 {
     auto al = [](uint64_t n, uint64_t sz) { return (std::max<uint64_t>(n, 1) * sz + 255) & ~255ull; };
     uint32_t sh = 0;
@@ -1241,11 +1243,11 @@ static uint64_t bt_bytes(uint32_t S, uint64_t total, uint32_t N, uint32_t num_pe
                  al(S, 4) * 2                                            /* top-N */
                  + al(hfx_topn_scratch_bytes(S, total), 1)               /* exact route */
                  + al(bmax, 4) * 3 + al(bmax + 1, 8);                    /* sparse blocks */
-    if (bt_is_dense(precision)) {
-        const uint64_t nseg = (S + CUT_SEG - 1) / CUT_SEG;
-        b += al(bt_dense_scratch(S), 1) + al((uint64_t)S + 1, 4) + al(nseg * CUT_SEG, 4) +
-             al(nseg, 4) + al(nseg + 1, 8);
-    }
+    const uint64_t nseg = (S + CUT_SEG - 1) / CUT_SEG;
+    if (rows || bt_is_dense(precision))
+        b += al((uint64_t)S + 1, 4) + al(nseg * CUT_SEG, 4) + al(nseg, 4) + al(nseg + 1, 8);
+    if (rows) b += al(5ull * S + 1, 4) + al(bt_planes_bytes(S), 1);
+    if (bt_is_dense(precision)) b += al(bt_dense_scratch(S), 1);
     return b;
 }
 
@@ -1339,7 +1341,7 @@ extern "C" int hfx_batch_plan(hfx_batch *b, const hfx_db *db, const hfx_spectra 
          * cannot fit (hfx_batch_split cuts a larger set into batches that do) */
         size_t fr = 0, tot = 0;
         HFX_CHECK_HIP(hipMemGetInfo(&fr, &tot));
-        const uint64_t need = bt_bytes(S, b->total, N, db->num_pep, HFX_BATCH_FP32_SPARSE);
+        const uint64_t need = bt_bytes(S, b->total, N, db->num_pep, HFX_BATCH_FP32_SPARSE, false);
         if (need > fr && hfx_spare_release()) HFX_CHECK_HIP(hipMemGetInfo(&fr, &tot));
         HFX_REQUIRE(need <= fr, HFX_ERR_NOMEM,
                     "hfx_batch_plan: %u spectra with %llu scores need %llu device bytes, %zu free "

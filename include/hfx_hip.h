@@ -612,10 +612,11 @@ int hfx_batch_plan_ix(hfx_batch *b, const hfx_pepix *ix, const hfx_spectra *sp, 
                       uint32_t N, uint32_t margin, void *stream);
 /* Device bytes a batch plan of S spectra with `total` scored pairs (the sum
  * of their window sizes, e.g. findSpecCandsByMass's return) allocates in
- * the given precision form, the per-database index excepted (host
+ * the given precision form, the per-database index and its rows excepted (host
  * arithmetic; Search.hs:427-433 sizes its work the same way).
  * hfx_batch_plan fails with HFX_ERR_NOMEM, allocating nothing, when its
- * batch exceeds the device's free memory. */
+ * batch exceeds the device's free memory without what the rows route takes (14 KB
+ * a spectrum) and with rows that no batch uses given back. */
 int hfx_batch_required_bytes(uint32_t S, uint64_t total, uint32_t N, uint32_t num_pep,
                              uint32_t precision, uint64_t *bytes);
 /* Execution.hs:77-93 groupScorePlan: cuts spectra 0..S-1 (score offsets
