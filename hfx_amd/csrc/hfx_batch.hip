@@ -1007,6 +1007,8 @@ extern "C" int hfx_batch_destroy(hfx_batch *b)
     return HFX_OK;
 }
 
+static int bt_ready_attached(hfx_batch *b, hipStream_t st);
+
 extern "C" int hfx_batch_use_index(hfx_batch *b, const hfx_pepix *ix)
 {
     HFX_REQUIRE(b, HFX_ERR_ARG, "hfx_batch_use_index: null batch");
@@ -1021,7 +1023,8 @@ extern "C" int hfx_batch_use_index(hfx_batch *b, const hfx_pepix *ix)
         (void)hipGraphDestroy(b->graph);
         b->graph = nullptr;
     }
-    return HFX_OK;
+    /* its rows now, so that no run waits or allocates for them */
+    return b->planned ? bt_ready_attached(b, nullptr) : HFX_OK;
 }
 
 /* Shape-bucketed autotuner results of this process: (S bucket, P bucket, L)
@@ -1187,9 +1190,12 @@ static int bt_ready(hfx_batch *b, hipStream_t st)
 {
     int rc = bt_need_index(b, st);
     if (rc || b->S == 0 || (b->rows_tried && (!b->use_rows || bt_rows_bufs(b)))) return rc;
+    /* (the null stream cannot be asked while another one is captured) */
     hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
-    HFX_CHECK_HIP(hipStreamIsCapturing(st, &cs));
-    if (cs != hipStreamCaptureStatusNone) return HFX_OK;
+    if (hipStreamIsCapturing(st, &cs) != hipSuccess || cs != hipStreamCaptureStatusNone) {
+        (void)hipGetLastError();
+        return HFX_OK;
+    }
     b->rows_tried = true;
     if (b->sp.x_stride > RW_MAXK || b->db.num_pep == 0) return HFX_OK;
     size_t fr = 0, tot = 0;

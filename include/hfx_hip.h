@@ -628,6 +628,9 @@ int hfx_batch_required_bytes(uint32_t S, uint64_t total, uint32_t N, uint32_t nu
 int hfx_batch_split(const uint64_t *h_off, uint32_t S, uint32_t N, uint32_t num_pep,
                     uint32_t precision, uint64_t budget, uint32_t *h_first, uint32_t cap,
                     uint32_t *num_batches);
+/* Attaches an index (null: none).  A planned batch takes its theoretical rows here,
+ * writing them on the null stream if it is the first to (waits for it); its runs then
+ * neither wait nor allocate. */
 int hfx_batch_use_index(hfx_batch *b, const hfx_pepix *ix);
 /* One batched search, every per-batch step on the device and without host
  * synchronisation or allocation: windows -> spectrum order (fragment charge

@@ -45,3 +45,19 @@ def test_a_plan_takes_what_required_bytes_says(env, form):
                                          getattr(first, form), C.byref(n)), "hfx_batch_required_bytes")
     # some thirty allocations, each rounded up to the driver's 2 MiB at most
     assert took <= n.value + (60 << 20)
+
+
+@pytest.mark.parametrize("form", ["FP32_SPARSE", "BF16X2_DENSE", "I8X3_DENSE"])
+def test_no_run_allocates_after_an_index_is_attached(env, form):
+    from hfx_amd import check, lib
+
+    pl, ctx, db, sp = env
+    pl.BatchSearch(ctx, db, sp, eps=3.0, topn=5, index=pl.PepIndex(ctx, db)).run()  # code is loaded
+    b = pl.BatchSearch(ctx, db, sp, eps=3.0, topn=5)
+    b.set_precision(getattr(b, form))
+    index = pl.PepIndex(ctx, db)
+    check(lib().hfx_batch_use_index(b.h, index.h), "hfx_batch_use_index")
+    before = free(pl)
+    b.run()
+    b.stream.sync()
+    assert free(pl) == before
