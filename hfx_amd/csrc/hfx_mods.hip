@@ -164,13 +164,22 @@ struct ModBits {
     }
 };
 
+/* the windows of a part of the modifications, [m0, m0 + M) of num_mod: the i-th of
+ * them, spectrum by spectrum */
+struct ModPart {
+    uint32_t m0, M, num_mod;
+    uint64_t pairs; /* spectra x M */
+    __device__ __forceinline__ uint64_t window(uint64_t i) const { return i / M * num_mod + m0 + i % M; }
+};
+
 /* modable peptides of every (spectrum, modification) window */
-__global__ void k_mod_counts(uint32_t *cnt, const uint32_t *begin, const uint32_t *end,
-                             uint32_t num_mod, uint64_t pairs, ModBits mb)
+__global__ void k_mod_counts(uint32_t *cnt, const uint32_t *begin, const uint32_t *end, ModPart p,
+                             ModBits mb)
 {
-    const uint64_t pr = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (pr >= pairs) return;
-    const uint32_t m = (uint32_t)(pr % num_mod), b = begin[pr], e = end[pr];
+    const uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= p.pairs) return;
+    const uint64_t pr = p.window(i);
+    const uint32_t m = (uint32_t)(i % p.M), b = begin[pr], e = end[pr];
     cnt[pr] = b < e ? mb.below(m, e) - mb.below(m, b) : 0u;
 }
 
@@ -186,12 +195,12 @@ __global__ void __launch_bounds__(256)
     k_mod_rows(uint32_t *__restrict__ out_pep, uint32_t *__restrict__ out_mod,
                uint32_t *__restrict__ out_cnt, const uint64_t *off,
                const uint32_t *__restrict__ idx_sorted, const uint32_t *begin, const uint32_t *end,
-               uint32_t num_mod, uint64_t pairs, const uint32_t *__restrict__ pcnt, uint32_t num_ma,
-               ModBits mb)
+               ModPart part, const uint32_t *__restrict__ pcnt, uint32_t num_ma, ModBits mb)
 {
-    const uint64_t pr = (uint64_t)blockIdx.x * 4 + threadIdx.x / HFX_WAVE;
-    if (pr >= pairs) return;
-    const uint32_t m = (uint32_t)(pr % num_mod), lane = hfx_lane();
+    const uint64_t i = (uint64_t)blockIdx.x * 4 + threadIdx.x / HFX_WAVE;
+    if (i >= part.pairs) return;
+    const uint64_t pr = part.window(i);
+    const uint32_t m = (uint32_t)(i % part.M), lane = hfx_lane();
     const uint32_t na = NA ? NA : num_ma;
     const uint32_t b = begin[pr], e = end[pr];
     const uint64_t *bits = mb.bits + (size_t)m * mb.W;
@@ -217,7 +226,7 @@ __global__ void __launch_bounds__(256)
                 for (uint32_t a = 0; a < (NA ? NA : 10u); ++a)
                     if (a < na) c[a] = from[a];
                 out_pep[p] = idx_sorted[k];
-                out_mod[p] = m;
+                out_mod[p] = part.m0 + m;
 #pragma unroll
                 for (uint32_t a = 0; a < (NA ? NA : 10u); ++a)
                     if (a < na) out_cnt[p * na + a] = c[a];
@@ -304,23 +313,44 @@ extern "C" uint32_t findModablePeptides(
         }
         for (uint32_t i = 0; i < g; ++i) npos = max(npos, ((uint32_t *)h)[i]);
     }
+    /* The bits and ranks take 12 bytes for 64 positions and a modification, however
+     * few of them a window holds: so many modifications at a time that they take no
+     * more than 64 MiB, or than the rows of all candidates would. */
     const uint32_t W = npos / 64 + 1;
+    const uint64_t room = max((uint64_t)num_cand_total * (20 + 4 * num_ma), 64ull << 20);
+    const uint32_t M = (uint32_t)min((uint64_t)num_mod, max(room / (12ull * W), 1ull));
     void *p;
-    const size_t words = (size_t)W * num_mod;
+    const size_t words = (size_t)W * M;
     const size_t bytes = words * 12 + (pairs + 1) * 8 + pairs * 4 + (size_t)npos * 4 * num_ma + 64;
     if (hfx_ctx_scratch(ctx, HFX_SLOT_MODS, bytes, &p) != HFX_OK) return 0;
     uint64_t *off = (uint64_t *)p, *bits = off + pairs + 1;
     uint32_t *rank = (uint32_t *)(bits + words), *cnt = rank + words, *pcnt = cnt + pairs;
     const ModBits mb{bits, rank, W};
-    hipLaunchKernelGGL(k_mod_bits, dim3((W + 3) / 4), t, 0, 0, pcnt, bits, W, d_pep_idx_r_sorted_raw,
-                       npos, d_ions, d_tc, d_tn, d_ma, num_ma, d_mod_ma_count, num_mod);
-    hipLaunchKernelGGL(k_mod_rank, dim3(num_mod), dim3(1024), 0, 0, rank, bits, W);
-    hipLaunchKernelGGL(k_mod_counts, dim3((uint32_t)((pairs + 255) / 256)), t, 0, 0, cnt, d_begin_raw,
-                       d_end_raw, num_mod, pairs, mb);
+    auto part = [&](uint32_t m0) {
+        const uint32_t m = min(M, num_mod - m0);
+        return ModPart{m0, m, num_mod, (uint64_t)num_spec * m};
+    };
+    auto find = [&](const ModPart &q) {
+        hipLaunchKernelGGL(k_mod_bits, dim3((W + 3) / 4), t, 0, 0, pcnt, bits, W, d_pep_idx_r_sorted_raw,
+                           npos, d_ions, d_tc, d_tn, d_ma, num_ma,
+                           d_mod_ma_count + (size_t)q.m0 * num_ma, q.M);
+        hipLaunchKernelGGL(k_mod_rank, dim3(q.M), dim3(1024), 0, 0, rank, bits, W);
+    };
+    for (uint64_t m0 = 0; m0 < num_mod; m0 += M) {
+        const ModPart q = part((uint32_t)m0);
+        find(q);
+        hipLaunchKernelGGL(k_mod_counts, dim3((uint32_t)((q.pairs + 255) / 256)), t, 0, 0, cnt,
+                           d_begin_raw, d_end_raw, q, mb);
+    }
     if (hfx_scan_offsets(ctx, off, cnt, (uint32_t)pairs, nullptr) != HFX_OK) return 0;
-    hipLaunchKernelGGL(num_ma == 4 ? k_mod_rows<4> : k_mod_rows<0>, dim3((uint32_t)((pairs + 3) / 4)), t, 0, 0, d_out_pep_idx_raw,
-                       d_out_pep_mod_idx_raw, d_out_pep_ma_count_raw, off, d_pep_idx_r_sorted_raw,
-                       d_begin_raw, d_end_raw, num_mod, pairs, pcnt, num_ma, mb);
+    for (uint64_t m0 = 0; m0 < num_mod; m0 += M) {
+        const ModPart q = part((uint32_t)m0);
+        if (M < num_mod) find(q);
+        hipLaunchKernelGGL(num_ma == 4 ? k_mod_rows<4> : k_mod_rows<0>,
+                           dim3((uint32_t)((q.pairs + 3) / 4)), t, 0, 0, d_out_pep_idx_raw,
+                           d_out_pep_mod_idx_raw, d_out_pep_ma_count_raw, off, d_pep_idx_r_sorted_raw,
+                           d_begin_raw, d_end_raw, q, pcnt, num_ma, mb);
+    }
     hipLaunchKernelGGL(k_mod_valid_scan, gs, t, 0, 0, d_out_spec_num_valid_scan, off, num_mod,
                        num_spec);
     uint64_t total = 0;
