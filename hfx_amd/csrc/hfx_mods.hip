@@ -81,6 +81,16 @@ __device__ __forceinline__ void d_unrank_comb(const uint32_t *tab, uint32_t *ans
     }
 }
 
+/* A kernel's instance for na modable acids: every number that prepare_ions packs (1
+ * to 7) has its own, whose loops over the acids keep their values in registers; up to
+ * 10, which these steps take, share one.  Finding the rows and unranking for 1,500
+ * spectra, us: one acid 93 and 17 by the shared instance, 90 and 16 by its own; three
+ * 124 and 36, 116 and 33; seven 337 and 173, 292 and 130. */
+#define MOD_NA(k, na) \
+    ((na) == 1 ? k<1> : (na) == 2 ? k<2> : (na) == 3 ? k<3> : (na) == 4 ? k<4> : (na) == 5 ? k<5> \
+     : (na) == 6 ? k<6> : (na) == 7 ? k<7> : k<0>)
+static_assert(HFX_MAX_MA == 7, "an instance for each packed number of acids");
+
 /* ------------------------------------------------------------------ */
 /* findModablePeptides                                                   */
 /* ------------------------------------------------------------------ */
@@ -190,7 +200,7 @@ __global__ void k_mod_counts(uint32_t *cnt, const uint32_t *begin, const uint32_
  * and 34 modifications; writing, scanning and compacting all of them took 1,300
  * us; the bits, their ranks, the counts and their scan take 60, this 78 (190
  * with a read of the bits, and of each acid's count, after every store). */
-template <uint32_t NA> /* num_ma, or 0: any */
+template <uint32_t NA> /* num_ma, or 0: any up to 10 */
 __global__ void __launch_bounds__(256)
     k_mod_rows(uint32_t *__restrict__ out_pep, uint32_t *__restrict__ out_mod,
                uint32_t *__restrict__ out_cnt, const uint64_t *off,
@@ -343,11 +353,11 @@ extern "C" uint32_t findModablePeptides(
                            d_begin_raw, d_end_raw, q, mb);
     }
     if (hfx_scan_offsets(ctx, off, cnt, (uint32_t)pairs, nullptr) != HFX_OK) return 0;
+    const auto rows = MOD_NA(k_mod_rows, num_ma);
     for (uint64_t m0 = 0; m0 < num_mod; m0 += M) {
         const ModPart q = part((uint32_t)m0);
         if (M < num_mod) find(q);
-        hipLaunchKernelGGL(num_ma == 4 ? k_mod_rows<4> : k_mod_rows<0>,
-                           dim3((uint32_t)((q.pairs + 3) / 4)), t, 0, 0, d_out_pep_idx_raw,
+        hipLaunchKernelGGL(rows, dim3((uint32_t)((q.pairs + 3) / 4)), t, 0, 0, d_out_pep_idx_raw,
                            d_out_pep_mod_idx_raw, d_out_pep_ma_count_raw, off, d_pep_idx_r_sorted_raw,
                            d_begin_raw, d_end_raw, q, pcnt, num_ma, mb);
     }
@@ -578,7 +588,7 @@ extern "C" void genModCands(uint32_t *d_out_mpep_unrank, const uint32_t *d_mod_m
         hfx_set_error("genModCands: num_ma %u outside 1..10", mod_num_ma);
         return;
     }
-    hipLaunchKernelGGL(mod_num_ma == 4 ? k_gen_mod_cands<4> : k_gen_mod_cands<0>, dim3((total + 255) / 256), dim3(256), 0, 0,
+    hipLaunchKernelGGL(MOD_NA(k_gen_mod_cands, mod_num_ma), dim3((total + 255) / 256), dim3(256), 0, 0,
                        d_out_mpep_unrank, d_mod_ma_count, d_mpep_ith_valid, d_mpep_rank,
                        d_mpep_mod_ma_count_sum_scan, d_pep_mod_idx, d_pep_ma_count,
                        d_pep_ma_num_comb_scan, total, mod_num_ma);
