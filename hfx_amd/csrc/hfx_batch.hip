@@ -937,13 +937,14 @@ struct hfx_batch {
     uint32_t *ord_cnt, *ord_tmp;
     uint64_t *ord_off;
     uint32_t precision; /* HFX_BATCH_FP32_SPARSE, _BF16X2_DENSE or _I8X3_DENSE */
-    uint32_t CH;        /* dense: candidates per work item */
+    uint32_t CH;        /* rows, dense: candidates per work item */
     uint8_t *dn_scratch; /* dense: hi/lo spectra, blocks (allocated with the dense form) */
     uint32_t *dn_bstart; /* dense: [S + 1] block starts in order (S past the last block) */
     uint32_t *cut_seg, *cut_n;
     uint64_t *cut_off;
     uint32_t nseg;
     bool dense_set;      /* a dense form was chosen since the plan */
+    bool chunk_set;      /* CH is the caller's or the tuner's */
     bool rows_tried, use_rows; /* scores come from the database's rows */
     RowSet *rs;                /* the set they are in, and what this batch reads of it */
     hfx_rows rows;
@@ -1028,19 +1029,34 @@ extern "C" int hfx_batch_use_index(hfx_batch *b, const hfx_pepix *ix)
 }
 
 /* Shape-bucketed autotuner results of this process: (S bucket, P bucket, L)
- * -> (G, C, threads). */
+ * -> (G, C, threads) of the ion-list kernel; the chunk of each precision form over
+ * rows, and of the dense forms' ladder kernels. */
+typedef std::tuple<int, int, uint32_t> tune_shape;
 static std::mutex g_tune_mu;
-static std::map<std::tuple<int, int, uint32_t>, std::tuple<uint32_t, uint32_t, uint32_t>> g_tune;
-static std::map<std::tuple<int, int, uint32_t>, uint32_t> g_tune_dense, g_tune_dense8;
+static std::map<tune_shape, std::tuple<uint32_t, uint32_t, uint32_t>> g_tune;
+struct TuneChunks {
+    const char *name; /* in the cache file */
+    uint32_t precision;
+    bool rows;
+    std::map<tune_shape, uint32_t> chunk;
+};
+static TuneChunks g_tune_chunks[] = {{"fp32", HFX_BATCH_FP32_SPARSE, true, {}},
+                                     {"bf16", HFX_BATCH_BF16X2_DENSE, true, {}},
+                                     {"int8", HFX_BATCH_I8X3_DENSE, true, {}},
+                                     {"bf16-ladder", HFX_BATCH_BF16X2_DENSE, false, {}},
+                                     {"int8-ladder", HFX_BATCH_I8X3_DENSE, false, {}}};
+/* null: the form without rows has no chunk */
+static std::map<tune_shape, uint32_t> *tune_chunks(uint32_t precision, bool rows)
+{
+    for (TuneChunks &t : g_tune_chunks)
+        if (t.precision == precision && t.rows == rows) return &t.chunk;
+    return nullptr;
+}
 
 /* the two dense forms share the ladders, block cut and work items */
 static inline bool bt_is_dense(uint32_t precision)
 {
     return precision == HFX_BATCH_BF16X2_DENSE || precision == HFX_BATCH_I8X3_DENSE;
-}
-static std::map<std::tuple<int, int, uint32_t>, uint32_t> &bt_tune_dense(uint32_t precision)
-{
-    return precision == HFX_BATCH_I8X3_DENSE ? g_tune_dense8 : g_tune_dense;
 }
 /* the dense forms' per-batch scratch: the larger of the two */
 static size_t bt_dense_scratch(uint32_t S)
@@ -1065,7 +1081,7 @@ static bool tune_dense_ok(uint32_t precision, uint32_t CH)
     return CH >= step && CH % step == 0 && CH <= 8192;
 }
 
-/* candidates a dense work item takes, untuned: by the rows the blocks read --
+/* candidates a work item takes over rows, untuned: by the rows the blocks read --
  * about a twelfth of the pairs, but every row of the database's two usual
  * levels once the batch covers it */
 static uint32_t bt_chunk(const hfx_batch *b)
@@ -1074,7 +1090,7 @@ static uint32_t bt_chunk(const hfx_batch *b)
     return hfx_rows_chunk(rows, (uint32_t)hfx_ctx_num_cus(b->ctx));
 }
 
-static std::tuple<int, int, uint32_t> tune_key(const hfx_batch *b)
+static tune_shape tune_key(const hfx_batch *b)
 {
     auto lg = [](uint64_t v) { int k = 0; while (v > 1) { v >>= 1; ++k; } return k; };
     return std::make_tuple(lg(b->S), lg(b->total), b->L);
@@ -1082,8 +1098,8 @@ static std::tuple<int, int, uint32_t> tune_key(const hfx_batch *b)
 
 /* The tuned shapes persist across processes when HFX_TUNE_CACHE names a
  * file: one line a shape, "sparse <S bucket> <pairs bucket> <levels> <G> <C>
- * <threads>", "bf16 ... <chunk>" or "int8 ... <chunk>" (other lines are
- * ignored).  It is read when a lookup first sees the path (its entries
+ * <threads>", or "fp32 ... <chunk>", "bf16", "int8" over rows, "bf16-ladder",
+ * "int8-ladder" without (other lines are ignored).  It is read when a lookup first sees the path (its entries
  * replace this process's for the same shapes) and rewritten whole, through a
  * temporary file and a rename, after each tuning.  Callers hold g_tune_mu. */
 static std::string g_tune_path;
@@ -1107,10 +1123,9 @@ static void tune_load_locked()
          * file) are skipped, never launched */
         if (n == 7 && !strcmp(kind, "sparse") && tune_sparse_ok(a, c, t))
             g_tune[key] = std::make_tuple((uint32_t)a, (uint32_t)c, (uint32_t)t);
-        else if (n == 5 && !strcmp(kind, "bf16") && tune_dense_ok(HFX_BATCH_BF16X2_DENSE, a))
-            g_tune_dense[key] = a;
-        else if (n == 5 && !strcmp(kind, "int8") && tune_dense_ok(HFX_BATCH_I8X3_DENSE, a))
-            g_tune_dense8[key] = a;
+        else if (n == 5)
+            for (TuneChunks &k : g_tune_chunks)
+                if (!strcmp(kind, k.name) && tune_dense_ok(k.precision, a)) k.chunk[key] = a;
     }
     fclose(f);
 }
@@ -1126,13 +1141,27 @@ static void tune_save_locked()
         fprintf(f, "sparse %d %d %u %u %u %u\n", std::get<0>(e.first), std::get<1>(e.first),
                 std::get<2>(e.first), std::get<0>(e.second), std::get<1>(e.second),
                 std::get<2>(e.second));
-    for (const auto &e : g_tune_dense)
-        fprintf(f, "bf16 %d %d %u %u\n", std::get<0>(e.first), std::get<1>(e.first),
-                std::get<2>(e.first), e.second);
-    for (const auto &e : g_tune_dense8)
-        fprintf(f, "int8 %d %d %u %u\n", std::get<0>(e.first), std::get<1>(e.first),
-                std::get<2>(e.first), e.second);
+    for (const TuneChunks &k : g_tune_chunks)
+        for (const auto &e : k.chunk)
+            fprintf(f, "%s %d %d %u %u\n", k.name, std::get<0>(e.first), std::get<1>(e.first),
+                    std::get<2>(e.first), e.second);
     if (fclose(f) == 0) rename(tmp.c_str(), g_tune_path.c_str());
+}
+
+/* The chunk of the current form, unless the caller or the tuner set one: tuned for
+ * batches of this shape, or by the rows it reads; 256 for the ladder kernels.  Until
+ * the rows are decided on they are taken to be there. */
+static void bt_pick_chunk(hfx_batch *b)
+{
+    if (b->chunk_set) return;
+    const bool rows = b->rows_tried ? b->use_rows : b->sp.x_stride <= RW_MAXK;
+    b->CH = rows ? bt_chunk(b) : 256u;
+    std::lock_guard<std::mutex> lk(g_tune_mu);
+    tune_load_locked();
+    if (auto *m = tune_chunks(b->precision, rows)) {
+        auto it = m->find(tune_key(b));
+        if (it != m->end()) b->CH = it->second;
+    }
 }
 
 /* the form of the peptide index the current precision reads */
@@ -1186,6 +1215,7 @@ static bool bt_rows(const hfx_batch *b) { return b->use_rows && bt_rows_bufs(b);
 /* the index, and its rows where they fit (decided once a plan, index and form, never
  * under capture: a batch captured by its caller without a run before it keeps
  * the other kernels) */
+static int bt_ready_rows(hfx_batch *b, hipStream_t st);
 static int bt_ready(hfx_batch *b, hipStream_t st)
 {
     int rc = bt_need_index(b, st);
@@ -1196,6 +1226,12 @@ static int bt_ready(hfx_batch *b, hipStream_t st)
         (void)hipGetLastError();
         return HFX_OK;
     }
+    rc = bt_ready_rows(b, st);
+    bt_pick_chunk(b);
+    return rc;
+}
+static int bt_ready_rows(hfx_batch *b, hipStream_t st)
+{
     b->rows_tried = true;
     if (b->sp.x_stride > RW_MAXK || b->db.num_pep == 0) return HFX_OK;
     size_t fr = 0, tot = 0;
@@ -1373,8 +1409,8 @@ extern "C" int hfx_batch_plan(hfx_batch *b, const hfx_db *db, const hfx_spectra 
     b->G = 8;
     b->C = 64;
     b->threads = 512;
-    b->CH = bt_chunk(b);
     b->precision = HFX_BATCH_FP32_SPARSE;
+    bt_pick_chunk(b);
     {
         std::lock_guard<std::mutex> lk(g_tune_mu);
         tune_load_locked();
@@ -1627,21 +1663,18 @@ extern "C" int hfx_batch_set_precision(hfx_batch *b, uint32_t precision)
     int rc;
     if (bt_is_dense(precision) && (rc = bt_dense_alloc(b))) return rc;
     if (bt_is_dense(precision)) b->dense_set = true;
-    if (bt_is_dense(precision) && precision != b->precision) {
-        /* the tuned chunk of this form for batches of this shape, if any */
-        std::lock_guard<std::mutex> lk(g_tune_mu);
-        tune_load_locked();
-        auto &m = bt_tune_dense(precision);
-        auto jt = m.find(tune_key(b));
-        b->CH = jt != m.end() ? jt->second : bt_chunk(b);
-    }
-    if (precision != b->precision && b->exec) {
+    const bool other = precision != b->precision;
+    if (other && b->exec) {
         (void)hipGraphExecDestroy(b->exec);
         b->exec = nullptr;
         (void)hipGraphDestroy(b->graph);
         b->graph = nullptr;
     }
     b->precision = precision;
+    if (other) {
+        b->chunk_set = false;
+        bt_pick_chunk(b);
+    }
     return bt_ready_attached(b, nullptr);
 }
 
@@ -1676,8 +1709,9 @@ extern "C" int hfx_batch_replay(hfx_batch *b, void *stream)
 
 /* Times the scoring kernel of the planned batch for each configuration in a
  * small grid and keeps the fastest; the choice is remembered for batches of
- * the same shape bucket in this process.  Sparse form: (G, C, threads);
- * dense form: the chunk of candidates per work item. */
+ * the same shape bucket in this process.  Over rows, any form, and in the dense
+ * ones: the chunk of candidates per work item; the FP32 form over ion lists: (G, C,
+ * threads). */
 extern "C" int hfx_batch_autotune(hfx_batch *b, void *stream, uint32_t *out_cfg)
 {
     HFX_REQUIRE(b && b->planned, HFX_ERR_ARG, "hfx_batch_autotune: batch not planned");
@@ -1707,9 +1741,17 @@ extern "C" int hfx_batch_autotune(hfx_batch *b, void *stream, uint32_t *out_cfg)
     };
     float best = 1e30f;
     uint32_t bG = b->G, bC = b->C, bT = b->threads, bCH = b->CH;
-    if (bt_is_dense(b->precision)) {
-        const uint32_t CHs[5] = {512, 1024, 2048, 4096, 8192};
-        for (uint32_t CH : CHs) {
+    const bool rows = bt_rows(b), chunks = rows || bt_is_dense(b->precision);
+    if (chunks) {
+        /* the untuned one is among them */
+        const uint32_t own = rows ? bt_chunk(b) : 256u;
+        const uint32_t CHs[6] = {512, 1024, 2048, 4096, 8192, own};
+        for (uint32_t i = 0; i < 6; ++i) {
+            const uint32_t CH = CHs[i];
+            bool seen = false;
+            for (uint32_t j = 0; j < i; ++j)
+                seen |= rows ? hfx_rows_item_tiles(CHs[j]) == hfx_rows_item_tiles(CH) : CHs[j] == CH;
+            if (seen) continue;
             b->CH = CH;
             float ms = 0;
             if ((rc = time2(&ms))) return rc;
@@ -1734,10 +1776,11 @@ extern "C" int hfx_batch_autotune(hfx_batch *b, void *stream, uint32_t *out_cfg)
     b->C = bC;
     b->threads = bT;
     b->CH = bCH;
+    b->chunk_set = chunks;
     {
         std::lock_guard<std::mutex> lk(g_tune_mu);
         tune_load_locked();
-        if (bt_is_dense(b->precision)) bt_tune_dense(b->precision)[tune_key(b)] = bCH;
+        if (chunks) (*tune_chunks(b->precision, rows))[tune_key(b)] = bCH;
         else g_tune[tune_key(b)] = std::make_tuple(bG, bC, bT);
         tune_save_locked();
     }
@@ -1755,7 +1798,7 @@ extern "C" int hfx_batch_autotune(hfx_batch *b, void *stream, uint32_t *out_cfg)
         if (bt_is_dense(b->precision)) {
             out_cfg[0] = 0;
             out_cfg[1] = bCH;
-            out_cfg[2] = 1024u; /* workgroup threads of both dense kernels */
+            out_cfg[2] = 1024u; /* workgroup threads of both ladder kernels */
         }
     }
     return HFX_OK;
@@ -1803,6 +1846,7 @@ extern "C" int hfx_batch_set_config(hfx_batch *b, uint32_t G, uint32_t C, uint32
                     "hfx_batch_set_config: dense chunk must be a multiple of %u in %u..8192",
                     step, step);
         b->CH = C;
+        b->chunk_set = true;
         return HFX_OK;
     }
     HFX_REQUIRE(tune_sparse_ok(G, C, threads), HFX_ERR_ARG,

@@ -31,6 +31,7 @@ struct hfx_rows {
 uint32_t hfx_rows_tiles(uint32_t num_pep);
 uint32_t hfx_rows_groups(uint32_t x_stride);
 uint32_t hfx_rows_chunk(uint64_t rows, uint32_t cus);
+uint32_t hfx_rows_item_tiles(uint32_t CH);
 /* spectra that are scored without rows (hfx_xcorr_rest), in any order */
 struct hfx_rest {
     uint32_t *list, *count; /* [S]; cleared before hfx_rows_split (hfx_cut_bufs) */
@@ -48,7 +49,8 @@ int hfx_rows_split(int mode, const hfx_spectra *sp, uint8_t *planes, float *qs, 
 int hfx_rows_build(uint32_t cus, const hfx_db *db, const hfx_rows *r, const uint32_t *flags,
                    void *stream);
 /* work items of the blocks bstart (num_spec + 1 entries, empty blocks at the
- * end) of CH candidates each, in scratch of hfx_rows_items_bytes(num_spec) */
+ * end) of hfx_rows_item_tiles(CH) tiles each, in scratch of
+ * hfx_rows_items_bytes(num_spec) */
 size_t hfx_rows_items_bytes(uint32_t S);
 int hfx_rows_blocks(hfx_ctx *ctx, void *scratch, const uint32_t *order, const uint32_t *bstart,
                     const uint32_t *begin, const uint32_t *num, const hfx_spectra *sp, uint32_t CH,

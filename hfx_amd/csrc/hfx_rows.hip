@@ -904,6 +904,14 @@ uint32_t hfx_rows_chunk(uint64_t rows, uint32_t cus)
     const uint64_t step = RM_WAVES * RM_T * RW_ROWS; /* every wave busy */
     return (uint32_t)std::min<uint64_t>(std::max<uint64_t>((c + step - 1) / step * step, step), 8192);
 }
+/* the tiles of a work item of CH candidates: a round of a workgroup's waves at least.
+ * The contraction of 20,000 spectra, three digits, by candidates an item: 512 1,216 us,
+ * 768 1,018, 1024 925, 1536 912, 2048 864, 2304 and 3072 897, 4096 911, 6144 975, 8192
+ * 1,040; whole rounds past the first gain nothing, 2048 is no multiple of 768. */
+uint32_t hfx_rows_item_tiles(uint32_t CH)
+{
+    return std::max((CH + RW_ROWS - 1) / RW_ROWS, (uint32_t)(RM_WAVES * RM_T));
+}
 
 int hfx_rows_split(int mode, const hfx_spectra *sp, uint8_t *planes, float *qs, uint32_t *lvl,
                    const hfx_rest *rest, uint32_t have, float2 *norms, float *scores,
@@ -962,7 +970,7 @@ int hfx_rows_blocks(hfx_ctx *ctx, void *scratch, const uint32_t *order, const ui
     uint64_t *off;
     rw_items(scratch, B, &tbeg, &tend, &binfo, &items, &off, &counter);
     hipStream_t st = hfx_stream(stream);
-    const uint32_t CT = std::max(CH / RW_ROWS, 1u);
+    const uint32_t CT = hfx_rows_item_tiles(CH);
     hipLaunchKernelGGL(k_rw_blocks, dim3((B + 15) / 16), dim3(256), 0, st, tbeg, tend, binfo, items,
                        counter, order, bstart, begin, num, *sp, B, CT);
     int rc = hfx_scan_offsets(ctx, off, items, B, stream);
@@ -1003,7 +1011,7 @@ int hfx_rows_scores(hfx_ctx *ctx, int mode, void *scratch, float *d_scores, cons
     a.order = order;
     a.bstart = bstart;
     a.B = S;
-    a.CT = std::max(CH / RW_ROWS, 1u);
+    a.CT = hfx_rows_item_tiles(CH);
     a.tbeg = tbeg;
     a.tend = tend;
     a.binfo = binfo;

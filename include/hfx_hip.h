@@ -648,10 +648,12 @@ int hfx_batch_set_precision(hfx_batch *b, uint32_t precision);
 /* capture hfx_batch_run on a non-null stream into a graph; replay it */
 int hfx_batch_capture(hfx_batch *b, void *stream);
 int hfx_batch_replay(hfx_batch *b, void *stream);
-/* time the scoring kernel over (spectra per block G, tile length C,
- * workgroup threads) -- dense form: candidates per work item C -- and keep
- * the fastest; out_cfg = {G, C, threads} ({0, C, workgroup threads} for the
- * dense forms: 1024 in both) */
+/* time the scoring kernel over its launch shapes and keep the fastest: over the
+ * index's rows, in every form, and in the dense forms the candidates a work item
+ * takes (over rows at least 768); without rows, FP32 form, (spectra per
+ * block G, tile length C, workgroup threads).  out_cfg = {0, candidates, 1024 (the
+ * threads of both ladder kernels' workgroups; 768 over rows)} for the dense forms,
+ * {G, C, threads} for the FP32 form, which rows do not use and leave as they are. */
 int hfx_batch_autotune(hfx_batch *b, void *stream, uint32_t *out_cfg);
 int hfx_batch_set_config(hfx_batch *b, uint32_t G, uint32_t C, uint32_t threads);
 /* one run, phase by phase, with event timings in ms (5 entries): {windows,
