@@ -17,7 +17,8 @@
  *
  * In FP64 the window sums are differences of the bins' prefix sums, as long as
  * every non-zero a is at least 2^-13 (its square at least 6e-12 of its region's
- * largest intensity): those sums are exact in any order.
+ * largest intensity) and all of them add up to less than 2^17 (2,621 bins at the
+ * largest value, 50): those sums are exact in any order.
  * Otherwise, and in FP32, they run over the bins that hold a peak only: a is nowhere
  * negative, so the zeros between them leave a left-to-right sum unchanged to
  * the last bit, and a spectrum of a few hundred peaks over 2,000 bins has about
@@ -174,11 +175,11 @@ __global__ void __launch_bounds__(PP_THREADS, PER <= 9 ? 8 : 6)
                 }
                 if (__ballot(!ok) && lane == 0) sh_odd = 1;
                 __syncthreads(); /* the bins have been read: their prefix sums may take their place */
-                whole = sh_odd == 0;
+                const double mine = lane < nch ? tot[lane] : 0.0;
+                const double run = pp_wave_incl(mine);
+                whole = sh_odd == 0 && pp_take(run, nch - 1) < 0x1p17;
                 if (whole) {
                     double *pb = (double *)sbin; /* sums of the bins below i <= nch * 64 */
-                    const double mine = lane < nch ? tot[lane] : 0.0;
-                    const double run = pp_wave_incl(mine);
 #pragma unroll
                     for (uint32_t q = 0; q < PER; ++q) {
                         const uint32_t c = wave + q * PP_WAVES;
