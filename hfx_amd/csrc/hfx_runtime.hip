@@ -166,7 +166,8 @@ hipError_t hfx_device_malloc(void **p, size_t bytes)
     hipError_t e = hipMalloc(p, bytes);
     if (e != hipErrorOutOfMemory) return e;
     (void)hipGetLastError();
-    return hfx_spare_release() ? hipMalloc(p, bytes) : e;
+    if (hfx_spare_release() && (e = hipMalloc(p, bytes)) != hipSuccess) (void)hipGetLastError();
+    return e;
 }
 
 int hfx_ctx_pinned(hfx_ctx *ctx, size_t bytes, void **out)

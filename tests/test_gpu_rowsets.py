@@ -83,3 +83,35 @@ def test_another_database_at_the_same_address_has_its_own_rows(orc, form):
     bound = (2.0**-16 + 210 * 2.0**-24) * scale + np.repeat(np.abs(x).max(1), res.num) * 50 * 8000 / 8355711
     assert (np.abs(res.scores - exact) <= bound + 1e-6).all()
     assert old.index is not None
+
+
+def test_rows_go_where_memory_is_short_and_come_back(orc):
+    """An allocation that cannot be had (a PiB) takes the rows that no batch uses, and those that
+    hfx_xcorr_sparse keeps; batches and calls after it write them again."""
+    from hfx_amd import lib
+    from hfx_amd import pipeline as pl
+
+    hdb = database(pl, 100_003, seed=14, longest=20)
+    x, lens, zmax, mass = spectra(pl, hdb, 4000, 600, seed=15)
+    ctx, db, sp = pl.Ctx(0), pl.DeviceDB(hdb), Spectra(pl, x, lens, np.minimum(zmax, 2), mass)
+    index = pl.PepIndex(ctx, db)
+
+    def run(b):
+        b.run()
+        return b.results(keep_scores=True).scores
+
+    b = pl.BatchSearch(ctx, db, sp, eps=3.0, topn=5, index=index)
+    plain = pl.PlainSearch(ctx, db, sp, eps=3.0, topn=5)
+    want, score = run(b), plain.run(keep_scores=True).scores
+    rows = 2 * ((100_003 + 15) // 16) * 9 * 1024
+    for _ in range(2):
+        full = free(pl)
+        p = C.c_void_p()
+        assert lib().hfx_malloc(C.byref(p), 1 << 50) != 0
+        assert free(pl) - full > (rows if b is None else 0)   # the plain call's; the idle set's too
+        if b is not None:
+            assert np.array_equal(run(b), want)               # a batch keeps the rows it uses
+            b = None
+        assert np.array_equal(plain.run(keep_scores=True).scores, score)
+    again = pl.BatchSearch(ctx, db, sp, eps=3.0, topn=5, index=index)
+    assert np.array_equal(run(again), want)
