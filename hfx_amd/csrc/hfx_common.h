@@ -95,13 +95,13 @@ enum {
 /* Scratch owned by a context: grown on demand, never shrunk. */
 int hfx_ctx_scratch(hfx_ctx *ctx, int slot, size_t bytes, void **out);
 /* the same for memory a caller can do without (HFX_SLOT_ROWS, _ROWS2), of the size
- * asked for: null (and no error left behind) when it would have to grow while
- * `stream` is being captured, past an eighth of the device's memory or past half
- * of what is free.  Only between hfx_ctx_spare_begin and _end, outside which
- * hfx_spare_release may take it back. */
+ * asked for: null (and no error left behind) when it would have to grow past an
+ * eighth of the device's memory or past half of what is free.  Only between
+ * hfx_ctx_spare_begin and _end, outside which hfx_spare_release may take it back, and
+ * never for a captured stream, whose graph would outlast it. */
 void hfx_ctx_spare_begin(hfx_ctx *ctx);
 void hfx_ctx_spare_end(hfx_ctx *ctx);
-void *hfx_ctx_scratch_spare(hfx_ctx *ctx, int slot, size_t bytes, void *stream);
+void *hfx_ctx_scratch_spare(hfx_ctx *ctx, int slot, size_t bytes);
 /* frees the current device's memory that nothing needs at the moment: spare
  * scratch of its contexts, theoretical rows that no batch uses.  True if there
  * was any. */

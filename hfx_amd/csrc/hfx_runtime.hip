@@ -101,14 +101,12 @@ int hfx_ctx_scratch(hfx_ctx *ctx, int slot, size_t bytes, void **out)
     return HFX_OK;
 }
 
-void *hfx_ctx_scratch_spare(hfx_ctx *ctx, int slot, size_t bytes, void *stream)
+void *hfx_ctx_scratch_spare(hfx_ctx *ctx, int slot, size_t bytes)
 {
     if (slot < 0 || slot >= HFX_SCRATCH_SLOTS) return nullptr;
     if (ctx->scratch[slot] && ctx->scratch_bytes[slot] >= bytes) return ctx->scratch[slot];
-    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
     size_t fr = 0, tot = 0;
-    if (hipStreamIsCapturing(hfx_stream(stream), &cs) != hipSuccess ||
-        cs != hipStreamCaptureStatusNone || hipMemGetInfo(&fr, &tot) != hipSuccess) {
+    if (hipMemGetInfo(&fr, &tot) != hipSuccess) {
         (void)hipGetLastError();
         return nullptr;
     }

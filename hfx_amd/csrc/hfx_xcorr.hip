@@ -423,7 +423,7 @@ static bool xr_pays(uint64_t total, uint32_t tiles)
 }
 
 /* *taken = 0: nothing done (too few pairs, rows longer than the form's, no
- * memory to spare) */
+ * memory to spare, a captured stream) */
 static int xcorr_rows(hfx_ctx *ctx, float *d_scores, const uint64_t *d_off,
                       const uint32_t *d_begin, const uint32_t *d_num, uint64_t total,
                       const hfx_db *db, const hfx_spectra *sp, void *stream, int *taken)
@@ -438,6 +438,14 @@ static int xcorr_rows(hfx_ctx *ctx, float *d_scores, const uint64_t *d_off,
     const uint32_t S = sp->num_spec;
     const uint32_t nt = hfx_rows_tiles(db->num_pep), G = hfx_rows_groups(sp->x_stride);
     if (!xr_pays(total, nt) || sp->x_stride > RW_MAXK || db->num_pep == 0) return HFX_OK;
+    /* a captured call keeps the packed kernel: a graph would hold these buffers, which
+     * a larger call replaces and a shortage of memory takes back */
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(hfx_stream(stream), &cs) != hipSuccess ||
+        cs != hipStreamCaptureStatusNone) {
+        (void)hipGetLastError();
+        return HFX_OK;
+    }
     const uint64_t nf = (uint64_t)HFX_MAX_CHARGE * nt;
     if (nf >= 0xffffffffull) return HFX_OK;
     /* the block cut never takes more rows than the windows one by one */
@@ -453,9 +461,9 @@ static int xcorr_rows(hfx_ctx *ctx, float *d_scores, const uint64_t *d_off,
         al(4 * nf), al(8 * nf + 8), al(nt + 4ull)};
     uint64_t bytes = 0;
     for (uint64_t z : sizes) bytes += z;
-    uint8_t *p = (uint8_t *)hfx_ctx_scratch_spare(ctx, HFX_SLOT_ROWS, bytes, stream);
+    uint8_t *p = (uint8_t *)hfx_ctx_scratch_spare(ctx, HFX_SLOT_ROWS, bytes);
     if (!p) return HFX_OK;
-    uint8_t *rows = (uint8_t *)hfx_ctx_scratch_spare(ctx, HFX_SLOT_ROWS2, slots * G * 1024ull, stream);
+    uint8_t *rows = (uint8_t *)hfx_ctx_scratch_spare(ctx, HFX_SLOT_ROWS2, slots * G * 1024ull);
     if (!rows) return HFX_OK;
     uint8_t *part[sizeof sizes / sizeof *sizes];
     for (size_t i = 0; i < sizeof sizes / sizeof *sizes; ++i) {
@@ -509,11 +517,12 @@ extern "C" int hfx_xcorr_sparse(hfx_ctx *ctx, float *d_scores, const uint64_t *d
     HfxPlainCands c{*db, d_begin, d_num, d_off};
     void *p = nullptr;
     int rc, taken = 0;
-    if ((rc = xcorr_rows(ctx, d_scores, d_off, d_begin, d_num, total, db, sp, stream, &taken)) ||
-        taken)
-        return rc;
+    /* whichever kernel scores: a captured call after this one finds the table there */
     if (sp->num_spec &&
         (rc = hfx_ctx_scratch(ctx, HFX_SLOT_TILES, xc_scratch_bytes(sp->num_spec), &p)) != HFX_OK)
+        return rc;
+    if ((rc = xcorr_rows(ctx, d_scores, d_off, d_begin, d_num, total, db, sp, stream, &taken)) ||
+        taken)
         return rc;
     return launch_xcorr(p, d_scores, c, total, sp, stream);
 }

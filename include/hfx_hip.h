@@ -293,8 +293,11 @@ int hfx_scan_offsets(hfx_ctx *ctx, uint64_t *d_off, const uint32_t *d_count, uin
  * four charge levels, 1.6 GB each for 2.7 M peptides, or for as many as the pairs
  * can need; 13 KB a spectrum) are kept by the context and given back where an
  * allocation of this library finds memory short.  Where it is short already, or the
- * stream is being captured before they exist, the call sums in FP32 without them, so
- * that two calls may differ in the last bit. */
+ * stream is being captured (a graph must not hold what a larger call replaces), the
+ * call sums in FP32 without them, so that two calls may differ in the last bit.  A
+ * captured call needs the context's tile table (12 bytes a spectrum, from any call
+ * before it of as many spectra) and holds it: a later call of more spectra replaces
+ * the table, and the graph must not be replayed after it. */
 int hfx_xcorr_sparse(hfx_ctx *ctx, float *d_scores, const uint64_t *d_off,
                      const uint32_t *d_begin, const uint32_t *d_num, uint64_t total,
                      const hfx_db *db, const hfx_spectra *sp, void *stream);
