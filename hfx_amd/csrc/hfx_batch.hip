@@ -1522,7 +1522,8 @@ static int bt_dense_prep(hfx_batch *b, hipStream_t st)
         return rc;
     if (bt_rows(b)) {
         return hfx_rows_split(bt_mode(b), &b->sp, bt_planes(b), bt_quanta(b), bt_levels(b), &rest,
-                              b->have, bt_norms(b), b->scores, b->score_off, b->num, (void *)st);
+                              b->have, bt_norms(b), b->scores, b->score_off, b->begin, b->num,
+                              b->db.num_pep, (void *)st);
     }
     return i8 ? hfx_dense8_split(&b->sp, b->dn_scratch, (void *)st)
               : hfx_dense_split(&b->sp, b->dn_scratch, (void *)st);

@@ -38,12 +38,14 @@ struct hfx_rest {
 };
 /* planes [S][RW_PLANES][RW_MAXK] and quanta of the spectra, and the charge level of
  * each, 0 for those put on the list `rest`: charges above `have`, the highest level
- * there are rows for; in RW_I8X6 spectra with a value that six digits do not hold.  norms
+ * there are rows for; windows past num_pep, the peptides there are rows of; in RW_I8X6
+ * spectra with a value that six digits do not hold.  norms
  * [S], if any: sum and max of |x|.  The num[s] scores of spectra whose charge is not
  * generated are set to 0, and nothing between one spectrum's scores and the next's */
 int hfx_rows_split(int mode, const hfx_spectra *sp, uint8_t *planes, float *qs, uint32_t *lvl,
                    const hfx_rest *rest, uint32_t have, float2 *norms, float *scores,
-                   const uint64_t *off, const uint32_t *num, void *stream);
+                   const uint64_t *off, const uint32_t *begin, const uint32_t *num, uint32_t num_pep,
+                   void *stream);
 /* writes the rows of the wanted levels (non-null) and tiles (flags
  * [HFX_MAX_CHARGE][ntiles], null: all) */
 int hfx_rows_build(uint32_t cus, const hfx_db *db, const hfx_rows *r, const uint32_t *flags,

@@ -80,14 +80,15 @@ __device__ __forceinline__ uint32_t rw_bf16(float f)
  * digit first) is the digit of bin 64 ks + rw_bin_of(kg, j); the BF16 planes (hi of bytes j < 8,
  * hi of j >= 8, lo, lo) hold eight BF16 in the 16 bytes of a k-group.
  * qs[s] = 2^-k.  norms (if any): sum and max of |x|.  A spectrum whose charge has no
- * rows (above `have`; a later one than those a batch was planned with) or, in the
- * FP32 form, one that the digits do not serve goes to the list `rest`, and its
- * lvl[s] is 0; the others' lvl[s] is their fragment charge. */
+ * rows (above `have`; a later one than those a batch was planned with), whose window
+ * passes the last peptide that has any (num_pep), or, in the FP32 form, which the
+ * digits do not serve, goes to the list `rest`, and its lvl[s] is 0; the others' lvl[s]
+ * is their fragment charge. */
 template <int MODE>
 __global__ void __launch_bounds__(256)
     k_rw_split(uint8_t *planes, float *qs, uint32_t *lvl, hfx_rest rest, uint32_t have,
-               float2 *norms, float *scores, const uint64_t *off, const uint32_t *num,
-               hfx_spectra sp)
+               float2 *norms, float *scores, const uint64_t *off, const uint32_t *begin,
+               const uint32_t *num, uint32_t num_pep, hfx_spectra sp)
 {
     constexpr uint32_t NP = RW_PLANES(MODE);
     __shared__ float red[2][256 / HFX_WAVE];
@@ -132,7 +133,7 @@ __global__ void __launch_bounds__(256)
     m = fmaxf(fmaxf(red[0][0], red[0][1]), fmaxf(red[0][2], red[0][3]));
     x1 = red[1][0] + red[1][1] + red[1][2] + red[1][3];
     if (tid == 0 && norms) norms[s] = make_float2(x1, m);
-    bool out = z > have;
+    bool out = z > have || (num[s] && (uint64_t)begin[s] + num[s] > num_pep);
     /* RW_I8X6, k: m 2^k in [2^45, 2^46), at most 126 */
     [[maybe_unused]] double sc6 = 1.0;
     if constexpr (MODE == RW_I8X6) {
@@ -915,7 +916,8 @@ uint32_t hfx_rows_item_tiles(uint32_t CH)
 
 int hfx_rows_split(int mode, const hfx_spectra *sp, uint8_t *planes, float *qs, uint32_t *lvl,
                    const hfx_rest *rest, uint32_t have, float2 *norms, float *scores,
-                   const uint64_t *off, const uint32_t *num, void *stream)
+                   const uint64_t *off, const uint32_t *begin, const uint32_t *num, uint32_t num_pep,
+                   void *stream)
 {
     HFX_REQUIRE(sp->x_stride <= RW_MAXK, HFX_ERR_ARG, "rows: spectra of up to %d bins", RW_MAXK);
     if (sp->num_spec == 0) return HFX_OK;
@@ -924,7 +926,8 @@ int hfx_rows_split(int mode, const hfx_spectra *sp, uint8_t *planes, float *qs, 
     const auto kernel = mode == RW_I8X3   ? k_rw_split<RW_I8X3>
                         : mode == RW_I8X6 ? k_rw_split<RW_I8X6>
                                           : k_rw_split<RW_BF16>;
-    hipLaunchKernelGGL(kernel, g, t, 0, st, planes, qs, lvl, *rest, have, norms, scores, off, num, *sp);
+    hipLaunchKernelGGL(kernel, g, t, 0, st, planes, qs, lvl, *rest, have, norms, scores, off, begin, num,
+                       num_pep, *sp);
     HFX_CHECK_LAUNCH();
     return HFX_OK;
 }

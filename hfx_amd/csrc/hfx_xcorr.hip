@@ -495,7 +495,7 @@ static int xcorr_rows(hfx_ctx *ctx, float *d_scores, const uint64_t *d_off,
     if ((rc = hfx_order_spectra(ctx, order, &ob, d_begin, sp->d_zmax, nullptr, S, stream)) ||
         (rc = hfx_cut_blocks(ctx, RW_NS(RW_I8X6), &cb, order, d_begin, d_num, sp->d_zmax, S, stream)) ||
         (rc = hfx_rows_split(RW_I8X6, sp, planes, qs, lvl, &rest, HFX_MAX_CHARGE, nullptr, d_scores,
-                             d_off, d_num, stream)) ||
+                             d_off, d_begin, d_num, db->num_pep, stream)) ||
         (rc = hfx_rows_blocks(ctx, items, order, cb.bstart, d_begin, d_num, &sq, CH, stream)) ||
         (rc = hfx_rows_mark(items, S, flags, nt, stream)) ||
         (rc = hfx_scan_offsets(ctx, (uint64_t *)r.slots, flags, (uint32_t)nf, stream)) ||

@@ -22,7 +22,7 @@ def search(orc):
     return hdb, x, lens, zmax, mass, ref, exact, scale
 
 
-@pytest.mark.parametrize("what", ["no masses", "any begin", "gaps"])
+@pytest.mark.parametrize("what", ["no masses", "any begin", "gaps", "fewer peptides"])
 def test_sparse_through_rows_reads_only_what_it_is_given(search, what):
     from hfx_amd import HfxSpectra, check as ok, lib
     from hfx_amd import pipeline as pl
@@ -39,9 +39,12 @@ def test_sparse_through_rows_reads_only_what_it_is_given(search, what):
         begin = np.where(num == 0, np.uint32(0xfffffff0), begin)
     if what == "gaps":
         off = off + 5 * np.arange(S + 1, dtype=np.uint64)
+    dd = type(db.desc)(*[getattr(db.desc, f) for f, _ in db.desc._fields_])
+    if what == "fewer peptides":   # the windows say where the candidates are
+        dd.num_pep = 70_000
     t = [pl.dev(v) for v in (off, begin, num)]
     out = pl.dev(np.full(int(off[-1]), 12345.0, np.float32))
-    ok(lib().hfx_xcorr_sparse(ctx.h, out.p, *[b.p for b in t], total, C.byref(db.desc), C.byref(d),
+    ok(lib().hfx_xcorr_sparse(ctx.h, out.p, *[b.p for b in t], total, C.byref(dd), C.byref(d),
                               None), "hfx_xcorr_sparse")
     pl.sync()
     got = pl.host(out, np.float32, int(off[-1]))
