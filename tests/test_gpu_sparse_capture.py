@@ -19,8 +19,6 @@ def free_rows(pl):
 
 
 def test_a_graph_and_larger_calls_afterwards(orc):
-    import torch
-
     from hfx_amd import check, lib
     from hfx_amd import pipeline as pl
 
@@ -43,9 +41,11 @@ def test_a_graph_and_larger_calls_afterwards(orc):
     score(big, 6000, None)   # the tile table, 12 bytes a spectrum, is there for the largest call
     score(out, half, None)
     pl.sync()
-    s, g = torch.cuda.Stream(), torch.cuda.CUDAGraph()
-    with torch.cuda.graph(g, stream=s, capture_error_mode="thread_local"):
-        score(out, half, s.cuda_stream)
+    hip, s, g, run = C.CDLL("libamdhip64.so"), pl.Stream(), C.c_void_p(), C.c_void_p()
+    assert hip.hipStreamBeginCapture(C.c_void_p(s.p), 1) == 0   # hipStreamCaptureModeThreadLocal
+    score(out, half, s.p)
+    assert hip.hipStreamEndCapture(C.c_void_p(s.p), C.byref(g)) == 0
+    assert hip.hipGraphInstantiate(C.byref(run), g, None, None, C.c_size_t(0)) == 0
     bound = FORMS["fp32"][0] * scale + 1e-6 + 2.0**-24 * np.abs(exact)
     for _ in range(3):
         score(big, 6000, None)
@@ -53,9 +53,10 @@ def test_a_graph_and_larger_calls_afterwards(orc):
         pl.sync()
         out.zero()
         pl.sync()
-        g.replay()
-        torch.cuda.synchronize()
+        assert hip.hipGraphLaunch(run, C.c_void_p(s.p)) == 0
+        pl.sync()
         got = pl.host(out, np.float32, n)
         assert (np.abs(got - exact[:n]) <= bound[:n]).all()
         got = pl.host(big, np.float32, len(exact))
         assert (np.abs(got - exact) <= bound).all()
+    assert hip.hipGraphExecDestroy(run) == 0 and hip.hipGraphDestroy(g) == 0
