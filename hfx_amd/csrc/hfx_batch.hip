@@ -7,21 +7,23 @@
  * candidate's peaks depend only on the peptide and the fragment charges, and
  * neighbouring precursors share most of their window, so a batch of thousands
  * of spectra here
- *   1. builds, once per batch, the sparse theoretical spectrum of every
- *      peptide any window touches, for fragment charge levels 1..L (level l =
- *      charges 1..l, max per bin): sorted uint16 entries bin | code << 14
- *      (k_ix_build, one wave per peptide, from the same ladder/bin code as the
- *      plain path), and the rows of 2-bit codes of the same peaks
- *      (hfx_rows.hip), which every form scores with where memory holds them;
- *   2. sorts the spectra by precursor mass and groups G consecutive spectra
- *      into blocks; a tile is (block, C consecutive candidates of the block's
- *      union window); a persistent kernel pulls tiles from an atomic counter
- *      (work stealing: heavy-tailed windows are cut into equal tiles), keeps
- *      the block's G spectra in LDS, streams each candidate's entries once
- *      (coalesced) and gathers every spectrum of the block that holds the
- *      candidate in its window, reducing the G partial sums with one
- *      reduce-scatter butterfly (with rows: blocks of up to sixteen ordered
- *      spectra contracted with the rows of their windows' hull);
+ *   1. writes, once per database, the theoretical spectrum of every peptide
+ *      for fragment charge levels 1..L (level l = charges 1..l, max per bin) as
+ *      rows of 2-bit codes (hfx_rows.hip), which every form scores with where
+ *      memory holds them; without them the FP32 form reads the same peaks as
+ *      sorted uint16 entries bin | code << 14 (k_ix_build, one wave per peptide,
+ *      from the same ladder/bin code as the plain path) and the dense forms the
+ *      b ladders;
+ *   2. sorts the spectra by fragment charge and precursor mass, cuts the order
+ *      into blocks of up to sixteen spectra (integer form; eight in the others)
+ *      and contracts each block with the rows of its windows' hull.  Without
+ *      rows, FP32 form: G consecutive spectra are a block; a tile is (block, C
+ *      consecutive candidates of the block's union window); a persistent kernel
+ *      pulls tiles from an atomic counter (work stealing: heavy-tailed windows
+ *      are cut into equal tiles), keeps the block's G spectra in LDS, streams
+ *      each candidate's entries once (coalesced) and gathers every spectrum of
+ *      the block that holds the candidate in its window, reducing the G partial
+ *      sums with one reduce-scatter butterfly;
  *   3. selects the top N with the exact re-score of hfx_topn (flagged spectra
  *      completed in the same launch sequence, no host round trip).
  * Scores land in the same layout as hfx_xcorr_sparse, so every result is

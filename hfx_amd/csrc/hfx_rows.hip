@@ -33,11 +33,11 @@
  *            spectra;
  *   RW_BF16  hi and lo BF16 of eight spectra, FP32 accumulation.
  *
- * Scoring kernels, 20,000 proteins (2.7 M peptides), before (rows written per
- * block into LDS, or per pair) and after: three digits, 20,000 spectra 1,978 ->
- * 864 us; BF16, 6,000 spectra 1,937 -> 773 us; FP32 batched, 4,000 spectra
- * 10,114 -> 570 us.  Writing two levels' rows of the database takes 0.87 ms,
- * once.
+ * Scoring kernels, 20,000 proteins (2.7 M peptides), with rows written per
+ * block into LDS (dense forms) or gathered per pair (FP32), and so: three digits,
+ * 20,000 spectra 1,978 and 864 us; BF16, 6,000 spectra 1,937 and 773; FP32 batched,
+ * 4,000 spectra 10,114 and 570.  Writing two levels' rows of the database takes
+ * 0.89 ms, once.
  */
 #include "hfx_cand.h"
 #include "hfx_rows.h"
@@ -235,11 +235,11 @@ __global__ void __launch_bounds__(256)
  * words.  Neither is emitted.  Words are cleared as they are emitted for the last
  * time.  Rows go out past the caches: they are read again only after gigabytes
  * of others.
- * Two levels of 2.7 M peptides (2.2 GB written, 0.7 GB of scattered reads): 1,340
+ * Two levels of 2.7 M peptides (2.4 GB written, 0.7 GB of scattered reads): 1,340
  * us with a workgroup of two waves a tile, no reads ahead and a lane a peptide
- * for residues, masses and sums; 880 us now (960 through the caches; 6
- * workgroups a CU 50 us more, 5 150 more).  Memory at 3.3 TB/s and vector
- * instructions (61 % of issue) share the rest. */
+ * for residues, masses and sums; 890 us so (960 through the caches; 6
+ * workgroups a CU 50 us more, 5 150 more).  Memory at 3.5 TB/s and vector
+ * instructions (69 % of issue; two thirds of the waves' cycles are waits) share it. */
 #define RB_THREADS 256
 #define RB_WAVES (RB_THREADS / HFX_WAVE)
 #define RB_PER_CU 7
@@ -612,15 +612,15 @@ __device__ __forceinline__ double rm_next(double h)
  * codes loaded while the current one is contracted.  A k-step of four tiles
  * costs 4 x 11 code lookups, 4 x planes matrix instructions and one fragment
  * read a plane.
- * The two kinds add up: vector and matrix instructions together fill 96 % of
- * the cycles, with rows from cache as well, and interleaving them by hand
- * changes nothing.  So what is not a lookup was taken out of the loop (copies of
- * the codes, per-lane addresses, FP64 folds) and a third wave a SIMD fills its
- * waits: three digits, 20,000 spectra 963 -> 881 (the wave) -> 864 us; BF16 850 ->
- * 812 -> 773.  Six digits take three matrix instructions a k-step of four tiles as
- * well, for half as many spectra: a plain search of 10,000 866 us, a batch of 4,000
- * 570 (four digits and sixteen spectra, which rounded the FP32 values below
- * max|x| / 128, 757 and 547).  Sixteen
+ * The two kinds add up: vector and matrix instructions take 49 and 39 % of the
+ * cycles with three digits, 52 and 39 with six, 70 and 22 in BF16 (20,000 spectra),
+ * and interleaving them by hand changes nothing.  So the loop holds lookups
+ * alone (no copies of the codes, per-lane addresses or FP64 folds), and a third
+ * wave a SIMD fills its waits: three digits, 20,000 spectra, 963 us with two waves
+ * and those, 864 so; BF16, 6,000 spectra, 850 and 773.  Six digits take three
+ * matrix instructions a k-step and tile as well, for half as many spectra: a plain
+ * search of 10,000 866 us, a batch of 4,000 570 (four digits and sixteen spectra,
+ * 757 and 547, round the FP32 values below max|x| / 128).  Sixteen
  * waves spill (983 us, three digits); three groups of codes on their way, also
  * across tiles, cost more scalar work than they hide (1,134). */
 template <int MODE>

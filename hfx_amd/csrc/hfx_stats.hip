@@ -533,10 +533,11 @@ ev_wide(const __attribute__((address_space(4))) void *args, EvShared &sh, uint32
 
 /* A workgroup a spectrum, eight of them a CU (64 registers, 4.5 KiB of LDS):
  * each step waits on the one before it (loads, least, counts, scan, logarithms,
- * sums), so the CU is kept busy by the other workgroups.  With the scores in
- * LDS four workgroups fitted, and keys in FP64 alone took a dozen FP64 operations
- * a score.  10,000 spectra of 4600 scores on average: 162 -> 70 us (185 MB,
- * 2.6 TB/s; 128 threads and 5120 scores held: 75, one wave and 4096: 110). */
+ * sums; half of a wave's cycles), so the CU is kept busy by the other workgroups,
+ * up to 0.97 vector instructions a SIMD every four cycles: they bound it.  With the
+ * scores in LDS four workgroups fit, and keys in FP64 alone take a dozen FP64
+ * operations a score.  10,000 spectra of 4600 scores on average: 162 us that way, 70
+ * so (185 MB, 2.6 TB/s; 128 threads and 5120 scores held: 75, one wave and 4096: 110). */
 __global__ __launch_bounds__(EV_THREADS, 8) void k_evfit(EvArgs a)
 {
     __shared__ __align__(16) EvShared sh;
@@ -1009,10 +1010,11 @@ struct SpModTop {
 };
 
 /* a wave a spectrum: its N matches, the flags of its row found here (E > 0) or
- * read from a.on (E = 0).  10,000 spectra of 2176 bins, top 5: 54 us, where the
- * flags took 53 us (31 steps of 36 ballots) and the matches 70 (a thread each).
- * The chains of reads and of select steps bound it, 24 waves a CU; 64 registers
- * for 32 waves spill (61 us). */
+ * read from a.on (E = 0).  10,000 spectra of 2176 bins, top 5: 54 us; in launches of
+ * their own the flags take 53 (31 steps of 36 ballots) and the matches 70 (a thread
+ * each).  The chains of reads and of select steps bound it: two thirds of the waves'
+ * cycles are waits and 36 % of the vector issue is used, 24 waves a CU at most; 64
+ * registers for 32 waves spill (61 us). */
 template <int E, class Top>
 __global__ __launch_bounds__(ST_THREADS) void k_sp_topn(SpArgs a, Top top, const float *x)
 {

@@ -27,15 +27,15 @@
  * rel0 = 80 * 2^-24 (<= 71 roundings per score), rel1 = 0; the dense BF16
  * scores pass their own (split error + one rounding per non-zero bin).
  *
- * One workgroup per spectrum did all three, a wave per candidate: half of its
- * time went to exact scores with a quarter of the lanes busy, and a spectrum
- * with 200 tied candidates held up a small batch by itself.
- * Now, select + exact + rank: 10,000 spectra, 1120 candidates each, top 10:
- * 127 + 124 + 15 us, against 445 us; 20,000 spectra, top 5: 157 + 136 + 15 us,
- * against 430 (179 where the selection reads the spectra for their norms); 250
- * spectra: 13 + 22 + 7 us, against 171.  The selection is a chain of short steps,
- * half of its waves waiting; the exact scores are bound by their FP64 terms and
- * the maps' LDS atomics.
+ * One workgroup per spectrum for all three, a wave per candidate, spends half of
+ * its time on exact scores with a quarter of the lanes busy, and a spectrum
+ * with 200 tied candidates holds up a small batch by itself.
+ * Select + exact + rank: 10,000 spectra, 1120 candidates each, top 10: 128 + 125 +
+ * 15 us, 445 in one kernel; 20,000 spectra, top 5: 159 + 135 + 15 us and 430 (179
+ * where the selection reads the spectra for their norms); 250 spectra: 13 + 21 + 7
+ * us and 171.  The selection is a chain of short steps (63 % of the waves' cycles
+ * are waits, 55 % of the vector issue is used); the exact scores are bound by their
+ * FP64 terms and the maps' LDS atomics.
  */
 #define HFX_TOPN_REL_F32 (80.0f * 5.9604644775390625e-08f)
 #include "hfx_pack.h"

@@ -54,7 +54,9 @@ __device__ __forceinline__ uint32_t find_segment(const uint64_t *off, uint32_t n
  *     scans the whole map, and the map is clean for the next pack;
  *   - the lanes' partial sums are reduced per candidate.
  * A candidate of more than 64 positions takes a wave of its own through the
- * general path (hfx_wave_peaks, hfx_wave_dot_f32). */
+ * general path (hfx_wave_peaks, hfx_wave_dot).
+ * 10.2 million modified candidates take 2,800 us, by vector instructions (1.02 a
+ * SIMD every four cycles) and LDS atomics (bank conflicts in a third of the cycles). */
 #define XP_THREADS 256
 #define XP_WAVES (XP_THREADS / HFX_WAVE)
 #define XP_CHUNK 128
@@ -407,15 +409,16 @@ int hfx_xcorr_rest(hfx_ctx *ctx, float *d_scores, const uint64_t *d_off, const u
 
 /* hfx_xcorr_sparse writes each candidate's theoretical row once and contracts the
  * rows with blocks of eight spectra (hfx_rows.hip, fixed point that holds them) instead
- * of building a row per pair, where that is quicker.  In ns: a pair costs 230 ps
- * to score by itself, 30 through its row; the rows' dozen launches 80,000 more
+ * of building a row per pair, where that is quicker.  In ns: a pair costs 0.2
+ * more to score by itself than through its row; the rows' dozen launches 80,000 more
  * than the packed kernel's three; a tile of the database 1/3 to look at and, if a
  * window holds it, 2.7 at each charge level to write and read (as many as the
- * pairs fill, at most two levels of all).  Measured, packed and rows, us: 2000
- * proteins, short peptides (7,293 tiles) 520,778 pairs 138 and 161, 1,043,828
- * pairs 243 and 174; longer ones (16,900 tiles) 365,831 pairs 156 and 181, 733,473
- * pairs 233 and 216; 20,000 proteins (73,000 and 170,000 tiles) 1,240,720 pairs
- * 268 and 333, 1,839,460 pairs 453 and 549; 46 million pairs 9,409 and 1,800. */
+ * pairs fill, at most two levels of all).  Measured, packed and rows, us: 2,000
+ * proteins, short peptides (7,293 tiles) 520,778 pairs 135 and 152, 1,043,828
+ * pairs 236 and 170; longer ones (17,089 tiles) 365,831 pairs 155 and 168, 733,473
+ * pairs 229 and 205; 20,000 proteins (72,760 and 170,538 tiles) 1,240,720 pairs
+ * 262 and 328, 2,546,519 475 and 462; 1,839,460 446 and 534, 3,771,758 812 and 772,
+ * 5,577,139 1,170 and 959, 45,788,296 9,120 and 1,790. */
 static bool xr_pays(uint64_t total, uint32_t tiles)
 {
     const uint64_t read = min(total / RW_ROWS, 2ull * tiles);

@@ -587,9 +587,11 @@ int hfx_format_scan(const hfx_scan_header *hdr, const hfx_match_row *rows, uint3
  *   levels 1..levels (level l = charges 1..l, max weight per bin), bins below
  *   max_len, as sorted uint16 entries bin | code << 14 (the FP32 batched
  *   form's input).
- * A batch that runs on the index adds the theoretical rows it scores with (a
- * KiB for each 256 bins of sixteen peptides, per charge level: 1.1 GB a level for
- * 2.7 M peptides), where the device's memory holds them.
+ * A batch on the index takes the theoretical rows it scores with, writing those
+ * that are not there yet, where the device's memory holds them: nine KiB for each
+ * sixteen peptides and charge level, 1.6 GB a level for 2.7 M peptides, one copy
+ * for all indexes over databases of the same contents.  Rows that no batch uses are
+ * given back where an allocation of this library finds memory short.
  * The reference has no counterpart: it rebuilds every theoretical spectrum
  * per (spectrum, candidate) pair (Search.hs:177-245).  Synchronises. */
 typedef struct hfx_pepix hfx_pepix;
